@@ -153,7 +153,7 @@ int derive(const hrn_kernel_desc* d, Derived* o) {
         return fail(HRN_E_BADPARAM, "colsum %d (caller-supplied column sums are an option of the u8s8 instances)", d->colsum);
     if (d->nt_store < 0 || d->nt_store > 1) return fail(HRN_E_BADPARAM, "nt_store %d (0 or 1)", d->nt_store);
     if (d->sched == 2 && (d->wm * d->wn != 8 || d->conv_window || d->persistent || d->split_k))
-        return fail(HRN_E_BADPARAM, "sched 2 (two wave groups) needs 8 waves and neither conv_window, persistent nor split_k");
+        return fail(HRN_E_BADPARAM, "sched 2 needs 8 waves and neither conv_window, persistent nor split_k");
     Derived r;
     r.es = d->dtype == HRN_DT_F16 ? 2 : 1;
     r.oes = (d->dtype == HRN_DT_F16 && !d->split_k) ? 2 : 4;

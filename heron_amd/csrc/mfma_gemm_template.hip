@@ -97,9 +97,9 @@ constexpr bool COLSUM = (HRN_DTYPE == 1) && (HRN_COLSUM != 0);
 #define HRN_NTSTORE 0
 #endif
 constexpr bool NTS = (HRN_NTSTORE != 0) && (HRN_SPLITK == 0);
-// Issue order of a k-step: 1 = the source order of the row groups is pinned (a scheduling fence after every row of
-// MFMAs), 0 = the compiler interleaves on its own, guided by group hints (one LDS read per few MFMAs), 2 = the two
-// wave groups of an 8-wave workgroup alternate between a memory phase and a matrix phase (see "SCHED 2" below).
+// Issue order of a k-step: 1 and 2 = the source order of the row groups is pinned (a scheduling fence after every row
+// of MFMAs), 0 = the compiler interleaves on its own, guided by group hints (one LDS read per few MFMAs).  Tiles that
+// PHASED (below) takes run the phased schedule whatever this says.
 #ifndef HRN_SCHED
 #define HRN_SCHED 1
 #endif
@@ -159,6 +159,14 @@ static_assert((NS - 1) * LPT <= 63, "vmcnt range");
 static_assert(NT <= 1024, "threads");
 static_assert(DT == 0 || NS * STAGE_BYTES >= WM * BN * 4, "column sums must fit the stages");
 
+// Phased schedule ("---- phased schedule" below) instead of the row-by-row one: 256x256 tiles of 128-byte rows in two
+// stages on 8 waves in a 2x4 or 4x2 grid.  These are the tiles of the large products, where the matrix pipes decide;
+// same card, 8192^3, row-by-row / phased: fp16 778 / 742 us (2x4, 16x16 MFMAs; 32x32: 884 / 842), u8 x s8 434 / 403 us
+// (4x2), fp16 4096^3 101.5 / 97.5.  The grids 8x1 and 1x8 would need 152 fragment registers beside the 128 accumulators, and
+// the uint8 path has no room for in-loop column sums, so both stay with the row-by-row schedule.
+constexpr bool PHASED = OP == 0 && BM == 256 && BN == 256 && BKB == 128 && NS == 2 && NW == 8 && (WM == 2 || WM == 4) &&
+                        !PERS && !SPLITK && (DT == 0 || COLSUM);
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
@@ -216,24 +224,6 @@ __device__ __forceinline__ v16i mfma(v4i x, v4i y, v16i c) {
 __device__ __forceinline__ v4i mfma(v4i x, v4i y, v4i c) {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(x, y, c, 0, 0, 0);
 }
-
-// In-place form for the two-group schedule: the accumulator is both source and destination, so its registers stay
-// where they are for the whole k-loop (with the intrinsic the register allocator is free to move them from step to
-// step, and with the single fragment buffer of that schedule it does, at the price of spills).  The compiler does not
-// know this instruction's latency: code that reads the accumulators afterwards starts with mfma_drain().
-__device__ __forceinline__ void mfma_inplace(v4i x, v4i y, v16f& c) {
-    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(x), "v"(y));
-}
-__device__ __forceinline__ void mfma_inplace(v4i x, v4i y, v4f& c) {
-    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(x), "v"(y));
-}
-__device__ __forceinline__ void mfma_inplace(v4i x, v4i y, v16i& c) {
-    asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, %0" : "+v"(c) : "v"(x), "v"(y));
-}
-__device__ __forceinline__ void mfma_inplace(v4i x, v4i y, v4i& c) {
-    asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(c) : "v"(x), "v"(y));
-}
-__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
 // Scheduling hints of one k-step (HRN_SCHED = 0): NR groups of {1 LDS read, NV/NR buffer loads, NMM/NR MFMAs}.
 template <int R, int NR, int NMM, int NV>
@@ -758,10 +748,12 @@ hrn_mfma_kernel(const HrnKArgs a) {
     };
 
     // ---- prologue: fill all stages, wait for tile 0 ----
+    if constexpr (!PHASED) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) issue_tile(s);
-    wait_and_barrier<(NS - 1) * LPT, 0>();
-    if constexpr (SCHED != 2) read_frags(0, 0, 0);
+        for (int s = 0; s < NS; ++s) issue_tile(s);
+        wait_and_barrier<(NS - 1) * LPT, 0>();
+        read_frags(0, 0, 0);
+    }
 
     int stage = 0;
     // One k-step: the MFMAs of register buffer `cur`, row-tile by row-tile, with the fragment reads of the next step
@@ -884,107 +876,159 @@ hrn_mfma_kernel(const HrnKArgs a) {
         }
         store_tile();
     };
-    // ---- SCHED 2: two wave groups half a k-step apart ("ping-pong") ----
-    // Waves w and w + 4 run on the same SIMD.  Group 0 (waves 0-3) and group 1 (waves 4-7) alternate between two kinds
-    // of phase, one barrier apart: a memory phase (read the fragments of one k-step from LDS into the single register
-    // buffer, flip the uint8 sign bits, add up the column sums) and a matrix phase (nothing but that step's MFMAs).
-    // While one wave of a SIMD multiplies, the other waits for LDS and for a slot in the vector-memory queue, so those
-    // waits never hold back an MFMA.  Phase 2s: group 0 multiplies step s, group 1 reads step s; phase 2s+1: group 0
-    // reads step s+1, group 1 multiplies step s.  The stage of k-tile t is free once group 1 has read its last step;
-    // in the phase after that every wave issues its share of the loads of k-tile t + NS, and every wave waits for its
-    // own loads of k-tile t + 1 at the end of the phase in which group 1 reads the last step of k-tile t.
-    // fragment reads of the step whose k-offset inside the stage row is `koff` bytes (a runtime value here: the
-    // k-loop of this schedule is not unrolled over the k-steps of a tile, so that every fragment register has one
-    // definition per iteration and stays where it is)
-    auto pp_mem = [&](const int stage_off, const int koff) __attribute__((always_inline)) {
-        const int gk = g16 ^ koff;
-        const char* pb = lds + stage_off + b_lane + gk;
-        const char* pa = lds + stage_off + a_lane + gk;
+    // ---- phased schedule (PHASED) ----
+    // Waves w and w + 4 share a SIMD.  Every wave alternates between a memory phase (fragment reads, tile fetches, waits)
+    // and a matrix phase (16 or 8 MFMAs, nothing else but the sign flips in their shadow), a barrier after each, and waves
+    // 4-7 enter the stream one barrier later: while one wave of a SIMD multiplies, the other moves data.
+    //   A wave tile is cut into 2x2 quadrants; one of them, over the whole k-tile, is a step.  X is the operand with more
+    // fragments, the steps of k-tile T are (X0,Y0) (X0,Y1) (X1,Y0) (X1,Y1).  Reads run one step ahead of their MFMAs and
+    // are spread evenly over the steps:
+    //   step 0: Y1 and a part of X1     step 1: the rest of X1     (of T)
+    //   step 2: a part of X0            step 3: Y0 and the rest of X0     (of T + 1)
+    // A half that has been read by everybody (it was read in step i, waited for in step i + 1) is refilled in step i + 2 or
+    // later: step 1 fetches X0 and Y0, step 2 Y1, step 3 X1 of T + 2.  So every fetch has four to five steps (about 1.2 us)
+    // to arrive, and a wait allows for the fetches that were issued after the half it is about.
+    //   8192^3: matrix pipes busy in 83 % (fp16) and 73 % (u8 x s8) of the cycles, 75 and 62 % with the row-by-row schedule;
+    // what bounds it then is power (the clock falls to 1.6 - 1.7 GHz): without the fetches in the loop the cycles fall
+    // by 4 %, the time by 12 %.
+    constexpr int HM = TM / 2, HN = TN / 2;                          // MFMA tiles of a half
+    constexpr bool XA = TM >= TN;                                    // X is A
+    constexpr int RA = HM * KS, RB = HN * KS;                        // fragments of a half
+    constexpr int RX = XA ? RA : RB, RY = XA ? RB : RA, XP = (RX - RY) / 2;   // XP: the part of X read beside a half of Y
+    v4i pa[2][PHASED ? HM : 1][KS], pb[2][PHASED ? HN : 1][KS];
+    auto phased_run = [&]() __attribute__((always_inline)) {
+        constexpr int LH = A_LPW / 2;                                // wave loads of a half (equal for A and B)
+        // row of the tile at which load q of half h starts: half h is rows [h*wt/2, (h+1)*wt/2) of every wave row's wt rows
+        auto row_of = [&](int wt, int h, int q) {
+            const int u = q * NW + wave, per = wt / 2 / RPI;
+            return (u / per) * wt + h * (wt / 2) + (u % per) * RPI;
+        };
+        // one descriptor per load, for the whole k-loop: its row block's base, and the bytes left from there
+        rsrc_t dA[2][LH], dB[2][LH];
+        int lA[2][LH], lB[2][LH];                                    // where the block goes in a stage
+        live_cur = true;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) fb[0][j] = *(const v4i*)(pb + j * MT * BKB);
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) fa[0][i] = *(const v4i*)(pa + i * MT * BKB);
-    };
-    auto pp_ready = [&](const int step) __attribute__((always_inline)) {      // after the reads have landed
-        if constexpr (DT == 1) {
-            // (as volatile statements, so that the sign flips stay in this phase: plain code may be moved past
-            // the barrier into the matrix phase)
-            const int flip = (int)0x80808080;
+            for (int q = 0; q < LH; ++q) {
+                dA[h][q] = block_rsrc(baseA, a_bytes, (uint32_t)(m0 + row_of(WTM, h, q)) * (uint32_t)a.lda * ES, 0, 0);
+                dB[h][q] = block_rsrc(baseB, b_bytes, (uint32_t)(n0 + row_of(WTN, h, q)) * (uint32_t)a.ldb * ES, 0, 0);
+                lA[h][q] = __builtin_amdgcn_readfirstlane(row_of(WTM, h, q) * BKB);
+                lB[h][q] = __builtin_amdgcn_readfirstlane(A_BYTES + row_of(WTN, h, q) * BKB);
+            }
+        const uint32_t chunkA = (uint32_t)((lpos ^ swz_of_row(row_of(WTM, 0, 0) + lrow)) * 16);
+        const uint32_t chunkB = (uint32_t)((lpos ^ swz_of_row(row_of(WTN, 0, 0) + lrow)) * 16);
+        const uint32_t offA = (uint32_t)lrow * (uint32_t)a.lda * ES + chunkA;
+        const uint32_t offB = (uint32_t)lrow * (uint32_t)a.ldb * ES + chunkB;
+        auto fetch = [&](auto isa, auto ragc, int h, int stg, int kt) __attribute__((always_inline)) {
+            constexpr bool IA = decltype(isa)::value;
+            const uint32_t ko = (uint32_t)kt * BKB;
+            uint32_t v = IA ? offA : offB;
+            if constexpr (decltype(ragc)::value) { if (ko + (IA ? chunkA : chunkB) >= Kb) v = OOB; }
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-                asm volatile("v_xor_b32 %0, %4, %0\n\tv_xor_b32 %1, %4, %1\n\tv_xor_b32 %2, %4, %2\n\tv_xor_b32 %3, %4, %3"
-                             : "+v"(fa[0][i].x), "+v"(fa[0][i].y), "+v"(fa[0][i].z), "+v"(fa[0][i].w) : "s"(flip));
-        }
-        bsum_step(0, step);
-    };
-    auto pp_mfma = [&]() __attribute__((always_inline)) {
-        __builtin_amdgcn_s_setprio(1);
+            for (int q = 0; q < LH; ++q)
+                load_chunk_to_lds(IA ? dA[h][q] : dB[h][q], lds + stg * STAGE_BYTES + (IA ? lA[h][q] : lB[h][q]), v, ko);
+        };
+        // fragments [from, to) of a half, in the order the MFMAs consume them (k-step outermost)
+        auto read = [&](auto isa, int h, int stg, int from, int to) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int r = from; r < to; ++r) {
+                if constexpr (decltype(isa)::value)
+                    pa[h][r % HM][r / HM] = *(const v4i*)(lds + stg * STAGE_BYTES + a_lane + (h * HM + r % HM) * MT * BKB + (g16 ^ (r / HM * KSB)));
+                else
+                    pb[h][r % HN][r / HN] = *(const v4i*)(lds + stg * STAGE_BYTES + b_lane + (h * HN + r % HN) * MT * BKB + (g16 ^ (r / HN * KSB)));
+            }
+        };
+        using X = std::integral_constant<bool, XA>;
+        using Y = std::integral_constant<bool, !XA>;
+        auto fence = [&]() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
+        auto bar = [&]() __attribute__((always_inline)) { fence(); asm volatile("s_barrier" ::: "memory"); fence(); };
+        // MFMAs of quadrant (A half h, B half g).  The uint8 sign flip of an A half happens at its first use (FLIP): the
+        // first fragment in the memory phase before, each other one in the shadow of its predecessor's MFMAs (all of them
+        // in the memory phases: 443 us instead of 413 for 8192^3).
+        auto flip_first = [&](int h) __attribute__((always_inline)) { if constexpr (DT == 1) pa[h][0][0] ^= (int)0x80808080; };
+        auto multiply = [&](auto flipc, int h, int g) __attribute__((always_inline)) {
+            constexpr bool FLIP = DT == 1 && decltype(flipc)::value;
 #pragma unroll
-            for (int j = 0; j < TN; ++j) mfma_inplace(fb[0][j], fa[0][i], acc[i][j]);
-        __builtin_amdgcn_s_setprio(0);
+            for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+                for (int i = 0; i < HM; ++i)
+#pragma unroll
+                    for (int j = 0; j < HN; ++j) {
+                        acc[h * HM + i][g * HN + j] = mfma(pb[g][j][kk], pa[h][i][kk], acc[h * HM + i][g * HN + j]);
+                        if constexpr (FLIP) {
+                            const int nr = kk * HM + i + 1;          // the next fragment, its registers spread over the HN MFMAs
+                            if (nr < RA) {
+#pragma unroll
+                                for (int r = 4 * j / HN; r < 4 * (j + 1) / HN; ++r) pa[h][nr % HM][nr / HM][r] ^= (int)0x80808080;
+                            }
+                            fence();
+                        }
+                    }
+        };
+        using Yes = std::integral_constant<bool, true>;
+        using No = std::integral_constant<bool, false>;
+        // one k-tile; LOAD: tile T + 2 is fetched (ragc: it may be the partly filled last one)
+        auto tile = [&](auto loadc, auto ragc, const int T) __attribute__((always_inline)) {
+            constexpr bool LOAD = decltype(loadc)::value;
+            const int stg = T & 1;
+            auto landed = [&]() __attribute__((always_inline)) { wait_only<63, 0>(); fence(); };   // the reads of the step before
+            landed();
+            read(Y{}, 1, stg, 0, RY);
+            read(X{}, 1, stg, 0, XP);
+            flip_first(0);
+            bar();
+            multiply(Yes{}, 0, 0);
+            bar();
+            landed();
+            read(X{}, 1, stg, XP, RX);
+            if constexpr (LOAD) { fetch(X{}, ragc, 0, stg, T + 2); fetch(Y{}, ragc, 0, stg, T + 2); }
+            if constexpr (!XA) flip_first(1);
+            fence();
+            wait_only<LOAD ? 5 * LH : 3 * LH, 15>();                 // X0 of T + 1
+            bar();
+            if constexpr (XA) multiply(No{}, 0, 1); else multiply(Yes{}, 1, 0);
+            bar();
+            landed();
+            read(X{}, 0, stg ^ 1, 0, RX - XP);
+            if constexpr (LOAD) fetch(Y{}, ragc, 1, stg, T + 2);
+            if constexpr (XA) flip_first(1);
+            fence();
+            wait_only<LOAD ? 5 * LH : 2 * LH, 15>();                 // Y0 of T + 1
+            bar();
+            if constexpr (XA) multiply(Yes{}, 1, 0); else multiply(No{}, 0, 1);
+            bar();
+            landed();
+            read(Y{}, 0, stg ^ 1, 0, RY);
+            read(X{}, 0, stg ^ 1, RX - XP, RX);
+            if constexpr (LOAD) fetch(X{}, ragc, 1, stg, T + 2);
+            fence();
+            wait_only<LOAD ? 4 * LH : 0, 15>();                      // Y1 and X1 of T + 1
+            bar();
+            multiply(No{}, 1, 1);
+            bar();
+        };
+        auto whole = [&](int kt) __attribute__((always_inline)) {    // tile kt into stage kt, in the order of the loop
+            auto all = [&](auto ragc) __attribute__((always_inline)) {
+                fetch(X{}, ragc, 0, kt, kt); fetch(Y{}, ragc, 0, kt, kt); fetch(Y{}, ragc, 1, kt, kt); fetch(X{}, ragc, 1, kt, kt);
+            };
+            if ((uint32_t)(kt + 1) * BKB > Kb) all(Yes{}); else all(No{});
+        };
+        whole(0);
+        if (KT > 1) { whole(1); wait_and_barrier<4 * LH, 0>(); }
+        else wait_and_barrier<0, 0>();
+        read(X{}, 0, 0, 0, RX);
+        read(Y{}, 0, 0, 0, RY);
+        if (wave >= NW / 2) bar();
+        fence();
+        int T = 0;
+        for (const int full = KT - 2 - (Kb % BKB != 0 ? 1 : 0); T < full; ++T) tile(Yes{}, No{}, T);
+        if (T + 2 < KT) { tile(Yes{}, Yes{}, T); ++T; }
+        for (; T < KT; ++T) tile(No{}, No{}, T);                     // (reads one tile past the end, of either stage: never used)
+        if (wave < NW / 2) bar();
     };
-    auto pp_fence = [&]() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
-    const bool grp1 = wave >= NW / 2;                     // wave-uniform: the group that runs one phase behind
-    // Both groups run the SAME instruction stream - read step s, barrier, multiply step s, barrier, read step s+1 ... -
-    // and group 1 enters it one barrier later, so the two are always in opposite kinds of phase.  Only the fetches of
-    // the next k-tile and the waits for them sit at group-dependent places of the stream (uniform branches around
-    // nothing but those), because they are tied to the moment at which a stage becomes free for BOTH groups.
-    auto pp_loads = [&]() __attribute__((always_inline)) {
-        const bool rag = begin_issue();
-        conv_tap();
-        if (rag) issue_loads(TrueC{}, stage, std::integral_constant<int, 0>{}, std::integral_constant<int, LPT>{});
-        else issue_loads(FalseC{}, stage, std::integral_constant<int, 0>{}, std::integral_constant<int, LPT>{});
-        end_issue();
-    };
-    auto pp_run = [&]() __attribute__((always_inline)) {
-        if (grp1) wait_and_barrier<63, 15>();            // group 1 enters the stream one phase later
-        pp_fence();
-        pp_mem(0, 0);
-        pp_fence();
-        wait_only<63, 0>();
-        pp_ready(0);
-        pp_fence();
-        if (KS == 1 && grp1) wait_only<(NS - 2) * LPT, 15>();
-        wait_and_barrier<63, 15>();
-        pp_fence();
-        int kk = 0;                                      // k-step inside the k-tile
-        const int steps = KT * KS;
-        for (int step = 0; step < steps; ++step) {
-            const bool last = (kk == KS - 1);
-            const int nkk = last ? 0 : kk + 1;
-            const bool next_last = (nkk == KS - 1);
-            const int next_stage = (stage + 1 == NS) ? 0 : stage + 1;
-            // ---- multiply step `step` (group 0: phase 2*step, group 1: one phase later) ----
-            if (last && grp1) pp_loads();                // the stage of this k-tile is free for both groups now
-            pp_fence();
-            pp_mfma();
-            pp_fence();
-            // before the next k-tile is published every wave's share of it has landed (group 0 waits here ...)
-            if (last && !grp1) wait_only<(NS - 2) * LPT, 15>();
-            wait_and_barrier<63, 15>();
-            pp_fence();
-            // ---- read step `step + 1` ----
-            pp_mem((last ? next_stage : stage) * STAGE_BYTES, nkk * KSB);
-            pp_fence();
-            if (last && !grp1) pp_loads();               // group 0 is one phase ahead: the stage is free only now
-            pp_fence();
-            wait_only<63, 0>();
-            pp_ready(step + 1);
-            pp_fence();
-            if (next_last && grp1) wait_only<(NS - 2) * LPT, 15>();      // (... group 1 here)
-            wait_and_barrier<63, 15>();
-            pp_fence();
-            kk = nkk;
-            if (last) stage = next_stage;
-        }
-        if (!grp1) wait_and_barrier<63, 15>();           // ... and group 0 leaves it one phase earlier
-    };
-    if constexpr (SCHED == 2) {
-        static_assert(SCHED != 2 || (NW == 8 && !CW && !PERS && !SPLITK), "the two-group schedule: 8 waves, plain launch");
-        pp_run();
-        mfma_drain();
+    if constexpr (PHASED) {
+        phased_run();
         store_tile();
     } else if constexpr (PERS) {
         for (int ct = blockIdx.x; ct < total; ct += (int)gridDim.x) {
