@@ -101,6 +101,12 @@ class Problem(ctypes.Structure):
                 ("bsum", ctypes.c_void_p)]
 
 
+class ConvView(ctypes.Structure):
+    """hrn_conv_view: channels-first result and zero-expanded input of a conv2d launch."""
+    _fields_ = [("out_plane", ctypes.c_int32), ("expand", ctypes.c_int32), ("in_h", ctypes.c_int32), ("in_w", ctypes.c_int32),
+                ("top", ctypes.c_int32), ("left", ctypes.c_int32)]
+
+
 def make_desc(dtype, op=HRN_OP_GEMM, bm=128, bn=128, bkb=128, wm=2, wn=2, mfma=32, stages=2, swizzle=1,
               epilogue=0, waves_per_eu=0, conv_window=0, persistent=0, split_k=0, sched=1, load_spread=2, colsum=0, nt_store=0):
     d = KernelDesc()
@@ -149,6 +155,7 @@ SYMBOLS = {
     "hrn_launch_conv2d_nhwc_f16": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_bmm_u8s8": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_conv2d_nhwc_u8s8": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
+    "hrn_launch_conv2d_chw": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(ConvView), _vp, _vp, _vp, _vp]),
     "hrn_launch_splitk_static": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_repeat": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _i, _vp]),
     "hrn_time": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _i, _i, _d, ctypes.POINTER(_d), _vp]),
@@ -388,6 +395,11 @@ class Module:
         self.bind_workspace(problem)
         self.bind_colsum(problem, b_ptr, stream)
         _check(self._launcher(problem)(self._h, ctypes.byref(problem), a_ptr, b_ptr, c_ptr, stream))
+
+    def launch_conv2d_chw(self, problem, view, a_ptr, b_ptr, c_ptr, stream=0):
+        """conv2d with a channels-first result and, where ``view.expand`` is set, a zero-expanded input (hrn_conv_view)."""
+        self.bind_colsum(problem, b_ptr, stream)
+        _check(lib().hrn_launch_conv2d_chw(self._h, ctypes.byref(problem), ctypes.byref(view), a_ptr, b_ptr, c_ptr, stream))
 
     def launch_splitk_static(self, problem, a_ptr, b_ptr, c_ptr, stream=0):
         """Split-K launch whose partial sums live in the library's own static device workspace (no allocation)."""

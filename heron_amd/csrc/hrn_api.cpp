@@ -41,6 +41,8 @@ struct HrnKArgs {  // must match mfma_gemm_template.hip
     int32_t cstride_w, cpad_w, cdil_w;
     int32_t split, kt_per_slice;
     const void* bsum;
+    int32_t out_plane;
+    int32_t expand_shift, in_h, in_w, top, left;
 };
 
 struct hrn_module {
@@ -48,9 +50,11 @@ struct hrn_module {
     hrn_kernel_info info;
     hipModule_t mod;
     hipFunction_t fn;
+    hipFunction_t fn_chw, fn_expand;   // conv2d: the kernels of hrn_launch_conv2d_chw (null where the instance has none)
     std::string path;
     int persist_grid;   // persistent instances: workgroups that fit the device at once (multiple of 8 when >= 8)
     int epi_bytes;      // LDS bytes of the epilogue region (column sums + strips)
+    int chw_bytes;      // the same of the channels-first epilogue
 };
 
 extern char** environ;
@@ -123,7 +127,7 @@ uint64_t fnv1a_file(const std::string& p) {
 }
 
 struct Derived {
-    int es, oes, nw, cpr, rpi, a_lpw, b_lpw, lpt, ksb, ks, tm, tn, stage_bytes, lds, epi_bytes;
+    int es, oes, nw, cpr, rpi, a_lpw, b_lpw, lpt, ksb, ks, tm, tn, stage_bytes, lds, epi_bytes, chw_bytes;
 };
 
 // Structural constraints of the template; the same conditions are static_asserts in the kernel.
@@ -195,6 +199,11 @@ int derive(const hrn_kernel_desc* d, Derived* o) {
             r.lds = std::max(r.lds, r.epi_bytes);
         }
     }
+    // channels-first epilogue: strips of mfma channels x at most 64 pixels (whole MFMA tiles of the wave tile)
+    int csw = 1;
+    for (int t = 64 / d->mfma; t > 1; --t)
+        if (r.tm % t == 0) { csw = t; break; }
+    r.chw_bytes = base + r.nw * d->mfma * (csw * d->mfma * r.oes + 16);
     // (a conv_window instance keeps the epilogue region in its dynamic LDS, where the window was)
     if (r.lds > 163840) return fail(HRN_E_BADPARAM, "LDS %d > 163840", r.lds);
     if (d->swizzle && (r.cpr << (d->swizzle - 1)) > d->mfma)
@@ -219,7 +228,9 @@ std::string desc_key(const hrn_kernel_desc* d, uint64_t srch) {
 }
 
 int parse_remark(const std::string& log, const char* tag) {
-    size_t p = log.find(tag);
+    // the figures of an instance are those of its main kernel
+    const size_t from = log.find("Function Name: hrn_mfma_kernel [");
+    size_t p = log.find(tag, from == std::string::npos ? 0 : from);
     if (p == std::string::npos) return -1;
     return atoi(log.c_str() + p + strlen(tag));
 }
@@ -359,6 +370,7 @@ void read_info(const std::string& path, hrn_kernel_info* o) {
 // What one launch consists of: the template kernel and, for a split-K instance, the pass that adds the K slices.
 struct LaunchPlan {
     HrnKArgs k;
+    hipFunction_t fn;
     unsigned grid, dyn_lds;
     int split;                 // K slices the grid covers (1 = the kernel writes C itself)
     void* C;                   // the caller's output
@@ -382,6 +394,7 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     HrnKArgs* k = &plan->k;
     plan->dyn_lds = 0;
     plan->split = 1;
+    plan->fn = mod ? mod->fn : nullptr;
     if (!mod || !p || !A || !B || !C) return fail(HRN_E_BADPARAM, "null argument");
     const hrn_kernel_desc& d = mod->desc;
     if (p->op != d.op) return fail(HRN_E_BADPARAM, "problem op %d does not match module op %d", p->op, d.op);
@@ -513,7 +526,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restri
 int run_plan(const hrn_module* mod, const hrn_problem* p, const LaunchPlan& plan, void* workspace, hipStream_t st) {
     size_t sz = sizeof plan.k;
     void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void*)&plan.k, HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz, HIP_LAUNCH_PARAM_END};
-    HIP_TRY(hipModuleLaunchKernel(mod->fn, plan.grid, 1, 1, (unsigned)mod->info.threads, 1, 1, plan.dyn_lds, st, nullptr, extra));
+    HIP_TRY(hipModuleLaunchKernel(plan.fn, plan.grid, 1, 1, (unsigned)mod->info.threads, 1, 1, plan.dyn_lds, st, nullptr, extra));
     if (mod->desc.split_k) {
         const int64_t count = (int64_t)p->batch * p->m * (p->n / 4);
         const unsigned blocks = (unsigned)std::min<int64_t>((count + 255) / 256, 256 * 32);
@@ -1220,6 +1233,7 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
         Derived dv;
         (void)derive(desc, &dv);        // compile_desc has validated the descriptor
         m->epi_bytes = dv.epi_bytes;
+        m->chw_bytes = dv.chw_bytes;
     }
     hipError_t e = hipModuleLoad(&m->mod, path.c_str());
     if (e != hipSuccess) {
@@ -1231,6 +1245,15 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
         (void)hipModuleUnload(m->mod);
         delete m;
         return fail(HRN_E_LOAD, "hipModuleGetFunction: %s", hipGetErrorString(e));
+    }
+    if (desc->op == HRN_OP_CONV2D && !desc->persistent && !desc->split_k) {
+        e = hipModuleGetFunction(&m->fn_chw, m->mod, "hrn_mfma_kernel_chw");
+        if (e == hipSuccess) e = hipModuleGetFunction(&m->fn_expand, m->mod, "hrn_mfma_kernel_chw_expand");
+        if (e != hipSuccess) {
+            (void)hipModuleUnload(m->mod);
+            delete m;
+            return fail(HRN_E_LOAD, "hipModuleGetFunction: %s", hipGetErrorString(e));
+        }
     }
     if (desc->split_k) {
         // hrn_launch_splitk_static finds the library's workspace of this device looked up already
@@ -1296,6 +1319,35 @@ int hrn_launch_bmm_u8s8(const hrn_module* mod, const hrn_problem* p, const void*
 int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, const void* In, const void* Filter, void* Out, void* stream) {
     if (mod && (mod->desc.dtype != HRN_DT_U8S8 || mod->desc.op != HRN_OP_CONV2D)) return fail(HRN_E_BADPARAM, "module is not a u8s8 conv2d");
     return launch(mod, p, In, Filter, Out, stream);
+}
+
+int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn_conv_view* view, const void* In, const void* Filter,
+                          void* Out, void* stream) {
+    if (!mod || !p || !view) return fail(HRN_E_BADPARAM, "null argument");
+    if (!mod->fn_chw) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k");
+    LaunchPlan plan;
+    int rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);
+    if (rc) return rc;
+    if (view->out_plane < 1 || p->m % view->out_plane)
+        return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
+    plan.fn = mod->fn_chw;
+    plan.k.out_plane = view->out_plane;
+    if (mod->desc.conv_window) {
+        plan.dyn_lds = std::max(plan.dyn_lds, (unsigned)mod->chw_bytes);
+        if ((int)plan.dyn_lds + mod->info.lds_bytes > 163840)
+            return fail(HRN_E_BADPARAM, "conv2d_chw: epilogue of %d bytes + %d static LDS exceeds 163840", mod->chw_bytes, mod->info.lds_bytes);
+    }
+    if (view->expand) {
+        if (view->expand < 1 || (view->expand & (view->expand - 1)) || view->in_h < 1 || view->in_w < 1 || view->top < 0 || view->left < 0 ||
+            ((int64_t)view->in_h - 1) * view->expand + view->top >= p->ch || ((int64_t)view->in_w - 1) * view->expand + view->left >= p->cw)
+            return fail(HRN_E_BADPARAM, "conv2d_chw: %d x %d pixels, %d apart (a power of two) from (%d, %d), do not lie in %d x %d",
+                        view->in_h, view->in_w, view->expand, view->top, view->left, p->ch, p->cw);
+        plan.fn = mod->fn_expand;
+        plan.k.in_h = view->in_h; plan.k.in_w = view->in_w;
+        plan.k.top = view->top; plan.k.left = view->left;
+        plan.k.expand_shift = __builtin_ctz((unsigned)view->expand);
+    }
+    return run_plan(mod, p, plan, nullptr, (hipStream_t)stream);
 }
 
 int hrn_launch_repeat(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, int count,

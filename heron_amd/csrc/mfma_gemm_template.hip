@@ -48,6 +48,9 @@ struct HrnKArgs {
     int32_t cstride_w, cpad_w, cdil_w;   // conv: the width-direction values (cstride/cpad/cdil are the height ones)
     int32_t split, kt_per_slice;         // split-K: number of K slices and k-tiles per slice
     const void* bsum;                    // uint8 path: per batch entry N column sums of B (sum_k B[n,k], int32), or null
+    int32_t out_plane;                   // CHW kernels: row m, column n of the result goes to C[m / out_plane][n][m % out_plane]
+    int32_t expand_shift;                // EXPAND kernels: the H x W input is not in memory: pixel (y, x) of the in_h x in_w
+    int32_t in_h, in_w, top, left;       // one that is stands at (top + (y << shift), left + (x << shift)), zeros elsewhere
 };
 #endif
 
@@ -149,6 +152,17 @@ constexpr int LDS_BYTES = PERS ? NS * STAGE_BYTES + EPI_BYTES
                                : ((CW || NS * STAGE_BYTES > EPI_BYTES) ? NS * STAGE_BYTES : EPI_BYTES);
 constexpr int STORES_PER_TILE = (EPI >= 1) ? TM * ESPLIT * (MT * (SW * OES / 16) / 64) : 0;   // store instructions per wave per output tile
 static_assert(EPI >= 0 && EPI <= 2 && TN % ESPLIT == 0, "epilogue kind");
+// Channels-first epilogue (CHW kernels): strips of MT channels x CSW pixels (whole MFMA tiles, at most 64)
+constexpr int chw_tiles() {
+    for (int d = 64 / MT; d > 1; --d)
+        if (TM % d == 0) return d;
+    return 1;
+}
+constexpr int CSW = chw_tiles() * MT;
+constexpr int CHW_PITCH = CSW * OES + 16;
+constexpr int CHW_BYTES = EPI_BASE + NW * MT * CHW_PITCH;
+constexpr int CHW_LDS_BYTES = (CW || NS * STAGE_BYTES > CHW_BYTES) ? NS * STAGE_BYTES : CHW_BYTES;
+
 static_assert(!PERS || (EPI >= 1 && !CW && !SPLITK && KS % 2 == 0), "persistent mode: staged epilogue, even k-steps");
 static_assert(!PERS || (NS - 2) * LPT + STORES_PER_TILE <= 63, "persistent mode: vmcnt range");
 static_assert(!SPLITK || !CW, "split-K uses the im2col load path");
@@ -238,14 +252,16 @@ __device__ __forceinline__ void sched_hint() {
     }
 }
 
-}  // namespace
-
-extern "C" __global__ void __launch_bounds__(NT)
-#if HRN_WPE > 0
-__attribute__((amdgpu_waves_per_eu(HRN_WPE, HRN_WPE)))
-#endif
-hrn_mfma_kernel(const HrnKArgs a) {
-    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+// The body of all kernels of an instance.
+//   CHW (conv): the result is stored channels first, see HrnKArgs::out_plane.  Such a result used to be the row-major one,
+// transposed by a pass of its own that read and wrote all of it once more.  The MFMAs are issued with their operands
+// exchanged, so that a lane holds 4 consecutive pixels of one channel.
+//   EXPAND (conv): the input of a transposed convolution, HrnKArgs::expand_shift; the zeros are not in memory.
+//   NCHW transposed conv 16 x 56x56x64 -> 111x111x128, stride 2: 77 us with the passes around the kernel, 39 us without
+// (50 MB of result; 28 us of it the kernel, 26 us when it stores rows).
+template <bool CHW, bool EXPAND>
+__device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
+    __shared__ __attribute__((aligned(1024))) char lds[CHW ? CHW_LDS_BYTES : LDS_BYTES];
     extern __shared__ __attribute__((aligned(1024))) char win[];   // window mode: input window, later the epilogue region
 
     const int tid = threadIdx.x;
@@ -284,11 +300,22 @@ hrn_mfma_kernel(const HrnKArgs a) {
     tile_coords(first_pid, c_bz, c_tile_m, c_tile_n);
     int m0 = c_tile_m * BM, n0 = c_tile_n * BN;
 
+    // conv: the input that is in memory, and the way from a position of the expanded one to it
+    const int in_h = EXPAND ? a.in_h : a.H, in_w = EXPAND ? a.in_w : a.W;
+    [[maybe_unused]] auto unexpand = [&](int& y, int& x) {
+        y -= a.top;
+        x -= a.left;
+        const bool hit = ((y | x) & ((1 << a.expand_shift) - 1)) == 0;
+        y >>= a.expand_shift;                                  // (a negative position stays negative)
+        x >>= a.expand_shift;
+        return hit && (unsigned)y < (unsigned)in_h && (unsigned)x < (unsigned)in_w;
+    };
+
     // ---- issue side: the tile whose k-tiles are being fetched (the same tile unless the launch is persistent) ----
     uint32_t a_bytes;
     const uint32_t b_bytes = (uint32_t)a.N * (uint32_t)a.ldb * ES;
     if constexpr (OP == 0) a_bytes = (uint32_t)a.M * (uint32_t)a.lda * ES;
-    else a_bytes = (uint32_t)(a.M / (a.HO * a.WO)) * (uint32_t)(a.H * a.W * a.CI) * ES;
+    else a_bytes = (uint32_t)(a.M / (a.HO * a.WO)) * (uint32_t)(in_h * in_w * a.CI) * ES;
     const char* baseA = (const char*)a.A;
     const char* baseB = (const char*)a.B;
     bool issue_alive = true;
@@ -357,7 +384,7 @@ hrn_mfma_kernel(const HrnKArgs a) {
 #pragma unroll
             for (int i = 0; i < A_LPW; ++i) {
                 const bool ok = m < a.M;
-                voffA[i] = (uint32_t)img * (uint32_t)(a.H * a.W * a.CI) * ES;
+                voffA[i] = (uint32_t)img * (uint32_t)(in_h * in_w * a.CI) * ES;
                 iy0[i] = ok ? oy * a.cstride - a.cpad : -(1 << 28);
                 ix0[i] = ox * a.cstride_w - a.cpad_w;
                 m += NW * RPI;
@@ -428,9 +455,11 @@ hrn_mfma_kernel(const HrnKArgs a) {
                     }
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, ks_cur);
                 } else if constexpr (!CW) {
-                    const int iy = iy0[i] + conv_iyr, ix = ix0[i] + conv_ixs;
-                    const bool ok = conv_kvalid && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-                    const uint32_t v = ok ? voffA[i] + (uint32_t)((iy * a.W + ix) * a.CI + cc) * ES : OOB;
+                    int iy = iy0[i] + conv_iyr, ix = ix0[i] + conv_ixs;
+                    bool ok = conv_kvalid;
+                    if constexpr (EXPAND) ok = ok && unexpand(iy, ix);
+                    else ok = ok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+                    const uint32_t v = ok ? voffA[i] + (uint32_t)((iy * in_w + ix) * a.CI + cc) * ES : OOB;
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, 0u);
                 }
             } else {
@@ -486,7 +515,15 @@ hrn_mfma_kernel(const HrnKArgs a) {
             const int wrow = L / cpp, pos = L - wrow * cpp;
             const int src = (pos & ~(CPR - 1)) | ((pos & (CPR - 1)) ^ swz_of_row(wrow));
             const int gp = gp0 + wrow;
-            const uint32_t v = (wrow < w_rows && gp >= 0) ? (uint32_t)gp * (uint32_t)w_pitch + src * 16 : OOB;
+            int px = gp;                                     // pixel in memory
+            bool ok = wrow < w_rows && gp >= 0;
+            if constexpr (EXPAND) {
+                const int img = gp / (a.H * a.W), rem = gp - img * (a.H * a.W);
+                int y = rem / a.W, x = rem - y * a.W;
+                ok = ok && unexpand(y, x);
+                px = (img * in_h + y) * in_w + x;
+            }
+            const uint32_t v = ok ? (uint32_t)px * (uint32_t)w_pitch + src * 16 : OOB;
             load_chunk_to_lds(rA, win + q * 1024, v, 0u);
         }
         // masks: pixel of fragment row i by one division, the following rows (MT further each) by carry
@@ -601,6 +638,7 @@ hrn_mfma_kernel(const HrnKArgs a) {
     // ---- epilogue of the compute-side tile (c_bz, m0, n0) ----
     // MFMA was issued as (B fragment, A fragment), so a lane holds 4 consecutive n for one m:
     //   m = lr, n = (r/4)*8 + lq*4 + r%4   (32x32)     m = lr, n = lq*4 + r   (16x16)
+    // (CHW: m and n exchanged)
     auto store_tile = [&]() __attribute__((always_inline)) {
         // the lane's coordinates, re-derived from values the compiler cannot trace back past this point: otherwise it
         // computes the epilogue's addresses in front of the k-loop and keeps them in registers all the way through it
@@ -649,7 +687,75 @@ hrn_mfma_kernel(const HrnKArgs a) {
             if constexpr (NTS) __builtin_nontemporal_store(val, ptr);
             else *ptr = val;
         };
-        if constexpr (EPI >= 1) {
+        if constexpr (CHW) {
+            // A wave parks MT channels x CSW pixels of its result in a private LDS strip and streams them out 16 bytes per
+            // lane along the pixels.  A piece starts at any element (a plane may be odd); the few that reach past the end of
+            // a plane or of the result go element by element.
+            if constexpr (DT == 0) wait_and_barrier<0, 0>();          // (the int8 path has synchronised above) stages are dead now
+            using oel_t = typename std::conditional<OES == 2, _Float16, int>::type;
+            typedef v4i piece_t __attribute__((aligned(2)));
+            char* strip = epi + EPI_BASE + wave * (MT * CHW_PITCH);
+            constexpr int CPRW = CSW * OES / 16, EPC = 16 / OES, IT = CSW / MT;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int nl = wn_idx * WTN + j * MT;
+                [[maybe_unused]] int bs = 0;
+                if constexpr (DT == 1) {
+                    bs = bs_lds[nl + lr_e];
+                    if constexpr (!COLSUM) {
+#pragma unroll
+                        for (int w = 1; w < WM; ++w) bs += bs_lds[w * BN + nl + lr_e];
+                    }
+                    bs *= 128;
+                }
+#pragma unroll
+                for (int ib = 0; ib < TM; ib += IT) {
+#pragma unroll
+                    for (int i = 0; i < IT; ++i)
+#pragma unroll
+                        for (int g = 0; g < ACC_N / 4; ++g) {
+                            char* dst = strip + lr_e * CHW_PITCH + (i * MT + g * 8 + lq_e * 4) * OES;
+                            if constexpr (DT == 0) {
+                                v4h o;
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) o[r] = (_Float16)acc[ib + i][j][g * 4 + r];
+                                *(v4h*)dst = o;
+                            } else {
+                                v4i o;
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) o[r] = acc[ib + i][j][g * 4 + r] + bs;
+                                *(v4i*)dst = o;
+                            }
+                        }
+                    asm volatile("" ::: "memory");     // LDS serves one wave's requests in order: the reads below see the writes
+#pragma unroll
+                    for (int it = 0; it < (MT * CPRW + 63) / 64; ++it) {
+                        const int c = it * 64 + lane_e;
+                        const int row = c / CPRW, cc2 = c % CPRW;
+                        const int n = n0 + nl + row;
+                        const int m = m0 + wm_idx * WTM + ib * MT + cc2 * EPC;
+                        if (c < MT * CPRW && n < a.N && m < a.M) {
+                            const v4i val = *(const v4i*)(strip + row * CHW_PITCH + cc2 * 16);
+                            const unsigned plane = (unsigned)a.out_plane, img = (unsigned)m / plane, px = (unsigned)m - img * plane;
+                            oel_t* dst = (oel_t*)a.C + ((int64_t)img * a.N + n) * plane + px;
+                            if (px + EPC <= plane && m + EPC <= a.M) {
+                                put((piece_t*)dst, val);
+                            } else {
+                                const oel_t* ve = (const oel_t*)&val;
+                                unsigned p = px;
+#pragma unroll
+                                for (int e = 0; e < EPC; ++e) {
+                                    if (m + e < a.M) *dst = ve[e];
+                                    ++dst;
+                                    if (++p == plane) { p = 0; dst += (int64_t)(a.N - 1) * plane; }
+                                }
+                            }
+                        }
+                    }
+                    asm volatile("" ::: "memory");
+                }
+            }
+        } else if constexpr (EPI >= 1) {
             // LDS-staged epilogue: a wave parks one MFMA row-tile (MT rows x SW columns) of its result in a private,
             // padded LDS strip, then streams it out with 16 bytes per lane_e, whole row segments per store instruction.
             if constexpr (DT == 0 && !PERS) wait_and_barrier<0, 0>();   // (the int8 path has synchronised above) stages are dead now
@@ -801,7 +907,7 @@ hrn_mfma_kernel(const HrnKArgs a) {
                 loads(std::integral_constant<int, f>{}, std::integral_constant<int, n>{});
             }
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = mfma(fb[cur][j], av, acc[i][j]);
+            for (int j = 0; j < TN; ++j) acc[i][j] = CHW ? mfma(av, fb[cur][j], acc[i][j]) : mfma(fb[cur][j], av, acc[i][j]);
             if constexpr (i + 1 < TM) av = a_operand(cur, i + 1);      // ready before the next row's MFMAs ask for it
             if constexpr (SCHED >= 1) __builtin_amdgcn_sched_barrier(0);
         };
@@ -1043,3 +1149,17 @@ hrn_mfma_kernel(const HrnKArgs a) {
         run_tile(false);
     }
 }
+
+}  // namespace
+
+#if HRN_WPE > 0
+#define HRN_ENTRY extern "C" __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(HRN_WPE, HRN_WPE)))
+#else
+#define HRN_ENTRY extern "C" __global__ void __launch_bounds__(NT)
+#endif
+
+HRN_ENTRY hrn_mfma_kernel(const HrnKArgs a) { hrn_mfma_body<false, false>(a); }
+#if HRN_OP == 1 && HRN_PERSIST == 0 && HRN_SPLITK == 0
+HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { hrn_mfma_body<true, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { hrn_mfma_body<true, true>(a); }
+#endif

@@ -411,6 +411,49 @@ ADAPTERS = {
 ACTIVATION_AS_IS = ('identity', 'c1d_nwc', 'c2d_hwio', 'c2d_krsc')
 
 
+# Adapters whose result reorder (pixels x channels -> channels first) the kernel does itself as it stores the result, with the
+# shape of that result: ``n`` images of ``ho`` x ``wo`` pixels
+CHANNELS_FIRST = {
+    'c1d_ncw': lambda info, n, co, ho, wo: (n, co, wo),
+    'c2d_nchw': lambda info, n, co, ho, wo: (n, co, ho, wo),
+    'c3d_ncdhw': lambda info, n, co, ho, wo: (info['depth']['N'], co, info['depth']['DO'], ho, wo),
+    't2d_nchw': lambda info, n, co, ho, wo: (n, co, ho, wo),
+}
+
+
+def _run_channels_first(mod, info, inputs, act, Bm, group_m, bsum):
+    """A channels-first convolution without passes over its result - and, transposed, without the zero-expanded input."""
+    c, t, X = info['conv'], info.get('transposed'), inputs[0]
+    f16 = mod.desc.dtype == B.HRN_DT_F16
+    view = B.ConvView()
+    if t is not None and t['stride'] & (t['stride'] - 1) == 0 and X.shape[0] <= 65535:
+        N, CI, H, W = X.shape
+        A = _channels_last(X.reshape(N, CI, H * W), c['CI'])
+        xshape = (N, c['H'], c['W'], c['CI'])
+        view.expand, view.in_h, view.in_w = t['stride'], H, W
+        view.top, view.left = (c['KH'] - 1) * t['dil'] - t['pad'], (c['KW'] - 1) * t['dil'] - t['pad']
+    else:
+        A = act(info, *inputs)
+        xshape = A.shape
+    _chk(A, torch.float16 if f16 else torch.uint8)
+    _chk(Bm, torch.float16 if f16 else torch.int8)
+    if xshape[3] != Bm.shape[3]:
+        raise ValueError("channel mismatch")
+    p = B.conv2d_problem(*xshape, *Bm.shape[:3], (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']), group_m)
+    if bsum is not None and mod.desc.colsum:
+        _chk(bsum, torch.int32)
+        if bsum.numel() != p.n:
+            raise ValueError("bsum holds %d sums, the filter has %d output channels" % (bsum.numel(), p.n))
+        p.bsum = bsum.data_ptr()
+    ho = (p.ch - ((p.kh - 1) * p.cdil + 1) + 2 * p.cpad) // p.cstride + 1
+    wo = (p.cw - ((p.kw - 1) * p.cdil_w + 1) + 2 * p.cpad_w) // p.cstride_w + 1
+    shape = CHANNELS_FIRST[info['adapter']](info, p.cn, p.n, ho, wo)
+    view.out_plane = p.m // shape[0]
+    out = _new(torch.empty, shape, dtype=torch.float16 if f16 else torch.int32, device=A.device)
+    _do(mod.launch_conv2d_chw, p, view, A.data_ptr(), Bm.data_ptr(), out.data_ptr(), _stream())
+    return out
+
+
 def prepare_constant(info, inputs):
     """The kernel's B operand of an operator: the reordered / padded filter or the generated right-hand side.  It
     depends on the weights and the shapes only, so a caller with fixed weights prepares it once."""
@@ -423,9 +466,12 @@ def run_operator(mod, info, inputs, group_m=8, split_k=0, constant=None, bsum=No
     ``info`` is the dictionary the operator definition handed to ``ctx.set_info``; ``mod`` an instance of the
     template that matches its kind and operator; ``constant`` a B operand from ``prepare_constant`` (made here when
     absent); ``bsum`` its column sums (``column_sums``) for a ``colsum`` instance."""
-    act, const, fin = ADAPTERS[info.get('adapter', 'identity')]
-    A = act(info, *inputs)
+    adapter = info.get('adapter', 'identity')
+    act, const, fin = ADAPTERS[adapter]
     Bm = const(info, *inputs) if constant is None else constant
+    if adapter in CHANNELS_FIRST and _native_ok(inputs[0]) and not (mod.desc.split_k or mod.desc.persistent):
+        return _run_channels_first(mod, info, inputs, act, Bm, group_m, bsum)
+    A = act(info, *inputs)
     if info['operator'] == 'conv2d_nhwc':
         c = info['conv']
         C = conv2d_nhwc(mod, A, Bm, (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']),

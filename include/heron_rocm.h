@@ -211,6 +211,23 @@ int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, con
 #define HRN_STATIC_WORKSPACE_BYTES (32u << 20)
 int hrn_launch_splitk_static(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* stream);
 
+/*
+ * conv2d whose result is stored channels first, and whose input may be zero-expanded on the way in: what the channels-first
+ * and transposed convolutions of the reference (ops/cuda/conv2d.py:9-135, conv1d.py:11-107, conv3d.py:10-115,
+ * conv2d_transposed.py:59-171) need around the NHWC kernel, without passes of their own.
+ *   out_plane: the m x n result of the GEMM view (pixels x channels) goes to Out[m / out_plane][n][m % out_plane], so
+ * out_plane is ho*wo for (n, co, ho, wo), and do*ho*wo where do successive images are the slices of a volume.
+ *   expand > 0 (a power of two): the problem's ch x cw input is not in memory; In holds (cn, in_h, in_w, ci), pixel (y, x)
+ * of which stands at (top + y*expand, left + x*expand) of ch x cw, everything else is zero.
+ * The instance is a conv2d one without persistent and split_k; p->ldc does not apply.
+ */
+typedef struct hrn_conv_view {
+    int32_t out_plane;
+    int32_t expand, in_h, in_w, top, left;
+} hrn_conv_view;
+int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn_conv_view* view, const void* In,
+                          const void* Filter, void* Out, void* stream);
+
 /* `count` back-to-back launches of the same problem from one host call (the inner loop of a time_evaluator
  * repeat, runner/measure_methods.py:138-145, without the events). */
 int hrn_launch_repeat(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C,
