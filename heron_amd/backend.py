@@ -11,6 +11,7 @@ import threading
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "librocm_heron.so")
+EXT_PATH = os.path.join(CSRC, "_hrn_torch.so")
 INCLUDE = os.path.join(os.path.dirname(_HERE), "include")
 
 HRN_DT_F16, HRN_DT_U8S8 = 0, 1
@@ -119,8 +120,9 @@ def make_desc(dtype, op=HRN_OP_GEMM, bm=128, bn=128, bkb=128, wm=2, wn=2, mfma=3
 
 
 def build_library(force=True, verbose=False):
-    """Compile ``csrc/hrn_api.cpp`` into ``csrc/librocm_heron.so`` with hipcc (cross-compiles without a GPU)."""
-    if os.path.exists(LIB_PATH) and not force:
+    """Compile ``csrc/hrn_api.cpp`` into ``csrc/librocm_heron.so`` with hipcc (cross-compiles without a GPU) and
+    ``csrc/hrn_torch.cpp``, the host path on torch tensors, into ``csrc/_hrn_torch.so`` beside it."""
+    if os.path.exists(LIB_PATH) and os.path.exists(EXT_PATH) and not force:
         return LIB_PATH
     hipcc = os.environ.get("HRN_HIPCC", "/opt/rocm/bin/hipcc")
     cmd = [hipcc, "-O2", "-fPIC", "-shared"] + HIPCC_FLAGS + [os.path.join(CSRC, "hrn_api.cpp"), "-o", LIB_PATH + ".tmp"]
@@ -128,14 +130,26 @@ def build_library(force=True, verbose=False):
     if r.returncode != 0:
         raise RuntimeError("building librocm_heron.so failed:\n" + r.stderr[-4000:])
     os.replace(LIB_PATH + ".tmp", LIB_PATH)
+    import sysconfig
+    from torch.utils import cpp_extension
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+    cmd += ["-I" + d for d in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]] if os.path.isdir(d)]
+    cmd += [os.path.join(CSRC, "hrn_torch.cpp")] + ["-L" + d for d in cpp_extension.library_paths("cuda") if os.path.isdir(d)]
+    cmd += ["-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python", "-lc10_hip", "-L" + CSRC, "-l:" + os.path.basename(LIB_PATH),
+            "-Wl,-rpath,$ORIGIN", "-o", EXT_PATH + ".tmp"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building _hrn_torch.so failed:\n" + r.stderr[-4000:])
+    os.replace(EXT_PATH + ".tmp", EXT_PATH)
     if verbose:
         print("built", LIB_PATH)
-    global _lib
-    _lib = None
+    global _lib, _ext
+    _lib = _ext = None
     return LIB_PATH
 
 
 _lib = None
+_ext = None
 _lock = threading.Lock()
 
 _vp, _i, _d = ctypes.c_void_p, ctypes.c_int, ctypes.c_double
@@ -193,6 +207,22 @@ def lib():
                 fn.argtypes = args
             _lib = L
     return _lib
+
+
+def ext():
+    """The host path on torch tensors (csrc/hrn_torch.cpp); raises if it has not been built."""
+    global _ext
+    if _ext is None:
+        lib()
+        import torch  # noqa: F401 - the extension links against the libraries torch has loaded
+        from importlib import machinery, util
+        if not os.path.exists(EXT_PATH):
+            raise HeronRocmError(HRN_E_LOAD, "%s is missing: run __graft_entry__.build() "
+                                 "(or heron_amd.backend.build_library())" % EXT_PATH)
+        spec = util.spec_from_file_location("_hrn_torch", EXT_PATH, loader=machinery.ExtensionFileLoader("_hrn_torch", EXT_PATH))
+        _ext = util.module_from_spec(spec)
+        spec.loader.exec_module(_ext)
+    return _ext
 
 
 def _check(rc):
@@ -347,6 +377,7 @@ class Module:
         h = _vp()
         _check(lib().hrn_build(ctypes.byref(desc), float(timeout_s), ctypes.byref(h)))
         self._h = h
+        self.native = (h.value, ctypes.addressof(desc))      # what the functions of ext() take for this instance
         info = KernelInfo()
         _check(lib().hrn_module_info(self._h, ctypes.byref(info)))
         self.info = info.as_dict()
@@ -434,6 +465,7 @@ class Module:
         if getattr(self, "_h", None):
             lib().hrn_module_free(self._h)
             self._h = None
+            self.native = (0, ctypes.addressof(self.desc))
         self._ws = None
         self._bs = None
 

@@ -8,7 +8,7 @@ from . import backend as B
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    return B.ext().stream()
 
 
 # While an OperatorPlan is being recorded, every library call of this module is also appended here (callable, arguments):
@@ -55,6 +55,10 @@ def gemm(mod, A, Bm, out=None, group_m=8, split_k=0, bsum=None):
     """C = A @ Bm.T for A (M,K), Bm (N,K), or batched (b,M,K) x (b,N,K) -> (b,M,N).  ``split_k`` is the number of
     K slices for a split-K instance (the module supplies the workspace).  ``bsum``: the column sums of Bm
     (``column_sums``) for a ``colsum`` instance; computed on the spot when absent."""
+    if _recording is None:
+        C = B.ext().gemm(*mod.native, group_m, split_k, A, Bm, out, bsum)
+        if C is not None:
+            return C if type(C) is not int else B._check(C)
     f16 = mod.desc.dtype == B.HRN_DT_F16
     _chk(A, torch.float16 if f16 else torch.uint8)
     _chk(Bm, torch.float16 if f16 else torch.int8)
@@ -87,6 +91,10 @@ def unpack_filter_blocked(Wb):
 
 def conv2d_nhwc(mod, X, Wt, stride=1, pad=0, dil=1, out=None, group_m=8, split_k=0, bsum=None):
     """X (N,H,W,CI), Wt KRSC (CO,KH,KW,CI) -> (N,HO,WO,CO): fp16 -> fp16, or uint8 x int8 -> int32."""
+    if _recording is None:
+        C = B.ext().conv2d(*mod.native, group_m, split_k, X, Wt, stride, pad, dil, out, bsum)
+        if C is not None:
+            return C if type(C) is not int else B._check(C)
     f16 = mod.desc.dtype == B.HRN_DT_F16
     _chk(X, torch.float16 if f16 else torch.uint8)
     _chk(Wt, torch.float16 if f16 else torch.int8)
