@@ -264,6 +264,17 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
     __shared__ __attribute__((aligned(1024))) char lds[CHW ? CHW_LDS_BYTES : LDS_BYTES];
     extern __shared__ __attribute__((aligned(1024))) char win[];   // window mode: input window, later the epilogue region
 
+    // every argument the start of the kernel needs, fetched at once: left to itself the compiler reads them where they are
+    // used and waits for memory several times before the first load is out (1700 - 1900 cycles, 850 like this)
+    if constexpr (TM * TN * ACC_N < 256) {      // (not where every register holds an accumulator)
+        asm volatile("" ::"s"(a.A), "s"(a.B), "s"(a.C), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.lda), "s"(a.ldb), "s"(a.ldc), "s"(a.sA), "s"(a.sB),
+                     "s"(a.sC), "s"(a.tiles_m), "s"(a.tiles_n), "s"(a.group_m), "s"(a.batch));
+        if constexpr (OP == 1)
+            asm volatile("" ::"s"(a.H), "s"(a.W), "s"(a.CI), "s"(a.HO), "s"(a.WO), "s"(a.KH), "s"(a.KW), "s"(a.cstride), "s"(a.cpad), "s"(a.cdil),
+                         "s"(a.cstride_w), "s"(a.cpad_w), "s"(a.cdil_w));
+        if constexpr (SPLITK) asm volatile("" ::"s"(a.split), "s"(a.kt_per_slice));
+        if constexpr (COLSUM) asm volatile("" ::"s"(a.bsum));
+    }
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -321,14 +332,25 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
     bool issue_alive = true;
 
     const int lrow = lane / CPR, lpos = lane % CPR;
-    // When the rows that successive load instructions of a wave cover (NW*RPI apart) share their swizzle phase, a
-    // lane's byte offset inside "its" row block is the same for every load and every tile: lane_off.  The row block
-    // itself - tile origin, wave, load index - is a scalar and goes into the buffer descriptor (base advanced by the
-    // block's byte offset, size reduced by it, so that rows past the end of the matrix still read as zeros).  The
-    // issue side then holds two vector registers instead of one per load and spends no vector ALU work per tile.
-    constexpr bool UNI = (SWZ == 0) || ((NW * RPI) % (CPR << (SWZ > 0 ? SWZ - 1 : 0))) == 0;
+    // Rows past the end of the matrix read as zeros.  Two ways to say which rows a load covers:
+    //   one vector register per load with the lane's byte offset (out of range for such rows), against one descriptor per
+    // operand - a load is then two instructions;
+    //   where accumulators and fragments leave no room for that, or a persistent launch would make the offsets again for
+    // every output tile (UNI), and the rows that successive loads of a wave cover
+    // (NW*RPI apart) share their swizzle phase: a lane's offset inside "its" row block is the same for every load, and the
+    // block - tile origin, wave, load index - goes into a descriptor per load, base advanced and size reduced by it.  That
+    // costs some ten scalar instructions a load, about 65 cycles of the issuing wave: a 64x64 tile of one wave needed
+    // 3050 cycles to issue the loads of its three stages, 2050 with the offsets in registers, and a k-tile of it 1390 instead
+    // of 860.
+    constexpr bool SAME_CHUNK = (SWZ == 0) || ((NW * RPI) % (CPR << (SWZ > 0 ? SWZ - 1 : 0))) == 0;
+    constexpr int WPS = (163840 / LDS_BYTES) * NW / 4;                     // waves per SIMD that LDS lets in: registers must not
+    constexpr int VGPRS = WPS >= 4 ? 128 : (WPS == 3 ? 168 : 256);         // keep any of them out
+    constexpr bool UNI = SAME_CHUNK && (PERS || TM * TN * ACC_N + 8 * (TM + TN) + LPT + 56 > VGPRS);
     constexpr bool UNI_A = UNI && OP == 0;
     const uint32_t lane_chunk = (uint32_t)((lpos ^ swz_of_row(wave * RPI + lrow)) * 16);
+    auto chunk_of = [&](int i) {                 // byte offset inside a row of the lane's chunk of load i
+        return SAME_CHUNK ? lane_chunk : (uint32_t)((lpos ^ swz_of_row((i * NW + wave) * RPI + lrow)) * 16);
+    };
     const uint32_t lane_offB = (uint32_t)lrow * (uint32_t)a.ldb * ES + lane_chunk;
     const uint32_t lane_offA = (uint32_t)lrow * (uint32_t)a.lda * ES + lane_chunk;
     uint32_t blkA = 0, blkB = 0;                 // byte offset of the wave's first row block of the issue-side tile
@@ -341,9 +363,9 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
     int issue_kt = 0;            // next k-tile (relative to kt0) of tile `itile` to fetch
 
     auto setup_issue = [&](int t) {
-        issue_alive = t < total;                      // past the last tile every fetch reads zeros
-        int bz, tile_m, tile_n;
-        tile_coords(issue_alive ? t : 0, bz, tile_m, tile_n);
+        issue_alive = !PERS || t < total;             // past the last tile every fetch reads zeros
+        int bz = c_bz, tile_m = c_tile_m, tile_n = c_tile_n;
+        if constexpr (PERS) tile_coords(issue_alive ? t : 0, bz, tile_m, tile_n);
         const int im0 = tile_m * BM, in0 = tile_n * BN;
         baseA = (const char*)a.A + (int64_t)bz * a.sA * ES;
         baseB = (const char*)a.B + (int64_t)bz * a.sB * ES;
@@ -352,10 +374,8 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
         } else {
 #pragma unroll
             for (int i = 0; i < B_LPW; ++i) {
-                const int row = (i * NW + wave) * RPI + lrow;
-                const int chunk = lpos ^ swz_of_row(row);
-                const int n = in0 + row;
-                voffB[i] = (n < a.N) ? (uint32_t)n * (uint32_t)a.ldb * ES + chunk * 16 : OOB;
+                const int n = in0 + (i * NW + wave) * RPI + lrow;
+                voffB[i] = (n < a.N) ? (uint32_t)n * (uint32_t)a.ldb * ES + chunk_of(i) : OOB;
             }
         }
         if constexpr (UNI_A) {
@@ -363,10 +383,8 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
         } else if constexpr (OP == 0) {
 #pragma unroll
             for (int i = 0; i < A_LPW; ++i) {
-                const int row = (i * NW + wave) * RPI + lrow;
-                const int chunk = lpos ^ swz_of_row(row);
-                const int m = im0 + row;
-                voffA[i] = (m < a.M) ? (uint32_t)m * (uint32_t)a.lda * ES + chunk * 16 : OOB;
+                const int m = im0 + (i * NW + wave) * RPI + lrow;
+                voffA[i] = (m < a.M) ? (uint32_t)m * (uint32_t)a.lda * ES + chunk_of(i) : OOB;
             }
         } else if constexpr (!CW) {
             static_assert(OP == 0 || CW || SWZ == 0 || ((NW * RPI) % (CPR << (SWZ > 0 ? SWZ - 1 : 0))) == 0,
@@ -449,10 +467,7 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
                     load_chunk_to_lds(block_rsrc(baseA, a_bytes, blkA, (uint32_t)a.lda * ES, i), sbase + (i * NW + wave) * 1024, v, ks_cur);
                 } else if constexpr (OP == 0) {
                     uint32_t v = voffA[i];
-                    if constexpr (RAG) {
-                        const int row = (i * NW + wave) * RPI + lrow;
-                        if (koff_rag + (uint32_t)((lpos ^ swz_of_row(row)) * 16) >= Kb) v = OOB;
-                    }
+                    if constexpr (RAG) { if (koff_rag + chunk_of(i) >= Kb) v = OOB; }
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, ks_cur);
                 } else if constexpr (!CW) {
                     int iy = iy0[i] + conv_iyr, ix = ix0[i] + conv_ixs;
@@ -470,10 +485,7 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
                     load_chunk_to_lds(block_rsrc(baseB, b_bytes, blkB, (uint32_t)a.ldb * ES, i), sbase + A_BYTES + (i * NW + wave) * 1024, v, ks_cur);
                 } else {
                     uint32_t v = voffB[i];
-                    if constexpr (RAG) {
-                        const int row = (i * NW + wave) * RPI + lrow;
-                        if (koff_rag + (uint32_t)((lpos ^ swz_of_row(row)) * 16) >= Kb) v = OOB;
-                    }
+                    if constexpr (RAG) { if (koff_rag + chunk_of(i) >= Kb) v = OOB; }
                     load_chunk_to_lds(rB_cur, sbase + A_BYTES + (i * NW + wave) * 1024, v, ks_cur);
                 }
             }
@@ -855,8 +867,8 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
 
     // ---- prologue: fill all stages, wait for tile 0 ----
     if constexpr (!PHASED) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) issue_tile(s);
+#pragma unroll 1
+        for (int s = 0; s < NS; ++s) issue_tile(s);           // (rolled: most of a short kernel is straight-line code run once)
         wait_and_barrier<(NS - 1) * LPT, 0>();
         read_frags(0, 0, 0);
     }
