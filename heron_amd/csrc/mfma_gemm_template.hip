@@ -257,8 +257,8 @@ __device__ __forceinline__ void sched_hint() {
 // transposed by a pass of its own that read and wrote all of it once more.  The MFMAs are issued with their operands
 // exchanged, so that a lane holds 4 consecutive pixels of one channel.
 //   EXPAND (conv): the input of a transposed convolution, HrnKArgs::expand_shift; the zeros are not in memory.
-//   NCHW transposed conv 16 x 56x56x64 -> 111x111x128, stride 2: 77 us with the passes around the kernel, 39 us without
-// (50 MB of result; 28 us of it the kernel, 26 us when it stores rows).
+//   NCHW transposed conv 16 x 56x56x64 -> 111x111x128, stride 2: 77 us with the passes around the kernel, 34 us without
+// (50 MB of result).
 template <bool CHW, bool EXPAND>
 __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
     __shared__ __attribute__((aligned(1024))) char lds[CHW ? CHW_LDS_BYTES : LDS_BYTES];
@@ -522,21 +522,45 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
         const int cpp = w_pitch / 16;                    // 16-byte chunks per pixel
         const int n_instr = (w_rows * cpp + 63) / 64;    // 1 KiB wave loads that cover the window
         const int gp0 = m0 - (a.cpad * a.W + a.cpad_w);  // input pixel index of window row 0
+        // A lane's chunk moves on by NW * 64 chunks from load to load.  Its window row and its position in the row (EXPAND:
+        // and the row's pixel) are divided out once and then carried: a division is some 40 instructions, and with three of
+        // them per load (and one per stored piece, see HOIST below) the transposed conv below took 38.0 us instead of 33.8.
+        const int d_row = NW * 64 / cpp, d_pos = NW * 64 - d_row * cpp;
+        int wrow = (wave * 64 + lane) / cpp, pos = wave * 64 + lane - wrow * cpp;
+        [[maybe_unused]] int w_img = 0, w_y = 0, w_x = 0, d_img = 0, d_y = 0, d_x = 0;
+        if constexpr (EXPAND) {
+            const int gp = gp0 + wrow;
+            w_img = gp / (a.H * a.W);
+            int rem = gp - w_img * (a.H * a.W);
+            if (rem < 0) { rem += a.H * a.W; --w_img; }
+            w_y = rem / a.W; w_x = rem - w_y * a.W;
+            d_img = d_row / (a.H * a.W);
+            const int d_rem = d_row - d_img * (a.H * a.W);
+            d_y = d_rem / a.W; d_x = d_rem - d_y * a.W;
+        }
         for (int q = wave; q < n_instr; q += NW) {
-            const int L = q * 64 + lane;
-            const int wrow = L / cpp, pos = L - wrow * cpp;
             const int src = (pos & ~(CPR - 1)) | ((pos & (CPR - 1)) ^ swz_of_row(wrow));
             const int gp = gp0 + wrow;
             int px = gp;                                     // pixel in memory
             bool ok = wrow < w_rows && gp >= 0;
             if constexpr (EXPAND) {
-                const int img = gp / (a.H * a.W), rem = gp - img * (a.H * a.W);
-                int y = rem / a.W, x = rem - y * a.W;
-                ok = ok && unexpand(y, x);
-                px = (img * in_h + y) * in_w + x;
+                int iy = w_y, ix = w_x;
+                ok = ok && unexpand(iy, ix);
+                px = (w_img * in_h + iy) * in_w + ix;
             }
             const uint32_t v = ok ? (uint32_t)px * (uint32_t)w_pitch + src * 16 : OOB;
             load_chunk_to_lds(rA, win + q * 1024, v, 0u);
+            pos += d_pos;
+            const int carry = pos >= cpp ? 1 : 0;
+            pos -= carry ? cpp : 0;
+            wrow += d_row + carry;
+            if constexpr (EXPAND) {                          // (each sum is less than twice its modulus)
+                w_x += d_x + carry;
+                w_y += d_y;
+                w_img += d_img;
+                if (w_x >= a.W) { w_x -= a.W; ++w_y; }
+                if (w_y >= a.H) { w_y -= a.H; ++w_img; }
+            }
         }
         // masks: pixel of fragment row i by one division, the following rows (MT further each) by carry
         const int hw = a.H * a.W;
@@ -708,6 +732,21 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
             typedef v4i piece_t __attribute__((aligned(2)));
             char* strip = epi + EPI_BASE + wave * (MT * CHW_PITCH);
             constexpr int CPRW = CSW * OES / 16, EPC = 16 / OES, IT = CSW / MT;
+            // where pixel m of the result lies: its image and its place in the plane.  Where a lane's pieces of a strip are the
+            // same pixels of other channels (HOIST), the division is made once per strip of pixels, not per piece
+            // (NCW conv1d 16 x 892 x 512 -> 512: 40.2 -> 38.2 us).
+            const unsigned plane = (unsigned)a.out_plane;
+            constexpr bool HOIST = 64 % CPRW == 0;
+            constexpr int NIB = HOIST ? TM / IT : 1;
+            unsigned h_img[NIB], h_px[NIB];
+            if constexpr (HOIST) {
+#pragma unroll
+                for (int b = 0; b < NIB; ++b) {
+                    const unsigned m = (unsigned)(m0 + wm_idx * WTM + b * CSW + (lane_e % CPRW) * EPC);
+                    h_img[b] = m / plane;
+                    h_px[b] = m - h_img[b] * plane;
+                }
+            }
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int nl = wn_idx * WTN + j * MT;
@@ -748,10 +787,12 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
                         const int m = m0 + wm_idx * WTM + ib * MT + cc2 * EPC;
                         if (c < MT * CPRW && n < a.N && m < a.M) {
                             const v4i val = *(const v4i*)(strip + row * CHW_PITCH + cc2 * 16);
-                            const unsigned plane = (unsigned)a.out_plane, img = (unsigned)m / plane, px = (unsigned)m - img * plane;
+                            const unsigned img = HOIST ? h_img[HOIST ? ib / IT : 0] : (unsigned)m / plane;
+                            const unsigned px = HOIST ? h_px[HOIST ? ib / IT : 0] : (unsigned)m - img * plane;
                             oel_t* dst = (oel_t*)a.C + ((int64_t)img * a.N + n) * plane + px;
                             if (px + EPC <= plane && m + EPC <= a.M) {
-                                put((piece_t*)dst, val);
+                                if constexpr (NTS) __builtin_nontemporal_store(val, (piece_t*)dst);
+                                else *(piece_t*)dst = val;
                             } else {
                                 const oel_t* ve = (const oel_t*)&val;
                                 unsigned p = px;

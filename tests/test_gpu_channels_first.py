@@ -37,12 +37,22 @@ class Ctx:
         pass
 
 
-@pytest.mark.parametrize("name", sorted(INSTANCES))
-def test_equals_the_separate_passes(name, hrn):
+# input windows whose position is carried from load to load: images smaller than a load's step, pixels of 24 chunks (no power of
+# two), one row or one column, a halo larger than the image, several images in a window
+WINDOW_CASES = [
+    ("t2d", [9, 2, 2, 64, 16, 1, 1, 2, 0, 1, 0]), ("t2d", [5, 1, 1, 64, 16, 3, 3, 2, 1, 1, 0]), ("t2d", [2, 9, 1, 192, 24, 3, 3, 4, 1, 1, 0]),
+    ("t2d", [3, 3, 11, 192, 64, 3, 3, 2, 1, 1, 0]), ("t2d", [40, 1, 2, 64, 8, 1, 1, 1, 0, 1, 0]), ("t2d", [1, 17, 15, 128, 64, 3, 3, 2, 1, 1, 0]),
+    ("c2d_nchw", [7, 3, 1, 192, 24, 3, 3, 1, 1, 1]), ("c2d_nchw", [2, 11, 13, 192, 64, 3, 3, 1, 1, 1]), ("c2d_nchw", [30, 1, 1, 64, 8, 5, 5, 1, 2, 1]),
+]
+
+
+@pytest.mark.parametrize("name,cases", [(n, CASES) for n in sorted(INSTANCES)] + [(n, WINDOW_CASES) for n in ("f16-window", "u8s8-window")],
+                         ids=sorted(INSTANCES) + ["f16-window-carry", "u8s8-window-carry"])
+def test_equals_the_separate_passes(name, cases, hrn):
     f16 = name.startswith("f16")
     mod = B.Module(INSTANCES[name])
     ran = 0
-    for op, args in CASES:
+    for op, args in cases:
         ctx = Ctx()
         getOpFromName(op)(ctx, *args, *(["float16"] * 2 if f16 else ["int8"] * 2))
         info, ref = ctx.info, ctx.info["reference_args"]
