@@ -169,6 +169,7 @@ SYMBOLS = {
     "hrn_launch_conv2d_nhwc_f16": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_bmm_u8s8": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_conv2d_nhwc_u8s8": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
+    "hrn_module_has_chw": (_i, [_vp]),
     "hrn_launch_conv2d_chw": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(ConvView), _vp, _vp, _vp, _vp]),
     "hrn_launch_splitk_static": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_repeat": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _i, _vp]),
@@ -378,6 +379,7 @@ class Module:
         _check(lib().hrn_build(ctypes.byref(desc), float(timeout_s), ctypes.byref(h)))
         self._h = h
         self.native = (h.value, ctypes.addressof(desc))      # what the functions of ext() take for this instance
+        self.has_chw = bool(lib().hrn_module_has_chw(h))     # launch_conv2d_chw takes it
         info = KernelInfo()
         _check(lib().hrn_module_info(self._h, ctypes.byref(info)))
         self.info = info.as_dict()

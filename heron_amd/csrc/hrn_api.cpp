@@ -128,6 +128,7 @@ uint64_t fnv1a_file(const std::string& p) {
 
 struct Derived {
     int es, oes, nw, cpr, rpi, a_lpw, b_lpw, lpt, ksb, ks, tm, tn, stage_bytes, lds, epi_bytes, chw_bytes;
+    bool has_chw;
 };
 
 // Structural constraints of the template; the same conditions are static_asserts in the kernel.
@@ -199,11 +200,14 @@ int derive(const hrn_kernel_desc* d, Derived* o) {
             r.lds = std::max(r.lds, r.epi_bytes);
         }
     }
-    // channels-first epilogue: strips of mfma channels x at most 64 pixels (whole MFMA tiles of the wave tile)
-    int csw = 1;
-    for (int t = 64 / d->mfma; t > 1; --t)
-        if (r.tm % t == 0) { csw = t; break; }
-    r.chw_bytes = base + r.nw * d->mfma * (csw * d->mfma * r.oes + 16);
+    // channels-first epilogue: strips of mfma channels x at most 64 pixels (whole MFMA tiles of the wave tile), as many as LDS
+    // holds beside what stays in it (a conv_window instance's stages)
+    const int stay = d->conv_window ? r.lds : 0;
+    auto chw = [&](int tiles) { return base + r.nw * d->mfma * (tiles * d->mfma * r.oes + 16); };
+    int tiles = 64 / d->mfma;
+    while (tiles > 1 && (r.tm % tiles || chw(tiles) + stay > 163840)) --tiles;
+    r.chw_bytes = chw(tiles);
+    r.has_chw = d->op == HRN_OP_CONV2D && !d->persistent && !d->split_k && r.chw_bytes + stay <= 163840;
     // (a conv_window instance keeps the epilogue region in its dynamic LDS, where the window was)
     if (r.lds > 163840) return fail(HRN_E_BADPARAM, "LDS %d > 163840", r.lds);
     if (d->swizzle && (r.cpr << (d->swizzle - 1)) > d->mfma)
@@ -1229,11 +1233,13 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
     memset(&m->info, 0, sizeof m->info);
     read_info(path.substr(0, path.size() - 6) + ".info", &m->info);
     m->info.threads = desc->wm * desc->wn * 64;
+    bool has_chw;
     {
         Derived dv;
         (void)derive(desc, &dv);        // compile_desc has validated the descriptor
         m->epi_bytes = dv.epi_bytes;
         m->chw_bytes = dv.chw_bytes;
+        has_chw = dv.has_chw;
     }
     hipError_t e = hipModuleLoad(&m->mod, path.c_str());
     if (e != hipSuccess) {
@@ -1246,7 +1252,7 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
         delete m;
         return fail(HRN_E_LOAD, "hipModuleGetFunction: %s", hipGetErrorString(e));
     }
-    if (desc->op == HRN_OP_CONV2D && !desc->persistent && !desc->split_k) {
+    if (has_chw) {
         e = hipModuleGetFunction(&m->fn_chw, m->mod, "hrn_mfma_kernel_chw");
         if (e == hipSuccess) e = hipModuleGetFunction(&m->fn_expand, m->mod, "hrn_mfma_kernel_chw_expand");
         if (e != hipSuccess) {
@@ -1321,10 +1327,12 @@ int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, con
     return launch(mod, p, In, Filter, Out, stream);
 }
 
+int hrn_module_has_chw(const hrn_module* mod) { return mod && mod->fn_chw ? 1 : 0; }
+
 int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn_conv_view* view, const void* In, const void* Filter,
                           void* Out, void* stream) {
     if (!mod || !p || !view) return fail(HRN_E_BADPARAM, "null argument");
-    if (!mod->fn_chw) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k");
+    if (!mod->fn_chw) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k whose strips fit into LDS");
     LaunchPlan plan;
     int rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);
     if (rc) return rc;
@@ -1332,11 +1340,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
         return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
     plan.fn = mod->fn_chw;
     plan.k.out_plane = view->out_plane;
-    if (mod->desc.conv_window) {
-        plan.dyn_lds = std::max(plan.dyn_lds, (unsigned)mod->chw_bytes);
-        if ((int)plan.dyn_lds + mod->info.lds_bytes > 163840)
-            return fail(HRN_E_BADPARAM, "conv2d_chw: epilogue of %d bytes + %d static LDS exceeds 163840", mod->chw_bytes, mod->info.lds_bytes);
-    }
+    if (mod->desc.conv_window) plan.dyn_lds = std::max(plan.dyn_lds, (unsigned)mod->chw_bytes);
     if (view->expand) {
         if (view->expand < 1 || (view->expand & (view->expand - 1)) || view->in_h < 1 || view->in_w < 1 || view->top < 0 || view->left < 0 ||
             ((int64_t)view->in_h - 1) * view->expand + view->top >= p->ch || ((int64_t)view->in_w - 1) * view->expand + view->left >= p->cw)

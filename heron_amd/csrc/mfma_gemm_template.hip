@@ -152,16 +152,18 @@ constexpr int LDS_BYTES = PERS ? NS * STAGE_BYTES + EPI_BYTES
                                : ((CW || NS * STAGE_BYTES > EPI_BYTES) ? NS * STAGE_BYTES : EPI_BYTES);
 constexpr int STORES_PER_TILE = (EPI >= 1) ? TM * ESPLIT * (MT * (SW * OES / 16) / 64) : 0;   // store instructions per wave per output tile
 static_assert(EPI >= 0 && EPI <= 2 && TN % ESPLIT == 0, "epilogue kind");
-// Channels-first epilogue (CHW kernels): strips of MT channels x CSW pixels (whole MFMA tiles, at most 64)
+// Channels-first epilogue (CHW kernels): strips of MT channels x CSW pixels (whole MFMA tiles, at most 64 pixels), as many as
+// LDS holds beside what stays in it (window mode: the stages)
 constexpr int chw_tiles() {
     for (int d = 64 / MT; d > 1; --d)
-        if (TM % d == 0) return d;
+        if (TM % d == 0 && EPI_BASE + NW * MT * (d * MT * OES + 16) + (CW ? NS * STAGE_BYTES : 0) <= 163840) return d;
     return 1;
 }
 constexpr int CSW = chw_tiles() * MT;
 constexpr int CHW_PITCH = CSW * OES + 16;
 constexpr int CHW_BYTES = EPI_BASE + NW * MT * CHW_PITCH;
 constexpr int CHW_LDS_BYTES = (CW || NS * STAGE_BYTES > CHW_BYTES) ? NS * STAGE_BYTES : CHW_BYTES;
+constexpr bool HAS_CHW = OP == 1 && !PERS && !SPLITK && CHW_BYTES + (CW ? NS * STAGE_BYTES : 0) <= 163840;
 
 static_assert(!PERS || (EPI >= 1 && !CW && !SPLITK && KS % 2 == 0), "persistent mode: staged epilogue, even k-steps");
 static_assert(!PERS || (NS - 2) * LPT + STORES_PER_TILE <= 63, "persistent mode: vmcnt range");
@@ -1203,6 +1205,12 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
     }
 }
 
+// a kernel that the instance has no room for is empty, and the host never launches it
+template <bool ROOM, bool CHW, bool EXPAND>
+__device__ __forceinline__ void body_if(const HrnKArgs& a) {
+    if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND>(a);
+}
+
 }  // namespace
 
 #if HRN_WPE > 0
@@ -1213,6 +1221,6 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
 
 HRN_ENTRY hrn_mfma_kernel(const HrnKArgs a) { hrn_mfma_body<false, false>(a); }
 #if HRN_OP == 1 && HRN_PERSIST == 0 && HRN_SPLITK == 0
-HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { hrn_mfma_body<true, false>(a); }
-HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { hrn_mfma_body<true, true>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { body_if<HAS_CHW, true, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { body_if<HAS_CHW, true, true>(a); }
 #endif

@@ -477,7 +477,7 @@ def run_operator(mod, info, inputs, group_m=8, split_k=0, constant=None, bsum=No
     adapter = info.get('adapter', 'identity')
     act, const, fin = ADAPTERS[adapter]
     Bm = const(info, *inputs) if constant is None else constant
-    if adapter in CHANNELS_FIRST and _native_ok(inputs[0]) and not (mod.desc.split_k or mod.desc.persistent):
+    if adapter in CHANNELS_FIRST and _native_ok(inputs[0]) and mod.has_chw:
         return _run_channels_first(mod, info, inputs, act, Bm, group_m, bsum)
     A = act(info, *inputs)
     if info['operator'] == 'conv2d_nhwc':

@@ -123,6 +123,11 @@ def int8_conv_descs():
     ]
 
 
+def chw_room_descs():
+    """A window instance whose channels-first strips of 64 pixels would not fit into LDS beside its stages."""
+    return [D(U8, CONV, 256, 256, 64, 4, 4, 32, 2, 1, win=1)]
+
+
 def persistent_descs():
     """Instances of the persistent (tile-stream) mode in the parity suite: short and long K streams, both element
     kinds, 2..4 stages, implicit-GEMM conv."""
@@ -156,8 +161,8 @@ BEST = {
 
 def all_shipped():
     seen, out = set(), []
-    for d in (parity_descs() + variant_descs() + int8_conv_descs() + persistent_descs() + persistent_twin_descs() + splitk_descs()
-              + list(BEST.values())):
+    for d in (parity_descs() + variant_descs() + int8_conv_descs() + chw_room_descs() + persistent_descs() + persistent_twin_descs()
+              + splitk_descs() + list(BEST.values())):
         if d.as_tuple() not in seen:
             seen.add(d.as_tuple())
             out.append(d)

@@ -219,12 +219,14 @@ int hrn_launch_splitk_static(const hrn_module* mod, const hrn_problem* p, const 
  * out_plane is ho*wo for (n, co, ho, wo), and do*ho*wo where do successive images are the slices of a volume.
  *   expand > 0 (a power of two): the problem's ch x cw input is not in memory; In holds (cn, in_h, in_w, ci), pixel (y, x)
  * of which stands at (top + y*expand, left + x*expand) of ch x cw, everything else is zero.
- * The instance is a conv2d one without persistent and split_k; p->ldc does not apply.
+ * The instance is a conv2d one for which hrn_module_has_chw says 1: not persistent, no split_k, and the strips of its
+ * epilogue fit into LDS; p->ldc does not apply.
  */
 typedef struct hrn_conv_view {
     int32_t out_plane;
     int32_t expand, in_h, in_w, top, left;
 } hrn_conv_view;
+int hrn_module_has_chw(const hrn_module* mod);
 int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn_conv_view* view, const void* In,
                           const void* Filter, void* Out, void* stream);
 
