@@ -49,8 +49,10 @@ struct hrn_module {
     hrn_kernel_desc desc;
     hrn_kernel_info info;
     hipModule_t mod;
-    hipFunction_t fn;
-    hipFunction_t fn_chw, fn_expand;   // conv2d: the kernels of hrn_launch_conv2d_chw (null where the instance has none)
+    // the instance's kernels, each plain and deep (a third stage); null where it has none or no room for it
+    hipFunction_t fn[2];
+    hipFunction_t fn_chw[2], fn_expand[2];   // conv2d: those of hrn_launch_conv2d_chw
+    int deep_grid;      // workgroups of the deep kernels that the device holds at once
     std::string path;
     int persist_grid;   // persistent instances: workgroups that fit the device at once (multiple of 8 when >= 8)
     int epi_bytes;      // LDS bytes of the epilogue region (column sums + strips)
@@ -127,8 +129,8 @@ uint64_t fnv1a_file(const std::string& p) {
 }
 
 struct Derived {
-    int es, oes, nw, cpr, rpi, a_lpw, b_lpw, lpt, ksb, ks, tm, tn, stage_bytes, lds, epi_bytes, chw_bytes;
-    bool has_chw;
+    int es, oes, nw, cpr, rpi, a_lpw, b_lpw, lpt, ksb, ks, tm, tn, stage_bytes, lds, epi_bytes, chw_bytes, deep_lds;
+    bool has_chw, has_deep;
 };
 
 // Structural constraints of the template; the same conditions are static_asserts in the kernel.
@@ -207,6 +209,9 @@ int derive(const hrn_kernel_desc* d, Derived* o) {
     int tiles = 64 / d->mfma;
     while (tiles > 1 && (r.tm % tiles || chw(tiles) + stay > 163840)) --tiles;
     r.chw_bytes = chw(tiles);
+    // deep kernels: a third stage
+    r.deep_lds = std::max(std::max(r.lds, r.chw_bytes), 3 * r.stage_bytes);
+    r.has_deep = d->stages == 2 && !d->conv_window && !d->persistent && 3 * r.stage_bytes <= 163840 && 2 * r.lpt <= 63;
     r.has_chw = d->op == HRN_OP_CONV2D && !d->persistent && !d->split_k && r.chw_bytes + stay <= 163840;
     // (a conv_window instance keeps the epilogue region in its dynamic LDS, where the window was)
     if (r.lds > 163840) return fail(HRN_E_BADPARAM, "LDS %d > 163840", r.lds);
@@ -374,6 +379,7 @@ void read_info(const std::string& path, hrn_kernel_info* o) {
 // What one launch consists of: the template kernel and, for a split-K instance, the pass that adds the K slices.
 struct LaunchPlan {
     HrnKArgs k;
+    bool deep;                 // the deep kernel of the instance
     hipFunction_t fn;
     unsigned grid, dyn_lds;
     int split;                 // K slices the grid covers (1 = the kernel writes C itself)
@@ -393,12 +399,22 @@ void split_shape(const hrn_kernel_desc& d, const hrn_problem* p, int* kt_per_sli
     *split = (kt_all + *kt_per_slice - 1) / *kt_per_slice;
 }
 
+// Two stages leave a k-tile's loads one k-tile of multiplication to arrive, enough from a near L2 but not from further away; two
+// stages were chosen so that several workgroups fit a CU, and a grid that the device holds at once with three has no other use
+// for that LDS.  128x128 fp16, 9 x 12 tiles, inputs of three calls in turn: 41.9 -> 33.8 us at 64 k-tiles, 16.3 -> 14.0 at 15,
+// 8.7 -> 8.9 at 4; 4 x 4 tiles 30.4 -> 22.5 at 40, 12.9 -> 13.0 at 20 (2.6 MB of operands).  The first tiles take 0.2 us longer per
+// stage (they are accepted at the L1's rate before the first product), so fewer than 6 k-tiles or 2 MB lose; four and five stages
+// are 1 - 4 % behind three, and instances that have three already lose 3 - 8 % with more.
+bool deep_fits(const hrn_module* mod, int64_t grid, int k_tiles, int64_t operand_bytes) {
+    return mod->fn[1] && grid <= mod->deep_grid && k_tiles >= 6 && operand_bytes >= (2 << 20);
+}
+
 int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
               size_t workspace_bytes, LaunchPlan* plan) {
     HrnKArgs* k = &plan->k;
     plan->dyn_lds = 0;
     plan->split = 1;
-    plan->fn = mod ? mod->fn : nullptr;
+    plan->deep = false;
     if (!mod || !p || !A || !B || !C) return fail(HRN_E_BADPARAM, "null argument");
     const hrn_kernel_desc& d = mod->desc;
     if (p->op != d.op) return fail(HRN_E_BADPARAM, "problem op %d does not match module op %d", p->op, d.op);
@@ -481,6 +497,11 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     }
     if (total <= 0 || total >= (1ll << 31)) return fail(HRN_E_BADPARAM, "grid size");
     plan->grid = (unsigned)total;
+    const int64_t b_bytes = (int64_t)p->n * p->k * es;
+    const int64_t a_bytes = d.op == HRN_OP_GEMM ? (int64_t)p->m * p->k * es : (int64_t)p->cn * p->ch * p->cw * p->ci * es;
+    plan->deep = deep_fits(mod, total, d.split_k ? k->kt_per_slice : (int)(((int64_t)p->k * es + d.bkb - 1) / d.bkb),
+                           p->batch * (a_bytes + b_bytes));
+    plan->fn = mod->fn[plan->deep];
     if (d.persistent) {
         if ((int64_t)p->n * oes % 16) return fail(HRN_E_BADPARAM, "persistent instances store whole 16-byte chunks: N*%d must be a multiple of 16", oes);
         if ((int64_t)p->m * p->ldc * oes >= (1ll << 31)) return fail(HRN_E_BADPARAM, "persistent: C exceeds 2 GiB per batch entry");
@@ -1233,34 +1254,39 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
     memset(&m->info, 0, sizeof m->info);
     read_info(path.substr(0, path.size() - 6) + ".info", &m->info);
     m->info.threads = desc->wm * desc->wn * 64;
-    bool has_chw;
+    Derived dv;
     {
-        Derived dv;
         (void)derive(desc, &dv);        // compile_desc has validated the descriptor
         m->epi_bytes = dv.epi_bytes;
         m->chw_bytes = dv.chw_bytes;
-        has_chw = dv.has_chw;
     }
     hipError_t e = hipModuleLoad(&m->mod, path.c_str());
     if (e != hipSuccess) {
         delete m;
         return fail(HRN_E_LOAD, "hipModuleLoad(%s): %s", path.c_str(), hipGetErrorString(e));
     }
-    e = hipModuleGetFunction(&m->fn, m->mod, "hrn_mfma_kernel");
+    const std::string kernel = "hrn_mfma_kernel";
+    const bool deep = dv.has_deep;
+    auto get = [&](hipFunction_t* f, const std::string& name) {
+        if (e == hipSuccess) e = hipModuleGetFunction(f, m->mod, name.c_str());
+    };
+    get(&m->fn[0], kernel);
+    if (deep) get(&m->fn[1], kernel + "_deep");
+    if (dv.has_chw) {
+        get(&m->fn_chw[0], kernel + "_chw");
+        get(&m->fn_expand[0], kernel + "_chw_expand");
+        if (deep) get(&m->fn_chw[1], kernel + "_chw_deep");
+        if (deep) get(&m->fn_expand[1], kernel + "_chw_expand_deep");
+    }
+    int dev = 0, cus = 0;
+    if (deep && e == hipSuccess) e = hipGetDevice(&dev);
+    if (deep && e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess) {
         (void)hipModuleUnload(m->mod);
         delete m;
         return fail(HRN_E_LOAD, "hipModuleGetFunction: %s", hipGetErrorString(e));
     }
-    if (has_chw) {
-        e = hipModuleGetFunction(&m->fn_chw, m->mod, "hrn_mfma_kernel_chw");
-        if (e == hipSuccess) e = hipModuleGetFunction(&m->fn_expand, m->mod, "hrn_mfma_kernel_chw_expand");
-        if (e != hipSuccess) {
-            (void)hipModuleUnload(m->mod);
-            delete m;
-            return fail(HRN_E_LOAD, "hipModuleGetFunction: %s", hipGetErrorString(e));
-        }
-    }
+    m->deep_grid = deep ? cus * (163840 / dv.deep_lds) : 0;
     if (desc->split_k) {
         // hrn_launch_splitk_static finds the library's workspace of this device looked up already
         void* ws = nullptr;
@@ -1271,7 +1297,7 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
     if (desc->persistent) {
         int per_cu = 0, dev = 0;
         hipDeviceProp_t pr;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->fn, m->info.threads, 0) != hipSuccess || per_cu < 1 ||
+        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->fn[0], m->info.threads, 0) != hipSuccess || per_cu < 1 ||
             hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&pr, dev) != hipSuccess) {
             (void)hipModuleUnload(m->mod);
             delete m;
@@ -1327,18 +1353,18 @@ int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, con
     return launch(mod, p, In, Filter, Out, stream);
 }
 
-int hrn_module_has_chw(const hrn_module* mod) { return mod && mod->fn_chw ? 1 : 0; }
+int hrn_module_has_chw(const hrn_module* mod) { return mod && mod->fn_chw[0] ? 1 : 0; }
 
 int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn_conv_view* view, const void* In, const void* Filter,
                           void* Out, void* stream) {
     if (!mod || !p || !view) return fail(HRN_E_BADPARAM, "null argument");
-    if (!mod->fn_chw) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k whose strips fit into LDS");
+    if (!mod->fn_chw[0]) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k whose strips fit into LDS");
     LaunchPlan plan;
     int rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);
     if (rc) return rc;
     if (view->out_plane < 1 || p->m % view->out_plane)
         return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
-    plan.fn = mod->fn_chw;
+    plan.fn = mod->fn_chw[plan.deep];
     plan.k.out_plane = view->out_plane;
     if (mod->desc.conv_window) plan.dyn_lds = std::max(plan.dyn_lds, (unsigned)mod->chw_bytes);
     if (view->expand) {
@@ -1346,7 +1372,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
             ((int64_t)view->in_h - 1) * view->expand + view->top >= p->ch || ((int64_t)view->in_w - 1) * view->expand + view->left >= p->cw)
             return fail(HRN_E_BADPARAM, "conv2d_chw: %d x %d pixels, %d apart (a power of two) from (%d, %d), do not lie in %d x %d",
                         view->in_h, view->in_w, view->expand, view->top, view->left, p->ch, p->cw);
-        plan.fn = mod->fn_expand;
+        plan.fn = mod->fn_expand[plan.deep];
         plan.k.in_h = view->in_h; plan.k.in_w = view->in_w;
         plan.k.top = view->top; plan.k.left = view->left;
         plan.k.expand_shift = __builtin_ctz((unsigned)view->expand);

@@ -183,6 +183,11 @@ static_assert(DT == 0 || NS * STAGE_BYTES >= WM * BN * 4, "column sums must fit 
 constexpr bool PHASED = OP == 0 && BM == 256 && BN == 256 && BKB == 128 && NS == 2 && NW == 8 && (WM == 2 || WM == 4) &&
                         !PERS && !SPLITK && (DT == 0 || COLSUM);
 
+// Deep kernels: an instance of two stages with a third one, for launches that leave its LDS free anyway and whose operands do
+// not come from a near L2 (hrn_api.cpp, deep_fits).
+constexpr int DEEP_NS = 3;
+constexpr bool HAS_DEEP = NS == 2 && !CW && !PERS && DEEP_NS * STAGE_BYTES <= 163840 && (DEEP_NS - 1) * LPT <= 63;
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
@@ -261,9 +266,13 @@ __device__ __forceinline__ void sched_hint() {
 //   EXPAND (conv): the input of a transposed convolution, HrnKArgs::expand_shift; the zeros are not in memory.
 //   NCHW transposed conv 16 x 56x56x64 -> 111x111x128, stride 2: 77 us with the passes around the kernel, 34 us without
 // (50 MB of result).
-template <bool CHW, bool EXPAND>
+//   DEEP: three stages instead of HRN_STAGES.
+template <bool CHW, bool EXPAND, bool DEEP>
 __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
-    __shared__ __attribute__((aligned(1024))) char lds[CHW ? CHW_LDS_BYTES : LDS_BYTES];
+    constexpr int NS = DEEP ? DEEP_NS : HRN_STAGES;
+    constexpr int OWN_LDS = CHW ? CHW_LDS_BYTES : LDS_BYTES;
+    constexpr int KERNEL_LDS = (DEEP && NS * STAGE_BYTES > OWN_LDS) ? NS * STAGE_BYTES : OWN_LDS;
+    __shared__ __attribute__((aligned(1024))) char lds[KERNEL_LDS];
     extern __shared__ __attribute__((aligned(1024))) char win[];   // window mode: input window, later the epilogue region
 
     // every argument the start of the kernel needs, fetched at once: left to itself the compiler reads them where they are
@@ -345,7 +354,7 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
     // 3050 cycles to issue the loads of its three stages, 2050 with the offsets in registers, and a k-tile of it 1390 instead
     // of 860.
     constexpr bool SAME_CHUNK = (SWZ == 0) || ((NW * RPI) % (CPR << (SWZ > 0 ? SWZ - 1 : 0))) == 0;
-    constexpr int WPS = (163840 / LDS_BYTES) * NW / 4;                     // waves per SIMD that LDS lets in: registers must not
+    constexpr int WPS = (163840 / (DEEP ? KERNEL_LDS : LDS_BYTES)) * NW / 4;                     // waves per SIMD that LDS lets in: registers must not
     constexpr int VGPRS = WPS >= 4 ? 128 : (WPS == 3 ? 168 : 256);         // keep any of them out
     constexpr bool UNI = SAME_CHUNK && (PERS || TM * TN * ACC_N + 8 * (TM + TN) + LPT + 56 > VGPRS);
     constexpr bool UNI_A = UNI && OP == 0;
@@ -1206,9 +1215,9 @@ __device__ __forceinline__ void hrn_mfma_body(const HrnKArgs& a) {
 }
 
 // a kernel that the instance has no room for is empty, and the host never launches it
-template <bool ROOM, bool CHW, bool EXPAND>
+template <bool ROOM, bool CHW, bool EXPAND, bool DEEP>
 __device__ __forceinline__ void body_if(const HrnKArgs& a) {
-    if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND>(a);
+    if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND, DEEP>(a);
 }
 
 }  // namespace
@@ -1219,8 +1228,11 @@ __device__ __forceinline__ void body_if(const HrnKArgs& a) {
 #define HRN_ENTRY extern "C" __global__ void __launch_bounds__(NT)
 #endif
 
-HRN_ENTRY hrn_mfma_kernel(const HrnKArgs a) { hrn_mfma_body<false, false>(a); }
-#if HRN_OP == 1 && HRN_PERSIST == 0 && HRN_SPLITK == 0
-HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { body_if<HAS_CHW, true, false>(a); }
-HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { body_if<HAS_CHW, true, true>(a); }
+HRN_ENTRY hrn_mfma_kernel(const HrnKArgs a) { hrn_mfma_body<false, false, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_deep(const HrnKArgs a) { body_if<HAS_DEEP, false, false, true>(a); }
+#if HRN_OP == 1
+HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { body_if<HAS_CHW, true, false, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_deep(const HrnKArgs a) { body_if<HAS_CHW && HAS_DEEP, true, false, true>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { body_if<HAS_CHW, true, true, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand_deep(const HrnKArgs a) { body_if<HAS_CHW && HAS_DEEP, true, true, true>(a); }
 #endif
