@@ -711,25 +711,64 @@ __global__ void __launch_bounds__(256) probe_copy_kernel(const pv4i* __restrict_
     for (; i < n16; i += stride) dst[i] = src[i];
 }
 
-// One lane per row: copies `c` elements of ES bytes and zero-fills up to `cp` elements, writing whole 16-byte words.
-template <int ES>
-__global__ void __launch_bounds__(256) pad_rows_kernel(const unsigned char* __restrict__ src, unsigned char* __restrict__ dst,
-                                                       size_t rows, int c, int cp) {
-    const size_t row = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= rows) return;
-    const unsigned char* in = src + row * (size_t)c * ES;
-    pv4i* out = (pv4i*)(dst + row * (size_t)cp * ES);
-    const int words = cp * ES / 16, live = c * ES;
-    for (int w = 0; w < words; ++w) {
-        unsigned int q[4] = {0u, 0u, 0u, 0u};
-        for (int b = 0; b < 16; b += ES) {
-            const int at = w * 16 + b;
-            if (at < live) {
-                const unsigned int v = ES == 2 ? (unsigned int)*(const unsigned short*)(in + at) : (unsigned int)in[at];
-                q[b / 4] |= v << (8 * (b % 4));
+template <int ES> struct ElemWord;          // an element, and 16 bytes of them at any element's address
+template <> struct ElemWord<1> { using T = unsigned char; typedef pv4i Piece __attribute__((aligned(1))); };
+template <> struct ElemWord<2> { using T = unsigned short; typedef pv4i Piece __attribute__((aligned(2))); };
+template <> struct ElemWord<4> { using T = unsigned int; typedef pv4i Piece __attribute__((aligned(4))); };
+
+// 16 bytes moved down by `bytes` < 16, zeros from above; and their first `bytes` <= 16 alone
+__device__ __forceinline__ pv4i drop_front(pv4i v, int bytes) {
+    unsigned long long q[2];
+    __builtin_memcpy(q, &v, 16);
+    const int sh = 8 * bytes;
+    if (sh >= 64) { q[0] = q[1] >> (sh - 64); q[1] = 0ull; }
+    else if (sh > 0) { q[0] = q[0] >> sh | q[1] << (64 - sh); q[1] >>= sh; }
+    __builtin_memcpy(&v, q, 16);
+    return v;
+}
+__device__ __forceinline__ pv4i keep_front(pv4i v, int bytes) {
+    unsigned long long q[2];
+    __builtin_memcpy(q, &v, 16);
+    if (bytes < 8) q[0] &= (1ull << (8 * bytes)) - 1;
+    if (bytes <= 8) q[1] = 0ull;
+    else if (bytes < 16) q[1] &= (1ull << (8 * bytes - 64)) - 1;
+    __builtin_memcpy(&v, q, 16);
+    return v;
+}
+
+// Rows of `c` elements copied into rows of `words` 16-byte words, zeros behind them: a lane per word, read with one 16-byte
+// access at whatever element it starts (what follows the row in memory is masked off; at the end of the last row the
+// access is moved back and its result down).  Bound by memory, below some 10 MB by the launch.  A lane used to copy a whole row
+// element by element, far apart from its neighbours' rows: fp16 8192 x 8191 3746 us, 46.5 us like this (5.8 TB/s);
+// 370 x 214 31.4 and 2.2 us, 401408 x 20 -> 24 19.5 and 6.9 us.
+template <int ES, typename IDX>
+__global__ void __launch_bounds__(256) pad_rows_kernel(const unsigned char* __restrict__ src, pv4i* __restrict__ dst, IDX total,
+                                                       IDX words, int c, int64_t elems) {
+    using Piece = typename ElemWord<ES>::Piece;
+    constexpr int V = 16 / ES;
+    for (IDX t = (IDX)blockIdx.x * 256 + threadIdx.x; t < total; t += (IDX)gridDim.x * 256) {
+        const IDX row = t / words;
+        const int at = (int)(t - row * words) * V;                      // element of the row the word starts with
+        const int live = min(max(c - at, 0), V);
+        const int64_t e = (int64_t)row * c + at, past = e + V - elems;  // elements by which the access passes the end
+        pv4i v = {0, 0, 0, 0};
+        if (live > 0) {
+            if (past <= 0) {
+                v = keep_front(*(const Piece*)(src + e * ES), live * ES);
+            } else if (elems >= V) {
+                v = keep_front(drop_front(*(const Piece*)(src + (elems - V) * ES), (int)past * ES), live * ES);
+            } else {                                                    // fewer elements than one access reads
+                unsigned long long q[2] = {0ull, 0ull};
+                for (int i = live - 1; i >= 0; --i) {
+                    unsigned long long x = 0;
+                    __builtin_memcpy(&x, src + (e + i) * ES, ES);
+                    q[1] = q[1] << (8 * ES) | q[0] >> (64 - 8 * ES);
+                    q[0] = q[0] << (8 * ES) | x;
+                }
+                __builtin_memcpy(&v, q, 16);
             }
         }
-        out[w] = pv4i{(int)q[0], (int)q[1], (int)q[2], (int)q[3]};
+        dst[t] = v;
     }
 }
 
@@ -817,11 +856,6 @@ __global__ void __launch_bounds__(256) gather_nd_kernel(const hrn_gather g, cons
 // Bound by memory.  16 x (512 x 892) fp16, 29 MB moved: 11.1 us with one element per lane through a 64 x 64 LDS tile,
 // 7.6 us like this (3.8 TB/s); 16 x (12321 x 128), odd row lengths, 101 MB: 48.8 and 31.3 us.  Rows need not be aligned: the
 // hardware takes 16-byte accesses at any element.
-template <int ES> struct ElemWord;          // an element, and 16 bytes of them at any element's address
-template <> struct ElemWord<1> { using T = unsigned char; typedef pv4i Piece __attribute__((aligned(1))); };
-template <> struct ElemWord<2> { using T = unsigned short; typedef pv4i Piece __attribute__((aligned(2))); };
-template <> struct ElemWord<4> { using T = unsigned int; typedef pv4i Piece __attribute__((aligned(4))); };
-
 template <int ES>
 __device__ __forceinline__ void store_piece(typename ElemWord<ES>::T* p, pv4i v, int n) {
     if (n >= 16 / ES) { *(typename ElemWord<ES>::Piece*)p = v; return; }
@@ -858,15 +892,7 @@ __global__ void __launch_bounds__(256) transpose_pad_kernel(const void* __restri
         }
         if (lack) {
 #pragma unroll
-            for (int i = 0; i < V; ++i) {
-                unsigned long long q[2];
-                __builtin_memcpy(q, &x[i], 16);
-                const int sh = 8 * ES * lack;
-                q[0] = sh >= 64 ? q[1] >> (sh - 64) : q[0] >> sh | q[1] << (64 - sh);
-                __builtin_memcpy(&x[i], q, 8);
-                q[1] = sh >= 64 ? 0ull : q[1] >> sh;
-                __builtin_memcpy((char*)&x[i] + 8, &q[1], 8);
-            }
+            for (int i = 0; i < V; ++i) x[i] = drop_front(x[i], lack * ES);
         }
     } else {
         unsigned long long q[V][2];
@@ -963,10 +989,16 @@ int hrn_pad_rows(const void* src, void* dst, size_t rows, int c, int cp, int ele
     if (!src || !dst || c < 1 || cp < c || (elem_bytes != 1 && elem_bytes != 2) || (cp * elem_bytes) % 16 || rows > ((size_t)1 << 40))
         return fail(HRN_E_BADPARAM, "pad_rows: %d -> %d elements of %d bytes (the padded row must be whole 16-byte words)", c, cp, elem_bytes);
     if (rows == 0) return HRN_OK;
-    const unsigned grid = (unsigned)((rows + 255) / 256);
+    const int64_t words = (int64_t)cp * elem_bytes / 16, total = (int64_t)rows * words, elems = (int64_t)rows * c;
+    const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 1 << 22);
     hipStream_t st = (hipStream_t)stream;
-    if (elem_bytes == 2) pad_rows_kernel<2><<<grid, 256, 0, st>>>((const unsigned char*)src, (unsigned char*)dst, rows, c, cp);
-    else pad_rows_kernel<1><<<grid, 256, 0, st>>>((const unsigned char*)src, (unsigned char*)dst, rows, c, cp);
+    auto run = [&](auto kernel, auto idx) {
+        using IDX = decltype(idx);
+        kernel<<<grid, 256, 0, st>>>((const unsigned char*)src, (pv4i*)dst, (IDX)total, (IDX)words, c, elems);
+    };
+    const bool narrow = total < (1ll << 31);
+    if (elem_bytes == 2) narrow ? run(pad_rows_kernel<2, uint32_t>, uint32_t()) : run(pad_rows_kernel<2, uint64_t>, uint64_t());
+    else narrow ? run(pad_rows_kernel<1, uint32_t>, uint32_t()) : run(pad_rows_kernel<1, uint64_t>, uint64_t());
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(HRN_E_LAUNCH, "pad_rows: %s", hipGetErrorString(e));
     return HRN_OK;
