@@ -409,6 +409,13 @@ bool deep_fits(const hrn_module* mod, int64_t grid, int k_tiles, int64_t operand
     return mod->fn[1] && grid <= mod->deep_grid && k_tiles >= 6 && operand_bytes >= (2 << 20);
 }
 
+// Extent of a convolution's result in one direction, 0 where the dilated filter is larger than the padded input: the division
+// truncates, so a numerator between -stride and 0 would count as one position.
+int conv_extent(int in, int k, int stride, int pad, int dil) {
+    const int64_t room = (int64_t)in - ((int64_t)(k - 1) * dil + 1) + 2 * (int64_t)pad;
+    return stride < 1 || room < 0 ? 0 : (int)(room / stride) + 1;
+}
+
 int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
               size_t workspace_bytes, LaunchPlan* plan) {
     HrnKArgs* k = &plan->k;
@@ -448,8 +455,8 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         if (p->cstride < 1 || p->cdil < 1 || p->cpad < 0 || p->cstride_w < 1 || p->cdil_w < 1 || p->cpad_w < 0)
             return fail(HRN_E_BADPARAM, "conv stride/pad/dilation (height %d/%d/%d, width %d/%d/%d)", p->cstride, p->cpad,
                         p->cdil, p->cstride_w, p->cpad_w, p->cdil_w);
-        const int ho = (p->ch - ((p->kh - 1) * p->cdil + 1) + 2 * p->cpad) / p->cstride + 1;
-        const int wo = (p->cw - ((p->kw - 1) * p->cdil_w + 1) + 2 * p->cpad_w) / p->cstride_w + 1;
+        const int ho = conv_extent(p->ch, p->kh, p->cstride, p->cpad, p->cdil);
+        const int wo = conv_extent(p->cw, p->kw, p->cstride_w, p->cpad_w, p->cdil_w);
         if (ho <= 0 || wo <= 0) return fail(HRN_E_BADPARAM, "conv output is empty");
         if (p->m != p->cn * ho * wo || p->n != p->co || p->k != p->kh * p->kw * p->ci)
             return fail(HRN_E_BADPARAM, "conv GEMM view (m,n,k)=(%d,%d,%d) inconsistent with the image shape", p->m, p->n, p->k);
@@ -1617,8 +1624,8 @@ void hrn_problem_conv2d_hw(hrn_problem* p, int n, int h, int w, int ci, int co, 
     p->cn = n; p->ch = h; p->cw = w; p->ci = ci; p->co = co; p->kh = kh; p->kw = kw;
     p->cstride = stride_h; p->cpad = pad_h; p->cdil = dil_h;
     p->cstride_w = stride_w; p->cpad_w = pad_w; p->cdil_w = dil_w;
-    const int ho = (stride_h > 0) ? (h - ((kh - 1) * dil_h + 1) + 2 * pad_h) / stride_h + 1 : 0;
-    const int wo = (stride_w > 0) ? (w - ((kw - 1) * dil_w + 1) + 2 * pad_w) / stride_w + 1 : 0;
+    const int ho = conv_extent(h, kh, stride_h, pad_h, dil_h);
+    const int wo = conv_extent(w, kw, stride_w, pad_w, dil_w);
     p->m = n * ho * wo; p->n = co; p->k = kh * kw * ci;
     p->lda = ci; p->ldb = p->k; p->ldc = co;
     p->group_m = 8;

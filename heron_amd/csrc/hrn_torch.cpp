@@ -164,9 +164,9 @@ PyObject* conv2d(PyObject*, PyObject* const* args, Py_ssize_t n) {
         hrn_problem_conv2d_hw(&p, (int)X->size(0), (int)X->size(1), (int)X->size(2), (int)X->size(3), (int)W->size(0), (int)W->size(1),
                               (int)W->size(2), (int)sh, (int)sw, (int)ph, (int)pw, (int)dh, (int)dw);
         p.group_m = (int32_t)v[0];
-        const int64_t ho = (X->size(1) - ((W->size(1) - 1) * dh + 1) + 2 * ph) / sh + 1;
-        const int64_t wo = (X->size(2) - ((W->size(2) - 1) * dw + 1) + 2 * pw) / sw + 1;
-        if (ho < 1 || wo < 1) Py_RETURN_NONE;
+        const int64_t room_h = X->size(1) - ((W->size(1) - 1) * dh + 1) + 2 * ph, room_w = X->size(2) - ((W->size(2) - 1) * dw + 1) + 2 * pw;
+        if (room_h < 0 || room_w < 0) Py_RETURN_NONE;           // (before the division, which truncates)
+        const int64_t ho = room_h / sh + 1, wo = room_w / sw + 1;
         at::Tensor C;
         if (args[9] != Py_None) {
             if (!tensor(args[9])) Py_RETURN_NONE;

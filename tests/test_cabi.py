@@ -93,6 +93,10 @@ def test_problem_helpers():
     assert (c.m, c.n, c.k) == (32 * 56 * 56, 64, 576)
     c = B.conv2d_problem(1, 15, 15, 8, 16, 3, 3, 2, 1, 1)
     assert c.m == 8 * 8
+    # a filter larger than the padded input has no position, also where it is so by less than the stride
+    for h, w, k, s, pad, dil in ((4, 4, 5, 2, 0, 1), (4, 9, 5, 2, 0, 1), (9, 4, 5, 3, 0, 1), (2, 2, 5, 4, 1, 1), (4, 4, 3, 3, 0, 2), (1, 1, 5, 2, 0, 1)):
+        assert B.conv2d_problem(2, h, w, 64, 8, k, k, s, pad, dil).m == 0
+    assert B.conv2d_problem(2, 5, 5, 64, 8, 5, 5, 2, 0, 1).m == 2
 
 
 def test_compile_without_gpu_and_shipped_instances_present():

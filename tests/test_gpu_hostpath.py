@@ -1,0 +1,36 @@
+"""What the native host path of hostops hands back or refuses, beside the plain calls the parity tests make."""
+import pytest
+import torch
+
+from heron_amd import backend as B
+from heron_amd import hostops, instances
+from heron_amd.ops.rocm import getOpFromName
+
+pytestmark = pytest.mark.gpu
+
+D, F16, U8, GEMM, CONV = instances.D, instances.F16, instances.U8, instances.GEMM, instances.CONV
+CONV_F16 = D(F16, CONV, *instances.PARITY_SHAPES[2])
+
+
+def half(*shape):
+    return torch.ones(shape, device="cuda", dtype=torch.float16)
+
+
+# the dilated filter is larger than the padded input by less than the stride, by the stride and by more than it; in one direction
+@pytest.mark.parametrize("h,w,k,stride,pad,dil", [(4, 4, 5, 2, 0, 1), (4, 9, 5, 2, 0, 1), (9, 4, 5, 2, 0, 1), (3, 3, 5, 2, 0, 1), (1, 1, 5, 2, 0, 1),
+                                                  (4, 4, 3, 3, 0, 2), (2, 2, 5, 4, 1, 1)])
+def test_filter_larger_than_the_input_is_refused(h, w, k, stride, pad, dil, hrn):
+    mod = B.Module(CONV_F16)
+    X, W = half(2, h, w, 64), half(8, k, k, 64)
+    print("empty", h, w, k, stride, pad, dil, flush=True)
+    for out in (None, half(2, 1, 1, 8)):
+        with pytest.raises((B.HeronRocmError, RuntimeError)):
+            hostops.conv2d_nhwc(mod, X, W, stride, pad, dil, out=out)
+        if out is not None:
+            assert torch.equal(out, half(2, 1, 1, 8))
+    # the same layer channels first, declared for a larger image
+    c = type("Ctx", (), dict(set_info=lambda self, i: setattr(self, "info", i), set_axis_map=lambda self, m: None))()
+    getOpFromName("c2d_nchw")(c, 2, 16, 16, 64, 8, k, k, stride, pad, dil, "float16", "float16")
+    with pytest.raises((B.HeronRocmError, RuntimeError)):
+        hostops.run_operator(mod, c.info, [half(2, 64, h, w), half(8, 64, k, k)])
+    mod.close()
