@@ -39,6 +39,9 @@ bool pair(PyObject* o, int64_t* h, int64_t* w) {
 
 const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
 
+// a tensor of its own on the argument's memory (undefined for anything else), usable without the interpreter lock
+at::Tensor held(PyObject* o) { return THPVariable_Check(o) ? THPVariable_Unpack(o) : at::Tensor(); }
+
 bool is(const at::Tensor* t, at::ScalarType dt) { return t && t->is_cuda() && t->scalar_type() == dt && t->is_contiguous(); }
 
 bool fits_int(int64_t v) { return v > 0 && v <= INT32_MAX; }
@@ -67,7 +70,7 @@ struct Instance {
 // stream order): split-K partial sums, column sums of B that the caller did not bring.
 struct Extras {
     at::Tensor workspace, bsum;
-    int add(const Instance& in, hrn_problem* p, const at::Tensor& B, PyObject* sums, int64_t split_k) {
+    int add(const Instance& in, hrn_problem* p, const at::Tensor& B, const at::Tensor& sums, int64_t split_k) {
         p->split_k = (int32_t)split_k;
         if (in.desc->split_k) {
             if (p->split_k < 1) p->split_k = 1;
@@ -78,8 +81,8 @@ struct Extras {
             p->workspace_bytes = (size_t)need;
         }
         if (in.desc->colsum) {
-            if (sums != Py_None) {
-                p->bsum = THPVariable_Unpack(sums).data_ptr();
+            if (sums.defined()) {
+                p->bsum = sums.data_ptr();
             } else {
                 bsum = at::empty({(int64_t)p->batch * p->n}, B.options().dtype(at::kInt));
                 p->bsum = bsum.data_ptr();
@@ -97,6 +100,13 @@ bool sums_fit(const Instance& in, PyObject* o, int64_t columns) {
     const at::Tensor* t = tensor(o);
     return is(t, at::kInt) && t->numel() == columns;
 }
+
+// The interpreter lock, given up while the native part of a call runs: allocation and launch can wait for the driver or for
+// room in a hardware queue, and other Python threads go on meanwhile.  Also taken back when an exception passes.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
 
 template <class F>
 PyObject* guarded(F f) {
@@ -124,21 +134,22 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (B->size(d + 1) != K || (d && B->size(0) != batch) || !fits_int(batch) || !fits_int(M) || !fits_int(N) || !fits_int(K) ||
             !sums_fit(in, args[7], batch * N))
             Py_RETURN_NONE;
-        at::Tensor C;
-        if (args[6] != Py_None) {
-            if (!tensor(args[6])) Py_RETURN_NONE;
-            C = *tensor(args[6]);
-        } else {
-            C = d ? at::empty({batch, M, N}, A->options().dtype(in.c)) : at::empty({M, N}, A->options().dtype(in.c));
+        if (args[6] != Py_None && !tensor(args[6])) Py_RETURN_NONE;
+        const at::Tensor a = held(args[4]), b = held(args[5]), sums = held(args[7]);
+        at::Tensor C = held(args[6]);
+        int rc;
+        {
+            Unlocked unlocked;
+            if (!C.defined()) C = d ? at::empty({batch, M, N}, a.options().dtype(in.c)) : at::empty({M, N}, a.options().dtype(in.c));
+            hrn_problem p;
+            hrn_problem_gemm(&p, (int)batch, (int)M, (int)N, (int)K);
+            p.group_m = (int32_t)v[0];
+            Extras x;
+            rc = x.add(in, &p, b, sums, v[1]);
+            if (rc == HRN_OK)
+                rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_bmm_f16(in.mod, &p, a.data_ptr(), b.data_ptr(), C.data_ptr(), stream())
+                                                  : hrn_launch_bmm_u8s8(in.mod, &p, a.data_ptr(), b.data_ptr(), C.data_ptr(), stream());
         }
-        hrn_problem p;
-        hrn_problem_gemm(&p, (int)batch, (int)M, (int)N, (int)K);
-        p.group_m = (int32_t)v[0];
-        Extras x;
-        int rc = x.add(in, &p, *B, args[7], v[1]);
-        if (rc == HRN_OK)
-            rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_bmm_f16(in.mod, &p, A->data_ptr(), B->data_ptr(), C.data_ptr(), stream())
-                                              : hrn_launch_bmm_u8s8(in.mod, &p, A->data_ptr(), B->data_ptr(), C.data_ptr(), stream());
         return rc == HRN_OK ? THPVariable_Wrap(C) : PyLong_FromLong(rc);
     });
 }
@@ -160,25 +171,25 @@ PyObject* conv2d(PyObject*, PyObject* const* args, Py_ssize_t n) {
         for (int i = 0; i < 4; ++i)
             if (!fits_int(X->size(i)) || !fits_int(W->size(i))) Py_RETURN_NONE;
         if (std::max({sh, sw, ph, pw, dh, dw}) > 1 << 20) Py_RETURN_NONE;
-        hrn_problem p;
-        hrn_problem_conv2d_hw(&p, (int)X->size(0), (int)X->size(1), (int)X->size(2), (int)X->size(3), (int)W->size(0), (int)W->size(1),
-                              (int)W->size(2), (int)sh, (int)sw, (int)ph, (int)pw, (int)dh, (int)dw);
-        p.group_m = (int32_t)v[0];
         const int64_t room_h = X->size(1) - ((W->size(1) - 1) * dh + 1) + 2 * ph, room_w = X->size(2) - ((W->size(2) - 1) * dw + 1) + 2 * pw;
         if (room_h < 0 || room_w < 0) Py_RETURN_NONE;           // (before the division, which truncates)
-        const int64_t ho = room_h / sh + 1, wo = room_w / sw + 1;
-        at::Tensor C;
-        if (args[9] != Py_None) {
-            if (!tensor(args[9])) Py_RETURN_NONE;
-            C = *tensor(args[9]);
-        } else {
-            C = at::empty({X->size(0), ho, wo, W->size(0)}, X->options().dtype(in.c));
+        if (args[9] != Py_None && !tensor(args[9])) Py_RETURN_NONE;
+        const at::Tensor x = held(args[4]), w = held(args[5]), sums = held(args[10]);
+        at::Tensor C = held(args[9]);
+        int rc;
+        {
+            Unlocked unlocked;
+            if (!C.defined()) C = at::empty({x.size(0), room_h / sh + 1, room_w / sw + 1, w.size(0)}, x.options().dtype(in.c));
+            hrn_problem p;
+            hrn_problem_conv2d_hw(&p, (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3), (int)w.size(0), (int)w.size(1),
+                                  (int)w.size(2), (int)sh, (int)sw, (int)ph, (int)pw, (int)dh, (int)dw);
+            p.group_m = (int32_t)v[0];
+            Extras e;
+            rc = e.add(in, &p, w, sums, v[1]);
+            if (rc == HRN_OK)
+                rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_conv2d_nhwc_f16(in.mod, &p, x.data_ptr(), w.data_ptr(), C.data_ptr(), stream())
+                                                  : hrn_launch_conv2d_nhwc_u8s8(in.mod, &p, x.data_ptr(), w.data_ptr(), C.data_ptr(), stream());
         }
-        Extras x;
-        int rc = x.add(in, &p, *W, args[10], v[1]);
-        if (rc == HRN_OK)
-            rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_conv2d_nhwc_f16(in.mod, &p, X->data_ptr(), W->data_ptr(), C.data_ptr(), stream())
-                                              : hrn_launch_conv2d_nhwc_u8s8(in.mod, &p, X->data_ptr(), W->data_ptr(), C.data_ptr(), stream());
         return rc == HRN_OK ? THPVariable_Wrap(C) : PyLong_FromLong(rc);
     });
 }

@@ -34,3 +34,40 @@ def test_filter_larger_than_the_input_is_refused(h, w, k, stride, pad, dil, hrn)
     with pytest.raises((B.HeronRocmError, RuntimeError)):
         hostops.run_operator(mod, c.info, [half(2, 64, h, w), half(8, 64, k, k)])
     mod.close()
+
+
+@pytest.mark.parametrize("entry", ["gemm", "conv2d"])
+def test_other_threads_run_during_a_call(entry, hrn):
+    """With no forced switch of the interpreter lock another thread gets on only where a call gives the lock up."""
+    import sys
+    import threading
+    import time
+    if entry == "gemm":
+        mod, args = B.Module(instances.BEST["small_f16"]), (half(512, 512), half(512, 512))
+        call = hostops.gemm
+    else:
+        mod, args = B.Module(CONV_F16), (half(4, 28, 28, 64), half(64, 3, 3, 64), 1, 1, 1)
+        call = hostops.conv2d_nhwc
+    turns, stop = [0], []
+
+    def other():
+        while not stop:
+            turns[0] += 1
+            time.sleep(0)
+
+    out = call(mod, *args)
+    thread, interval = threading.Thread(target=other), sys.getswitchinterval()
+    try:
+        sys.setswitchinterval(1000.0)
+        thread.start()
+        before, end = turns[0], time.monotonic() + 5.0
+        while turns[0] == before and time.monotonic() < end:
+            call(mod, *args, out=out)
+        ran = turns[0] - before
+    finally:
+        sys.setswitchinterval(interval)
+        stop.append(True)
+        thread.join()
+    torch.cuda.synchronize()
+    assert ran > 0
+    mod.close()
