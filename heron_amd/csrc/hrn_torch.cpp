@@ -11,6 +11,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/heron_rocm.h"
@@ -108,12 +109,13 @@ struct Unlocked {
     ~Unlocked() { PyEval_RestoreThread(state); }
 };
 
+// C++ exceptions become the Python ones that torch makes of them (torch.OutOfMemoryError when the allocator is out of memory).
 template <class F>
 PyObject* guarded(F f) {
     try {
         return f();
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (...) {
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }

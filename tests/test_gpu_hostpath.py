@@ -71,3 +71,17 @@ def test_other_threads_run_during_a_call(entry, hrn):
     torch.cuda.synchronize()
     assert ran > 0
     mod.close()
+
+
+def test_out_of_memory_keeps_its_type(hrn):
+    """A result that no card holds: torch's allocator refuses it and its exception arrives as such."""
+    mod = B.Module(instances.BEST["small_f16"])
+    A = half(1 << 20, 16)                       # 2 TiB of results
+    with pytest.raises(torch.OutOfMemoryError):
+        hostops.gemm(mod, A, A)
+    mod.close()
+    mod = B.Module(CONV_F16)
+    X, W = half(1 << 18, 2, 2, 16), half(1 << 20, 1, 1, 16)
+    with pytest.raises(torch.OutOfMemoryError):
+        hostops.conv2d_nhwc(mod, X, W)
+    mod.close()
