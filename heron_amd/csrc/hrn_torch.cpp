@@ -8,6 +8,7 @@
 #include <Python.h>
 
 #include <algorithm>
+#include <initializer_list>
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
@@ -44,6 +45,16 @@ const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariab
 at::Tensor held(PyObject* o) { return THPVariable_Check(o) ? THPVariable_Unpack(o) : at::Tensor(); }
 
 bool is(const at::Tensor* t, at::ScalarType dt) { return t && t->is_cuda() && t->scalar_type() == dt && t->is_contiguous(); }
+
+// a caller's result tensor: None, or on the operands' device, of the result's type, contiguous and large enough
+bool result_fits(PyObject* o, const at::Tensor& operand, at::ScalarType dt, std::initializer_list<int64_t> shape) {
+    if (o == Py_None) return true;
+    const at::Tensor* t = tensor(o);
+    if (!is(t, dt) || t->device() != operand.device()) return false;
+    int64_t room = t->numel();
+    for (int64_t d : shape) room /= d;                          // (the product of the extents may not fit)
+    return room >= 1;
+}
 
 bool fits_int(int64_t v) { return v > 0 && v <= INT32_MAX; }
 
@@ -136,7 +147,7 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (B->size(d + 1) != K || (d && B->size(0) != batch) || !fits_int(batch) || !fits_int(M) || !fits_int(N) || !fits_int(K) ||
             !sums_fit(in, args[7], batch * N))
             Py_RETURN_NONE;
-        if (args[6] != Py_None && !tensor(args[6])) Py_RETURN_NONE;
+        if (!result_fits(args[6], *A, in.c, {batch, M, N})) Py_RETURN_NONE;
         const at::Tensor a = held(args[4]), b = held(args[5]), sums = held(args[7]);
         at::Tensor C = held(args[6]);
         int rc;
@@ -175,13 +186,14 @@ PyObject* conv2d(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (std::max({sh, sw, ph, pw, dh, dw}) > 1 << 20) Py_RETURN_NONE;
         const int64_t room_h = X->size(1) - ((W->size(1) - 1) * dh + 1) + 2 * ph, room_w = X->size(2) - ((W->size(2) - 1) * dw + 1) + 2 * pw;
         if (room_h < 0 || room_w < 0) Py_RETURN_NONE;           // (before the division, which truncates)
-        if (args[9] != Py_None && !tensor(args[9])) Py_RETURN_NONE;
+        const int64_t ho = room_h / sh + 1, wo = room_w / sw + 1;
+        if (!result_fits(args[9], *X, in.c, {X->size(0), ho, wo, W->size(0)})) Py_RETURN_NONE;
         const at::Tensor x = held(args[4]), w = held(args[5]), sums = held(args[10]);
         at::Tensor C = held(args[9]);
         int rc;
         {
             Unlocked unlocked;
-            if (!C.defined()) C = at::empty({x.size(0), room_h / sh + 1, room_w / sw + 1, w.size(0)}, x.options().dtype(in.c));
+            if (!C.defined()) C = at::empty({x.size(0), ho, wo, w.size(0)}, x.options().dtype(in.c));
             hrn_problem p;
             hrn_problem_conv2d_hw(&p, (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3), (int)w.size(0), (int)w.size(1),
                                   (int)w.size(2), (int)sh, (int)sw, (int)ph, (int)pw, (int)dh, (int)dw);

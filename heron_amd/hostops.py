@@ -2,6 +2,8 @@
 
 torch is plumbing only (device memory and streams); every multiply goes through the C ABI.
 """
+import math
+
 import torch
 
 from . import backend as B
@@ -38,6 +40,13 @@ def _chk(t, dtype):
         raise ValueError("expected a contiguous CUDA tensor of %s, got %s %s" % (dtype, t.dtype, t.device))
 
 
+def _chk_out(out, operand, dtype, shape):
+    """A caller's result tensor is written as ``shape``, whatever view of the memory it is."""
+    _chk(out, dtype)
+    if out.device != operand.device or out.numel() < math.prod(shape):
+        raise ValueError("out holds %d elements on %s, the result is %s on %s" % (out.numel(), out.device, tuple(shape), operand.device))
+
+
 def column_sums(Bm):
     """Column sums of an int8 operand (N,K) / (b,N,K) / KRSC filter (CO,KH,KW,CI): int32 (N,) / (b,N) / (CO,).  What a
     ``colsum`` instance takes with the weights; with fixed weights it is computed once."""
@@ -54,7 +63,8 @@ def column_sums(Bm):
 def gemm(mod, A, Bm, out=None, group_m=8, split_k=0, bsum=None):
     """C = A @ Bm.T for A (M,K), Bm (N,K), or batched (b,M,K) x (b,N,K) -> (b,M,N).  ``split_k`` is the number of
     K slices for a split-K instance (the module supplies the workspace).  ``bsum``: the column sums of Bm
-    (``column_sums``) for a ``colsum`` instance; computed on the spot when absent."""
+    (``column_sums``) for a ``colsum`` instance; computed on the spot when absent.  ``out``: a contiguous tensor of the
+    result's type with room for it, on A's device."""
     if _recording is None:
         C = B.ext().gemm(*mod.native, group_m, split_k, A, Bm, out, bsum)
         if C is not None:
@@ -70,6 +80,8 @@ def gemm(mod, A, Bm, out=None, group_m=8, split_k=0, bsum=None):
     oshape = (batch, M, N) if A.dim() == 3 else (M, N)
     if out is None:
         out = _new(torch.empty, oshape, dtype=torch.float16 if f16 else torch.int32, device=A.device)
+    else:
+        _chk_out(out, A, torch.float16 if f16 else torch.int32, oshape)
     p = B.gemm_problem(batch, M, N, K, group_m, split_k)
     if bsum is not None and mod.desc.colsum:
         _chk(bsum, torch.int32)
@@ -108,6 +120,8 @@ def conv2d_nhwc(mod, X, Wt, stride=1, pad=0, dil=1, out=None, group_m=8, split_k
     wo = (W - ((KW - 1) * dw + 1) + 2 * pw) // sw + 1
     if out is None:
         out = _new(torch.empty, (N, ho, wo, CO), dtype=torch.float16 if f16 else torch.int32, device=X.device)
+    else:
+        _chk_out(out, X, torch.float16 if f16 else torch.int32, (N, ho, wo, CO))
     if bsum is not None and mod.desc.colsum:
         _chk(bsum, torch.int32)
         if bsum.numel() != CO:

@@ -85,3 +85,26 @@ def test_out_of_memory_keeps_its_type(hrn):
     with pytest.raises(torch.OutOfMemoryError):
         hostops.conv2d_nhwc(mod, X, W)
     mod.close()
+
+
+@pytest.mark.parametrize("entry", ["gemm", "bmm", "conv2d"])
+def test_results_of_the_caller(entry, hrn):
+    """``out`` is any contiguous tensor of the result's type with room for it; everything else is refused before a launch."""
+    if entry == "conv2d":
+        mod, args, shape, call = B.Module(CONV_F16), (half(2, 5, 7, 64), half(8, 3, 3, 64), 1, 1, 1), (2, 5, 7, 8), hostops.conv2d_nhwc
+    else:
+        b = (3,) if entry == "bmm" else ()
+        mod, args, shape, call = B.Module(instances.BEST["small_f16"]), (half(*b, 33, 64), half(*b, 40, 64)), b + (33, 40), hostops.gemm
+    want = call(mod, *args)
+    assert want.shape == shape
+    n = want.numel()
+    for out in (torch.zeros_like(want), torch.zeros(n, device="cuda").half(), torch.zeros(n + 5, device="cuda").half()):
+        got = call(mod, *args, out=out)
+        assert got is out and torch.equal(out.flatten()[:n], want.flatten()) and not out.flatten()[n:].any()
+    wide = torch.zeros(shape[:-1] + (2 * shape[-1],), device="cuda").half()
+    for out in (torch.zeros(shape, dtype=torch.float16), torch.zeros(n - 1, device="cuda").half(), wide[..., :shape[-1]],
+                torch.zeros(shape, device="cuda"), torch.zeros(shape, device="cuda", dtype=torch.bfloat16)):
+        with pytest.raises(ValueError):
+            call(mod, *args, out=out)
+        assert not out.any()
+    mod.close()
