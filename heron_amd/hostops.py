@@ -443,7 +443,7 @@ CHANNELS_FIRST = {
 }
 
 
-def _run_channels_first(mod, info, inputs, act, Bm, group_m, bsum):
+def _run_channels_first(mod, info, inputs, act, Bm, group_m, split_k, bsum):
     """A channels-first convolution without passes over its result - and, transposed, without the zero-expanded input."""
     c, t, X = info['conv'], info.get('transposed'), inputs[0]
     f16 = mod.desc.dtype == B.HRN_DT_F16
@@ -461,7 +461,8 @@ def _run_channels_first(mod, info, inputs, act, Bm, group_m, bsum):
     _chk(Bm, torch.float16 if f16 else torch.int8)
     if xshape[3] != Bm.shape[3]:
         raise ValueError("channel mismatch")
-    p = B.conv2d_problem(*xshape, *Bm.shape[:3], (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']), group_m)
+    p = B.conv2d_problem(*xshape, *Bm.shape[:3], (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']), group_m,
+                         split_k)
     if bsum is not None and mod.desc.colsum:
         _chk(bsum, torch.int32)
         if bsum.numel() != p.n:
@@ -492,7 +493,7 @@ def run_operator(mod, info, inputs, group_m=8, split_k=0, constant=None, bsum=No
     act, const, fin = ADAPTERS[adapter]
     Bm = const(info, *inputs) if constant is None else constant
     if adapter in CHANNELS_FIRST and _native_ok(inputs[0]) and mod.has_chw:
-        return _run_channels_first(mod, info, inputs, act, Bm, group_m, bsum)
+        return _run_channels_first(mod, info, inputs, act, Bm, group_m, split_k, bsum)
     A = act(info, *inputs)
     if info['operator'] == 'conv2d_nhwc':
         c = info['conv']

@@ -16,6 +16,12 @@ def half(*shape):
     return torch.ones(shape, device="cuda", dtype=torch.float16)
 
 
+def declared(op, args, dtype="float16"):
+    ctx = type("Ctx", (), dict(set_info=lambda self, i: setattr(self, "info", i), set_axis_map=lambda self, m: None))()
+    getOpFromName(op)(ctx, *args, dtype, dtype)
+    return ctx.info
+
+
 # the dilated filter is larger than the padded input by less than the stride, by the stride and by more than it; in one direction
 @pytest.mark.parametrize("h,w,k,stride,pad,dil", [(4, 4, 5, 2, 0, 1), (4, 9, 5, 2, 0, 1), (9, 4, 5, 2, 0, 1), (3, 3, 5, 2, 0, 1), (1, 1, 5, 2, 0, 1),
                                                   (4, 4, 3, 3, 0, 2), (2, 2, 5, 4, 1, 1)])
@@ -29,10 +35,9 @@ def test_filter_larger_than_the_input_is_refused(h, w, k, stride, pad, dil, hrn)
         if out is not None:
             assert torch.equal(out, half(2, 1, 1, 8))
     # the same layer channels first, declared for a larger image
-    c = type("Ctx", (), dict(set_info=lambda self, i: setattr(self, "info", i), set_axis_map=lambda self, m: None))()
-    getOpFromName("c2d_nchw")(c, 2, 16, 16, 64, 8, k, k, stride, pad, dil, "float16", "float16")
+    info = declared("c2d_nchw", [2, 16, 16, 64, 8, k, k, stride, pad, dil])
     with pytest.raises((B.HeronRocmError, RuntimeError)):
-        hostops.run_operator(mod, c.info, [half(2, 64, h, w), half(8, 64, k, k)])
+        hostops.run_operator(mod, info, [half(2, 64, h, w), half(8, 64, k, k)])
     mod.close()
 
 
@@ -107,4 +112,20 @@ def test_results_of_the_caller(entry, hrn):
         with pytest.raises(ValueError):
             call(mod, *args, out=out)
         assert not out.any()
+    mod.close()
+
+
+CHANNELS_FIRST = {"c1d": [2, 9, 64, 8, 3, 1, 1, 1], "c2d_nchw": [2, 5, 6, 64, 8, 3, 3, 1, 1, 1], "c3d": [2, 3, 5, 6, 16, 8, 3, 3, 3, 1, 1, 1],
+                  "t2d": [2, 5, 6, 64, 8, 3, 3, 2, 1, 1, 0]}
+
+
+@pytest.mark.parametrize("op", sorted(CHANNELS_FIRST))
+def test_slices_of_k_need_an_instance_built_for_them(op, hrn):
+    mod, info = B.Module(CONV_F16), declared(op, CHANNELS_FIRST[op])
+    X, F = half(*info["reference_args"]["input"]), half(*info["reference_args"]["filter"])
+    want = hostops.run_operator(mod, info, [X, F])
+    assert torch.equal(hostops.run_operator(mod, info, [X, F], split_k=1), want)
+    for split_k in (2, 8):
+        with pytest.raises(B.HeronRocmError):
+            hostops.run_operator(mod, info, [X, F], split_k=split_k)
     mod.close()
