@@ -471,7 +471,7 @@ def _run_channels_first(mod, info, inputs, act, Bm, group_m, split_k, bsum):
     ho = (p.ch - ((p.kh - 1) * p.cdil + 1) + 2 * p.cpad) // p.cstride + 1
     wo = (p.cw - ((p.kw - 1) * p.cdil_w + 1) + 2 * p.cpad_w) // p.cstride_w + 1
     shape = CHANNELS_FIRST[info['adapter']](info, p.cn, p.n, ho, wo)
-    view.out_plane = p.m // shape[0]
+    view.out_plane = p.m // max(1, shape[0])               # (no images: the library refuses the empty problem)
     out = _new(torch.empty, shape, dtype=torch.float16 if f16 else torch.int32, device=A.device)
     _do(mod.launch_conv2d_chw, p, view, A.data_ptr(), Bm.data_ptr(), out.data_ptr(), _stream())
     return out

@@ -129,3 +129,12 @@ def test_slices_of_k_need_an_instance_built_for_them(op, hrn):
         with pytest.raises(B.HeronRocmError):
             hostops.run_operator(mod, info, [X, F], split_k=split_k)
     mod.close()
+
+
+@pytest.mark.parametrize("op", sorted(CHANNELS_FIRST))
+def test_no_images_are_refused_by_the_library(op, hrn):
+    mod, info = B.Module(CONV_F16), declared(op, CHANNELS_FIRST[op])
+    empty = half(0, *info["reference_args"]["input"][1:])
+    with pytest.raises(B.HeronRocmError):
+        hostops.run_operator(mod, info, [empty, half(*info["reference_args"]["filter"])])
+    mod.close()
