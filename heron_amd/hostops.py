@@ -459,9 +459,10 @@ def _run_channels_first(mod, info, inputs, act, Bm, group_m, split_k, bsum):
         xshape = A.shape
     _chk(A, torch.float16 if f16 else torch.uint8)
     _chk(Bm, torch.float16 if f16 else torch.int8)
-    if xshape[3] != Bm.shape[3]:
+    CO, KH, KW, CI = Bm.shape
+    if xshape[3] != CI:
         raise ValueError("channel mismatch")
-    p = B.conv2d_problem(*xshape, *Bm.shape[:3], (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']), group_m,
+    p = B.conv2d_problem(*xshape, CO, KH, KW, (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']), group_m,
                          split_k)
     if bsum is not None and mod.desc.colsum:
         _chk(bsum, torch.int32)
@@ -471,7 +472,9 @@ def _run_channels_first(mod, info, inputs, act, Bm, group_m, split_k, bsum):
     ho = (p.ch - ((p.kh - 1) * p.cdil + 1) + 2 * p.cpad) // p.cstride + 1
     wo = (p.cw - ((p.kw - 1) * p.cdil_w + 1) + 2 * p.cpad_w) // p.cstride_w + 1
     shape = CHANNELS_FIRST[info['adapter']](info, p.cn, p.n, ho, wo)
-    view.out_plane = p.m // max(1, shape[0])               # (no images: the library refuses the empty problem)
+    if p.m > 0 and math.prod(shape) != p.m * p.n:          # (an empty problem is refused by the library)
+        raise RuntimeError("the operator was declared with a result of %s, its input makes %d pixels" % (shape, p.m))
+    view.out_plane = p.m // max(1, shape[0])
     out = _new(torch.empty, shape, dtype=torch.float16 if f16 else torch.int32, device=A.device)
     _do(mod.launch_conv2d_chw, p, view, A.data_ptr(), Bm.data_ptr(), out.data_ptr(), _stream())
     return out

@@ -138,3 +138,14 @@ def test_no_images_are_refused_by_the_library(op, hrn):
     with pytest.raises(B.HeronRocmError):
         hostops.run_operator(mod, info, [empty, half(*info["reference_args"]["filter"])])
     mod.close()
+
+
+@pytest.mark.parametrize("images", [1, 3, 4])
+def test_volumes_of_another_number_than_declared_are_refused(images, hrn):
+    """conv3d takes the number of volumes from its declaration; the result has room for those."""
+    mod, info = B.Module(CONV_F16), declared("c3d", CHANNELS_FIRST["c3d"])
+    shape = info["reference_args"]["input"]
+    assert shape[0] == 2
+    with pytest.raises(RuntimeError):
+        hostops.run_operator(mod, info, [half(images, *shape[1:]), half(*info["reference_args"]["filter"])])
+    mod.close()
