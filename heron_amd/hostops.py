@@ -448,12 +448,18 @@ def _run_channels_first(mod, info, inputs, act, Bm, group_m, split_k, bsum):
     c, t, X = info['conv'], info.get('transposed'), inputs[0]
     f16 = mod.desc.dtype == B.HRN_DT_F16
     view = B.ConvView()
-    if t is not None and t['stride'] & (t['stride'] - 1) == 0 and X.shape[0] <= 65535:
+    expand = False
+    if t is not None and X.dim() == 4:
         N, CI, H, W = X.shape
+        s, top, left = t['stride'], (c['KH'] - 1) * t['dil'] - t['pad'], (c['KW'] - 1) * t['dil'] - t['pad']
+        # what hrn_conv_view takes: a stride that is a power of two, every pixel inside the expanded image; the gather pass
+        # takes the others and drops what lies outside
+        expand = (s & (s - 1) == 0 and N <= 65535 and top >= 0 and left >= 0 and H > 0 and W > 0 and
+                  (H - 1) * s + top < c['H'] and (W - 1) * s + left < c['W'])
+    if expand:
         A = _channels_last(X.reshape(N, CI, H * W), c['CI'])
         xshape = (N, c['H'], c['W'], c['CI'])
-        view.expand, view.in_h, view.in_w = t['stride'], H, W
-        view.top, view.left = (c['KH'] - 1) * t['dil'] - t['pad'], (c['KW'] - 1) * t['dil'] - t['pad']
+        view.expand, view.in_h, view.in_w, view.top, view.left = s, H, W, top, left
     else:
         A = act(info, *inputs)
         xshape = A.shape

@@ -149,3 +149,17 @@ def test_volumes_of_another_number_than_declared_are_refused(images, hrn):
     with pytest.raises(RuntimeError):
         hostops.run_operator(mod, info, [half(images, *shape[1:]), half(*info["reference_args"]["filter"])])
     mod.close()
+
+
+@pytest.mark.parametrize("shape", [(2, 64, 7, 6), (2, 64, 5, 9), (3, 64, 8, 8), (1, 64, 2, 3)])
+def test_transposed_conv_of_another_image_than_declared(shape, hrn):
+    """The expanded image has the declared extents: pixels beyond them are dropped, missing ones are zeros."""
+    mod, info = B.Module(CONV_F16), declared("t2d", CHANNELS_FIRST["t2d"])
+    gen = torch.Generator(device="cuda").manual_seed(shape[2])
+    X = torch.randn(shape, device="cuda", generator=gen).half()
+    F = torch.randn(info["reference_args"]["filter"], device="cuda", generator=gen).half()
+    c = info["conv"]
+    act, const, fin = hostops.ADAPTERS[info["adapter"]]
+    want = fin(info, hostops.conv2d_nhwc(mod, act(info, X, F), const(info, X, F), 1, 0, (c["dil"], c["dil_w"])))
+    assert torch.equal(hostops.run_operator(mod, info, [X, F]), want)
+    mod.close()
