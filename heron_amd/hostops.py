@@ -47,6 +47,17 @@ def _chk_out(out, operand, dtype, shape):
         raise ValueError("out holds %d elements on %s, the result is %s on %s" % (out.numel(), out.device, tuple(shape), operand.device))
 
 
+def _slice_workspace(mod, p, operand):
+    """Split-K instances: the partial sums of this call.  A recorded plan keeps them with its buffers: the module's own
+    workspace is replaced by a larger launch of the same module."""
+    if mod.desc.split_k:
+        p.split_k = max(1, p.split_k)
+        need = B.splitk_workspace_bytes(mod.desc, p)
+        ws = _new(torch.empty, (max(need, 16),), dtype=torch.uint8, device=operand.device)
+        p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+        return ws
+
+
 def column_sums(Bm):
     """Column sums of an int8 operand (N,K) / (b,N,K) / KRSC filter (CO,KH,KW,CI): int32 (N,) / (b,N) / (CO,).  What a
     ``colsum`` instance takes with the weights; with fixed weights it is computed once."""
@@ -88,6 +99,7 @@ def gemm(mod, A, Bm, out=None, group_m=8, split_k=0, bsum=None):
         if bsum.numel() != batch * N:
             raise ValueError("bsum holds %d sums, B has %d columns" % (bsum.numel(), batch * N))
         p.bsum = bsum.data_ptr()
+    ws = _slice_workspace(mod, p, A)                        # noqa: F841 - alive until the launch
     _do(mod.launch, p, A.data_ptr(), Bm.data_ptr(), out.data_ptr(), _stream())
     return out
 
@@ -127,6 +139,7 @@ def conv2d_nhwc(mod, X, Wt, stride=1, pad=0, dil=1, out=None, group_m=8, split_k
         if bsum.numel() != CO:
             raise ValueError("bsum holds %d sums, the filter has %d output channels" % (bsum.numel(), CO))
         p.bsum = bsum.data_ptr()
+    ws = _slice_workspace(mod, p, X)                        # noqa: F841 - alive until the launch
     _do(mod.launch, p, X.data_ptr(), Wt.data_ptr(), out.data_ptr(), _stream())
     return out
 

@@ -163,3 +163,23 @@ def test_transposed_conv_of_another_image_than_declared(shape, hrn):
     want = fin(info, hostops.conv2d_nhwc(mod, act(info, X, F), const(info, X, F), 1, 0, (c["dil"], c["dil_w"])))
     assert torch.equal(hostops.run_operator(mod, info, [X, F]), want)
     mod.close()
+
+
+def test_a_recorded_split_k_plan_owns_its_workspace(hrn):
+    mod, info = B.Module(instances.splitk_descs()[4]), declared("c2d_nchw", [2, 7, 7, 64, 64, 3, 3, 1, 1, 1])
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    X = torch.randn(info["reference_args"]["input"], device="cuda", generator=gen).half()
+    F = torch.randn(info["reference_args"]["filter"], device="cuda", generator=gen).half()
+    plan = hostops.OperatorPlan(mod, info, [X, F], split_k=3)
+    want = plan.run().clone()
+    bound = [a.workspace for _, args in plan.steps for a in args if isinstance(a, B.Problem)]
+    assert bound and all(any(b.data_ptr() <= w < b.data_ptr() + b.numel() * b.element_size() for b in plan.buffers) for w in bound)
+    # a larger launch of the same module in between, and fresh tensors on whatever memory it freed
+    p = B.conv2d_problem(64, 28, 28, 64, 64, 3, 3, 1, 1, 1, split_k=3)
+    big = half(64, 28, 28, 64), half(64, 3, 3, 64), half(64, 28, 28, 64)
+    mod.launch(p, *(t.data_ptr() for t in big), hostops._stream())
+    other = [torch.full((1 << 18,), 7.0, device="cuda") for _ in range(8)]
+    plan.out.zero_()
+    assert torch.equal(plan.run(), want)
+    assert all(bool((t == 7.0).all()) for t in other)
+    mod.close()
