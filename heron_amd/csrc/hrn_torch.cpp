@@ -41,9 +41,6 @@ bool pair(PyObject* o, int64_t* h, int64_t* w) {
 
 const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
 
-// a tensor of its own on the argument's memory (undefined for anything else), usable without the interpreter lock
-at::Tensor held(PyObject* o) { return THPVariable_Check(o) ? THPVariable_Unpack(o) : at::Tensor(); }
-
 bool is(const at::Tensor* t, at::ScalarType dt) { return t && t->is_cuda() && t->scalar_type() == dt && t->is_contiguous(); }
 
 // a caller's result tensor: None, or on the operands' device, of the result's type, contiguous and large enough
@@ -82,7 +79,7 @@ struct Instance {
 // stream order): split-K partial sums, column sums of B that the caller did not bring.
 struct Extras {
     at::Tensor workspace, bsum;
-    int add(const Instance& in, hrn_problem* p, const at::Tensor& B, const at::Tensor& sums, int64_t split_k) {
+    int add(const Instance& in, hrn_problem* p, const at::Tensor& B, const at::Tensor* sums, int64_t split_k) {
         p->split_k = (int32_t)split_k;
         if (in.desc->split_k) {
             if (p->split_k < 1) p->split_k = 1;
@@ -93,8 +90,8 @@ struct Extras {
             p->workspace_bytes = (size_t)need;
         }
         if (in.desc->colsum) {
-            if (sums.defined()) {
-                p->bsum = sums.data_ptr();
+            if (sums) {
+                p->bsum = sums->data_ptr();
             } else {
                 bsum = at::empty({(int64_t)p->batch * p->n}, B.options().dtype(at::kInt));
                 p->bsum = bsum.data_ptr();
@@ -114,7 +111,8 @@ bool sums_fit(const Instance& in, PyObject* o, int64_t columns) {
 }
 
 // The interpreter lock, given up while the native part of a call runs: allocation and launch can wait for the driver or for
-// room in a hardware queue, and other Python threads go on meanwhile.  Also taken back when an exception passes.
+// room in a hardware queue, and other Python threads go on meanwhile.  Also taken back when an exception passes.  The caller
+// holds the arguments, so their tensors stay.
 struct Unlocked {
     PyThreadState* state = PyEval_SaveThread();
     ~Unlocked() { PyEval_RestoreThread(state); }
@@ -148,20 +146,21 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
             !sums_fit(in, args[7], batch * N))
             Py_RETURN_NONE;
         if (!result_fits(args[6], *A, in.c, {batch, M, N})) Py_RETURN_NONE;
-        const at::Tensor a = held(args[4]), b = held(args[5]), sums = held(args[7]);
-        at::Tensor C = held(args[6]);
+        const at::Tensor* sums = tensor(args[7]);
+        at::Tensor C;
+        if (args[6] != Py_None) C = *tensor(args[6]);
         int rc;
         {
             Unlocked unlocked;
-            if (!C.defined()) C = d ? at::empty({batch, M, N}, a.options().dtype(in.c)) : at::empty({M, N}, a.options().dtype(in.c));
+            if (!C.defined()) C = d ? at::empty({batch, M, N}, A->options().dtype(in.c)) : at::empty({M, N}, A->options().dtype(in.c));
             hrn_problem p;
             hrn_problem_gemm(&p, (int)batch, (int)M, (int)N, (int)K);
             p.group_m = (int32_t)v[0];
             Extras x;
-            rc = x.add(in, &p, b, sums, v[1]);
+            rc = x.add(in, &p, *B, sums, v[1]);
             if (rc == HRN_OK)
-                rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_bmm_f16(in.mod, &p, a.data_ptr(), b.data_ptr(), C.data_ptr(), stream())
-                                                  : hrn_launch_bmm_u8s8(in.mod, &p, a.data_ptr(), b.data_ptr(), C.data_ptr(), stream());
+                rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_bmm_f16(in.mod, &p, A->data_ptr(), B->data_ptr(), C.data_ptr(), stream())
+                                                  : hrn_launch_bmm_u8s8(in.mod, &p, A->data_ptr(), B->data_ptr(), C.data_ptr(), stream());
         }
         return rc == HRN_OK ? THPVariable_Wrap(C) : PyLong_FromLong(rc);
     });
@@ -188,21 +187,22 @@ PyObject* conv2d(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (room_h < 0 || room_w < 0) Py_RETURN_NONE;           // (before the division, which truncates)
         const int64_t ho = room_h / sh + 1, wo = room_w / sw + 1;
         if (!result_fits(args[9], *X, in.c, {X->size(0), ho, wo, W->size(0)})) Py_RETURN_NONE;
-        const at::Tensor x = held(args[4]), w = held(args[5]), sums = held(args[10]);
-        at::Tensor C = held(args[9]);
+        const at::Tensor* sums = tensor(args[10]);
+        at::Tensor C;
+        if (args[9] != Py_None) C = *tensor(args[9]);
         int rc;
         {
             Unlocked unlocked;
-            if (!C.defined()) C = at::empty({x.size(0), ho, wo, w.size(0)}, x.options().dtype(in.c));
+            if (!C.defined()) C = at::empty({X->size(0), ho, wo, W->size(0)}, X->options().dtype(in.c));
             hrn_problem p;
-            hrn_problem_conv2d_hw(&p, (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3), (int)w.size(0), (int)w.size(1),
-                                  (int)w.size(2), (int)sh, (int)sw, (int)ph, (int)pw, (int)dh, (int)dw);
+            hrn_problem_conv2d_hw(&p, (int)X->size(0), (int)X->size(1), (int)X->size(2), (int)X->size(3), (int)W->size(0),
+                                  (int)W->size(1), (int)W->size(2), (int)sh, (int)sw, (int)ph, (int)pw, (int)dh, (int)dw);
             p.group_m = (int32_t)v[0];
-            Extras e;
-            rc = e.add(in, &p, w, sums, v[1]);
+            Extras x;
+            rc = x.add(in, &p, *W, sums, v[1]);
             if (rc == HRN_OK)
-                rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_conv2d_nhwc_f16(in.mod, &p, x.data_ptr(), w.data_ptr(), C.data_ptr(), stream())
-                                                  : hrn_launch_conv2d_nhwc_u8s8(in.mod, &p, x.data_ptr(), w.data_ptr(), C.data_ptr(), stream());
+                rc = in.desc->dtype == HRN_DT_F16 ? hrn_launch_conv2d_nhwc_f16(in.mod, &p, X->data_ptr(), W->data_ptr(), C.data_ptr(), stream())
+                                                  : hrn_launch_conv2d_nhwc_u8s8(in.mod, &p, X->data_ptr(), W->data_ptr(), C.data_ptr(), stream());
         }
         return rc == HRN_OK ? THPVariable_Wrap(C) : PyLong_FromLong(rc);
     });
