@@ -169,6 +169,7 @@ SYMBOLS = {
     "hrn_launch_conv2d_nhwc_f16": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_bmm_u8s8": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_conv2d_nhwc_u8s8": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
+    "hrn_compile_chw": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
     "hrn_module_has_chw": (_i, [_vp]),
     "hrn_launch_conv2d_chw": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(ConvView), _vp, _vp, _vp, _vp]),
     "hrn_launch_splitk_static": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
@@ -254,6 +255,12 @@ def compile_desc(desc, timeout_s=0.0):
     buf = ctypes.create_string_buffer(4096)
     _check(lib().hrn_compile(ctypes.byref(desc), float(timeout_s), buf, 4096))
     return buf.value.decode()
+
+
+def compile_chw(desc, expand, timeout_s=0.0):
+    """hipcc the channels-first kernels of a conv2d instance (``expand``: those for zero-expanded inputs) into the cache;
+    nothing to do for an instance that has none."""
+    _check(lib().hrn_compile_chw(ctypes.byref(desc), 1 if expand else 0, float(timeout_s)))
 
 
 def gemm_problem(batch, m, n, k, group_m=8, split_k=0):

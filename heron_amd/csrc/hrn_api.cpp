@@ -45,13 +45,25 @@ struct HrnKArgs {  // must match mfma_gemm_template.hip
     int32_t expand_shift, in_h, in_w, top, left;
 };
 
+// An instance's kernels lie in up to three code objects, so that a caller pays the compiler only for those it launches: a
+// 128x128 im2col conv instance takes 1.8 s for its own, 5.1 s for all.
+enum { PART_MAIN, PART_CHW, PART_EXPAND, PARTS };
+const char* const kPartKernel[PARTS] = {"hrn_mfma_kernel", "hrn_mfma_kernel_chw", "hrn_mfma_kernel_chw_expand"};
+const char* const kPartFile[PARTS] = {"", "_chw", "_expand"};
+
+struct CodeObject {
+    hipModule_t mod = nullptr;
+    hipFunction_t fn[2] = {};       // plain and deep (a third stage); null where the instance has no room for it
+};
+
 struct hrn_module {
     hrn_kernel_desc desc;
     hrn_kernel_info info;
-    hipModule_t mod;
-    // the instance's kernels, each plain and deep (a third stage); null where it has none or no room for it
-    hipFunction_t fn[2];
-    hipFunction_t fn_chw[2], fn_expand[2];   // conv2d: those of hrn_launch_conv2d_chw
+    mutable CodeObject part[PARTS]; // those of hrn_launch_conv2d_chw are there from hrn_build on or from their first launch
+    mutable std::mutex part_mutex;
+    bool has_chw, has_deep;
+    int device;                     // the code objects are loaded on
+    double timeout_s;               // of a compilation
     int deep_grid;      // workgroups of the deep kernels that the device holds at once
     std::string path;
     int persist_grid;   // persistent instances: workgroups that fit the device at once (multiple of 8 when >= 8)
@@ -294,10 +306,11 @@ int run_hipcc(const std::vector<std::string>& args, const std::string& log_path,
     return HRN_OK;
 }
 
-int compile_desc(const hrn_kernel_desc* d, double timeout_s, std::string* out_path) {
+int compile_desc(const hrn_kernel_desc* d, int part, double timeout_s, std::string* out_path) {
     Derived dv;
     int rc = derive(d, &dv);
     if (rc) return rc;
+    if (part != PART_MAIN && !dv.has_chw) return fail(HRN_E_BADPARAM, "the instance has no channels-first kernels");
     const std::string src = kernel_source();
     if (!file_exists(src)) return fail(HRN_E_BUILD, "kernel template not found: %s", src.c_str());
     const std::string dir = cache_dir();
@@ -306,11 +319,11 @@ int compile_desc(const hrn_kernel_desc* d, double timeout_s, std::string* out_pa
     const std::string extra = env_or("HRN_HIPCC_FLAGS", "");
     uint64_t srch = fnv1a_file(src);
     for (unsigned char ch : extra) { srch ^= ch; srch *= 1099511628211ull; }
-    const std::string key = desc_key(d, srch);
+    const std::string key = desc_key(d, srch) + kPartFile[part];
     const std::string co = dir + "/" + key + ".hsaco";
     const std::string info = dir + "/" + key + ".info";
     *out_path = co;
-    if (file_exists(co) && file_exists(info)) return HRN_OK;
+    if (file_exists(co) && (part != PART_MAIN || file_exists(info))) return HRN_OK;
 
     char tmp[64];
     snprintf(tmp, sizeof tmp, ".tmp%d_%lx", (int)getpid(), (unsigned long)pthread_self());
@@ -331,6 +344,7 @@ int compile_desc(const hrn_kernel_desc* d, double timeout_s, std::string* out_pa
     def("HRN_LSPREAD", d->load_spread);
     def("HRN_COLSUM", d->colsum);
     def("HRN_NTSTORE", d->nt_store);
+    def("HRN_PART", part);
     {
         std::stringstream es(extra);
         std::string tok;
@@ -342,12 +356,12 @@ int compile_desc(const hrn_kernel_desc* d, double timeout_s, std::string* out_pa
     rc = run_hipcc(args, log, timeout_s);
     if (rc) { unlink(co_tmp.c_str()); unlink(log.c_str()); return rc; }
 
-    std::ifstream lf(log);
-    std::stringstream ss;
-    ss << lf.rdbuf();
-    const std::string ls = ss.str();
     const std::string info_tmp = info + tmp;
-    {
+    if (part == PART_MAIN) {
+        std::ifstream lf(log);
+        std::stringstream ss;
+        ss << lf.rdbuf();
+        const std::string ls = ss.str();
         std::ofstream o(info_tmp);
         o << "vgprs " << parse_remark(ls, " VGPRs: ") << "\n"
           << "agprs " << parse_remark(ls, "AGPRs: ") << "\n"
@@ -358,8 +372,43 @@ int compile_desc(const hrn_kernel_desc* d, double timeout_s, std::string* out_pa
     }
     unlink(log.c_str());
     if (rename(co_tmp.c_str(), co.c_str()) != 0) return fail(HRN_E_BUILD, "rename %s failed", co.c_str());
-    rename(info_tmp.c_str(), info.c_str());
+    if (part == PART_MAIN) rename(info_tmp.c_str(), info.c_str());
     return HRN_OK;
+}
+
+int load_part(const std::string& path, int part, bool deep, CodeObject* out) {
+    CodeObject c;
+    hipError_t e = hipModuleLoad(&c.mod, path.c_str());
+    if (e != hipSuccess) return fail(HRN_E_LOAD, "hipModuleLoad(%s): %s", path.c_str(), hipGetErrorString(e));
+    const std::string name = kPartKernel[part];
+    e = hipModuleGetFunction(&c.fn[0], c.mod, name.c_str());
+    if (e == hipSuccess && deep) e = hipModuleGetFunction(&c.fn[1], c.mod, (name + "_deep").c_str());
+    if (e != hipSuccess) {
+        (void)hipModuleUnload(c.mod);
+        return fail(HRN_E_LOAD, "hipModuleGetFunction(%s): %s", name.c_str(), hipGetErrorString(e));
+    }
+    *out = c;
+    return HRN_OK;
+}
+
+// The channels-first kernels of a module: compiled and loaded here if hrn_build did not find them in the cache.
+int chw_kernels(const hrn_module* m, int part, const CodeObject** out) {
+    std::lock_guard<std::mutex> lock(m->part_mutex);
+    *out = &m->part[part];
+    if (m->part[part].mod) return HRN_OK;
+    std::string path;
+    int rc = compile_desc(&m->desc, part, m->timeout_s, &path);
+    if (rc) return rc;
+    int dev = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    // (loading allocates, which a thread that captures a stream may otherwise not do)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    hipError_t e = dev == m->device ? hipSuccess : hipSetDevice(m->device);
+    rc = e == hipSuccess ? load_part(path, part, m->has_deep, &m->part[part]) : fail(HRN_E_LOAD, "hipSetDevice: %s", hipGetErrorString(e));
+    if (dev != m->device) (void)hipSetDevice(dev);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return rc;
 }
 
 void read_info(const std::string& path, hrn_kernel_info* o) {
@@ -406,7 +455,7 @@ void split_shape(const hrn_kernel_desc& d, const hrn_problem* p, int* kt_per_sli
 // stage (they are accepted at the L1's rate before the first product), so fewer than 6 k-tiles or 2 MB lose; four and five stages
 // are 1 - 4 % behind three, and instances that have three already lose 3 - 8 % with more.
 bool deep_fits(const hrn_module* mod, int64_t grid, int k_tiles, int64_t operand_bytes) {
-    return mod->fn[1] && grid <= mod->deep_grid && k_tiles >= 6 && operand_bytes >= (2 << 20);
+    return mod->has_deep && grid <= mod->deep_grid && k_tiles >= 6 && operand_bytes >= (2 << 20);
 }
 
 // Extent of a convolution's result in one direction, 0 where the dilated filter is larger than the padded input: the division
@@ -508,7 +557,7 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     const int64_t a_bytes = d.op == HRN_OP_GEMM ? (int64_t)p->m * p->k * es : (int64_t)p->cn * p->ch * p->cw * p->ci * es;
     plan->deep = deep_fits(mod, total, d.split_k ? k->kt_per_slice : (int)(((int64_t)p->k * es + d.bkb - 1) / d.bkb),
                            p->batch * (a_bytes + b_bytes));
-    plan->fn = mod->fn[plan->deep];
+    plan->fn = mod->part[PART_MAIN].fn[plan->deep];
     if (d.persistent) {
         if ((int64_t)p->n * oes % 16) return fail(HRN_E_BADPARAM, "persistent instances store whole 16-byte chunks: N*%d must be a multiple of 16", oes);
         if ((int64_t)p->m * p->ldc * oes >= (1ll << 31)) return fail(HRN_E_BADPARAM, "persistent: C exceeds 2 GiB per batch entry");
@@ -1333,7 +1382,7 @@ int hrn_lds_bytes(const hrn_kernel_desc* desc) {
 
 int hrn_compile(const hrn_kernel_desc* desc, double timeout_s, char* path_out, size_t path_cap) {
     std::string path;
-    int rc = compile_desc(desc, timeout_s, &path);
+    int rc = compile_desc(desc, PART_MAIN, timeout_s, &path);
     if (rc) return rc;
     if (path_out) {
         if (path.size() + 1 > path_cap)
@@ -1343,11 +1392,19 @@ int hrn_compile(const hrn_kernel_desc* desc, double timeout_s, char* path_out, s
     return HRN_OK;
 }
 
+int hrn_compile_chw(const hrn_kernel_desc* desc, int expand, double timeout_s) {
+    Derived d;
+    int rc = derive(desc, &d);
+    if (rc || !d.has_chw) return rc;
+    std::string path;
+    return compile_desc(desc, expand ? PART_EXPAND : PART_CHW, timeout_s, &path);
+}
+
 int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
     if (!out) return fail(HRN_E_BADPARAM, "null out");
     *out = nullptr;
     std::string path;
-    int rc = compile_desc(desc, timeout_s, &path);
+    int rc = compile_desc(desc, PART_MAIN, timeout_s, &path);
     if (rc) return rc;
     int n = 0;
     if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) return fail(HRN_E_NODEVICE, "no HIP device");
@@ -1363,47 +1420,36 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
         m->epi_bytes = dv.epi_bytes;
         m->chw_bytes = dv.chw_bytes;
     }
-    hipError_t e = hipModuleLoad(&m->mod, path.c_str());
-    if (e != hipSuccess) {
-        delete m;
-        return fail(HRN_E_LOAD, "hipModuleLoad(%s): %s", path.c_str(), hipGetErrorString(e));
+    m->has_chw = dv.has_chw;
+    m->has_deep = dv.has_deep;
+    m->timeout_s = timeout_s;
+    rc = load_part(path, PART_MAIN, dv.has_deep, &m->part[PART_MAIN]);
+    const std::string stem = path.substr(0, path.size() - 6);
+    for (int part = PART_CHW; part < PARTS && !rc; ++part) {
+        const std::string co = stem + kPartFile[part] + ".hsaco";
+        if (dv.has_chw && file_exists(co)) rc = load_part(co, part, dv.has_deep, &m->part[part]);
     }
-    const std::string kernel = "hrn_mfma_kernel";
-    const bool deep = dv.has_deep;
-    auto get = [&](hipFunction_t* f, const std::string& name) {
-        if (e == hipSuccess) e = hipModuleGetFunction(f, m->mod, name.c_str());
-    };
-    get(&m->fn[0], kernel);
-    if (deep) get(&m->fn[1], kernel + "_deep");
-    if (dv.has_chw) {
-        get(&m->fn_chw[0], kernel + "_chw");
-        get(&m->fn_expand[0], kernel + "_chw_expand");
-        if (deep) get(&m->fn_chw[1], kernel + "_chw_deep");
-        if (deep) get(&m->fn_expand[1], kernel + "_chw_expand_deep");
+    int cus = 0;
+    if (!rc) {
+        hipError_t e = hipGetDevice(&m->device);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->device);
+        if (e != hipSuccess) rc = fail(HRN_E_LOAD, "device query: %s", hipGetErrorString(e));
     }
-    int dev = 0, cus = 0;
-    if (deep && e == hipSuccess) e = hipGetDevice(&dev);
-    if (deep && e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) {
-        (void)hipModuleUnload(m->mod);
-        delete m;
-        return fail(HRN_E_LOAD, "hipModuleGetFunction: %s", hipGetErrorString(e));
-    }
-    m->deep_grid = deep ? cus * (163840 / dv.deep_lds) : 0;
+    if (rc) { hrn_module_free(m); return rc; }
+    m->deep_grid = dv.has_deep ? cus * (163840 / dv.deep_lds) : 0;
     if (desc->split_k) {
         // hrn_launch_splitk_static finds the library's workspace of this device looked up already
         void* ws = nullptr;
         rc = static_scratch(&ws);
-        if (rc) { (void)hipModuleUnload(m->mod); delete m; return rc; }
+        if (rc) { hrn_module_free(m); return rc; }
     }
     m->persist_grid = 0;
     if (desc->persistent) {
         int per_cu = 0, dev = 0;
         hipDeviceProp_t pr;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->fn[0], m->info.threads, 0) != hipSuccess || per_cu < 1 ||
-            hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&pr, dev) != hipSuccess) {
-            (void)hipModuleUnload(m->mod);
-            delete m;
+        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->part[PART_MAIN].fn[0], m->info.threads, 0) != hipSuccess ||
+            per_cu < 1 || hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&pr, dev) != hipSuccess) {
+            hrn_module_free(m);
             return fail(HRN_E_LOAD, "occupancy query failed: %s", hipGetErrorString(hipGetLastError()));
         }
         m->persist_grid = per_cu * pr.multiProcessorCount;
@@ -1420,7 +1466,8 @@ int hrn_module_info(const hrn_module* mod, hrn_kernel_info* out) {
 
 void hrn_module_free(hrn_module* mod) {
     if (!mod) return;
-    (void)hipModuleUnload(mod->mod);
+    for (CodeObject& c : mod->part)
+        if (c.mod) (void)hipModuleUnload(c.mod);
     delete mod;
 }
 
@@ -1456,18 +1503,17 @@ int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, con
     return launch(mod, p, In, Filter, Out, stream);
 }
 
-int hrn_module_has_chw(const hrn_module* mod) { return mod && mod->fn_chw[0] ? 1 : 0; }
+int hrn_module_has_chw(const hrn_module* mod) { return mod && mod->has_chw ? 1 : 0; }
 
 int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn_conv_view* view, const void* In, const void* Filter,
                           void* Out, void* stream) {
     if (!mod || !p || !view) return fail(HRN_E_BADPARAM, "null argument");
-    if (!mod->fn_chw[0]) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k whose strips fit into LDS");
+    if (!mod->has_chw) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k whose strips fit into LDS");
     LaunchPlan plan;
     int rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);
     if (rc) return rc;
     if (view->out_plane < 1 || p->m % view->out_plane)
         return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
-    plan.fn = mod->fn_chw[plan.deep];
     plan.k.out_plane = view->out_plane;
     if (mod->desc.conv_window) plan.dyn_lds = std::max(plan.dyn_lds, (unsigned)mod->chw_bytes);
     if (view->expand) {
@@ -1475,11 +1521,14 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
             ((int64_t)view->in_h - 1) * view->expand + view->top >= p->ch || ((int64_t)view->in_w - 1) * view->expand + view->left >= p->cw)
             return fail(HRN_E_BADPARAM, "conv2d_chw: %d x %d pixels, %d apart (a power of two) from (%d, %d), do not lie in %d x %d",
                         view->in_h, view->in_w, view->expand, view->top, view->left, p->ch, p->cw);
-        plan.fn = mod->fn_expand[plan.deep];
         plan.k.in_h = view->in_h; plan.k.in_w = view->in_w;
         plan.k.top = view->top; plan.k.left = view->left;
         plan.k.expand_shift = __builtin_ctz((unsigned)view->expand);
     }
+    const CodeObject* kernels;
+    rc = chw_kernels(mod, view->expand ? PART_EXPAND : PART_CHW, &kernels);
+    if (rc) return rc;
+    plan.fn = kernels->fn[plan.deep];
     return run_plan(mod, p, plan, nullptr, (hipStream_t)stream);
 }
 

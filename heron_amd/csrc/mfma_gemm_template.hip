@@ -1218,7 +1218,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     }
 }
 
-// a kernel that the instance has no room for is empty, and the host never launches it
+// a deep kernel that the instance has no room for is empty, and the host never launches it
 template <bool ROOM, bool CHW, bool EXPAND, bool DEEP>
 __device__ __forceinline__ void body_if(BodyArgs a) {
     if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND, DEEP>(a);
@@ -1232,11 +1232,20 @@ __device__ __forceinline__ void body_if(BodyArgs a) {
 #define HRN_ENTRY extern "C" __global__ void __launch_bounds__(NT)
 #endif
 
+// Which kernels this code object holds: those of the instance's own launches, the channels-first ones, or those that also
+// expand their input.
+#ifndef HRN_PART
+#define HRN_PART 0
+#endif
+static_assert(HRN_PART == 0 || HAS_CHW, "the channels-first kernels of this instance have no room");
+
+#if HRN_PART == 0
 HRN_ENTRY hrn_mfma_kernel(const HrnKArgs a) { hrn_mfma_body<false, false, false>(a); }
 HRN_ENTRY hrn_mfma_kernel_deep(const HrnKArgs a) { body_if<HAS_DEEP, false, false, true>(a); }
-#if HRN_OP == 1
-HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { body_if<HAS_CHW, true, false, false>(a); }
-HRN_ENTRY hrn_mfma_kernel_chw_deep(const HrnKArgs a) { body_if<HAS_CHW && HAS_DEEP, true, false, true>(a); }
-HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { body_if<HAS_CHW, true, true, false>(a); }
-HRN_ENTRY hrn_mfma_kernel_chw_expand_deep(const HrnKArgs a) { body_if<HAS_CHW && HAS_DEEP, true, true, true>(a); }
+#elif HRN_PART == 1
+HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { hrn_mfma_body<true, false, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_deep(const HrnKArgs a) { body_if<HAS_DEEP, true, false, true>(a); }
+#else
+HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { hrn_mfma_body<true, true, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand_deep(const HrnKArgs a) { body_if<HAS_DEEP, true, true, true>(a); }
 #endif

@@ -169,18 +169,22 @@ def all_shipped():
     return out
 
 
-def _compile_one(tup):
+def _compile_one(job):
+    tup, part = job
     d = B.make_desc(*tup)
     try:
+        if part:
+            return tup, B.compile_chw(d, part == 2, 300.0), None
         return tup, B.compile_desc(d, 300.0), None
     except Exception as e:  # noqa: BLE001 - reported to the caller
         return tup, None, str(e)
 
 
 def precompile(descs, jobs=None, verbose=False):
-    """Compile descriptors into the cache with ``jobs`` parallel hipcc workers; returns the failures."""
+    """Compile descriptors into the cache with ``jobs`` parallel hipcc workers, conv instances with their channels-first
+    kernels; returns the failures."""
     jobs = jobs or min(8, os.cpu_count() or 1)
-    tups = [d.as_tuple() for d in descs]
+    tups = [(d.as_tuple(), part) for d in descs for part in ((0, 1, 2) if d.op == CONV else (0,))]
     failures = []
     with ProcessPoolExecutor(max_workers=jobs) as ex:
         for tup, path, err in ex.map(_compile_one, tups):

@@ -34,11 +34,24 @@ def _problem_to_dict(p):
     return {name: int(getattr(p, name)) for name, _ in p._fields_ if name not in ("workspace", "workspace_bytes", "bsum")}
 
 
-def _compile_worker(desc_tuple, timeout_s):
+_CHANNELS_FIRST = ('c1d_ncw', 'c2d_nchw', 'c3d_ncdhw', 't2d_nchw')       # hostops.CHANNELS_FIRST, without importing torch
+
+
+def _compile_view(desc, adapter, timeout_s):
+    """The kernels that hostops.run_operator launches for an operator whose result is channels first."""
+    from .. import backend as B
+    if adapter is None or adapter.get('adapter') not in _CHANNELS_FIRST:
+        return
+    t = adapter.get('transposed')
+    B.compile_chw(desc, t is not None and t['stride'] & (t['stride'] - 1) == 0, timeout_s)
+
+
+def _compile_worker(desc_tuple, timeout_s, adapter=None):
     from .. import backend as B
     t0 = time.time()
     try:
         B.compile_desc(B.make_desc(*desc_tuple), timeout_s)
+        _compile_view(B.make_desc(*desc_tuple), adapter, timeout_s)
         return None, time.time() - t0
     except B.HeronRocmError as e:
         return (e.code, str(e)), time.time() - t0
@@ -75,9 +88,9 @@ class HipBuilder:
                 prepared.append((None, None, None, (MeasureErrorNo.INSTANTIATION_ERROR, repr(e)), t0, None))
         ex = self._executor()
         futures = {}
-        for tup, _, _, err, _, _ in prepared:
+        for tup, _, _, err, _, adapter in prepared:
             if err is None and tup not in futures:
-                futures[tup] = ex.submit(_compile_worker, tup, float(self.timeout))
+                futures[tup] = ex.submit(_compile_worker, tup, float(self.timeout), adapter)
         results = []
         for tup, prob, arg_info, err, t0, adapter in prepared:
             if err is None:
@@ -393,6 +406,7 @@ class HipRunner:
         time_evaluator; returns the mean seconds per launch."""
         from .. import backend as B
         B.compile_desc(s.to_desc(), 300.0)
+        _compile_view(s.to_desc(), s.info, 300.0)
         req = ("measure", s.to_desc().as_tuple(), _problem_to_dict(s.to_problem()),
                [(tuple(t.shape), t.dtype) for t in args], number, repeat, float(min_repeat_ms), None, None, 0.1, cold,
                dict(s.info) if s.info.get('adapter', 'identity') != 'identity' else None)

@@ -166,6 +166,12 @@ int hrn_check_desc(const hrn_kernel_desc* desc);
  */
 int hrn_compile(const hrn_kernel_desc* desc, double timeout_s, char* path_out, size_t path_cap);
 
+/*
+ * The kernels hrn_launch_conv2d_chw launches, without (expand 0) or with a zero-expanded input: code objects of their own,
+ * compiled ahead like the instance itself.  Nothing to do for an instance without them (HRN_OK).
+ */
+int hrn_compile_chw(const hrn_kernel_desc* desc, int expand, double timeout_s);
+
 /* hrn_compile + load on the current device.  Stands in for the module loader of
  * runner/measure_methods.py:129-130. */
 int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out);
@@ -220,7 +226,8 @@ int hrn_launch_splitk_static(const hrn_module* mod, const hrn_problem* p, const 
  *   expand > 0 (a power of two): the problem's ch x cw input is not in memory; In holds (cn, in_h, in_w, ci), pixel (y, x)
  * of which stands at (top + y*expand, left + x*expand) of ch x cw, everything else is zero.
  * The instance is a conv2d one for which hrn_module_has_chw says 1: not persistent, no split_k, and the strips of its
- * epilogue fit into LDS; p->ldc does not apply.
+ * epilogue fit into LDS; p->ldc does not apply.  Kernels that hrn_compile_chw has not put into the cache before hrn_build are
+ * compiled by the first launch that needs them.
  */
 typedef struct hrn_conv_view {
     int32_t out_plane;

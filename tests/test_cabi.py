@@ -106,6 +106,36 @@ def test_compile_without_gpu_and_shipped_instances_present():
     assert os.path.exists(path[:-6] + ".info")
 
 
+def test_channels_first_kernels_are_compiled_apart(tmp_path, monkeypatch):
+    """A conv instance alone is one code object; the channels-first kernels are compiled for those that ask, and an instance
+    without them has nothing to compile."""
+    monkeypatch.setenv("HRN_CACHE_DIR", str(tmp_path))
+    conv = instances.D(instances.F16, instances.CONV, 64, 64, 64, 2, 2, 32, 2, 2)
+
+    def built():
+        return sorted(f.name for f in tmp_path.glob("*.hsaco"))
+    own = os.path.basename(B.compile_desc(conv, 120.0))
+    assert built() == [own]
+    B.compile_chw(conv, False, 120.0)
+    assert built() == sorted([own, own[:-6] + "_chw.hsaco"])
+    B.compile_chw(conv, True, 120.0)
+    assert built() == sorted([own, own[:-6] + "_chw.hsaco", own[:-6] + "_expand.hsaco"])
+    for d in (instances.BEST["small"], instances.splitk_descs()[4], instances.D(instances.F16, instances.CONV, 128, 64, 128, 2, 1, 32, 2, 1, epi=1, pers=1)):
+        B.compile_chw(d, False, 120.0)
+    assert len(built()) == 3
+    # the builder compiles what the operator launches
+    from heron_amd import hostops
+    from heron_amd.runner import measure_methods as mm
+    assert set(mm._CHANNELS_FIRST) == set(hostops.CHANNELS_FIRST)
+    for info, kinds in (({'adapter': 'c2d_hwio'}, 0), ({'adapter': 'c1d_ncw'}, 1), ({'adapter': 't2d_nchw', 'transposed': {'stride': 3}}, 1),
+                        ({'adapter': 't2d_nchw', 'transposed': {'stride': 2}}, 2)):
+        for f in tmp_path.iterdir():
+            f.unlink()
+        err, _ = mm._compile_worker(conv.as_tuple(), 120.0, info)
+        want = {0: [own], 1: [own, own[:-6] + "_chw.hsaco"], 2: [own, own[:-6] + "_expand.hsaco"]}[kinds]
+        assert err is None and built() == sorted(want)
+
+
 def test_compile_error_paths(tmp_path, monkeypatch):
     """A path buffer that is too small, a compiler that fails and a compiler that outlives the limit are reported as
     errors with a message; nothing is left in the cache for them."""

@@ -183,3 +183,36 @@ def test_a_recorded_split_k_plan_owns_its_workspace(hrn):
     assert torch.equal(plan.run(), want)
     assert all(bool((t == 7.0).all()) for t in other)
     mod.close()
+
+
+@pytest.mark.parametrize("captured", [False, True])
+def test_channels_first_kernels_of_an_instance_not_prepared_for_them(captured, hrn, tmp_path, monkeypatch):
+    """hrn_build finds no such code objects in the cache: the first launch compiles and loads them, also inside a capture."""
+    monkeypatch.setenv("HRN_CACHE_DIR", str(tmp_path))
+    mod, full = B.Module(CONV_F16), {}
+    monkeypatch.undo()
+    ready = B.Module(CONV_F16)
+    monkeypatch.setenv("HRN_CACHE_DIR", str(tmp_path))
+    for op in ("c2d_nchw", "t2d"):
+        info = declared(op, CHANNELS_FIRST[op])
+        gen = torch.Generator(device="cuda").manual_seed(11)
+        X = torch.randn(info["reference_args"]["input"], device="cuda", generator=gen).half()
+        F = torch.randn(info["reference_args"]["filter"], device="cuda", generator=gen).half()
+        weights = hostops.prepare_constant(info, [X, F])
+        want = hostops.run_operator(ready, info, [X, F], constant=weights)
+        torch.cuda.synchronize()
+        if captured:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                got = hostops.run_operator(mod, info, [X, F], constant=weights)
+            for _ in range(3):
+                got.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(got, want)
+        else:
+            assert torch.equal(hostops.run_operator(mod, info, [X, F], constant=weights), want)
+        full[op] = len(list(tmp_path.glob("*.hsaco")))
+    assert full == {"c2d_nchw": 2, "t2d": 3}
+    mod.close()
+    ready.close()
