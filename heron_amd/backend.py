@@ -172,6 +172,7 @@ SYMBOLS = {
     "hrn_compile_chw": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
     "hrn_module_has_chw": (_i, [_vp]),
     "hrn_launch_conv2d_chw": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(ConvView), _vp, _vp, _vp, _vp]),
+    "hrn_launch_is_deep": (_i, [_vp, ctypes.POINTER(Problem)]),
     "hrn_launch_splitk_static": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_launch_repeat": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _i, _vp]),
     "hrn_time": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _i, _i, _d, ctypes.POINTER(_d), _vp]),
@@ -435,6 +436,13 @@ class Module:
         self.bind_workspace(problem)
         self.bind_colsum(problem, b_ptr, stream)
         _check(self._launcher(problem)(self._h, ctypes.byref(problem), a_ptr, b_ptr, c_ptr, stream))
+
+    def is_deep(self, problem):
+        """Whether a launch of ``problem`` takes the instance's deep kernel."""
+        rc = lib().hrn_launch_is_deep(self._h, ctypes.byref(problem))
+        if rc < 0:
+            _check(rc)
+        return rc == 1
 
     def launch_conv2d_chw(self, problem, view, a_ptr, b_ptr, c_ptr, stream=0):
         """conv2d with a channels-first result and, where ``view.expand`` is set, a zero-expanded input (hrn_conv_view)."""

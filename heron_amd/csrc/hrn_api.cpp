@@ -221,10 +221,12 @@ int derive(const hrn_kernel_desc* d, Derived* o) {
     int tiles = 64 / d->mfma;
     while (tiles > 1 && (r.tm % tiles || chw(tiles) + stay > 163840)) --tiles;
     r.chw_bytes = chw(tiles);
-    // deep kernels: a third stage
+    r.has_chw = d->op == HRN_OP_CONV2D && !d->persistent && !d->split_k && r.chw_bytes + stay <= 163840;
+    // deep kernels: a third stage.  The strips count for every instance, also where it has no channels-first kernels: for one
+    // whose strips are more than its stages (u8 x s8 128x128 tiles, 64-byte rows, 8 waves: 71 and 48 KiB) the grids of two to
+    // three workgroups a CU lose 1 - 2.7 % with three stages at 8 and 16 k-tiles and gain 0.4 - 0.9 % at 64.
     r.deep_lds = std::max(std::max(r.lds, r.chw_bytes), 3 * r.stage_bytes);
     r.has_deep = d->stages == 2 && !d->conv_window && !d->persistent && 3 * r.stage_bytes <= 163840 && 2 * r.lpt <= 63;
-    r.has_chw = d->op == HRN_OP_CONV2D && !d->persistent && !d->split_k && r.chw_bytes + stay <= 163840;
     // (a conv_window instance keeps the epilogue region in its dynamic LDS, where the window was)
     if (r.lds > 163840) return fail(HRN_E_BADPARAM, "LDS %d > 163840", r.lds);
     if (d->swizzle && (r.cpr << (d->swizzle - 1)) > d->mfma)
@@ -449,8 +451,8 @@ void split_shape(const hrn_kernel_desc& d, const hrn_problem* p, int* kt_per_sli
 }
 
 // Two stages leave a k-tile's loads one k-tile of multiplication to arrive, enough from a near L2 but not from further away; two
-// stages were chosen so that several workgroups fit a CU, and a grid that the device holds at once with three has no other use
-// for that LDS.  128x128 fp16, 9 x 12 tiles, inputs of three calls in turn: 41.9 -> 33.8 us at 64 k-tiles, 16.3 -> 14.0 at 15,
+// stages were chosen so that several workgroups fit a CU, and a grid whose LDS the device has at once with three (deep_lds) has
+// no other use for it.  128x128 fp16, 9 x 12 tiles, inputs of three calls in turn: 41.9 -> 33.8 us at 64 k-tiles, 16.3 -> 14.0 at 15,
 // 8.7 -> 8.9 at 4; 4 x 4 tiles 30.4 -> 22.5 at 40, 12.9 -> 13.0 at 20 (2.6 MB of operands).  The first tiles take 0.2 us longer per
 // stage (they are accepted at the L1's rate before the first product), so fewer than 6 k-tiles or 2 MB lose; four and five stages
 // are 1 - 4 % behind three, and instances that have three already lose 3 - 8 % with more.
@@ -1501,6 +1503,23 @@ int hrn_launch_bmm_u8s8(const hrn_module* mod, const hrn_problem* p, const void*
 int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, const void* In, const void* Filter, void* Out, void* stream) {
     if (mod && (mod->desc.dtype != HRN_DT_U8S8 || mod->desc.op != HRN_OP_CONV2D)) return fail(HRN_E_BADPARAM, "module is not a u8s8 conv2d");
     return launch(mod, p, In, Filter, Out, stream);
+}
+
+int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p) {
+    if (!mod || !p) return fail(HRN_E_BADPARAM, "null argument");
+    // (the operands' addresses decide nothing; what a launch would have to bring is filled in)
+    void* any = (void*)(uintptr_t)256;
+    hrn_problem q = *p;
+    if (mod->desc.colsum && !q.bsum) q.bsum = any;
+    if (mod->desc.split_k) {
+        q.split_k = std::max(1, q.split_k);
+        const int64_t need = hrn_splitk_workspace_bytes(&mod->desc, &q);
+        if (need < 0) return (int)need;
+        q.workspace_bytes = (size_t)need;
+    }
+    LaunchPlan plan;
+    int rc = fill_args(mod, &q, any, any, any, any, q.workspace_bytes, &plan);
+    return rc ? rc : (plan.deep ? 1 : 0);
 }
 
 int hrn_module_has_chw(const hrn_module* mod) { return mod && mod->has_chw ? 1 : 0; }

@@ -128,6 +128,16 @@ def chw_room_descs():
     return [D(U8, CONV, 256, 256, 64, 4, 4, 32, 2, 1, win=1)]
 
 
+def deep_descs():
+    """Two-stage instances with one k-step per k-tile: the register buffers alternate per tile, in the deep kernels over
+    three stages."""
+    return [
+        D(F16, GEMM, 128, 128, 64, 2, 2, 16, 2, 3),
+        D(U8, GEMM, 128, 128, 64, 2, 2, 16, 2, 3, epi=1),
+        D(F16, CONV, 128, 64, 64, 2, 2, 16, 2, 3, epi=1),
+    ]
+
+
 def persistent_descs():
     """Instances of the persistent (tile-stream) mode in the parity suite: short and long K streams, both element
     kinds, 2..4 stages, implicit-GEMM conv."""
@@ -161,8 +171,8 @@ BEST = {
 
 def all_shipped():
     seen, out = set(), []
-    for d in (parity_descs() + variant_descs() + int8_conv_descs() + chw_room_descs() + persistent_descs() + persistent_twin_descs()
-              + splitk_descs() + list(BEST.values())):
+    for d in (parity_descs() + variant_descs() + int8_conv_descs() + chw_room_descs() + deep_descs() + persistent_descs()
+              + persistent_twin_descs() + splitk_descs() + list(BEST.values())):
         if d.as_tuple() not in seen:
             seen.add(d.as_tuple())
             out.append(d)

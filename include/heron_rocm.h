@@ -202,6 +202,12 @@ int hrn_launch_bmm_u8s8(const hrn_module* mod, const hrn_problem* p, const void*
 int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, const void* In, const void* Filter, void* Out, void* stream);
 
 /*
+ * Which kernel a launch of `p` takes: 1 = the deep one (an instance of two stages carries a kernel with a third, for grids that
+ * leave its LDS free), 0 = the plain one, negative = the launch would be refused.  hrn_launch_conv2d_chw decides alike.
+ */
+int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
+
+/*
  * Split-K launch that allocates nothing.  No counterpart in the reference; it is for callers that cannot allocate
  * device memory around a launch (code under HIP graph capture, tight serving loops, harnesses that forbid it).  Same as
  * launching a split_k instance through the entry points above, except that the partial sums go to a workspace that
