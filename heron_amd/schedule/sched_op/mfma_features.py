@@ -94,6 +94,22 @@ def featurize(info, values):
     return feats
 
 
+def inert_knobs(info, values):
+    """Knob variables that the kernel template does not read at this point, at their defaults: points that differ in nothing
+    else are the same kernel.  The tiles of the template's phased schedule (PHASED there) run it whatever the issue order and
+    the load spread are."""
+    stage = info['stage_name']
+    v = {k: _get(values, stage, k, True) for k in KNOBS}
+    bm, bn = _get(values, stage, 'block_m', False), _get(values, stage, 'block_n', False)
+    phased = (info['operator'] != 'conv2d_nhwc' and bm == bn == 256 and v['block_k_bytes'] == 128 and v['lds_stages'] == 2 and
+              v['wave_m'] * v['wave_n'] == 8 and v['wave_m'] in (2, 4) and not v['persistent'] and v['split_k'] <= 1 and
+              (info['kind'] == 'f16' or v['column_sums'] == 1))
+    if not phased:
+        return {}
+    key = "P#ST:%s,AX:None,PA:%s"
+    return {key % (stage, 'issue_order'): 1, key % (stage, 'load_spread'): 2}
+
+
 def view_of_values(info, values):
     """``info`` with the GEMM view of the task the point was solved for (a record of another task of the same
     operator carries that task's padded extents: cover - waste of each tiled axis; the batch is taken as equal)."""

@@ -11,6 +11,7 @@ import os
 from ..schedule.constraints import KnobManager
 from ..schedule.context import buildContext
 from ..schedule.sched_op import TemplateSchedule, get_op_methods, sched_via_rule
+from ..utils import Code, DeCode
 
 
 class Task:
@@ -116,6 +117,16 @@ class Task:
         from ..schedule.sched_op.mfma_features import featurize, view_of_values
         info = self.template_info if own_shape else view_of_values(self.template_info, values)
         return featurize(info, values)
+
+    def instance_code(self, code):
+        """A point's text form with the knobs that the template does not read there at their defaults: equal for points
+        that make the same kernel, so that a search builds and times it once."""
+        if self.template_info is None or self.config is None or self.config.codegen_type != 'GPU_MFMA':
+            return code
+        from ..schedule.sched_op.mfma_features import inert_knobs
+        names, point = list(self.knob_manager.solver.vals), DeCode(code)
+        inert = inert_knobs(self.template_info, dict(zip(names, point)))
+        return Code([inert.get(n, v) for n, v in zip(names, point)]) if inert else code
 
     def coupled_moves(self, knob_manager):
         """(label, knob dictionary) pairs a few coordinated knob changes away from the point ``knob_manager`` holds

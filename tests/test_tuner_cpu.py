@@ -631,3 +631,65 @@ def test_coupled_moves_reach_the_other_row_length_and_the_other_mfma_edge():
     assert any(m['mfma'] == 32 and m['tile_m'] == 2 and m['tile_n'] == 4 and m['block_k_bytes'] == 64 for m in feasible)
     # every move keeps the block tile: rows per wave tile x wave grid unchanged
     assert all(m['tile_m'] * m['mfma'] == 64 and m['tile_n'] * m['mfma'] == 128 for m in map(short, moves))
+
+
+def _code_of(path):
+    """The machine code of a code object: the .text section of the ELF image inside the offload bundle."""
+    import struct
+    blob = open(path, "rb").read()
+    elf = blob[blob.index(b"\x7fELF"):]
+    shoff, = struct.unpack_from("<Q", elf, 40)
+    size, count, names = struct.unpack_from("<HHH", elf, 58)
+    heads = [struct.unpack_from("<IIQQQQ", elf, shoff + i * size) for i in range(count)]
+    table = heads[names][4]
+    for name, _, _, _, off, length in heads:
+        if elf[table + name:elf.index(b"\0", table + name)] == b".text":
+            return elf[off:off + length]
+    raise AssertionError("no code in " + path)
+
+
+def test_points_of_one_kernel_are_searched_once(tmp_path, monkeypatch):
+    """Where the phased schedule leaves issue order and load spread without effect, points that differ in them only count as
+    one kernel: they compile to the same code, and the search drops them as measured; other tiles keep them apart."""
+    from heron_amd.sample import Sample
+    from heron_amd.tuner.tuner import Tuner
+    from heron_amd.utils import Code
+    monkeypatch.setenv("HRN_CACHE_DIR", str(tmp_path))
+    cfg = Config()
+    cfg.codegen_type = 'GPU_MFMA'
+    t = Task("t", getOpFromName("gemm"), [8192, 8192, 8192, "int8", "int8"], "rocm")
+    t.config = cfg
+    t.make_stage_schedules()
+    base = dict(mfma=16, wave_m=4, wave_n=2, tile_m=4, tile_n=8, block_k_bytes=128, lds_stages=2, lds_swizzle=1, persistent=0, split_k=1,
+                conv_window=0, epilogue=0, column_sums=1, issue_order=1, load_spread=2)
+
+    def sample(**change):
+        s = Sample(t)
+        knobs = {}
+        for n in s.knob_manager.knob_names:
+            short = n.split("PA:")[-1]
+            knobs[n] = dict(base, **change).get(short, s.knob_manager.get_knob_candidates(n)[0])
+        point, valid = s.knob_manager.validate(knobs)
+        assert valid, change
+        s.point, s.valid, s.stmt_code, s.predict = point, True, Code(point), 0.0
+        return s
+
+    def kernel(s):
+        sched, _ = t.instantiate(copy.deepcopy(s.knob_manager))
+        return _code_of(B.compile_desc(sched.to_desc(), 120.0))
+
+    class Buf:
+        perfs = {}
+    env = type("Env", (), dict(perf_buffer=Buf, task=t))
+    tuner = Tuner(cfg)
+    phased = [sample(), sample(issue_order=0), sample(load_spread=0), sample(issue_order=0, load_spread=3)]
+    assert len({s.stmt_code for s in phased}) == 4 and len({kernel(s) for s in phased}) == 1
+    assert tuner.FilterSamples(phased, env) == phased[:1]
+    Buf.perfs = {phased[3].stmt_code: 1.0}
+    assert tuner.FilterSamples(phased, env) == []
+    near = tuner.one_knob_neighbours(env, phased[1], skip=[phased[1].stmt_code])
+    assert near and not any(t.instance_code(s.stmt_code) == t.instance_code(phased[0].stmt_code) for s in near)
+    # column sums in the loop: not phased
+    Buf.perfs = {}
+    rows = [sample(column_sums=0), sample(column_sums=0, issue_order=0), sample(column_sums=0, load_spread=0)]
+    assert len({kernel(s) for s in rows}) == 3 and tuner.FilterSamples(rows, env) == rows
