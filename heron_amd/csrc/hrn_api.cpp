@@ -171,8 +171,6 @@ int derive(const hrn_kernel_desc* d, Derived* o) {
     if (d->colsum < 0 || d->colsum > 1 || (d->colsum && d->dtype != HRN_DT_U8S8))
         return fail(HRN_E_BADPARAM, "colsum %d (caller-supplied column sums are an option of the u8s8 instances)", d->colsum);
     if (d->nt_store < 0 || d->nt_store > 1) return fail(HRN_E_BADPARAM, "nt_store %d (0 or 1)", d->nt_store);
-    if (d->sched == 2 && (d->wm * d->wn != 8 || d->conv_window || d->persistent || d->split_k))
-        return fail(HRN_E_BADPARAM, "sched 2 needs 8 waves and neither conv_window, persistent nor split_k");
     Derived r;
     r.es = d->dtype == HRN_DT_F16 ? 2 : 1;
     r.oes = (d->dtype == HRN_DT_F16 && !d->split_k) ? 2 : 4;
@@ -242,11 +240,14 @@ int derive(const hrn_kernel_desc* d, Derived* o) {
     return HRN_OK;
 }
 
+// the issue order the template is built with: 2 is another name of 1
+int issue_order(const hrn_kernel_desc* d) { return d->sched ? 1 : 0; }
+
 std::string desc_key(const hrn_kernel_desc* d, uint64_t srch) {
     char b[256];
     snprintf(b, sizeof b, "hrn_d%d_o%d_m%dn%dk%d_w%dx%d_t%d_s%d_z%d_e%d_p%d_c%d_r%d_k%d_i%d_l%d_b%d_n%d_%08x", d->dtype, d->op, d->bm, d->bn,
              d->bkb, d->wm, d->wn, d->mfma, d->stages, d->swizzle, d->epilogue, d->waves_per_eu, d->conv_window,
-             d->persistent, d->split_k, d->sched, d->load_spread, d->colsum, d->nt_store, (unsigned)(srch ^ (srch >> 32)));
+             d->persistent, d->split_k, issue_order(d), d->load_spread, d->colsum, d->nt_store, (unsigned)(srch ^ (srch >> 32)));
     return b;
 }
 
@@ -342,7 +343,7 @@ int compile_desc(const hrn_kernel_desc* d, int part, double timeout_s, std::stri
     def("HRN_CONVWIN", d->conv_window);
     def("HRN_PERSIST", d->persistent);
     def("HRN_SPLITK", d->split_k);
-    def("HRN_SCHED", d->sched);
+    def("HRN_SCHED", issue_order(d));
     def("HRN_LSPREAD", d->load_spread);
     def("HRN_COLSUM", d->colsum);
     def("HRN_NTSTORE", d->nt_store);

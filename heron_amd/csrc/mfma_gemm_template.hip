@@ -100,8 +100,8 @@ constexpr bool COLSUM = (HRN_DTYPE == 1) && (HRN_COLSUM != 0);
 #define HRN_NTSTORE 0
 #endif
 constexpr bool NTS = (HRN_NTSTORE != 0) && (HRN_SPLITK == 0);
-// Issue order of a k-step: 1 and 2 = the source order of the row groups is pinned (a scheduling fence after every row
-// of MFMAs), 0 = the compiler interleaves on its own, guided by group hints (one LDS read per few MFMAs).  Tiles that
+// Issue order of a k-step: 1 = the source order of the row groups is pinned (a scheduling fence after every row of
+// MFMAs), 0 = the compiler interleaves on its own, guided by group hints (one LDS read per few MFMAs).  Tiles that
 // PHASED (below) takes run the phased schedule whatever this says.
 #ifndef HRN_SCHED
 #define HRN_SCHED 1

@@ -87,10 +87,10 @@ typedef struct hrn_kernel_desc {
                              output tiles).  Not with persistent or conv_window. */
     int32_t sched;        /* issue order of a k-step: 1 = the template's own interleaving of fragment reads, tile loads
                              and MFMAs is pinned with scheduling fences, 0 = left to the compiler under group hints,
-                             2 = as 1 (8 waves, no conv_window / persistent / split_k).  256x256 tiles of 128-byte rows
-                             in two stages on 2x4 or 4x2 waves (GEMM; fp16, or u8s8 with colsum) run the template's
-                             phased schedule in any case: the two waves of a SIMD alternate between a phase that only
-                             moves data and one that only multiplies */
+                             2 = another name of 1 (the same code object).  256x256 tiles of 128-byte rows in two stages
+                             on 2x4 or 4x2 waves (GEMM; fp16, or u8s8 with colsum) run the template's phased schedule in
+                             any case: the two waves of a SIMD alternate between a phase that only moves data and one that
+                             only multiplies */
     int32_t load_spread;  /* with sched = 1: how far the wave loads of the next k-tile are spread over the MFMA rows of the
                              step that issues them: 0 = all right behind the barrier, 1 = over a quarter of the rows,
                              2 = half, 3 = all but the last two (smoother demand on the L2, later arrival) */

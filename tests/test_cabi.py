@@ -195,3 +195,15 @@ def test_gather_rejects_bad_maps_without_a_gpu():
     assert L.hrn_gather_nd(ctypes.byref(g), p, None, p, None) == B.HRN_E_BADPARAM
     g = B.make_gather(2, (0, 8), [(4, 8, {0: 1}), (8, 1, {1: 1})])                          # nothing to do is not an error
     assert L.hrn_gather_nd(ctypes.byref(g), p, None, p, None) == 0
+
+
+def test_second_name_of_the_pinned_issue_order():
+    """sched 2 names the code object of sched 1, for every instance that has one."""
+    conv = dict(op=B.HRN_OP_CONV2D, bm=64, bn=64, bkb=64, swizzle=2)
+    for kw in (dict(bm=64, bn=64, wm=1, wn=1, stages=3), conv):
+        paths = []
+        for sched in (1, 2):
+            d = B.make_desc(B.HRN_DT_F16, sched=sched, **kw)
+            assert B.check_desc(d)
+            paths.append(B.compile_desc(d, 120.0))
+        assert paths[0] == paths[1]
