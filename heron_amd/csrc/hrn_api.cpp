@@ -990,8 +990,10 @@ __global__ void __launch_bounds__(256) transpose_pad_kernel(const void* __restri
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= tiles) return;
     const int lane = threadIdx.x & 63;
-    const int r0 = (t / tiles_c) * TILE + (lane >> 3) * V, c0 = (t % tiles_c) * TILE + (lane & 7) * V;
-    if (c0 >= cols || r0 >= rp) return;
+    const unsigned row0 = (unsigned)(t / tiles_c) * TILE + (lane >> 3) * V;          // (either may pass 2^31 by a tile)
+    const unsigned col0 = (unsigned)(t % tiles_c) * TILE + (lane & 7) * V;
+    if (col0 >= (unsigned)cols || row0 >= (unsigned)rp) return;
+    const int r0 = (int)row0, c0 = (int)col0;
     const T* in = (const T*)src + blockIdx.z * (size_t)rows * cols + (size_t)r0 * cols + c0;
     T* out = (T*)dst + blockIdx.z * (size_t)cols * rp + (size_t)c0 * rp + r0;
     pv4i x[V];                               // rows of the block
@@ -1131,7 +1133,6 @@ int hrn_transpose_pad(const void* src, void* dst, int batch, int rows, int cols,
         (elem_bytes != 1 && elem_bytes != 2 && elem_bytes != 4))
         return fail(HRN_E_BADPARAM, "transpose_pad: batch %d, %d x %d -> %d x %d, %d-byte elements", batch, rows, cols, cols, rows_padded, elem_bytes);
     if (batch == 0) return HRN_OK;
-    if (((int64_t)rows_padded + 63) / 64 > 65535) return fail(HRN_E_BADPARAM, "transpose_pad: %d rows are more than 65535 tiles", rows_padded);
     const int64_t tile = 8 * (16 / elem_bytes), tiles_c = (cols + tile - 1) / tile, tiles = tiles_c * ((rows_padded + tile - 1) / tile);
     if (tiles >= (1ll << 31)) return fail(HRN_E_BADPARAM, "transpose_pad: %d x %d is more than one launch covers", rows_padded, cols);
     const dim3 grid((unsigned)((tiles + 3) / 4), 1, batch);

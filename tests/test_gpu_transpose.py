@@ -22,3 +22,14 @@ def test_edges(dtype, hrn):
         B.transpose_pad(x.data_ptr(), out.data_ptr(), b, r, c, rp, x.element_size(), st)
         torch.cuda.synchronize()
         assert torch.equal(out, torch.nn.functional.pad(x.permute(0, 2, 1), (0, rp - r))), (dtype, b, r, c, rp)
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.float16, torch.int32])
+def test_more_rows_than_one_grid_dimension_of_tiles(dtype, hrn):
+    rows, cols = 65535 * 64 + 9, 3
+    x = torch.randint(0, 120, (rows, cols), device="cuda").to(dtype)
+    for rp in (rows, rows + 7):
+        out = torch.full((cols, rp), 9, dtype=dtype, device="cuda")
+        print("transpose", dtype, rows, cols, rp, flush=True)
+        B.transpose_pad(x.data_ptr(), out.data_ptr(), 1, rows, cols, rp, x.element_size(), torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(out, torch.nn.functional.pad(x.t(), (0, rp - rows)))
