@@ -127,6 +127,18 @@ def chw_room_descs():
     return [D(U8, CONV, 256, 256, 64, 4, 4, 32, 2, 1, win=1)]
 
 
+def phased_descs():
+    """256x256 tiles of the phased schedule that no other list holds: uint8 with B the operand of more fragments, 32x32 MFMAs
+    on both wave grids."""
+    return [
+        D(U8, GEMM, 256, 256, 128, 4, 2, 16, 2, 1, colsum=1),
+        D(U8, GEMM, 256, 256, 128, 4, 2, 32, 2, 1, epi=1, colsum=1),
+        D(U8, GEMM, 256, 256, 128, 2, 4, 32, 2, 1, colsum=1),
+        D(F16, GEMM, 256, 256, 128, 2, 4, 32, 2, 1),
+        D(F16, GEMM, 256, 256, 128, 4, 2, 32, 2, 1, epi=1),
+    ]
+
+
 def deep_descs():
     """Two-stage instances with one k-step per k-tile: the register buffers alternate per tile, in the deep kernels over
     three stages."""
@@ -170,8 +182,8 @@ BEST = {
 
 def all_shipped():
     seen, out = set(), []
-    for d in (parity_descs() + variant_descs() + int8_conv_descs() + chw_room_descs() + deep_descs() + persistent_descs()
-              + persistent_twin_descs() + splitk_descs() + list(BEST.values())):
+    for d in (parity_descs() + variant_descs() + int8_conv_descs() + chw_room_descs() + phased_descs() + deep_descs()
+              + persistent_descs() + persistent_twin_descs() + splitk_descs() + list(BEST.values())):
         if d.as_tuple() not in seen:
             seen.add(d.as_tuple())
             out.append(d)

@@ -1,12 +1,13 @@
 """The phased schedule of the 256x256 tiles: K from one chunk over one, two and three k-tiles to a ragged last one, M and N
-around the tile edge, both wave grids, against the host references (uint8 bit-exact)."""
+around the tile edge, both wave grids and both MFMA shapes in either element type, against the host references (uint8
+bit-exact)."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
 from heron_amd import backend as B
-from heron_amd import hostops, instances, workloads
+from heron_amd import hostops, instances, tuned, workloads
 from parity_checks import check_f16
 
 pytestmark = pytest.mark.gpu
@@ -16,6 +17,13 @@ INSTANCES = {
     "f16-4x2": D(F16, GEMM, 256, 256, 128, 4, 2, 16, 2, 1, epi=2, sched=2),
     "f16-2x4": D(F16, GEMM, 256, 256, 128, 2, 4, 16, 2, 2),
     "u8s8-2x4": D(U8, GEMM, 256, 256, 128, 2, 4, 16, 2, 1, colsum=1),
+    "u8s8-4x2": instances.phased_descs()[0],
+    "u8s8-4x2-32x32": instances.phased_descs()[1],
+    "u8s8-2x4-32x32": instances.phased_descs()[2],
+    "f16-2x4-32x32": instances.phased_descs()[3],
+    "f16-4x2-32x32": instances.phased_descs()[4],
+    "u8s8-tuned": tuned.load("gemm_u8s8_8192").desc,
+    "f16-tuned": tuned.load("gemm_f16_8192").desc,
 }
 
 
