@@ -1062,9 +1062,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     // A half that has been read by everybody (it was read in step i, waited for in step i + 1) is refilled in step i + 2 or
     // later: step 1 fetches X0 and Y0, step 2 Y1, step 3 X1 of T + 2.  So every fetch has four to five steps (about 1.2 us)
     // to arrive, and a wait allows for the fetches that were issued after the half it is about.
-    //   8192^3: matrix pipes busy in 83 % (fp16) and 73 % (u8 x s8) of the cycles, 75 and 62 % with the row-by-row schedule;
-    // what bounds it then is power (the clock falls to 1.6 - 1.7 GHz): without the fetches in the loop the cycles fall
-    // by 4 %, the time by 12 %.
+    //   8192^3: matrix pipes busy in 81 % (fp16) and 73 % (u8 x s8) of the cycles, 73 - 76 and 60 % with the row-by-row
+    // schedule; what bounds it then is power (the clock falls to 1.7 - 1.8 GHz): without the fetches in the loop the cycles fall
+    // by 8.5 and 5 %, the time by 14 and 12 %.
     constexpr int HM = TM / 2, HN = TN / 2;                          // MFMA tiles of a half
     constexpr bool XA = TM >= TN;                                    // X is A
     constexpr int RA = HM * KS, RB = HN * KS;                        // fragments of a half
