@@ -990,10 +990,8 @@ __global__ void __launch_bounds__(256) transpose_pad_kernel(const void* __restri
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= tiles) return;
     const int lane = threadIdx.x & 63;
-    const unsigned row0 = (unsigned)(t / tiles_c) * TILE + (lane >> 3) * V;          // (either may pass 2^31 by a tile)
-    const unsigned col0 = (unsigned)(t % tiles_c) * TILE + (lane & 7) * V;
-    if (col0 >= (unsigned)cols || row0 >= (unsigned)rp) return;
-    const int r0 = (int)row0, c0 = (int)col0;
+    const int r0 = (t / tiles_c) * TILE + (lane >> 3) * V, c0 = (t % tiles_c) * TILE + (lane & 7) * V;
+    if (c0 >= cols || r0 >= rp) return;
     const T* in = (const T*)src + blockIdx.z * (size_t)rows * cols + (size_t)r0 * cols + c0;
     T* out = (T*)dst + blockIdx.z * (size_t)cols * rp + (size_t)c0 * rp + r0;
     pv4i x[V];                               // rows of the block
@@ -1134,7 +1132,9 @@ int hrn_transpose_pad(const void* src, void* dst, int batch, int rows, int cols,
         return fail(HRN_E_BADPARAM, "transpose_pad: batch %d, %d x %d -> %d x %d, %d-byte elements", batch, rows, cols, cols, rows_padded, elem_bytes);
     if (batch == 0) return HRN_OK;
     const int64_t tile = 8 * (16 / elem_bytes), tiles_c = (cols + tile - 1) / tile, tiles = tiles_c * ((rows_padded + tile - 1) / tile);
-    if (tiles >= (1ll << 31)) return fail(HRN_E_BADPARAM, "transpose_pad: %d x %d is more than one launch covers", rows_padded, cols);
+    // (32-bit rows and columns, up to a tile past the end)
+    if (tiles >= (1ll << 31) || rows_padded > INT32_MAX - tile || cols > INT32_MAX - tile)
+        return fail(HRN_E_BADPARAM, "transpose_pad: %d x %d is more than one launch covers", rows_padded, cols);
     const dim3 grid((unsigned)((tiles + 3) / 4), 1, batch);
     hipStream_t st = (hipStream_t)stream;
     if (elem_bytes == 1) transpose_pad_kernel<1><<<grid, 256, 0, st>>>(src, dst, rows, cols, rows_padded, (int)tiles_c, (int)tiles);

@@ -172,6 +172,9 @@ def test_prestage_entry_points_reject_bad_arguments_without_a_gpu():
     assert L.hrn_transpose_pad(p, p, 1, 8, 8, 8, 3, None) == B.HRN_E_BADPARAM   # 3-byte elements
     assert L.hrn_transpose_pad(p, p, 70000, 8, 8, 8, 2, None) == B.HRN_E_BADPARAM
     assert L.hrn_transpose_pad(p, p, 0, 8, 8, 8, 2, None) == 0
+    # 32-bit rows and columns: a tile past the end of either has to be one too
+    assert L.hrn_transpose_pad(p, p, 1, 1, 2 ** 31 - 1, 1, 1, None) == B.HRN_E_BADPARAM
+    assert L.hrn_transpose_pad(p, p, 1, 1, 1, 2 ** 31 - 1, 4, None) == B.HRN_E_BADPARAM
     out = ctypes.c_double()
     assert L.hrn_probe_launch(0, 10, ctypes.byref(out), None) == B.HRN_E_BADPARAM
     assert L.hrn_probe_launch(256, 10, None, None) == B.HRN_E_BADPARAM
