@@ -1218,7 +1218,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     }
 }
 
-// a deep kernel that the instance has no room for is empty, and the host never launches it
+// a kernel that the instance has no room for is empty, and the host never launches it
+// (all but the main kernel go through here, also where there is always room: called directly, the body of the channels-first
+// kernel is scheduled 0.6 % slower, NCW conv1d 16 x 892 x 512 -> 512 30.56 -> 30.73 us)
 template <bool ROOM, bool CHW, bool EXPAND, bool DEEP>
 __device__ __forceinline__ void body_if(BodyArgs a) {
     if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND, DEEP>(a);
@@ -1237,15 +1239,14 @@ __device__ __forceinline__ void body_if(BodyArgs a) {
 #ifndef HRN_PART
 #define HRN_PART 0
 #endif
-static_assert(HRN_PART == 0 || HAS_CHW, "the channels-first kernels of this instance have no room");
 
 #if HRN_PART == 0
 HRN_ENTRY hrn_mfma_kernel(const HrnKArgs a) { hrn_mfma_body<false, false, false>(a); }
 HRN_ENTRY hrn_mfma_kernel_deep(const HrnKArgs a) { body_if<HAS_DEEP, false, false, true>(a); }
 #elif HRN_PART == 1
-HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { hrn_mfma_body<true, false, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { body_if<HAS_CHW, true, false, false>(a); }
 HRN_ENTRY hrn_mfma_kernel_chw_deep(const HrnKArgs a) { body_if<HAS_DEEP, true, false, true>(a); }
 #else
-HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { hrn_mfma_body<true, true, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { body_if<HAS_CHW, true, true, false>(a); }
 HRN_ENTRY hrn_mfma_kernel_chw_expand_deep(const HrnKArgs a) { body_if<HAS_DEEP, true, true, true>(a); }
 #endif
