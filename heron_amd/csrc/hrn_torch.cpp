@@ -57,16 +57,16 @@ bool fits_int(int64_t v) { return v > 0 && v <= INT32_MAX; }
 
 void* stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
 
-// A loaded instance: the handle and the descriptor (addresses, as Module hands them over).
+// A loaded instance: the handle and the descriptor (addresses, the tuple that Module hands over).
 struct Instance {
     const hrn_module* mod;
     const hrn_kernel_desc* desc;
     at::ScalarType a, b, c;
-    bool read(PyObject* const* args) {
-        int64_t v[2];
-        if (!ints(args, 0, 2, v)) return false;
-        mod = (const hrn_module*)v[0];
-        desc = (const hrn_kernel_desc*)v[1];
+    bool read(PyObject* native) {
+        if (!PyTuple_Check(native) || PyTuple_GET_SIZE(native) != 2) return false;
+        mod = (const hrn_module*)PyLong_AsVoidPtr(PyTuple_GET_ITEM(native, 0));
+        desc = (const hrn_kernel_desc*)PyLong_AsVoidPtr(PyTuple_GET_ITEM(native, 1));
+        if (PyErr_Occurred() || !desc) return false;
         const bool f16 = desc->dtype == HRN_DT_F16;
         a = f16 ? at::kHalf : at::kByte;
         b = f16 ? at::kHalf : at::kChar;
@@ -129,26 +129,26 @@ PyObject* guarded(F f) {
     }
 }
 
-// gemm(handle, desc, group_m, split_k, A, B, out, bsum)
+// gemm(native, group_m, split_k, A, B, out, bsum)
 PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         Instance in;
         int64_t v[2];
-        if (n != 8 || !in.read(args) || !ints(args, 2, 2, v)) {
+        if (n != 7 || !in.read(args[0]) || !ints(args, 1, 2, v)) {
             PyErr_Clear();
             Py_RETURN_NONE;
         }
-        const at::Tensor *A = tensor(args[4]), *B = tensor(args[5]);
+        const at::Tensor *A = tensor(args[3]), *B = tensor(args[4]);
         if (!is(A, in.a) || !is(B, in.b) || A->dim() != B->dim() || (A->dim() != 2 && A->dim() != 3)) Py_RETURN_NONE;
         const int d = (int)A->dim() - 2;
         const int64_t batch = d ? A->size(0) : 1, M = A->size(d), K = A->size(d + 1), N = B->size(d);
         if (B->size(d + 1) != K || (d && B->size(0) != batch) || !fits_int(batch) || !fits_int(M) || !fits_int(N) || !fits_int(K) ||
-            !sums_fit(in, args[7], batch * N))
+            !sums_fit(in, args[6], batch * N))
             Py_RETURN_NONE;
-        if (!result_fits(args[6], *A, in.c, {batch, M, N})) Py_RETURN_NONE;
-        const at::Tensor* sums = tensor(args[7]);
+        if (!result_fits(args[5], *A, in.c, {batch, M, N})) Py_RETURN_NONE;
+        const at::Tensor* sums = tensor(args[6]);
         at::Tensor C;
-        if (args[6] != Py_None) C = *tensor(args[6]);
+        if (args[5] != Py_None) C = *tensor(args[5]);
         int rc;
         {
             Unlocked unlocked;
@@ -166,19 +166,19 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
-// conv2d(handle, desc, group_m, split_k, X, W, stride, pad, dil, out, bsum)
+// conv2d(native, group_m, split_k, X, W, stride, pad, dil, out, bsum)
 PyObject* conv2d(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         Instance in;
         int64_t v[2], sh, sw, ph, pw, dh, dw;
-        if (n != 11 || !in.read(args) || !ints(args, 2, 2, v) || !pair(args[6], &sh, &sw) || !pair(args[7], &ph, &pw) ||
-            !pair(args[8], &dh, &dw)) {
+        if (n != 10 || !in.read(args[0]) || !ints(args, 1, 2, v) || !pair(args[5], &sh, &sw) || !pair(args[6], &ph, &pw) ||
+            !pair(args[7], &dh, &dw)) {
             PyErr_Clear();
             Py_RETURN_NONE;
         }
-        const at::Tensor *X = tensor(args[4]), *W = tensor(args[5]);
+        const at::Tensor *X = tensor(args[3]), *W = tensor(args[4]);
         if (!is(X, in.a) || !is(W, in.b) || X->dim() != 4 || W->dim() != 4 || X->size(3) != W->size(3) || sh < 1 || sw < 1 || ph < 0 ||
-            pw < 0 || dh < 1 || dw < 1 || !sums_fit(in, args[10], W->size(0)))
+            pw < 0 || dh < 1 || dw < 1 || !sums_fit(in, args[9], W->size(0)))
             Py_RETURN_NONE;
         for (int i = 0; i < 4; ++i)
             if (!fits_int(X->size(i)) || !fits_int(W->size(i))) Py_RETURN_NONE;
@@ -186,10 +186,10 @@ PyObject* conv2d(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const int64_t room_h = X->size(1) - ((W->size(1) - 1) * dh + 1) + 2 * ph, room_w = X->size(2) - ((W->size(2) - 1) * dw + 1) + 2 * pw;
         if (room_h < 0 || room_w < 0) Py_RETURN_NONE;           // (before the division, which truncates)
         const int64_t ho = room_h / sh + 1, wo = room_w / sw + 1;
-        if (!result_fits(args[9], *X, in.c, {X->size(0), ho, wo, W->size(0)})) Py_RETURN_NONE;
-        const at::Tensor* sums = tensor(args[10]);
+        if (!result_fits(args[8], *X, in.c, {X->size(0), ho, wo, W->size(0)})) Py_RETURN_NONE;
+        const at::Tensor* sums = tensor(args[9]);
         at::Tensor C;
-        if (args[9] != Py_None) C = *tensor(args[9]);
+        if (args[8] != Py_None) C = *tensor(args[8]);
         int rc;
         {
             Unlocked unlocked;
@@ -214,8 +214,8 @@ PyObject* current_stream(PyObject*, PyObject*) {
 }
 
 PyMethodDef methods[] = {
-    {"gemm", (PyCFunction)(void (*)(void))gemm, METH_FASTCALL, "gemm(handle, desc, group_m, split_k, A, B, out, bsum)"},
-    {"conv2d", (PyCFunction)(void (*)(void))conv2d, METH_FASTCALL, "conv2d(handle, desc, group_m, split_k, X, W, stride, pad, dil, out, bsum)"},
+    {"gemm", (PyCFunction)(void (*)(void))gemm, METH_FASTCALL, "gemm(native, group_m, split_k, A, B, out, bsum)"},
+    {"conv2d", (PyCFunction)(void (*)(void))conv2d, METH_FASTCALL, "conv2d(native, group_m, split_k, X, W, stride, pad, dil, out, bsum)"},
     {"stream", current_stream, METH_NOARGS, "handle of torch's current stream"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -77,7 +77,7 @@ def gemm(mod, A, Bm, out=None, group_m=8, split_k=0, bsum=None):
     (``column_sums``) for a ``colsum`` instance; computed on the spot when absent.  ``out``: a contiguous tensor of the
     result's type with room for it, on A's device."""
     if _recording is None:
-        C = (B._ext or B.ext()).gemm(*mod.native, group_m, split_k, A, Bm, out, bsum)
+        C = (B._ext or B.ext()).gemm(mod.native, group_m, split_k, A, Bm, out, bsum)
         if C is not None:
             return C if type(C) is not int else B._check(C)
     f16 = mod.desc.dtype == B.HRN_DT_F16
@@ -116,7 +116,7 @@ def unpack_filter_blocked(Wb):
 def conv2d_nhwc(mod, X, Wt, stride=1, pad=0, dil=1, out=None, group_m=8, split_k=0, bsum=None):
     """X (N,H,W,CI), Wt KRSC (CO,KH,KW,CI) -> (N,HO,WO,CO): fp16 -> fp16, or uint8 x int8 -> int32."""
     if _recording is None:
-        C = (B._ext or B.ext()).conv2d(*mod.native, group_m, split_k, X, Wt, stride, pad, dil, out, bsum)
+        C = (B._ext or B.ext()).conv2d(mod.native, group_m, split_k, X, Wt, stride, pad, dil, out, bsum)
         if C is not None:
             return C if type(C) is not int else B._check(C)
     f16 = mod.desc.dtype == B.HRN_DT_F16
