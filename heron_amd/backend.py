@@ -178,6 +178,7 @@ SYMBOLS = {
     "hrn_time": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _i, _i, _d, ctypes.POINTER(_d), _vp]),
     "hrn_time_cold": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp, ctypes.c_size_t, _i, ctypes.POINTER(_d), _vp]),
     "hrn_splitk_workspace_bytes": (ctypes.c_int64, [ctypes.POINTER(KernelDesc), ctypes.POINTER(Problem)]),
+    "hrn_splitk_workspace_fast_bytes": (ctypes.c_int64, [ctypes.POINTER(KernelDesc), ctypes.POINTER(Problem)]),
     "hrn_problem_gemm": (None, [ctypes.POINTER(Problem), _i, _i, _i, _i]),
     "hrn_problem_conv2d": (None, [ctypes.POINTER(Problem)] + [_i] * 10),
     "hrn_problem_conv2d_hw": (None, [ctypes.POINTER(Problem)] + [_i] * 13),
@@ -272,9 +273,11 @@ def gemm_problem(batch, m, n, k, group_m=8, split_k=0):
     return p
 
 
-def splitk_workspace_bytes(desc, problem):
-    """Bytes of device workspace a split-K launch of ``desc`` on ``problem`` needs (0 for other instances)."""
-    n = lib().hrn_splitk_workspace_bytes(ctypes.byref(desc), ctypes.byref(problem))
+def splitk_workspace_bytes(desc, problem, fast=False):
+    """Bytes of device workspace a split-K launch of ``desc`` on ``problem`` needs (0 for other instances); ``fast``: with the
+    room that lets the launch add the slices up without a second one."""
+    size = lib().hrn_splitk_workspace_fast_bytes if fast else lib().hrn_splitk_workspace_bytes
+    n = size(ctypes.byref(desc), ctypes.byref(problem))
     if n < 0:
         _check(int(n))
     return int(n)
@@ -399,7 +402,7 @@ class Module:
             return problem
         if problem.split_k < 1:
             problem.split_k = 1
-        need = splitk_workspace_bytes(self.desc, problem)
+        need = splitk_workspace_bytes(self.desc, problem, fast=True)
         ws = getattr(self, "_ws", None)
         if ws is None or ws.numel() < need:
             import torch

@@ -17,11 +17,13 @@
 #include <algorithm>
 #include <chrono>
 #include <cstdarg>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <fstream>
 #include <mutex>
+#include <random>
 #include <sstream>
 #include <string>
 #include <thread>
@@ -43,6 +45,11 @@ struct HrnKArgs {  // must match mfma_gemm_template.hip
     const void* bsum;
     int32_t out_plane;
     int32_t expand_shift, in_h, in_w, top, left;
+    void* out;
+    int64_t out_stride;
+    uint64_t* arrivals;
+    uint64_t ticket;
+    int32_t out_ld;
 };
 
 // An instance's kernels lie in up to three code objects, so that a caller pays the compiler only for those it launches: a
@@ -451,6 +458,22 @@ void split_shape(const hrn_kernel_desc& d, const hrn_problem* p, int* kt_per_sli
     *split = (kt_all + *kt_per_slice - 1) / *kt_per_slice;
 }
 
+// Where the workspace holds one more word per output tile, the slice that reaches a tile last adds them all up, and the launch of
+// splitk_reduce_kernel falls away.  A word counts arrivals in its low 16 bits; above them is a number of the launch's own, so that
+// nothing has to be zero before.  The numbers grow from one launch to the next and are high, so that raising a word to one
+// almost always takes effect; words that never were an arrival count equal one with the odds of 43 random bits.
+constexpr int kMaxArrivals = 65535;
+int64_t output_tiles(const hrn_kernel_desc& d, const hrn_problem* p) {
+    return (int64_t)((p->m + d.bm - 1) / d.bm) * ((p->n + d.bn - 1) / d.bn) * p->batch;
+}
+uint64_t next_ticket() {
+    static std::atomic<uint64_t> next{[] {
+        std::random_device r;
+        return (15ull << 44) | ((((uint64_t)r() << 32) | r()) >> 21);
+    }()};
+    return next.fetch_add(1, std::memory_order_relaxed) << 16;
+}
+
 // Two stages leave a k-tile's loads one k-tile of multiplication to arrive, enough from a near L2 but not from further away; two
 // stages were chosen so that several workgroups fit a CU, and a grid whose LDS the device has at once with three (deep_lds) has
 // no other use for it.  128x128 fp16, 9 x 12 tiles, inputs of three calls in turn: 41.9 -> 33.8 us at 64 k-tiles, 16.3 -> 14.0 at 15,
@@ -550,6 +573,11 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         k->C = workspace; k->ldc = p->n; k->sC = (int64_t)p->m * p->n;
         k->split = split; k->kt_per_slice = kps;
         plan->split = split;
+        if (split <= kMaxArrivals && (int64_t)workspace_bytes >= need + total * 8) {
+            k->out = C; k->out_ld = p->ldc; k->out_stride = p->stride_c;
+            k->arrivals = (uint64_t*)((char*)workspace + need);
+            k->ticket = next_ticket();
+        }
         total *= split;
     } else if (p->split_k > 1) {
         return fail(HRN_E_BADPARAM, "problem.split_k = %d but the instance was not built with split_k", p->split_k);
@@ -576,7 +604,8 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
 }
 
 // Adds the K slices of a split-K launch: C[b,m,n] = sum_z ws[z,b,m,n], converted to the output type.  One lane per
-// 4 consecutive n (N is a multiple of 4): 16-byte reads, 8- or 16-byte writes.
+// 4 consecutive n (N is a multiple of 4): 16-byte reads, 8- or 16-byte writes.  For workspaces without a word per output tile;
+// the same additions as fold_slices of the template, bit for bit.
 typedef float rv4f __attribute__((ext_vector_type(4)));
 typedef int rv4i __attribute__((ext_vector_type(4)));
 typedef _Float16 rv4h __attribute__((ext_vector_type(4)));
@@ -593,15 +622,14 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restri
         const int b = (int)(bm / M), m = (int)(bm - (int64_t)b * M);
         const int64_t src = bm * N + (int64_t)q * 4;
         const int64_t dst = (int64_t)b * stride_c + (int64_t)m * ldc + (int64_t)q * 4;
+        using sum_t = typename std::conditional<F16, rv4f, rv4i>::type;
+        sum_t acc = *(const sum_t*)((const char*)ws + src * 4);
+        for (int z = 1; z < split; ++z) acc += *(const sum_t*)((const char*)ws + (z * slice + src) * 4);
         if constexpr (F16) {
-            rv4f acc = *(const rv4f*)((const float*)ws + src);
-            for (int z = 1; z < split; ++z) acc += *(const rv4f*)((const float*)ws + z * slice + src);
             rv4h o;
             for (int r = 0; r < 4; ++r) o[r] = (_Float16)acc[r];
             *(rv4h*)((_Float16*)C + dst) = o;
         } else {
-            rv4i acc = *(const rv4i*)((const int*)ws + src);
-            for (int z = 1; z < split; ++z) acc += *(const rv4i*)((const int*)ws + z * slice + src);
             *(rv4i*)((int*)C + dst) = acc;
         }
     }
@@ -611,7 +639,7 @@ int run_plan(const hrn_module* mod, const hrn_problem* p, const LaunchPlan& plan
     size_t sz = sizeof plan.k;
     void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void*)&plan.k, HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz, HIP_LAUNCH_PARAM_END};
     HIP_TRY(hipModuleLaunchKernel(plan.fn, plan.grid, 1, 1, (unsigned)mod->info.threads, 1, 1, plan.dyn_lds, st, nullptr, extra));
-    if (mod->desc.split_k) {
+    if (mod->desc.split_k && !plan.k.arrivals) {
         const int64_t count = (int64_t)p->batch * p->m * (p->n / 4);
         const unsigned blocks = (unsigned)std::min<int64_t>((count + 255) / 256, 256 * 32);
         if (mod->desc.dtype == HRN_DT_F16)
@@ -1675,6 +1703,13 @@ int64_t hrn_splitk_workspace_bytes(const hrn_kernel_desc* desc, const hrn_proble
     int kps, split;
     split_shape(*desc, p, &kps, &split);
     return splitk_bytes(p, split);
+}
+
+int64_t hrn_splitk_workspace_fast_bytes(const hrn_kernel_desc* desc, const hrn_problem* p) {
+    const int64_t need = hrn_splitk_workspace_bytes(desc, p);
+    if (need <= 0) return need;
+    if (desc->bm < 1 || desc->bn < 1) return fail(HRN_E_BADPARAM, "tile %dx%d", desc->bm, desc->bn);
+    return need + output_tiles(*desc, p) * 8;
 }
 
 void hrn_problem_gemm(hrn_problem* p, int batch, int m, int n, int k) {

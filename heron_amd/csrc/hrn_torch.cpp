@@ -83,7 +83,7 @@ struct Extras {
         p->split_k = (int32_t)split_k;
         if (in.desc->split_k) {
             if (p->split_k < 1) p->split_k = 1;
-            const int64_t need = hrn_splitk_workspace_bytes(in.desc, p);
+            const int64_t need = hrn_splitk_workspace_fast_bytes(in.desc, p);
             if (need < 0) return (int)need;
             workspace = at::empty({need}, B.options().dtype(at::kByte));
             p->workspace = workspace.data_ptr();

@@ -51,6 +51,12 @@ struct HrnKArgs {
     int32_t out_plane;                   // CHW kernels: row m, column n of the result goes to C[m / out_plane][n][m % out_plane]
     int32_t expand_shift;                // EXPAND kernels: the H x W input is not in memory: pixel (y, x) of the in_h x in_w
     int32_t in_h, in_w, top, left;       // one that is stands at (top + (y << shift), left + (x << shift)), zeros elsewhere
+    // split-K: the result and what tells the last slice of a tile to add them all up; arrivals null: a kernel behind this one does
+    void* out;
+    int64_t out_stride;                  // batch stride of the result, elements
+    uint64_t* arrivals;                  // one word per output tile, of any content
+    uint64_t ticket;                     // of this launch, its low 16 bits zero
+    int32_t out_ld;
 };
 #endif
 
@@ -221,6 +227,8 @@ __device__ __forceinline__ void wait_only() {
 }
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+constexpr int AGENT_SCOPE = 16;             // cache policy (sc1): a load or store that all XCDs of the device see
 
 // raw buffer (stride 0): a lane offset >= `bytes` reads as zero instead of touching memory (the scalar offset of a
 // load is not part of that check)
@@ -734,9 +742,13 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         };
 
         char* Cb = (char*)a.C + ((int64_t)slice * a.batch + c_bz) * a.sC * OES;
+        [[maybe_unused]] const rsrc_t rsrcC = make_rsrc(Cb, (uint32_t)a.M * (uint32_t)a.ldc * OES);
         auto put = [&](auto* ptr, auto val) __attribute__((always_inline)) {
             if constexpr (NTS) __builtin_nontemporal_store(val, ptr);
             else *ptr = val;
+        };
+        [[maybe_unused]] auto put_partial = [&](int m, int n, auto val) __attribute__((always_inline)) {
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rsrcC, (m * a.ldc + n) * 4, 0, AGENT_SCOPE);
         };
         if constexpr (CHW) {
             // A wave parks MT channels x CSW pixels of its result in a private LDS strip and streams them out 16 bytes per
@@ -827,7 +839,6 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             // LDS-staged epilogue: a wave parks one MFMA row-tile (MT rows x SW columns) of its result in a private,
             // padded LDS strip, then streams it out with 16 bytes per lane_e, whole row segments per store instruction.
             if constexpr (DT == 0 && !PERS) wait_and_barrier<0, 0>();   // (the int8 path has synchronised above) stages are dead now
-            [[maybe_unused]] const rsrc_t rsrcC = make_rsrc(Cb, (uint32_t)a.M * (uint32_t)a.ldc * OES);
             char* strip = epi + EPI_BASE + wave * (MT * EPI_PITCH);
             constexpr int CPRW = SW * OES / 16;                // 16-byte chunks per strip row
             constexpr int EPC = 16 / OES;                      // output elements per chunk
@@ -873,7 +884,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                         if constexpr (PERS) {
                             // always issued, so that every wave has exactly STORES_PER_TILE stores per tile in flight
                             const uint32_t off = (m < a.M && n + EPC <= a.N) ? (uint32_t)(m * a.ldc + n) * OES : OOB;
-                            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(unsigned int __attribute__((ext_vector_type(4))), val), rsrcC, (int)off, 0, NTS ? 2 : 0);
+                            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rsrcC, (int)off, 0, NTS ? 2 : 0);
+                        } else if constexpr (SPLITK) {
+                            if (m < a.M && n < a.N) put_partial(m, n, val);
                         } else {
                             char* dst = Cb + ((int64_t)m * a.ldc + n) * OES;
                             if (m < a.M) {
@@ -906,19 +919,116 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                                 v4f o;
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r];
-                                put((v4f*)dst, o);
+                                put_partial(m, n, o);
                             } else {
                                 const v4i bs = colsum4(nl);
                                 v4i o;
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r] + 128 * bs[r];
-                                put((v4i*)dst, o);
+                                if constexpr (SPLITK) put_partial(m, n, o);
+                                else put((v4i*)dst, o);
                             }
                         }
                     }
                 }
             }
         }
+    };
+
+    // ---- split-K: the last slice of an output tile adds all of them up ----
+    // Every slice stores its partial sums so that all XCDs see them, waits for the stores and counts itself in at the tile's
+    // word.  Nobody waits for anybody: whoever counts last reads the slices (its own among them) and writes the result.  The
+    // word may hold anything before: greet() raises it to this launch's ticket with no arrivals (tickets grow and are high numbers),
+    // while the partial sums are on their way; only where it was higher does arrive() find something else, and installs the ticket
+    // itself.  The last slice takes the arrivals back, for a replay of the launch from a graph.  Slices are
+    // added in their order, as by splitk_reduce_kernel, the launch behind this one that workspaces without the words get.
+    //   What it costs is three trips to memory, one of them the stores' that a kernel's end waits for anyway; a launch of its own cost
+    // the call 3.5 us of host time and the device 2.7 - 4.6 us.  Loads and stores carry their scope themselves: fences instead
+    // empty the L2s (1.3 - 5.4 us more).  fp16, per call: 32x4096x4096 in 4 slices 10.8 -> 10.4 us (7.7 without any sum),
+    // 86x2648x576 in 2 9.0 -> 7.3, 540x784x864 in 2 8.8 -> 8.2, variance of 15x128x36x36 in 76 32.1 -> 19.1.
+    [[maybe_unused]] auto greet = [&]() __attribute__((always_inline)) {
+        if (tid == 0) (void)__hip_atomic_fetch_max(a.arrivals + first_pid, a.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    [[maybe_unused]] auto arrive = [&]() __attribute__((always_inline)) {      // (one lane)
+        uint64_t* const word = a.arrivals + first_pid;
+        uint64_t n = __hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - a.ticket;
+        if (n >= 0x10000) {                                           // not of this launch (compare-and-swap alone: 0.7 us per slice)
+            uint64_t seen = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), next;
+            do {
+                n = seen - a.ticket < 0x10000 ? seen - a.ticket : 0;
+                next = a.ticket + n + 1;
+            } while (!__hip_atomic_compare_exchange_strong(word, &seen, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        }
+        const bool last = n + 1 == (uint64_t)a.split;
+        if (last) __hip_atomic_store(word, a.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return last;
+    };
+    [[maybe_unused]] auto fold_slices = [&]() __attribute__((always_inline)) {
+        using sum_t = typename std::conditional<DT == 0, v4f, v4i>::type;
+        wait_only<0, 0>();                                            // the stores of this wave have arrived
+        __syncthreads();
+        int* const flag = (int*)lds;
+        if (tid == 0) *flag = arrive();
+        __syncthreads();
+        const bool last = *flag != 0;
+        if (!last) return;
+        asm volatile("" ::: "memory");
+        const int cpr = min(BN, a.N - n0) / 4, count = min(BM, a.M - m0) * cpr;   // 16-byte pieces of the tile
+        const float inv = 1.0f / (float)cpr;
+        const uint32_t slice_bytes = (uint32_t)a.M * (uint32_t)a.N * 4;
+        const int64_t step = (int64_t)a.batch * a.sC * 4;
+        // U pieces of a lane at a time, Z slices of each on the way
+        auto fold = [&](auto uc, auto zc) __attribute__((always_inline)) {
+            constexpr int U = decltype(uc)::value, Z = decltype(zc)::value;
+#pragma unroll 1
+            for (int v0 = tid; v0 < count; v0 += U * NT) {
+                int m[U], n[U];
+                uint32_t off[U];
+                sum_t sum[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int v = v0 + u * NT, row = (int)(((float)v + 0.5f) * inv);      // v / cpr (v is below 2^16, so the quotient is exact)
+                    m[u] = m0 + row;
+                    n[u] = n0 + (v - row * cpr) * 4;
+                    off[u] = v < count ? (uint32_t)(m[u] * a.N + n[u]) * 4 : OOB;
+                    sum[u] = sum_t{0, 0, 0, 0};
+                }
+                const char* part = (const char*)a.C + (int64_t)c_bz * a.sC * 4;
+#pragma unroll 1
+                for (int z0 = 0; z0 < a.split; z0 += Z, part += Z * step) {
+                    sum_t t[Z][U];
+#pragma unroll
+                    for (int z = 0; z < Z; ++z)
+                        if (z0 + z < a.split) {
+                            const rsrc_t r = make_rsrc(part + z * step, slice_bytes);
+#pragma unroll
+                            for (int u = 0; u < U; ++u) t[z][u] = __builtin_bit_cast(sum_t, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[u], 0, AGENT_SCOPE));
+                        }
+#pragma unroll
+                    for (int z = 0; z < Z; ++z)
+                        if (z0 + z < a.split) {
+#pragma unroll
+                            for (int u = 0; u < U; ++u) sum[u] += t[z][u];
+                        }
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (v0 + u * NT < count) {
+                        const int64_t at = (int64_t)c_bz * a.out_stride + (int64_t)m[u] * a.out_ld + n[u];
+                        if constexpr (DT == 0) {
+                            v4h o;
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) o[r] = (_Float16)sum[u][r];
+                            *(v4h*)((_Float16*)a.out + at) = o;
+                        } else {
+                            *(v4i*)((int*)a.out + at) = __builtin_bit_cast(v4i, sum[u]);
+                        }
+                    }
+                }
+            }
+        };
+        if (count > NT) fold(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+        else fold(std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
     };
 
     // ---- prologue: fill all stages, wait for tile 0 ----
@@ -1047,6 +1157,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             tiles(FalseC{}, 0, cut, stores_between);
             if (kt_rag >= 0) tiles(TrueC{}, cut, min(cut + 1, KT), stores_between);
             tiles(FalseC{}, kt_rag >= 0 ? min(cut + 1, KT) : cut, KT, stores_between);
+        }
+        if constexpr (SPLITK) {
+            if (a.arrivals) greet();
         }
         store_tile();
     };
@@ -1215,6 +1328,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         }
     } else {
         run_tile(false);
+        if constexpr (SPLITK) {
+            if (a.arrivals) fold_slices();
+        }
     }
 }
 

@@ -52,7 +52,7 @@ def _slice_workspace(mod, p, operand):
     workspace is replaced by a larger launch of the same module."""
     if mod.desc.split_k:
         p.split_k = max(1, p.split_k)
-        need = B.splitk_workspace_bytes(mod.desc, p)
+        need = B.splitk_workspace_bytes(mod.desc, p, fast=True)
         ws = _new(torch.empty, (max(need, 16),), dtype=torch.uint8, device=operand.device)
         p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
         return ws

@@ -364,6 +364,13 @@ int hrn_probe_copy(const void* src, void* dst, size_t bytes, int repeat, double*
  */
 int64_t hrn_splitk_workspace_bytes(const hrn_kernel_desc* desc, const hrn_problem* p);
 
+/*
+ * The same with room for one 8-byte word per output tile behind the partial sums.  A launch whose workspace is this large adds the
+ * slices up itself (the slice that finishes a tile last does); with less room a second launch adds them, 2.5 - 4 us more.  Both
+ * give the same bits.  The words need no content before the launch.
+ */
+int64_t hrn_splitk_workspace_fast_bytes(const hrn_kernel_desc* desc, const hrn_problem* p);
+
 /* Fills an hrn_problem for the plain cases (packed row-major operands). */
 void hrn_problem_gemm(hrn_problem* p, int batch, int m, int n, int k);
 void hrn_problem_conv2d(hrn_problem* p, int n, int h, int w, int ci, int co, int kh, int kw,
