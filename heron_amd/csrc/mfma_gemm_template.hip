@@ -7,7 +7,7 @@
 //               1: conv2d NHWC x KRSC as implicit GEMM (M = n*ho*wo, N = co, K = kh*kw*ci)
 //   HRN_BM/BN   workgroup tile, HRN_BKB bytes of K per LDS row, HRN_WM x HRN_WN wave grid,
 //   HRN_MFMA    32 | 16 (MFMA tile edge), HRN_STAGES LDS stages, HRN_SWZ LDS chunk swizzle,
-//   HRN_EPI     0 stores straight from the accumulator registers, 1 LDS-staged epilogue with 16-byte coalesced
+//   HRN_EPI     0 result of any alignment, staged where there is room, 1 LDS-staged epilogue with 16-byte coalesced
 //               stores, 2 the same with half-width staging strips, HRN_WPE waves-per-SIMD hint, HRN_CONVWIN conv input window in LDS, HRN_PERSIST persistent
 //               launch, HRN_SPLITK K split over several workgroups with raw partial sums as output.
 //
@@ -66,7 +66,6 @@ constexpr int DT = HRN_DTYPE;
 constexpr int OP = HRN_OP;
 constexpr int BM = HRN_BM, BN = HRN_BN, BKB = HRN_BKB;
 constexpr int WM = HRN_WM, WN = HRN_WN, MT = HRN_MFMA, NS = HRN_STAGES, SWZ = HRN_SWZ;
-constexpr int EPI = HRN_EPI;
 // Conv window mode (HRN_OP=1, stride 1, dilation 1, 'same' padding): instead of fetching an im2col tile of A for every
 // filter tap, the workgroup loads ONCE the window of input pixels its BM output pixels can reach (a contiguous range
 // of BM + 2*(pad_h*W + pad_w) pixels, all channels) and every tap reads its operand fragments from that window at a row offset
@@ -143,6 +142,14 @@ static_assert((CW || ((BM / RPI) % NW == 0 && A_LPW >= 1)) && (BN / RPI) % NW ==
 static_assert(!CW || OP == 1, "window mode is a conv2d load path");
 static_assert(BM % (WM * MT) == 0 && BN % (WN * MT) == 0, "wave tile");
 static_assert(NS >= 2 && NS <= 5, "stages");
+// HRN_EPI = 0 stages fp16 results as well, where the strips fit into the LDS of the stages: lanes that store what the MFMAs leave them
+// with write 8 bytes here and there, 32 bytes of a row per instruction at best, and with the non-temporal hint each of them on
+// its own.  (32-bit results go out 16 bytes at a time either way; staged, one wave's 64x64 tile of them takes 0.4 us longer.)  Unlike HRN_EPI = 1 it takes rows of any alignment.  fp16, 128x128 tiles, stored non-temporally / not: 2000x2000x1024
+// 25.4 / 16.4 -> 13.0 us, 3000x2304x512 34.5 / 15.6 -> 11.9, 4000x1024x512 19.7 / 13.1 -> 8.2.
+constexpr bool ANY_ALIGNMENT = HRN_EPI == 0;
+constexpr bool STAGE_DIRECT = HRN_EPI == 0 && OES == 2 && !CW && !PERS && (MT * (WTN * OES / 16)) % 64 == 0 &&
+                              NW * MT * (WTN * OES + 16) <= NS * STAGE_BYTES;
+constexpr int EPI = STAGE_DIRECT ? 1 : HRN_EPI;
 // LDS-staged epilogue: per wave a strip of MT rows x WTN outputs, rows padded by 16 bytes; in front of the strips the
 // uint8 path keeps the column sums of B, one row of BN sums per wave row (each wave row sums its share of the k-steps)
 // (HRN_EPI = 2: strips of half the wave tile's width, filled and written out twice per row-tile - half the LDS)
@@ -842,6 +849,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             char* strip = epi + EPI_BASE + wave * (MT * EPI_PITCH);
             constexpr int CPRW = SW * OES / 16;                // 16-byte chunks per strip row
             constexpr int EPC = 16 / OES;                      // output elements per chunk
+            typedef v4i any_t __attribute__((aligned(OES)));
+            using piece_t = typename std::conditional<ANY_ALIGNMENT, any_t, v4i>::type;
             constexpr int TNS = TN / ESPLIT;                   // MFMA column tiles per strip
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -890,7 +899,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                         } else {
                             char* dst = Cb + ((int64_t)m * a.ldc + n) * OES;
                             if (m < a.M) {
-                                if (n + EPC <= a.N) put((v4i*)dst, val);
+                                if (n + EPC <= a.N) put((piece_t*)dst, val);
                                 else if (OES == 2 && n + 4 <= a.N) put((long*)dst, (long)(((long)(uint32_t)val.y << 32) | (uint32_t)val.x));
                             }
                         }

@@ -73,8 +73,8 @@ typedef struct hrn_kernel_desc {
     int32_t mfma;       /* 32 -> 32x32x(16 f16|32 i8), 16 -> 16x16x(32 f16|64 i8) */
     int32_t stages;     /* LDS stages of the A/B tiles, 2..5 (2 = double buffer) */
     int32_t swizzle;    /* LDS 16-byte-chunk XOR swizzle: 0 none, 1 row, 2 row/2, 3 row/4 */
-    int32_t epilogue;   /* 0 = store accumulators straight from registers, 1 = stage C through LDS strips as wide as
-                           the wave tile, 2 = through strips of half that width (half the LDS) */
+    int32_t epilogue;   /* 0 = C of any alignment, fp16 staged through LDS where the stages have room for the strips, otherwise
+                           straight from the registers, 1 = 16-byte aligned C, staged through strips as wide as the wave tile, 2 = through strips of half that width (half the LDS) */
     int32_t waves_per_eu; /* 0 = let the compiler pick, else occupancy hint 1..4 */
     int32_t conv_window;  /* conv2d only: 1 = keep the reachable input window in LDS and read every filter tap from it
                              (needs stride 1, dilation 1, 'same' padding, CI*2 a multiple of bkb) instead of im2col tiles */
