@@ -171,6 +171,10 @@ SYMBOLS = {
     "hrn_launch_conv2d_nhwc_u8s8": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
     "hrn_compile_chw": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
     "hrn_module_has_chw": (_i, [_vp]),
+    "hrn_tiles": (_i, [ctypes.POINTER(KernelDesc), ctypes.POINTER(KernelDesc), _i]),
+    "hrn_compile_tiles": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
+    "hrn_launch_tile": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(KernelDesc)]),
+    "hrn_module_own_tiles": (None, [_vp, _i]),
     "hrn_launch_conv2d_chw": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(ConvView), _vp, _vp, _vp, _vp]),
     "hrn_launch_is_deep": (_i, [_vp, ctypes.POINTER(Problem)]),
     "hrn_launch_splitk_static": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
@@ -257,6 +261,15 @@ def compile_desc(desc, timeout_s=0.0):
     buf = ctypes.create_string_buffer(4096)
     _check(lib().hrn_compile(ctypes.byref(desc), float(timeout_s), buf, 4096))
     return buf.value.decode()
+
+
+def tiles(desc):
+    """The instances whose tiles launches of ``desc`` may take instead of its own (hrn_tiles)."""
+    out = (KernelDesc * 8)()
+    n = lib().hrn_tiles(ctypes.byref(desc), out, 8)
+    if n < 0:
+        _check(n)
+    return [KernelDesc.from_buffer_copy(out[i]) for i in range(n)]
 
 
 def compile_chw(desc, expand, timeout_s=0.0):
@@ -382,13 +395,16 @@ def probe_copy(src_ptr, dst_ptr, nbytes, repeat=10, stream=0):
 
 
 class Module:
-    """One loaded template instance (``hrn_module``)."""
+    """One loaded template instance (``hrn_module``).  Launches whose grid leaves most of the device idle take another tile of
+    the same instance (``launch_tile``) unless ``own_tiles`` is set."""
 
-    def __init__(self, desc, timeout_s=0.0):
+    def __init__(self, desc, timeout_s=0.0, own_tiles=False):
         self.desc = desc
         h = _vp()
         _check(lib().hrn_build(ctypes.byref(desc), float(timeout_s), ctypes.byref(h)))
         self._h = h
+        if own_tiles:
+            lib().hrn_module_own_tiles(h, 1)
         self.native = (h.value, ctypes.addressof(desc))      # what the functions of ext() take for this instance
         self.has_chw = bool(lib().hrn_module_has_chw(h))     # launch_conv2d_chw takes it
         info = KernelInfo()
@@ -439,6 +455,12 @@ class Module:
         self.bind_workspace(problem)
         self.bind_colsum(problem, b_ptr, stream)
         _check(self._launcher(problem)(self._h, ctypes.byref(problem), a_ptr, b_ptr, c_ptr, stream))
+
+    def launch_tile(self, problem):
+        """The descriptor of the instance whose kernel a launch of ``problem`` takes."""
+        out = KernelDesc()
+        _check(lib().hrn_launch_tile(self._h, ctypes.byref(problem), ctypes.byref(out)))
+        return out
 
     def is_deep(self, problem):
         """Whether a launch of ``problem`` takes the instance's deep kernel."""

@@ -63,8 +63,17 @@ struct CodeObject {
     hipFunction_t fn[2] = {};       // plain and deep (a third stage); null where the instance has no room for it
 };
 
+constexpr int kMaxFits = 6;
+
 struct hrn_module {
     hrn_kernel_desc desc;
+    int cus;                        // of the device
+    // the instance's tile cut for grids that leave the device idle (fitting_tiles): built at the first launch that takes one
+    int fits, first_half;
+    hrn_kernel_desc fit_desc[kMaxFits];
+    mutable std::atomic<hrn_module*> fit[kMaxFits];
+    mutable bool fit_failed[kMaxFits];
+    std::atomic<bool> own_tiles;    // launches keep to the instance's own tile
     hrn_kernel_info info;
     mutable CodeObject part[PARTS]; // those of hrn_launch_conv2d_chw are there from hrn_build on or from their first launch
     mutable std::mutex part_mutex;
@@ -491,6 +500,94 @@ int conv_extent(int in, int k, int stride, int pad, int dil) {
     return stride < 1 || room < 0 ? 0 : (int)(room / stride) + 1;
 }
 
+// ---- other tiles of an instance ----
+// A grid of at most half as many tiles as the device has CUs leaves half of it idle, and what bounds such a launch is what one
+// CU fetches and multiplies.  The instance's tile is then cut in halves, the longer side first, down to 64x64, until the
+// grid passes half the CUs; cut tiles keep the MFMA shape and the order along K, so the result is the same bit for bit.  A tile of one
+// to three waves that has a CU to itself is given more: they cannot issue its fetches fast enough.  Cut tiles have a wave
+// per SIMD, two from 128x64 on; with an input window one row of MFMA tiles per wave.
+//   u8 x s8 1111x1500x2064 (108 tiles of 128x128 -> 216 of 64x128) 16.9 -> 11.9 us; 96x200x608 (64x64, one wave -> four) 6.4 -> 4.5;
+// conv fp16 16x27x27x128 -> 80 (128x64, two waves -> eight) 18.1 -> 12.9; window convs 8x28x31x64 -> 64, 5x5 (14 tiles of 512x64 ->
+// 109 of 64x64) 25.4 -> 12.7 and u8 22x16x16x192 -> 80 (44 of 256x64 -> 176) 15.5 -> 10.7.  Above the line: fp16 2000x2000x1024 (256 tiles
+// of 128x128) 13.0 us, 15.0 with 64x128.
+bool with_waves(hrn_kernel_desc d, hrn_kernel_desc* out) {
+    const int two[4][2] = {{4, 2}, {2, 4}, {2, 2}, {4, 1}}, wide[4][2] = {{2, 4}, {4, 2}, {2, 2}, {1, 4}}, one[4][2] = {{2, 2}, {4, 1}, {1, 4}, {2, 1}};
+    const int win[4][2] = {{d.bm / d.mfma, 1}, {d.bm / d.mfma / 2, 1}, {2, 2}, {2, 1}};
+    const auto& list = d.conv_window ? win : d.bm * d.bn < 8192 ? one : d.bn > d.bm ? wide : two;
+    d.waves_per_eu = 0;
+    for (int epi = d.epilogue; epi >= std::min(d.epilogue, 1); --epi)
+        for (const auto& w : list) {
+            d.wm = w[0]; d.wn = w[1]; d.epilogue = epi;
+            if (derive(&d, nullptr) == HRN_OK) { *out = d; return true; }
+        }
+    return false;
+}
+
+// fit_desc[0]: the own tile with more waves, if it has few; then the halves.  Returns how many there are; *first_half is where
+// the halves begin.
+int cut_tiles(const hrn_kernel_desc& own, hrn_kernel_desc* out, int* first_half) {
+    int n = 0;
+    *first_half = 0;
+    if (own.persistent || own.split_k) return 0;
+    const std::string keep = g_err;
+    if (own.wm * own.wn < 4 && with_waves(own, &out[n]) && out[n].wm * out[n].wn >= 4) ++n;
+    *first_half = n;
+    hrn_kernel_desc d = own;
+    while (n < kMaxFits && (d.bm > 64 || d.bn > 64)) {
+        if (d.bm > 64 && (d.bm >= d.bn || d.bn <= 64)) d.bm /= 2;
+        else d.bn /= 2;
+        if (d.bm % 64 || d.bn % 64 || !with_waves(d, &d)) break;
+        out[n++] = d;
+    }
+    g_err = keep;
+    return n;
+}
+
+int64_t tiles_of(const hrn_kernel_desc& d, const hrn_problem* p) {
+    return (((int64_t)p->m + d.bm - 1) / d.bm) * (((int64_t)p->n + d.bn - 1) / d.bn) * p->batch;
+}
+
+// which of the instance's tiles a launch takes: -1 its own
+int fitting_tiles(const hrn_module* m, const hrn_problem* p) {
+    if (!p || p->m < 1 || p->n < 1 || p->batch < 1 || m->fits == 0 || m->own_tiles.load(std::memory_order_relaxed)) return -1;
+    const int halves = m->first_half;
+    int pick = -1;
+    const hrn_kernel_desc* d = &m->desc;
+    for (int i = halves; i < m->fits && tiles_of(*d, p) * 2 <= m->cus; ++i) { pick = i; d = &m->fit_desc[i]; }
+    if (pick < 0 && halves == 1 && tiles_of(m->desc, p) <= m->cus) pick = 0;
+    return pick;
+}
+
+int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out);
+
+// The module whose kernel a launch takes.  One that cannot be built or does not take the problem leaves the launch to the
+// instance itself.
+const hrn_module* fitting(const hrn_module* m, const hrn_problem* p) {
+    const int i = fitting_tiles(m, p);
+    if (i < 0) return m;
+    if (const hrn_module* f = m->fit[i].load(std::memory_order_acquire)) return f;
+    std::lock_guard<std::mutex> lock(m->part_mutex);
+    if (const hrn_module* f = m->fit[i].load(std::memory_order_acquire)) return f;
+    if (m->fit_failed[i]) return m;
+    hrn_module* f = nullptr;
+    int dev = 0;
+    const std::string keep = g_err;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;       // (see chw_kernels)
+    bool ok = hipGetDevice(&dev) == hipSuccess && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (ok) {
+        ok = (dev == m->device || hipSetDevice(m->device) == hipSuccess) && build_module(&m->fit_desc[i], m->timeout_s, &f) == HRN_OK;
+        if (dev != m->device) (void)hipSetDevice(dev);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    if (!ok) {
+        m->fit_failed[i] = true;
+        g_err = keep;
+        return m;
+    }
+    m->fit[i].store(f, std::memory_order_release);
+    return f;
+}
+
 int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
               size_t workspace_bytes, LaunchPlan* plan) {
     HrnKArgs* k = &plan->k;
@@ -635,6 +732,19 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restri
     }
 }
 
+// fill_args for the kernel that the launch takes; *mod becomes its module
+int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, const void* B, void* C, LaunchPlan* plan) {
+    void* ws = p ? p->workspace : nullptr;
+    const size_t ws_bytes = p ? p->workspace_bytes : 0;
+    int rc = fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);          // (the instance says what is refused)
+    if (rc) return rc;
+    const hrn_module* f = fitting(*mod, p);
+    if (f == *mod) return HRN_OK;
+    if (fill_args(f, p, A, B, C, ws, ws_bytes, plan)) return fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);
+    *mod = f;
+    return HRN_OK;
+}
+
 int run_plan(const hrn_module* mod, const hrn_problem* p, const LaunchPlan& plan, void* workspace, hipStream_t st) {
     size_t sz = sizeof plan.k;
     void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void*)&plan.k, HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz, HIP_LAUNCH_PARAM_END};
@@ -687,7 +797,7 @@ int static_scratch(void** out, int* dev_out = nullptr) {
 
 int launch(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* stream) {
     LaunchPlan plan;
-    int rc = fill_args(mod, p, A, B, C, p ? p->workspace : nullptr, p ? p->workspace_bytes : 0, &plan);
+    int rc = plan_launch(&mod, p, A, B, C, &plan);
     if (rc) return rc;
     return run_plan(mod, p, plan, p->workspace, (hipStream_t)stream);
 }
@@ -1432,7 +1542,50 @@ int hrn_compile_chw(const hrn_kernel_desc* desc, int expand, double timeout_s) {
     return compile_desc(desc, expand ? PART_EXPAND : PART_CHW, timeout_s, &path);
 }
 
+int hrn_compile_tiles(const hrn_kernel_desc* desc, int part, double timeout_s) {
+    int rc = derive(desc, nullptr);
+    if (rc) return rc;
+    hrn_kernel_desc fit[kMaxFits];
+    int first_half = 0;
+    const int n = cut_tiles(*desc, fit, &first_half);
+    for (int i = 0; i < n; ++i) {
+        Derived dv;
+        (void)derive(&fit[i], &dv);
+        std::string path;
+        if (part == PART_MAIN || dv.has_chw) rc = compile_desc(&fit[i], part, timeout_s, &path);
+        if (rc) return rc;
+    }
+    return n;
+}
+
+int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap) {
+    int rc = derive(desc, nullptr);
+    if (rc) return rc;
+    hrn_kernel_desc fit[kMaxFits];
+    int first_half = 0;
+    const int n = cut_tiles(*desc, fit, &first_half);
+    for (int i = 0; i < n && i < cap; ++i) out[i] = fit[i];
+    return n;
+}
+
+int hrn_launch_tile(const hrn_module* mod, const hrn_problem* p, hrn_kernel_desc* out) {
+    if (!mod || !p || !out) return fail(HRN_E_BADPARAM, "null argument");
+    *out = fitting(mod, p)->desc;
+    return HRN_OK;
+}
+
+void hrn_module_own_tiles(hrn_module* mod, int on) {
+    if (mod) mod->own_tiles.store(on != 0, std::memory_order_relaxed);
+}
+
 int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
+    return build_module(desc, timeout_s, out);
+}
+
+}  // extern "C"
+
+namespace {
+int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
     if (!out) return fail(HRN_E_BADPARAM, "null out");
     *out = nullptr;
     std::string path;
@@ -1452,6 +1605,9 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
         m->epi_bytes = dv.epi_bytes;
         m->chw_bytes = dv.chw_bytes;
     }
+    m->fits = cut_tiles(*desc, m->fit_desc, &m->first_half);
+    for (int i = 0; i < kMaxFits; ++i) { m->fit[i].store(nullptr); m->fit_failed[i] = false; }
+    m->own_tiles.store(false);
     m->has_chw = dv.has_chw;
     m->has_deep = dv.has_deep;
     m->timeout_s = timeout_s;
@@ -1468,6 +1624,7 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
         if (e != hipSuccess) rc = fail(HRN_E_LOAD, "device query: %s", hipGetErrorString(e));
     }
     if (rc) { hrn_module_free(m); return rc; }
+    m->cus = cus;
     m->deep_grid = dv.has_deep ? cus * (163840 / dv.deep_lds) : 0;
     if (desc->split_k) {
         // hrn_launch_splitk_static finds the library's workspace of this device looked up already
@@ -1489,6 +1646,9 @@ int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
     *out = m;
     return HRN_OK;
 }
+}  // namespace
+
+extern "C" {
 
 int hrn_module_info(const hrn_module* mod, hrn_kernel_info* out) {
     if (!mod || !out) return fail(HRN_E_BADPARAM, "null argument");
@@ -1498,6 +1658,7 @@ int hrn_module_info(const hrn_module* mod, hrn_kernel_info* out) {
 
 void hrn_module_free(hrn_module* mod) {
     if (!mod) return;
+    for (auto& f : mod->fit) hrn_module_free(f.load());
     for (CodeObject& c : mod->part)
         if (c.mod) (void)hipModuleUnload(c.mod);
     delete mod;
@@ -1547,8 +1708,9 @@ int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p) {
         if (need < 0) return (int)need;
         q.workspace_bytes = (size_t)need;
     }
+    q.workspace = any;
     LaunchPlan plan;
-    int rc = fill_args(mod, &q, any, any, any, any, q.workspace_bytes, &plan);
+    int rc = plan_launch(&mod, &q, any, any, any, &plan);
     return rc ? rc : (plan.deep ? 1 : 0);
 }
 
@@ -1559,7 +1721,15 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
     if (!mod || !p || !view) return fail(HRN_E_BADPARAM, "null argument");
     if (!mod->has_chw) return fail(HRN_E_BADPARAM, "conv2d_chw takes a conv2d instance without persistent and split_k whose strips fit into LDS");
     LaunchPlan plan;
-    int rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);
+    hrn_problem q = *p;
+    q.workspace = nullptr;
+    q.workspace_bytes = 0;
+    const hrn_module* own = mod;
+    int rc = plan_launch(&mod, &q, In, Filter, Out, &plan);
+    if (!rc && !mod->has_chw) {
+        mod = own;
+        rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);
+    }
     if (rc) return rc;
     if (view->out_plane < 1 || p->m % view->out_plane)
         return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
@@ -1585,7 +1755,7 @@ int hrn_launch_repeat(const hrn_module* mod, const hrn_problem* p, const void* A
                       void* stream) {
     if (count < 1) return fail(HRN_E_BADPARAM, "count %d", count);
     LaunchPlan plan;
-    int rc = fill_args(mod, p, A, B, C, p ? p->workspace : nullptr, p ? p->workspace_bytes : 0, &plan);
+    int rc = plan_launch(&mod, p, A, B, C, &plan);
     if (rc) return rc;
     for (int i = 0; i < count; ++i) {
         rc = run_plan(mod, p, plan, p->workspace, (hipStream_t)stream);

@@ -203,9 +203,12 @@ def _compile_one(job):
 
 def precompile(descs, jobs=None, verbose=False):
     """Compile descriptors into the cache with ``jobs`` parallel hipcc workers, conv instances with their channels-first
-    kernels; returns the failures."""
+    kernels, each with the other tiles its launches may take; returns the failures."""
     jobs = jobs or min(8, os.cpu_count() or 1)
-    tups = [(d.as_tuple(), part) for d in descs for part in ((0, 1, 2) if d.op == CONV else (0,))]
+    every = {d.as_tuple(): d for d in descs}
+    for d in descs:
+        every.update((t.as_tuple(), t) for t in B.tiles(d))
+    tups = [(t, part) for t, d in every.items() for part in ((0, 1, 2) if d.op == CONV else (0,))]
     failures = []
     with ProcessPoolExecutor(max_workers=jobs) as ex:
         for tup, path, err in ex.map(_compile_one, tups):

@@ -242,7 +242,7 @@ def _server_main(conn, device_id):
             if desc_tuple not in mods:
                 if len(mods) > 64:
                     mods.pop(next(iter(mods))).close()
-                mods[desc_tuple] = B.Module(B.make_desc(*desc_tuple))
+                mods[desc_tuple] = B.Module(B.make_desc(*desc_tuple), own_tiles=True)
             mod = mods[desc_tuple]
             p = B.Problem()
             for k, v in prob.items():

@@ -208,6 +208,20 @@ int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, con
 int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
 
 /*
+ * A launch of at most half as many tiles as the device has CUs takes the instance's tile cut in halves (same MFMA shape, same order
+ * along K: same result bit for bit), and a tile of few waves that has a CU to itself takes more of them; persistent and split-K
+ * instances keep theirs.  Such a tile is an instance of its own, compiled and loaded at the first launch that takes it unless
+ * the cache holds it.  hrn_tiles lists those of an instance (returns how many, at most `cap` are written), hrn_compile_tiles
+ * compiles them ahead (part 0: the kernels of plain launches, 1 and 2: those of hrn_launch_conv2d_chw without and with
+ * expand), hrn_launch_tile says which a launch takes, and hrn_module_own_tiles(mod, 1) keeps a module to its own, as a search
+ * over tiles needs.
+ */
+int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap);
+int hrn_compile_tiles(const hrn_kernel_desc* desc, int part, double timeout_s);
+int hrn_launch_tile(const hrn_module* mod, const hrn_problem* p, hrn_kernel_desc* out);
+void hrn_module_own_tiles(hrn_module* mod, int on);
+
+/*
  * Split-K launch that allocates nothing.  No counterpart in the reference; it is for callers that cannot allocate
  * device memory around a launch (code under HIP graph capture, tight serving loops, harnesses that forbid it).  Same as
  * launching a split_k instance through the entry points above, except that the partial sums go to a workspace that

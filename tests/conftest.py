@@ -12,6 +12,19 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
+# files that test the kernels of the very instances they name, on problems small enough for another tile of them
+OWN_TILES = {"test_gpu_parity", "test_gpu_phased", "test_gpu_deep", "test_gpu_fuzz", "test_gpu_channels_first", "test_gpu_colsum",
+             "test_gpu_direct_epilogue", "test_gpu_splitk_fold"}
+
+
+@pytest.fixture(autouse=True)
+def own_tiles(request, monkeypatch):
+    if request.module.__name__.rpartition(".")[2] in OWN_TILES:
+        from heron_amd import backend
+        init = backend.Module.__init__
+        monkeypatch.setattr(backend.Module, "__init__", lambda self, desc, timeout_s=0.0, own_tiles=True: init(self, desc, timeout_s, own_tiles))
+
+
 @pytest.fixture(scope="session")
 def hrn():
     """The ctypes backend; GPU tests fail (not skip) when the HIP library is missing."""
