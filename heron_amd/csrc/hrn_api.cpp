@@ -69,7 +69,7 @@ struct hrn_module {
     hrn_kernel_desc desc;
     int cus;                        // of the device
     // the instance's tile cut for grids that leave the device idle (fitting_tiles): built at the first launch that takes one
-    int fits, first_half;
+    int fits, first_half, end_half;
     hrn_kernel_desc fit_desc[kMaxFits];
     mutable std::atomic<hrn_module*> fit[kMaxFits];
     mutable bool fit_failed[kMaxFits];
@@ -504,7 +504,8 @@ int conv_extent(int in, int k, int stride, int pad, int dil) {
 // A grid of at most half as many tiles as the device has CUs leaves half of it idle, and what bounds such a launch is what one
 // CU fetches and multiplies.  The instance's tile is then cut in halves, the longer side first, down to 64x64, until the
 // grid passes half the CUs; cut tiles keep the MFMA shape and the order along K, so the result is the same bit for bit.  A tile of one
-// to three waves that has a CU to itself is given more: they cannot issue its fetches fast enough.  Cut tiles have a wave
+// to three waves that has a CU to itself is given more, from three k-tiles on: they cannot issue its fetches fast enough (u8 64^3, one
+// k-tile: 4.1 us with one wave, 3.9 - 4.7 with four, as the launches then run dry).  Cut tiles have a wave
 // per SIMD, two from 128x64 on; with an input window one row of MFMA tiles per wave.
 //   u8 x s8 1111x1500x2064 (108 tiles of 128x128 -> 216 of 64x128) 16.9 -> 11.9 us; 96x200x608 (64x64, one wave -> four) 6.4 -> 4.5;
 // conv fp16 16x27x27x128 -> 80 (128x64, two waves -> eight) 18.1 -> 12.9; window convs 8x28x31x64 -> 64, 5x5 (14 tiles of 512x64 ->
@@ -523,21 +524,37 @@ bool with_waves(hrn_kernel_desc d, hrn_kernel_desc* out) {
     return false;
 }
 
-// fit_desc[0]: the own tile with more waves, if it has few; then the halves.  Returns how many there are; *first_half is where
-// the halves begin.
-int cut_tiles(const hrn_kernel_desc& own, hrn_kernel_desc* out, int* first_half) {
+// Of an input window's tile whose workgroup has a CU to itself (more than half of the LDS), the phases - window in, filter taps,
+// result out - take turns: half the rows leave room for a second workgroup, whose phases fill the gaps.  Row-major results with as many
+// waves as before, channels-first ones with half (their strips are as long as a wave has rows) and two stages (a third workgroup).
+//   fp16 512x64 -> 256x64, 3x3: 64x56x56x64 -> 128 52.5 -> 41.1 us, 128x56x56x64 -> 64 52.0 -> 42.2, 32x56x56x64 -> 64 15.5 -> 14.5; 1x1
+// 16x111x111x64 -> 128 22.3 -> 18.7; transposed conv 16x56x56x64 -> 128, stride 2, channels first 35.7 -> 31.0 (25.5 with stores that
+// allocate, see the template).
+constexpr int kOnePerCu = 163840 / 2;
+
+// fit_desc[0]: the own tile with more waves, if it has few; then the halves, [*first_half, *end_half); behind them the half of
+// a window's tile for channels-first results.  Returns how many there are.
+int cut_tiles(const hrn_kernel_desc& own, hrn_kernel_desc* out, int* first_half, int* end_half) {
     int n = 0;
-    *first_half = 0;
+    *first_half = *end_half = 0;
     if (own.persistent || own.split_k) return 0;
     const std::string keep = g_err;
     if (own.wm * own.wn < 4 && with_waves(own, &out[n]) && out[n].wm * out[n].wn >= 4) ++n;
     *first_half = n;
     hrn_kernel_desc d = own;
-    while (n < kMaxFits && (d.bm > 64 || d.bn > 64)) {
+    while (n < kMaxFits - 1 && (d.bm > 64 || d.bn > 64)) {
         if (d.bm > 64 && (d.bm >= d.bn || d.bn <= 64)) d.bm /= 2;
         else d.bn /= 2;
         if (d.bm % 64 || d.bn % 64 || !with_waves(d, &d)) break;
         out[n++] = d;
+    }
+    *end_half = n;
+    d = own;
+    if (own.conv_window && own.wm > 1) {
+        d.bm /= 2; d.wm /= 2;
+        d.stages = 2;
+        d.waves_per_eu = 0;
+        if (derive(&d, nullptr) == HRN_OK) out[n++] = d;
     }
     g_err = keep;
     return n;
@@ -547,14 +564,16 @@ int64_t tiles_of(const hrn_kernel_desc& d, const hrn_problem* p) {
     return (((int64_t)p->m + d.bm - 1) / d.bm) * (((int64_t)p->n + d.bn - 1) / d.bn) * p->batch;
 }
 
-// which of the instance's tiles a launch takes: -1 its own
-int fitting_tiles(const hrn_module* m, const hrn_problem* p) {
+// which of the instance's tiles a launch takes: -1 its own (`lds`: what a workgroup of that needs)
+int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw, int lds) {
     if (!p || p->m < 1 || p->n < 1 || p->batch < 1 || m->fits == 0 || m->own_tiles.load(std::memory_order_relaxed)) return -1;
     const int halves = m->first_half;
     int pick = -1;
     const hrn_kernel_desc* d = &m->desc;
-    for (int i = halves; i < m->fits && tiles_of(*d, p) * 2 <= m->cus; ++i) { pick = i; d = &m->fit_desc[i]; }
-    if (pick < 0 && halves == 1 && tiles_of(m->desc, p) <= m->cus) pick = 0;
+    for (int i = halves; i < m->end_half && tiles_of(*d, p) * 2 <= m->cus; ++i) { pick = i; d = &m->fit_desc[i]; }
+    if (pick < 0 && m->desc.conv_window && lds > kOnePerCu) pick = chw ? (m->fits > m->end_half ? m->end_half : -1) : (halves < m->end_half ? halves : -1);
+    const int64_t row_bytes = (int64_t)p->k * (m->desc.dtype == HRN_DT_F16 ? 2 : 1);
+    if (pick < 0 && halves == 1 && tiles_of(m->desc, p) <= m->cus && row_bytes > 2 * m->desc.bkb) pick = 0;
     return pick;
 }
 
@@ -562,8 +581,8 @@ int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out
 
 // The module whose kernel a launch takes.  One that cannot be built or does not take the problem leaves the launch to the
 // instance itself.
-const hrn_module* fitting(const hrn_module* m, const hrn_problem* p) {
-    const int i = fitting_tiles(m, p);
+const hrn_module* fitting(const hrn_module* m, const hrn_problem* p, bool chw, int lds) {
+    const int i = fitting_tiles(m, p, chw, lds);
     if (i < 0) return m;
     if (const hrn_module* f = m->fit[i].load(std::memory_order_acquire)) return f;
     std::lock_guard<std::mutex> lock(m->part_mutex);
@@ -733,16 +752,33 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restri
 }
 
 // fill_args for the kernel that the launch takes; *mod becomes its module
-int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, const void* B, void* C, LaunchPlan* plan) {
+int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, const void* B, void* C, LaunchPlan* plan, bool chw = false) {
     void* ws = p ? p->workspace : nullptr;
     const size_t ws_bytes = p ? p->workspace_bytes : 0;
     int rc = fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);          // (the instance says what is refused)
     if (rc) return rc;
-    const hrn_module* f = fitting(*mod, p);
+    const hrn_module* f = fitting(*mod, p, chw, (*mod)->info.lds_bytes + (int)plan->dyn_lds);
     if (f == *mod) return HRN_OK;
     if (fill_args(f, p, A, B, C, ws, ws_bytes, plan)) return fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);
     *mod = f;
     return HRN_OK;
+}
+
+// The plan of a launch that is not made: the operands' addresses decide nothing, and what a launch would have to bring is filled in.
+int launch_plan_only(const hrn_module** mod, const hrn_problem* p, LaunchPlan* plan) {
+    void* any = (void*)(uintptr_t)256;
+    hrn_problem q = *p;
+    const hrn_kernel_desc& d = (*mod)->desc;
+    if (d.colsum && !q.bsum) q.bsum = any;
+    q.workspace = any;
+    q.workspace_bytes = 0;
+    if (d.split_k && q.m > 0 && q.n > 0 && q.k > 0 && q.batch > 0) {
+        q.split_k = std::max(1, q.split_k);
+        int kps, split;
+        split_shape(d, &q, &kps, &split);
+        q.workspace_bytes = (size_t)splitk_bytes(&q, split);
+    }
+    return plan_launch(mod, &q, any, any, any, plan);
 }
 
 int run_plan(const hrn_module* mod, const hrn_problem* p, const LaunchPlan& plan, void* workspace, hipStream_t st) {
@@ -1546,8 +1582,8 @@ int hrn_compile_tiles(const hrn_kernel_desc* desc, int part, double timeout_s) {
     int rc = derive(desc, nullptr);
     if (rc) return rc;
     hrn_kernel_desc fit[kMaxFits];
-    int first_half = 0;
-    const int n = cut_tiles(*desc, fit, &first_half);
+    int first_half, end_half;
+    const int n = cut_tiles(*desc, fit, &first_half, &end_half);
     for (int i = 0; i < n; ++i) {
         Derived dv;
         (void)derive(&fit[i], &dv);
@@ -1562,15 +1598,18 @@ int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap) {
     int rc = derive(desc, nullptr);
     if (rc) return rc;
     hrn_kernel_desc fit[kMaxFits];
-    int first_half = 0;
-    const int n = cut_tiles(*desc, fit, &first_half);
+    int first_half, end_half;
+    const int n = cut_tiles(*desc, fit, &first_half, &end_half);
     for (int i = 0; i < n && i < cap; ++i) out[i] = fit[i];
     return n;
 }
 
 int hrn_launch_tile(const hrn_module* mod, const hrn_problem* p, hrn_kernel_desc* out) {
     if (!mod || !p || !out) return fail(HRN_E_BADPARAM, "null argument");
-    *out = fitting(mod, p)->desc;
+    LaunchPlan plan;
+    int rc = launch_plan_only(&mod, p, &plan);
+    if (rc) return rc;
+    *out = mod->desc;
     return HRN_OK;
 }
 
@@ -1605,7 +1644,7 @@ int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out
         m->epi_bytes = dv.epi_bytes;
         m->chw_bytes = dv.chw_bytes;
     }
-    m->fits = cut_tiles(*desc, m->fit_desc, &m->first_half);
+    m->fits = cut_tiles(*desc, m->fit_desc, &m->first_half, &m->end_half);
     for (int i = 0; i < kMaxFits; ++i) { m->fit[i].store(nullptr); m->fit_failed[i] = false; }
     m->own_tiles.store(false);
     m->has_chw = dv.has_chw;
@@ -1698,19 +1737,8 @@ int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, con
 
 int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p) {
     if (!mod || !p) return fail(HRN_E_BADPARAM, "null argument");
-    // (the operands' addresses decide nothing; what a launch would have to bring is filled in)
-    void* any = (void*)(uintptr_t)256;
-    hrn_problem q = *p;
-    if (mod->desc.colsum && !q.bsum) q.bsum = any;
-    if (mod->desc.split_k) {
-        q.split_k = std::max(1, q.split_k);
-        const int64_t need = hrn_splitk_workspace_bytes(&mod->desc, &q);
-        if (need < 0) return (int)need;
-        q.workspace_bytes = (size_t)need;
-    }
-    q.workspace = any;
     LaunchPlan plan;
-    int rc = plan_launch(&mod, &q, any, any, any, &plan);
+    int rc = launch_plan_only(&mod, p, &plan);
     return rc ? rc : (plan.deep ? 1 : 0);
 }
 
@@ -1725,7 +1753,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
     q.workspace = nullptr;
     q.workspace_bytes = 0;
     const hrn_module* own = mod;
-    int rc = plan_launch(&mod, &q, In, Filter, Out, &plan);
+    int rc = plan_launch(&mod, &q, In, Filter, Out, &plan, true);
     if (!rc && !mod->has_chw) {
         mod = own;
         rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);

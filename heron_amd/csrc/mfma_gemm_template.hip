@@ -770,6 +770,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             // same pixels of other channels (HOIST), the division is made once per strip of pixels, not per piece
             // (NCW conv1d 16 x 892 x 512 -> 512: 40.2 -> 38.2 us).
             const unsigned plane = (unsigned)a.out_plane;
+            // Planes that are no whole lines begin and end strips inside them: such stores go through the L2, which joins the pieces
+            // (transposed conv with planes of 111x111, 256x64 tiles: 31.0 us with the non-temporal hint, 25.5 without).
+            [[maybe_unused]] const bool whole_lines = plane * OES % 128 == 0;
             constexpr bool HOIST = 64 % CPRW == 0;
             constexpr int NIB = HOIST ? TM / IT : 1;
             unsigned h_img[NIB], h_px[NIB];
@@ -825,7 +828,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                             const unsigned px = HOIST ? h_px[HOIST ? ib / IT : 0] : (unsigned)m - img * plane;
                             oel_t* dst = (oel_t*)a.C + ((int64_t)img * a.N + n) * plane + px;
                             if (px + EPC <= plane && m + EPC <= a.M) {
-                                if constexpr (NTS) __builtin_nontemporal_store(val, (piece_t*)dst);
+                                if (NTS && whole_lines) __builtin_nontemporal_store(val, (piece_t*)dst);
                                 else *(piece_t*)dst = val;
                             } else {
                                 const oel_t* ve = (const oel_t*)&val;

@@ -213,7 +213,7 @@ int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
  * instances keep theirs.  Such a tile is an instance of its own, compiled and loaded at the first launch that takes it unless
  * the cache holds it.  hrn_tiles lists those of an instance (returns how many, at most `cap` are written), hrn_compile_tiles
  * compiles them ahead (part 0: the kernels of plain launches, 1 and 2: those of hrn_launch_conv2d_chw without and with
- * expand), hrn_launch_tile says which a launch takes, and hrn_module_own_tiles(mod, 1) keeps a module to its own, as a search
+ * expand), hrn_launch_tile says which a row-major launch takes, and hrn_module_own_tiles(mod, 1) keeps a module to its own, as a search
  * over tiles needs.
  */
 int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap);

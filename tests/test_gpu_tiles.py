@@ -50,17 +50,18 @@ def test_gemm(name, hrn):
         A, W = _operands(f16, (b, m, k), (b, n, k), i)
         if b == 1:
             A, W = A[0], W[0]
-        p = B.gemm_problem(b, m, n, k)
-        assert not _cut(own, p)
-        t = mod.launch_tile(p)
-        taken.add((t.bm, t.bn, t.wm, t.wn))
-        tiles = -(-m // d.bm) * -(-n // d.bn) * b
-        assert _cut(mod, p) == (tiles <= (256 if d.wm * d.wn < 4 else 128) and bool(B.tiles(d)))
         if (n % 8 and f16) and d.epilogue:
             for x in (mod, own):
                 with pytest.raises(B.HeronRocmError):
                     hostops.gemm(x, A, W)
             continue
+        p = B.gemm_problem(b, m, n, k)
+        assert not _cut(own, p)
+        t = mod.launch_tile(p)
+        taken.add((t.bm, t.bn, t.wm, t.wn))
+        tiles = -(-m // d.bm) * -(-n // d.bn) * b
+        few_waves = d.wm * d.wn < 4 and k * (2 if f16 else 1) > 2 * d.bkb
+        assert _cut(mod, p) == (tiles <= (256 if few_waves else 128 if d.bm > 64 or d.bn > 64 else 0))
         print("tiles gemm", name, (b, m, n, k), t.as_tuple(), flush=True)
         bsum = hostops.column_sums(W) if d.colsum else None
         assert torch.equal(hostops.gemm(mod, A, W, bsum=bsum), hostops.gemm(own, A, W, bsum=bsum))
@@ -83,7 +84,7 @@ def test_conv(name, hrn):
         print("tiles conv", name, cases[i], flush=True)
         bsum = hostops.column_sums(F) if d.colsum else None
         assert torch.equal(hostops.conv2d_nhwc(mod, X, F, s, pd, dl, bsum=bsum), hostops.conv2d_nhwc(own, X, F, s, pd, dl, bsum=bsum))
-    assert 2 <= cut < len(cases) or not f16
+    assert cut >= 2 and (cut < len(cases) or d.conv_window)
     mod.close()
     own.close()
 
