@@ -208,6 +208,156 @@ PyObject* conv2d(PyObject*, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
+// ---- the passes and the channels-first launch of hostops.run_operator ----
+// An eager conv3d spent 30 us of Python and ctypes on three kernels of 16 us.
+bool plain(const at::Tensor* t) {
+    return t && t->is_cuda() && t->is_contiguous() && (t->element_size() == 1 || t->element_size() == 2 || t->element_size() == 4);
+}
+
+// channels_last(x, cp): (N, C, L) -> (N, L, cp)
+PyObject* channels_last(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        int64_t cp;
+        if (n != 2 || !ints(args, 1, 1, &cp)) {
+            PyErr_Clear();
+            Py_RETURN_NONE;
+        }
+        const at::Tensor* x = tensor(args[0]);
+        if (!plain(x) || x->dim() != 3) Py_RETURN_NONE;
+        const int64_t N = x->size(0), C = x->size(1), L = x->size(2);
+        if (!fits_int(N) || !fits_int(C) || !fits_int(L) || !fits_int(cp) || N > 65535) Py_RETURN_NONE;
+        at::Tensor out;
+        int rc;
+        {
+            Unlocked unlocked;
+            out = at::empty({N, L, cp}, x->options());
+            rc = hrn_transpose_pad(x->data_ptr(), out.data_ptr(), (int)N, (int)C, (int)L, (int)cp, (int)x->element_size(), stream());
+        }
+        return rc == HRN_OK ? THPVariable_Wrap(out) : PyLong_FromLong(rc);
+    });
+}
+
+// integers of a tuple or list, at most `cap`; -1: something else
+int int_list(PyObject* o, int64_t* out, int cap) {
+    if (!PyTuple_Check(o) && !PyList_Check(o)) return -1;
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(o);
+    if (n > cap) return -1;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        out[i] = PyLong_AsLongLong(PySequence_Fast_GET_ITEM(o, i));
+        if (out[i] == -1 && PyErr_Occurred()) return -1;
+    }
+    return (int)n;
+}
+
+// gather(src, out, dst_dim, coords, dst_stride, dst_live, op, aux): backend.make_gather and the pass; HRN_OK or its error code
+PyObject* gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        hrn_gather g = {};
+        int64_t op;
+        auto parse = [&]() {
+            if (n != 8 || !ints(args, 6, 1, &op)) return false;
+            const int nd = int_list(args[2], g.dst_dim, HRN_GATHER_DIMS);
+            if (nd < 1 || !PyList_Check(args[3])) return false;
+            const Py_ssize_t ns = PyList_GET_SIZE(args[3]);
+            if (ns < 1 || ns > HRN_GATHER_DIMS) return false;
+            int64_t stride = 1;
+            for (int d = nd - 1; d >= 0; --d) {
+                g.dst_stride[d] = stride;
+                g.dst_live[d] = g.dst_dim[d];
+                stride *= g.dst_dim[d];
+            }
+            if (args[4] != Py_None && int_list(args[4], g.dst_stride, HRN_GATHER_DIMS) != nd) return false;
+            if (args[5] != Py_None && int_list(args[5], g.dst_live, HRN_GATHER_DIMS) != nd) return false;
+            for (Py_ssize_t s = 0; s < ns; ++s) {
+                PyObject* e = PyList_GET_ITEM(args[3], s);
+                if (!PyTuple_Check(e)) return false;
+                const Py_ssize_t len = PyTuple_GET_SIZE(e);
+                if (len < 3 || len > 5 || !PyDict_Check(PyTuple_GET_ITEM(e, 2))) return false;
+                int64_t v[5] = {0, 0, 0, 0, 1};
+                for (Py_ssize_t i = 0; i < len; ++i) {
+                    if (i == 2) continue;
+                    v[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(e, i));
+                    if (v[i] == -1 && PyErr_Occurred()) return false;
+                }
+                g.src_dim[s] = v[0]; g.src_stride[s] = v[1]; g.add[s] = v[3]; g.div[s] = v[4];
+                PyObject *key, *val;
+                Py_ssize_t pos = 0;
+                while (PyDict_Next(PyTuple_GET_ITEM(e, 2), &pos, &key, &val)) {
+                    const long long d = PyLong_AsLongLong(key), m = PyLong_AsLongLong(val);
+                    if (PyErr_Occurred() || d < 0 || d >= nd) return false;
+                    g.mul[s][d] = m;
+                }
+            }
+            g.ndim = nd;
+            g.nsrc = (int32_t)ns;
+            g.op = (int32_t)op;
+            return true;
+        };
+        const at::Tensor *src = n == 8 ? tensor(args[0]) : nullptr, *out = n == 8 ? tensor(args[1]) : nullptr;
+        const at::Tensor* aux = n == 8 ? tensor(args[7]) : nullptr;
+        if (!plain(src) || !plain(out) || (!aux && args[7] != Py_None) || (aux && !plain(aux)) || !parse()) {
+            PyErr_Clear();
+            Py_RETURN_NONE;
+        }
+        g.elem_bytes = (int32_t)src->element_size();
+        int rc;
+        {
+            Unlocked unlocked;
+            rc = hrn_gather_nd(&g, src->data_ptr(), aux ? aux->data_ptr() : nullptr, out->data_ptr(), stream());
+        }
+        return PyLong_FromLong(rc);
+    });
+}
+
+// conv_chw(native, group_m, split_k, X, xshape, W, stride, pad, dil, view, shape, bsum): hrn_launch_conv2d_chw with a fresh result of
+// `shape`; view: (expand, in_h, in_w, top, left)
+PyObject* conv_chw(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        Instance in;
+        int64_t v[2], x4[4], vw[5], shape[5], sh, sw, ph, pw, dh, dw;
+        int dims = -1;
+        if (n != 12 || !in.read(args[0]) || !ints(args, 1, 2, v) || int_list(args[4], x4, 4) != 4 || !pair(args[6], &sh, &sw) ||
+            !pair(args[7], &ph, &pw) || !pair(args[8], &dh, &dw) || int_list(args[9], vw, 5) != 5 || (dims = int_list(args[10], shape, 5)) < 2) {
+            PyErr_Clear();
+            Py_RETURN_NONE;
+        }
+        const at::Tensor *X = tensor(args[3]), *W = tensor(args[5]);
+        if (!is(X, in.a) || !is(W, in.b) || W->dim() != 4 || x4[3] != W->size(3) || sh < 1 || sw < 1 || ph < 0 || pw < 0 || dh < 1 || dw < 1 ||
+            in.desc->split_k || !sums_fit(in, args[11], W->size(0)))
+            Py_RETURN_NONE;
+        for (int i = 0; i < 4; ++i)
+            if (!fits_int(x4[i]) || !fits_int(W->size(i))) Py_RETURN_NONE;
+        // (what is in memory: the pixels before the expansion)
+        if (X->numel() != x4[0] * (vw[0] > 0 ? vw[1] * vw[2] : x4[1] * x4[2]) * x4[3]) Py_RETURN_NONE;
+        if (std::max({sh, sw, ph, pw, dh, dw}) > 1 << 20) Py_RETURN_NONE;
+        for (int64_t e : vw)
+            if (e < 0 || e > INT32_MAX) Py_RETURN_NONE;
+        hrn_problem p;
+        hrn_problem_conv2d_hw(&p, (int)x4[0], (int)x4[1], (int)x4[2], (int)x4[3], (int)W->size(0), (int)W->size(1), (int)W->size(2), (int)sh,
+                              (int)sw, (int)ph, (int)pw, (int)dh, (int)dw);
+        p.group_m = (int32_t)v[0];
+        int64_t count = 1;
+        for (int i = 0; i < dims; ++i) {
+            if (!fits_int(shape[i])) Py_RETURN_NONE;
+            count *= shape[i];
+            if (count > INT64_MAX >> 32) Py_RETURN_NONE;
+        }
+        if (p.m < 1 || count != (int64_t)p.m * p.n || p.m % shape[0]) Py_RETURN_NONE;
+        hrn_conv_view view = {(int32_t)(p.m / shape[0]), (int32_t)vw[0], (int32_t)vw[1], (int32_t)vw[2], (int32_t)vw[3], (int32_t)vw[4]};
+        const at::Tensor* sums = tensor(args[11]);
+        at::Tensor C;
+        int rc;
+        {
+            Unlocked unlocked;
+            C = at::empty(at::IntArrayRef(shape, dims), X->options().dtype(in.c));
+            Extras x;
+            rc = x.add(in, &p, *W, sums, v[1]);
+            if (rc == HRN_OK) rc = hrn_launch_conv2d_chw(in.mod, &p, &view, X->data_ptr(), W->data_ptr(), C.data_ptr(), stream());
+        }
+        return rc == HRN_OK ? THPVariable_Wrap(C) : PyLong_FromLong(rc);
+    });
+}
+
 // stream(): the current stream's handle
 PyObject* current_stream(PyObject*, PyObject*) {
     return guarded([&]() -> PyObject* { return PyLong_FromVoidPtr(stream()); });
@@ -216,6 +366,10 @@ PyObject* current_stream(PyObject*, PyObject*) {
 PyMethodDef methods[] = {
     {"gemm", (PyCFunction)(void (*)(void))gemm, METH_FASTCALL, "gemm(native, group_m, split_k, A, B, out, bsum)"},
     {"conv2d", (PyCFunction)(void (*)(void))conv2d, METH_FASTCALL, "conv2d(native, group_m, split_k, X, W, stride, pad, dil, out, bsum)"},
+    {"channels_last", (PyCFunction)(void (*)(void))channels_last, METH_FASTCALL, "channels_last(x, cp)"},
+    {"gather", (PyCFunction)(void (*)(void))gather, METH_FASTCALL, "gather(src, out, dst_dim, coords, dst_stride, dst_live, op, aux)"},
+    {"conv_chw", (PyCFunction)(void (*)(void))conv_chw, METH_FASTCALL,
+     "conv_chw(native, group_m, split_k, X, xshape, W, stride, pad, dil, view, shape, bsum)"},
     {"stream", current_stream, METH_NOARGS, "handle of torch's current stream"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -168,6 +168,12 @@ def _native_ok(t):
 def _gather(src, out, dst_dim, coords, dst_stride=None, dst_live=None, op=B.GATHER_COPY, aux=None):
     """One pass of the library's affine gather from ``src`` into ``out`` (both contiguous device tensors; see
     backend.make_gather for ``coords``)."""
+    if _recording is None:
+        rc = (B._ext or B.ext()).gather(src, out, dst_dim, coords, dst_stride, dst_live, op, aux)
+        if rc is not None:
+            if rc:
+                B._check(rc)
+            return out
     g = B.make_gather(src.element_size(), dst_dim, coords, dst_stride, dst_live, op)
     _do(B.gather_nd, g, src.data_ptr(), out.data_ptr(), aux.data_ptr() if aux is not None else None, _stream())
     return out
@@ -177,6 +183,10 @@ def _channels_last(x3, cp=None):
     """(N, C, L) -> (N, L, cp): channels become the last axis, zero-padded to ``cp`` (one pass of the library)."""
     N, C, L = x3.shape
     cp = cp or C
+    if _recording is None and x3.is_cuda:
+        out = (B._ext or B.ext()).channels_last(x3, cp)
+        if out is not None:
+            return out if type(out) is not int else B._check(out)
     if _native_ok(x3) and N <= 65535 and L > 0:
         out = _new(torch.empty, (N, L, cp), dtype=x3.dtype, device=x3.device)
         _do(B.transpose_pad, x3.data_ptr(), out.data_ptr(), N, C, L, cp, x3.element_size(), _stream())
@@ -476,13 +486,23 @@ def _run_channels_first(mod, info, inputs, act, Bm, group_m, split_k, bsum):
     else:
         A = act(info, *inputs)
         xshape = A.shape
+    stride, pad, dil = (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w'])
+    if _recording is None and Bm.dim() == 4:
+        n, h, w, _ = xshape
+        CO, KH, KW, _ = Bm.shape
+        ho = (h - ((KH - 1) * dil[0] + 1) + 2 * pad[0]) // stride[0] + 1
+        wo = (w - ((KW - 1) * dil[1] + 1) + 2 * pad[1]) // stride[1] + 1
+        at = (t['stride'], H, W, top, left) if expand else (0, 0, 0, 0, 0)
+        C = (B._ext or B.ext()).conv_chw(mod.native, group_m, split_k, A, tuple(xshape), Bm, stride, pad, dil, at,
+                                         CHANNELS_FIRST[info['adapter']](info, n, CO, ho, wo), bsum)
+        if C is not None:
+            return C if type(C) is not int else B._check(C)
     _chk(A, torch.float16 if f16 else torch.uint8)
     _chk(Bm, torch.float16 if f16 else torch.int8)
     CO, KH, KW, CI = Bm.shape
     if xshape[3] != CI:
         raise ValueError("channel mismatch")
-    p = B.conv2d_problem(*xshape, CO, KH, KW, (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']), group_m,
-                         split_k)
+    p = B.conv2d_problem(*xshape, CO, KH, KW, stride, pad, dil, group_m, split_k)
     if bsum is not None and mod.desc.colsum:
         _chk(bsum, torch.int32)
         if bsum.numel() != p.n:
