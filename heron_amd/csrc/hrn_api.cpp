@@ -504,11 +504,12 @@ int conv_extent(int in, int k, int stride, int pad, int dil) {
 // A grid of at most half as many tiles as the device has CUs leaves half of it idle, and what bounds such a launch is what one
 // CU fetches and multiplies.  The instance's tile is then cut in halves, the longer side first, down to 64x64, until the
 // grid passes half the CUs; cut tiles keep the MFMA shape and the order along K, so the result is the same bit for bit.  A tile of one
-// to three waves that has a CU to itself is given more, from three k-tiles on: they cannot issue its fetches fast enough (u8 64^3, one
-// k-tile: 4.1 us with one wave, 3.9 - 4.7 with four, as the launches then run dry).  Cut tiles have a wave
+// to three waves is given more: they cannot issue its fetches fast enough.  Up to 6 tiles per CU that was measured; not for one
+// or two k-tiles on at most as many tiles as CUs (u8 64^3: 4.1 us with one wave, 3.9 - 4.7 with four, as the launches then run dry),
+// nor on larger grids for channels-first results, whose strips are as long as a wave has rows.  Cut tiles have a wave
 // per SIMD, two from 128x64 on; with an input window one row of MFMA tiles per wave.
-//   u8 x s8 1111x1500x2064 (108 tiles of 128x128 -> 216 of 64x128) 16.9 -> 11.9 us; 96x200x608 (64x64, one wave -> four) 6.4 -> 4.5;
-// conv fp16 16x27x27x128 -> 80 (128x64, two waves -> eight) 18.1 -> 12.9; window convs 8x28x31x64 -> 64, 5x5 (14 tiles of 512x64 ->
+//   u8 x s8 1111x1500x2064 (108 tiles of 128x128 -> 216 of 64x128) 16.9 -> 11.9 us; 96x200x608 (64x64, one wave -> four) 6.4 -> 4.5, 4096x800x2048 26.0 -> 19.2;
+// conv fp16 16x27x27x128 -> 80 (128x64, two waves -> eight) 18.1 -> 12.9, 1x1 32x56x56x96 -> 64 14.0 -> 10.9; window convs 8x28x31x64 -> 64, 5x5 (14 tiles of 512x64 ->
 // 109 of 64x64) 25.4 -> 12.7 and u8 22x16x16x192 -> 80 (44 of 256x64 -> 176) 15.5 -> 10.7.  Above the line: fp16 2000x2000x1024 (256 tiles
 // of 128x128) 13.0 us, 15.0 with 64x128.
 bool with_waves(hrn_kernel_desc d, hrn_kernel_desc* out) {
@@ -572,8 +573,8 @@ int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw, int lds) 
     const hrn_kernel_desc* d = &m->desc;
     for (int i = halves; i < m->end_half && tiles_of(*d, p) * 2 <= m->cus; ++i) { pick = i; d = &m->fit_desc[i]; }
     if (pick < 0 && m->desc.conv_window && lds > kOnePerCu) pick = chw ? (m->fits > m->end_half ? m->end_half : -1) : (halves < m->end_half ? halves : -1);
-    const int64_t row_bytes = (int64_t)p->k * (m->desc.dtype == HRN_DT_F16 ? 2 : 1);
-    if (pick < 0 && halves == 1 && tiles_of(m->desc, p) <= m->cus && row_bytes > 2 * m->desc.bkb) pick = 0;
+    const int64_t row_bytes = (int64_t)p->k * (m->desc.dtype == HRN_DT_F16 ? 2 : 1), tiles = tiles_of(m->desc, p);
+    if (pick < 0 && halves == 1 && tiles <= 6 * (int64_t)m->cus && (tiles <= m->cus ? row_bytes > 2 * m->desc.bkb : !chw)) pick = 0;
     return pick;
 }
 

@@ -209,7 +209,7 @@ int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
 
 /*
  * A launch of at most half as many tiles as the device has CUs takes the instance's tile cut in halves (same MFMA shape, same order
- * along K: same result bit for bit), and a tile of few waves that has a CU to itself takes more of them; persistent and split-K
+ * along K: same result bit for bit), and a tile of one to three waves takes more of them on grids of at most six tiles a CU; persistent and split-K
  * instances keep theirs.  Such a tile is an instance of its own, compiled and loaded at the first launch that takes it unless
  * the cache holds it.  hrn_tiles lists those of an instance (returns how many, at most `cap` are written), hrn_compile_tiles
  * compiles them ahead (part 0: the kernels of plain launches, 1 and 2: those of hrn_launch_conv2d_chw without and with

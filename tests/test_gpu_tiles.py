@@ -46,7 +46,7 @@ def test_gemm(name, hrn):
     mod, own, f16 = B.Module(d), B.Module(d, own_tiles=True), d.dtype == F16
     taken = set()
     for i, (b, m, n, k) in enumerate([(1, 64, 64, 64), (1, 1, 4, 16), (1, 65, 68, 1040), (1, 1111, 1500, 2064), (3, 130, 36, 304), (1, 2048, 1024, 256),
-                                      (1, 1025, 2052, 128), (40, 182, 64, 96), (1, 4100, 4100, 80)]):
+                                      (1, 1025, 2052, 128), (1, 2049, 580, 208), (40, 182, 64, 96), (1, 4100, 4100, 80)]):
         A, W = _operands(f16, (b, m, k), (b, n, k), i)
         if b == 1:
             A, W = A[0], W[0]
@@ -60,8 +60,8 @@ def test_gemm(name, hrn):
         t = mod.launch_tile(p)
         taken.add((t.bm, t.bn, t.wm, t.wn))
         tiles = -(-m // d.bm) * -(-n // d.bn) * b
-        few_waves = d.wm * d.wn < 4 and k * (2 if f16 else 1) > 2 * d.bkb
-        assert _cut(mod, p) == (tiles <= (256 if few_waves else 128 if d.bm > 64 or d.bn > 64 else 0))
+        few_waves = d.wm * d.wn < 4 and (256 < tiles <= 6 * 256 or (tiles <= 256 and k * (2 if f16 else 1) > 2 * d.bkb))
+        assert _cut(mod, p) == (few_waves or (tiles <= 128 and (d.bm > 64 or d.bn > 64)))
         print("tiles gemm", name, (b, m, n, k), t.as_tuple(), flush=True)
         bsum = hostops.column_sums(W) if d.colsum else None
         assert torch.equal(hostops.gemm(mod, A, W, bsum=bsum), hostops.gemm(own, A, W, bsum=bsum))
