@@ -61,6 +61,9 @@ const char* const kPartFile[PARTS] = {"", "_chw", "_expand"};
 struct CodeObject {
     hipModule_t mod = nullptr;
     hipFunction_t fn[2] = {};       // plain and deep (a third stage); null where the instance has no room for it
+    std::string path;               // of the file, where the cache holds it
+    std::atomic<bool> ready{false}; // loaded
+    bool failed = false;            // to load (tiles of an instance only)
 };
 
 constexpr int kMaxFits = 6;
@@ -68,11 +71,11 @@ constexpr int kMaxFits = 6;
 struct hrn_module {
     hrn_kernel_desc desc;
     int cus;                        // of the device
-    // the instance's tile cut for grids that leave the device idle (fitting_tiles): built at the first launch that takes one
+    // the instance's other tiles (fitting_tiles): those whose code objects the cache held in hrn_build, each loaded at the first
+    // launch that takes it; null: not in the cache
     int fits, first_half, end_half;
     hrn_kernel_desc fit_desc[kMaxFits];
-    mutable std::atomic<hrn_module*> fit[kMaxFits];
-    mutable bool fit_failed[kMaxFits];
+    hrn_module* fit[kMaxFits];
     std::atomic<bool> own_tiles;    // launches keep to the instance's own tile
     hrn_kernel_info info;
     mutable CodeObject part[PARTS]; // those of hrn_launch_conv2d_chw are there from hrn_build on or from their first launch
@@ -81,7 +84,6 @@ struct hrn_module {
     int device;                     // the code objects are loaded on
     double timeout_s;               // of a compilation
     int deep_grid;      // workgroups of the deep kernels that the device holds at once
-    std::string path;
     int persist_grid;   // persistent instances: workgroups that fit the device at once (multiple of 8 when >= 8)
     int epi_bytes;      // LDS bytes of the epilogue region (column sums + strips)
     int chw_bytes;      // the same of the channels-first epilogue
@@ -325,6 +327,13 @@ int run_hipcc(const std::vector<std::string>& args, const std::string& log_path,
     return HRN_OK;
 }
 
+// what the template is compiled from: its text and extra compiler flags (e.g. -D switches of the template under study)
+uint64_t template_hash(const std::string& src, const std::string& extra) {
+    uint64_t h = fnv1a_file(src);
+    for (unsigned char ch : extra) { h ^= ch; h *= 1099511628211ull; }
+    return h;
+}
+
 int compile_desc(const hrn_kernel_desc* d, int part, double timeout_s, std::string* out_path) {
     Derived dv;
     int rc = derive(d, &dv);
@@ -334,11 +343,8 @@ int compile_desc(const hrn_kernel_desc* d, int part, double timeout_s, std::stri
     if (!file_exists(src)) return fail(HRN_E_BUILD, "kernel template not found: %s", src.c_str());
     const std::string dir = cache_dir();
     mkdir(dir.c_str(), 0755);
-    // extra compiler flags (e.g. -D switches of the template under study) are part of the instance's identity
     const std::string extra = env_or("HRN_HIPCC_FLAGS", "");
-    uint64_t srch = fnv1a_file(src);
-    for (unsigned char ch : extra) { srch ^= ch; srch *= 1099511628211ull; }
-    const std::string key = desc_key(d, srch) + kPartFile[part];
+    const std::string key = desc_key(d, template_hash(src, extra)) + kPartFile[part];
     const std::string co = dir + "/" + key + ".hsaco";
     const std::string info = dir + "/" + key + ".info";
     *out_path = co;
@@ -396,18 +402,35 @@ int compile_desc(const hrn_kernel_desc* d, int part, double timeout_s, std::stri
 }
 
 int load_part(const std::string& path, int part, bool deep, CodeObject* out) {
-    CodeObject c;
-    hipError_t e = hipModuleLoad(&c.mod, path.c_str());
+    hipModule_t mod = nullptr;
+    hipFunction_t fn[2] = {};
+    hipError_t e = hipModuleLoad(&mod, path.c_str());
     if (e != hipSuccess) return fail(HRN_E_LOAD, "hipModuleLoad(%s): %s", path.c_str(), hipGetErrorString(e));
     const std::string name = kPartKernel[part];
-    e = hipModuleGetFunction(&c.fn[0], c.mod, name.c_str());
-    if (e == hipSuccess && deep) e = hipModuleGetFunction(&c.fn[1], c.mod, (name + "_deep").c_str());
+    e = hipModuleGetFunction(&fn[0], mod, name.c_str());
+    if (e == hipSuccess && deep) e = hipModuleGetFunction(&fn[1], mod, (name + "_deep").c_str());
     if (e != hipSuccess) {
-        (void)hipModuleUnload(c.mod);
+        (void)hipModuleUnload(mod);
         return fail(HRN_E_LOAD, "hipModuleGetFunction(%s): %s", name.c_str(), hipGetErrorString(e));
     }
-    *out = c;
+    out->mod = mod;
+    out->fn[0] = fn[0]; out->fn[1] = fn[1];
+    out->ready.store(true, std::memory_order_release);
     return HRN_OK;
+}
+
+// load_part outside hrn_build: on the module's device, also while this thread captures a stream (loading allocates, which such a
+// thread may otherwise not do).  Holds part_mutex.
+int load_late(const hrn_module* m, const std::string& path, int part) {
+    int dev = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    hipError_t e = dev == m->device ? hipSuccess : hipSetDevice(m->device);
+    const int rc = e == hipSuccess ? load_part(path, part, m->has_deep, &m->part[part]) : fail(HRN_E_LOAD, "hipSetDevice: %s", hipGetErrorString(e));
+    if (dev != m->device) (void)hipSetDevice(dev);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return rc;
 }
 
 // The channels-first kernels of a module: compiled and loaded here if hrn_build did not find them in the cache.
@@ -417,17 +440,23 @@ int chw_kernels(const hrn_module* m, int part, const CodeObject** out) {
     if (m->part[part].mod) return HRN_OK;
     std::string path;
     int rc = compile_desc(&m->desc, part, m->timeout_s, &path);
-    if (rc) return rc;
-    int dev = 0;
-    HIP_TRY(hipGetDevice(&dev));
-    // (loading allocates, which a thread that captures a stream may otherwise not do)
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-    hipError_t e = dev == m->device ? hipSuccess : hipSetDevice(m->device);
-    rc = e == hipSuccess ? load_part(path, part, m->has_deep, &m->part[part]) : fail(HRN_E_LOAD, "hipSetDevice: %s", hipGetErrorString(e));
-    if (dev != m->device) (void)hipSetDevice(dev);
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    return rc;
+    return rc ? rc : load_late(m, path, part);
+}
+
+// The same of a tile of an instance (hrn_module.fit), which no launch compiles; false: the launch is the instance's own.
+bool tile_kernels(const hrn_module* f, int part) {
+    CodeObject& c = f->part[part];
+    if (c.ready.load(std::memory_order_acquire)) return true;
+    std::lock_guard<std::mutex> lock(f->part_mutex);
+    if (c.ready.load(std::memory_order_acquire)) return true;
+    if (c.failed) return false;
+    const std::string keep = g_err;
+    c.failed = load_late(f, c.path, part) != HRN_OK;
+    if (c.failed) {
+        g_err = keep;
+        (void)hipGetLastError();        // (no error of the launch)
+    }
+    return !c.failed;
 }
 
 void read_info(const std::string& path, hrn_kernel_info* o) {
@@ -578,36 +607,6 @@ int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw, int lds) 
     return pick;
 }
 
-int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out);
-
-// The module whose kernel a launch takes.  One that cannot be built or does not take the problem leaves the launch to the
-// instance itself.
-const hrn_module* fitting(const hrn_module* m, const hrn_problem* p, bool chw, int lds) {
-    const int i = fitting_tiles(m, p, chw, lds);
-    if (i < 0) return m;
-    if (const hrn_module* f = m->fit[i].load(std::memory_order_acquire)) return f;
-    std::lock_guard<std::mutex> lock(m->part_mutex);
-    if (const hrn_module* f = m->fit[i].load(std::memory_order_acquire)) return f;
-    if (m->fit_failed[i]) return m;
-    hrn_module* f = nullptr;
-    int dev = 0;
-    const std::string keep = g_err;
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;       // (see chw_kernels)
-    bool ok = hipGetDevice(&dev) == hipSuccess && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    if (ok) {
-        ok = (dev == m->device || hipSetDevice(m->device) == hipSuccess) && build_module(&m->fit_desc[i], m->timeout_s, &f) == HRN_OK;
-        if (dev != m->device) (void)hipSetDevice(dev);
-        (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-    if (!ok) {
-        m->fit_failed[i] = true;
-        g_err = keep;
-        return m;
-    }
-    m->fit[i].store(f, std::memory_order_release);
-    return f;
-}
-
 int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
               size_t workspace_bytes, LaunchPlan* plan) {
     HrnKArgs* k = &plan->k;
@@ -705,7 +704,6 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     const int64_t a_bytes = d.op == HRN_OP_GEMM ? (int64_t)p->m * p->k * es : (int64_t)p->cn * p->ch * p->cw * p->ci * es;
     plan->deep = deep_fits(mod, total, d.split_k ? k->kt_per_slice : (int)(((int64_t)p->k * es + d.bkb - 1) / d.bkb),
                            p->batch * (a_bytes + b_bytes));
-    plan->fn = mod->part[PART_MAIN].fn[plan->deep];
     if (d.persistent) {
         if ((int64_t)p->n * oes % 16) return fail(HRN_E_BADPARAM, "persistent instances store whole 16-byte chunks: N*%d must be a multiple of 16", oes);
         if ((int64_t)p->m * p->ldc * oes >= (1ll << 31)) return fail(HRN_E_BADPARAM, "persistent: C exceeds 2 GiB per batch entry");
@@ -718,6 +716,29 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         plan->grid = (unsigned)g;
     }
     return HRN_OK;
+}
+
+// A module of `desc` with nothing loaded yet, whose code objects lie at `stem`: the main one is there.
+hrn_module* module_of(const hrn_kernel_desc* desc, const std::string& stem, double timeout_s, int dev, int cus) {
+    hrn_module* m = new hrn_module();
+    Derived dv;
+    (void)derive(desc, &dv);            // (the caller has validated the descriptor)
+    m->desc = *desc;
+    read_info(stem + ".info", &m->info);
+    m->info.threads = desc->wm * desc->wn * 64;
+    m->epi_bytes = dv.epi_bytes;
+    m->chw_bytes = dv.chw_bytes;
+    m->has_chw = dv.has_chw;
+    m->has_deep = dv.has_deep;
+    m->timeout_s = timeout_s;
+    m->device = dev;
+    m->cus = cus;
+    m->deep_grid = dv.has_deep ? cus * (163840 / dv.deep_lds) : 0;
+    for (int part = PART_MAIN; part < PARTS; ++part) {
+        const std::string co = stem + kPartFile[part] + ".hsaco";
+        if (part == PART_MAIN || (dv.has_chw && file_exists(co))) m->part[part].path = co;
+    }
+    return m;
 }
 
 // Adds the K slices of a split-K launch: C[b,m,n] = sum_z ws[z,b,m,n], converted to the output type.  One lane per
@@ -752,21 +773,30 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restri
     }
 }
 
-// fill_args for the kernel that the launch takes; *mod becomes its module
-int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, const void* B, void* C, LaunchPlan* plan, bool chw = false) {
+// fill_args for the kernel that the launch takes; *mod becomes its module.  `load`: the kernel is about to be launched.  A tile whose
+// kernel the cache does not hold, that cannot be loaded or that does not take the problem leaves the launch to the instance itself.
+int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, const void* B, void* C, LaunchPlan* plan, int part, bool load) {
     void* ws = p ? p->workspace : nullptr;
     const size_t ws_bytes = p ? p->workspace_bytes : 0;
     int rc = fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);          // (the instance says what is refused)
     if (rc) return rc;
-    const hrn_module* f = fitting(*mod, p, chw, (*mod)->info.lds_bytes + (int)plan->dyn_lds);
-    if (f == *mod) return HRN_OK;
-    if (fill_args(f, p, A, B, C, ws, ws_bytes, plan)) return fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);
-    *mod = f;
-    return HRN_OK;
+    const int i = fitting_tiles(*mod, p, part != PART_MAIN, (*mod)->info.lds_bytes + (int)plan->dyn_lds);
+    const hrn_module* f = i < 0 ? nullptr : (*mod)->fit[i];
+    if (f && !f->part[part].path.empty() && (!load || tile_kernels(f, part))) {
+        const std::string keep = g_err;
+        if (fill_args(f, p, A, B, C, ws, ws_bytes, plan) == HRN_OK) {
+            *mod = f;
+        } else {
+            g_err = keep;
+            rc = fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);
+        }
+    }
+    if (load && part == PART_MAIN) plan->fn = (*mod)->part[part].fn[plan->deep];
+    return rc;
 }
 
 // The plan of a launch that is not made: the operands' addresses decide nothing, and what a launch would have to bring is filled in.
-int launch_plan_only(const hrn_module** mod, const hrn_problem* p, LaunchPlan* plan) {
+int launch_plan_only(const hrn_module** mod, const hrn_problem* p, LaunchPlan* plan, int part = PART_MAIN) {
     void* any = (void*)(uintptr_t)256;
     hrn_problem q = *p;
     const hrn_kernel_desc& d = (*mod)->desc;
@@ -779,7 +809,7 @@ int launch_plan_only(const hrn_module** mod, const hrn_problem* p, LaunchPlan* p
         split_shape(d, &q, &kps, &split);
         q.workspace_bytes = (size_t)splitk_bytes(&q, split);
     }
-    return plan_launch(mod, &q, any, any, any, plan);
+    return plan_launch(mod, &q, any, any, any, plan, part, false);
 }
 
 int run_plan(const hrn_module* mod, const hrn_problem* p, const LaunchPlan& plan, void* workspace, hipStream_t st) {
@@ -834,7 +864,7 @@ int static_scratch(void** out, int* dev_out = nullptr) {
 
 int launch(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* stream) {
     LaunchPlan plan;
-    int rc = plan_launch(&mod, p, A, B, C, &plan);
+    int rc = plan_launch(&mod, p, A, B, C, &plan, PART_MAIN, true);
     if (rc) return rc;
     return run_plan(mod, p, plan, p->workspace, (hipStream_t)stream);
 }
@@ -1619,13 +1649,6 @@ void hrn_module_own_tiles(hrn_module* mod, int on) {
 }
 
 int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
-    return build_module(desc, timeout_s, out);
-}
-
-}  // extern "C"
-
-namespace {
-int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {
     if (!out) return fail(HRN_E_BADPARAM, "null out");
     *out = nullptr;
     std::string path;
@@ -1633,39 +1656,22 @@ int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out
     if (rc) return rc;
     int n = 0;
     if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) return fail(HRN_E_NODEVICE, "no HIP device");
-    hrn_module* m = new hrn_module();
-    m->desc = *desc;
-    m->path = path;
-    memset(&m->info, 0, sizeof m->info);
-    read_info(path.substr(0, path.size() - 6) + ".info", &m->info);
-    m->info.threads = desc->wm * desc->wn * 64;
-    Derived dv;
-    {
-        (void)derive(desc, &dv);        // compile_desc has validated the descriptor
-        m->epi_bytes = dv.epi_bytes;
-        m->chw_bytes = dv.chw_bytes;
-    }
-    m->fits = cut_tiles(*desc, m->fit_desc, &m->first_half, &m->end_half);
-    for (int i = 0; i < kMaxFits; ++i) { m->fit[i].store(nullptr); m->fit_failed[i] = false; }
-    m->own_tiles.store(false);
-    m->has_chw = dv.has_chw;
-    m->has_deep = dv.has_deep;
-    m->timeout_s = timeout_s;
-    rc = load_part(path, PART_MAIN, dv.has_deep, &m->part[PART_MAIN]);
-    const std::string stem = path.substr(0, path.size() - 6);
-    for (int part = PART_CHW; part < PARTS && !rc; ++part) {
-        const std::string co = stem + kPartFile[part] + ".hsaco";
-        if (dv.has_chw && file_exists(co)) rc = load_part(co, part, dv.has_deep, &m->part[part]);
-    }
-    int cus = 0;
-    if (!rc) {
-        hipError_t e = hipGetDevice(&m->device);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->device);
-        if (e != hipSuccess) rc = fail(HRN_E_LOAD, "device query: %s", hipGetErrorString(e));
-    }
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return fail(HRN_E_LOAD, "device query: %s", hipGetErrorString(e));
+    hrn_module* m = module_of(desc, path.substr(0, path.size() - 6), timeout_s, dev, cus);
+    for (int part = PART_MAIN; part < PARTS && !rc; ++part)
+        if (!m->part[part].path.empty()) rc = load_part(m->part[part].path, part, m->has_deep, &m->part[part]);
     if (rc) { hrn_module_free(m); return rc; }
-    m->cus = cus;
-    m->deep_grid = dv.has_deep ? cus * (163840 / dv.deep_lds) : 0;
+    m->fits = cut_tiles(*desc, m->fit_desc, &m->first_half, &m->end_half);
+    if (m->fits) {
+        const uint64_t hash = template_hash(kernel_source(), env_or("HRN_HIPCC_FLAGS", ""));
+        for (int i = 0; i < m->fits; ++i) {
+            const std::string stem = cache_dir() + "/" + desc_key(&m->fit_desc[i], hash);
+            if (file_exists(stem + ".hsaco") && file_exists(stem + ".info")) m->fit[i] = module_of(&m->fit_desc[i], stem, timeout_s, dev, cus);
+        }
+    }
     if (desc->split_k) {
         // hrn_launch_splitk_static finds the library's workspace of this device looked up already
         void* ws = nullptr;
@@ -1674,10 +1680,10 @@ int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out
     }
     m->persist_grid = 0;
     if (desc->persistent) {
-        int per_cu = 0, dev = 0;
+        int per_cu = 0;
         hipDeviceProp_t pr;
         if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->part[PART_MAIN].fn[0], m->info.threads, 0) != hipSuccess ||
-            per_cu < 1 || hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&pr, dev) != hipSuccess) {
+            per_cu < 1 || hipGetDeviceProperties(&pr, dev) != hipSuccess) {
             hrn_module_free(m);
             return fail(HRN_E_LOAD, "occupancy query failed: %s", hipGetErrorString(hipGetLastError()));
         }
@@ -1686,9 +1692,6 @@ int build_module(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out
     *out = m;
     return HRN_OK;
 }
-}  // namespace
-
-extern "C" {
 
 int hrn_module_info(const hrn_module* mod, hrn_kernel_info* out) {
     if (!mod || !out) return fail(HRN_E_BADPARAM, "null argument");
@@ -1698,7 +1701,7 @@ int hrn_module_info(const hrn_module* mod, hrn_kernel_info* out) {
 
 void hrn_module_free(hrn_module* mod) {
     if (!mod) return;
-    for (auto& f : mod->fit) hrn_module_free(f.load());
+    for (hrn_module* f : mod->fit) hrn_module_free(f);
     for (CodeObject& c : mod->part)
         if (c.mod) (void)hipModuleUnload(c.mod);
     delete mod;
@@ -1753,12 +1756,8 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
     hrn_problem q = *p;
     q.workspace = nullptr;
     q.workspace_bytes = 0;
-    const hrn_module* own = mod;
-    int rc = plan_launch(&mod, &q, In, Filter, Out, &plan, true);
-    if (!rc && !mod->has_chw) {
-        mod = own;
-        rc = fill_args(mod, p, In, Filter, Out, nullptr, 0, &plan);
-    }
+    const int part = view->expand ? PART_EXPAND : PART_CHW;
+    int rc = plan_launch(&mod, &q, In, Filter, Out, &plan, part, true);
     if (rc) return rc;
     if (view->out_plane < 1 || p->m % view->out_plane)
         return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
@@ -1774,7 +1773,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
         plan.k.expand_shift = __builtin_ctz((unsigned)view->expand);
     }
     const CodeObject* kernels;
-    rc = chw_kernels(mod, view->expand ? PART_EXPAND : PART_CHW, &kernels);
+    rc = chw_kernels(mod, part, &kernels);
     if (rc) return rc;
     plan.fn = kernels->fn[plan.deep];
     return run_plan(mod, p, plan, nullptr, (hipStream_t)stream);
@@ -1784,7 +1783,7 @@ int hrn_launch_repeat(const hrn_module* mod, const hrn_problem* p, const void* A
                       void* stream) {
     if (count < 1) return fail(HRN_E_BADPARAM, "count %d", count);
     LaunchPlan plan;
-    int rc = plan_launch(&mod, p, A, B, C, &plan);
+    int rc = plan_launch(&mod, p, A, B, C, &plan, PART_MAIN, true);
     if (rc) return rc;
     for (int i = 0; i < count; ++i) {
         rc = run_plan(mod, p, plan, p->workspace, (hipStream_t)stream);
@@ -1810,6 +1809,7 @@ int hrn_launch_splitk_static(const hrn_module* mod, const hrn_problem* p, const 
     LaunchPlan plan;
     rc = fill_args(mod, p, A, B, C, ws, (size_t)HRN_STATIC_WORKSPACE_BYTES, &plan);
     if (rc) return rc;
+    plan.fn = mod->part[PART_MAIN].fn[plan.deep];
     // Every call on a GPU shares that GPU's one workspace.  Calls on one stream are ordered by the stream; a call on
     // another stream is made to wait for the previous user (an event recorded behind each call), so calls from several
     // streams or threads are serialised on the device instead of racing.

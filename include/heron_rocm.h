@@ -209,12 +209,14 @@ int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
 
 /*
  * A launch of at most half as many tiles as the device has CUs takes the instance's tile cut in halves (same MFMA shape, same order
- * along K: same result bit for bit), and a tile of one to three waves takes more of them on grids of at most six tiles a CU; persistent and split-K
- * instances keep theirs.  Such a tile is an instance of its own, compiled and loaded at the first launch that takes it unless
- * the cache holds it.  hrn_tiles lists those of an instance (returns how many, at most `cap` are written), hrn_compile_tiles
+ * along K: same result bit for bit), a tile of one to three waves takes more of them on grids of at most six tiles a CU, and a conv window
+ * tile that has a CU to itself takes half the rows; persistent and split-K instances keep theirs.  Such a tile is an instance of its own.
+ * hrn_build looks which of them the cache holds; only those are taken, each loaded (never compiled) at the first launch that does, and
+ * a launch whose kernel the cache lacks or that cannot be loaded is the instance's own.  hrn_tiles lists those of an instance (returns
+ * how many, at most `cap` are written), for hrn_compile and hrn_compile_chw; hrn_compile_tiles
  * compiles them ahead (part 0: the kernels of plain launches, 1 and 2: those of hrn_launch_conv2d_chw without and with
- * expand), hrn_launch_tile says which a row-major launch takes, and hrn_module_own_tiles(mod, 1) keeps a module to its own, as a search
- * over tiles needs.
+ * expand), hrn_launch_tile says which a row-major launch takes without loading it, and hrn_module_own_tiles(mod, 1) keeps a module to its own,
+ * as a search over tiles needs.
  */
 int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap);
 int hrn_compile_tiles(const hrn_kernel_desc* desc, int part, double timeout_s);

@@ -14,7 +14,7 @@ def pytest_configure(config):
 
 # files that test the kernels of the very instances they name, on problems small enough for another tile of them
 OWN_TILES = {"test_gpu_parity", "test_gpu_phased", "test_gpu_deep", "test_gpu_fuzz", "test_gpu_channels_first", "test_gpu_colsum",
-             "test_gpu_direct_epilogue", "test_gpu_splitk_fold", "test_gpu_hostpath"}
+             "test_gpu_direct_epilogue", "test_gpu_splitk_fold"}
 
 
 @pytest.fixture(autouse=True)

@@ -2,9 +2,9 @@
 tile: equal bit for bit over grids on both sides of the rule, ragged M, N and K, batches, im2col and window convs, channels first
 and expanded input; what an instance refuses, it refuses whatever tile the launch would take; capture with tiles that are
 not loaded yet."""
-import ctypes
+import os
+import shutil
 
-import numpy as np
 import pytest
 import torch
 
@@ -34,6 +34,14 @@ def _operands(f16, a, b, seed):
         return torch.randn(a, device="cuda", generator=gen).half(), torch.randn(b, device="cuda", generator=gen).half()
     return (torch.randint(0, 256, a, device="cuda", generator=gen, dtype=torch.uint8),
             torch.randint(-128, 128, b, device="cuda", generator=gen, dtype=torch.int8))
+
+
+def _declared(op, args, f16):
+    """(info, inputs) of an operator"""
+    ctx = type("Ctx", (), dict(set_info=lambda self, i: setattr(self, "info", i), set_axis_map=lambda self, m: None))()
+    getOpFromName(op)(ctx, *args, *(["float16"] * 2 if f16 else ["int8"] * 2))
+    ref = ctx.info["reference_args"]
+    return ctx.info, list(_operands(f16, ref["input"], ref["filter"], len(args)))
 
 
 def _cut(mod, p):
@@ -95,12 +103,10 @@ def test_channels_first(name, hrn):
     mod, own, f16 = B.Module(d), B.Module(d, own_tiles=True), d.dtype == F16
     for op, args in [("c2d_nchw", [3, 13, 11, 64, 72, 3, 3, 1, 1, 1]), ("c1d", [2, 301, 64, 64, 3, 1, 1, 1]), ("t2d", [2, 9, 7, 64, 96, 1, 1, 2, 0, 1, 0]),
                      ("t2d", [16, 56, 56, 64, 128, 1, 1, 2, 0, 1, 0]), ("t2d", [2, 9, 7, 128, 40, 3, 3, 2, 1, 1, 1])]:
-        ctx = type("Ctx", (), dict(set_info=lambda self, i: setattr(self, "info", i), set_axis_map=lambda self, m: None))()
-        getOpFromName(op)(ctx, *args, *(["float16"] * 2 if f16 else ["int8"] * 2))
-        info, c = ctx.info, ctx.info["conv"]
+        info, inputs = _declared(op, args, f16)
+        c = info["conv"]
         if d.conv_window and (2 * c["pad"] != c["KH"] - 1 or 2 * c["pad_w"] != c["KW"] - 1):
             continue
-        inputs = list(_operands(f16, info["reference_args"]["input"], info["reference_args"]["filter"], len(args)))
         print("tiles channels first", name, op, args, flush=True)
         assert torch.equal(hostops.run_operator(mod, info, inputs), hostops.run_operator(own, info, inputs))
     mod.close()
@@ -134,5 +140,85 @@ def test_first_launch_under_capture(hrn):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, hostops.gemm(own, A, W, bsum=bsum))
+    mod.close()
+    own.close()
+
+
+def _copy_parts(tmp, *parts):
+    """A cache that holds these (descriptor, kernels) and nothing else; kernels: "main", "chw" or "expand"."""
+    for d, part in parts:
+        stem = B.compile_desc(d)[:-len(".hsaco")]
+        for end in (".hsaco", ".info") if part == "main" else ("_%s.hsaco" % part,):
+            shutil.copy(stem + end, tmp)
+
+
+@pytest.fixture
+def no_compiler(tmp_path, monkeypatch):
+    """An empty cache, and a compiler that only leaves a mark."""
+    cache, script, mark = tmp_path / "cache", tmp_path / "hipcc", tmp_path / "called"
+    cache.mkdir()
+    script.write_text("#!/bin/sh\ntouch %s\nexit 1\n" % mark)
+    script.chmod(0o755)
+
+    def use():
+        monkeypatch.setenv("HRN_CACHE_DIR", str(cache))
+        monkeypatch.setenv("HRN_HIPCC", str(script))
+    return cache, use, mark
+
+
+def test_a_launch_compiles_no_tile(no_compiler, hrn):
+    """An instance whose tiles are not in the cache launches its own, and neither the launch nor the questions about it compile."""
+    cache, use, mark = no_compiler
+    d = GEMMS["u8-128"]
+    _copy_parts(cache, (d, "main"))
+    A, W = _operands(False, (300, 528), (260, 528), 3)
+    bsum, p = hostops.column_sums(W), B.gemm_problem(1, 300, 260, 528)
+    own = B.Module(d, own_tiles=True)
+    want = hostops.gemm(own, A, W, bsum=bsum)
+    use()
+    mod = B.Module(d)
+    assert not _cut(mod, p) and mod.is_deep(p) == own.is_deep(p)
+    assert torch.equal(hostops.gemm(mod, A, W, bsum=bsum), want)
+    assert not mark.exists()
+    mod.close()
+    own.close()
+
+
+def test_channels_first_without_the_tiles_kernels(no_compiler, hrn):
+    """A channels-first launch whose tile lies in the cache without channels-first kernels takes the instance's own."""
+    cache, use, mark = no_compiler
+    d = CONVS["f16-128"]
+    info, inputs = _declared("c2d_nchw", [2, 5, 6, 64, 8, 3, 3, 1, 1, 1], True)
+    own = B.Module(d, own_tiles=True)
+    want = hostops.run_operator(own, info, inputs)
+    _copy_parts(cache, (d, "main"), (d, "chw"), *((t, "main") for t in B.tiles(d)))
+    use()
+    mod = B.Module(d)
+    assert torch.equal(hostops.run_operator(mod, info, inputs), want)
+    assert not mark.exists()
+    mod.close()
+    own.close()
+
+
+def test_a_tile_that_cannot_be_loaded(no_compiler, hrn):
+    """A code object without the kernel it should hold leaves the launch to the instance, and no error behind."""
+    cache, use, mark = no_compiler
+    d = CONVS["f16-128"]
+    p = B.conv2d_problem(2, 5, 6, 64, 8, 3, 3, 1, 1, 1)
+    X, F = _operands(True, (2, 5, 6, 64), (8, 3, 3, 64), 1)
+    own = B.Module(d, own_tiles=True)
+    want = hostops.conv2d_nhwc(own, X, F, 1, 1, 1)
+    _copy_parts(cache, (d, "main"), *((t, "main") for t in B.tiles(d)))
+    for t in B.tiles(d):
+        stem = os.path.basename(B.compile_desc(t))[:-len(".hsaco")]
+        shutil.copy(B.compile_desc(d)[:-len(".hsaco")] + "_chw.hsaco", cache / (stem + ".hsaco"))
+    use()
+    mod = B.Module(d)
+    assert _cut(mod, p)
+    for _ in range(2):
+        assert torch.equal(hostops.conv2d_nhwc(mod, X, F, 1, 1, 1), want)
+    assert "hipModule" not in B.lib().hrn_last_error().decode()
+    torch.zeros(4, device="cuda").add_(1)
+    torch.cuda.synchronize()
     mod.close()
     own.close()
