@@ -396,7 +396,7 @@ def probe_copy(src_ptr, dst_ptr, nbytes, repeat=10, stream=0):
 
 class Module:
     """One loaded template instance (``hrn_module``).  Launches whose grid leaves half of the device idle, tiles of one to three
-    waves on grids of at most six tiles a CU and conv windows that fill a CU's LDS take another tile of the same instance
+    waves on grids of at most six tiles a CU and conv windows that fill a CU's LDS where two halves would fit take another tile of the same instance
     (``launch_tile``, same bits) where the cache holds it, unless ``own_tiles`` is set."""
 
     def __init__(self, desc, timeout_s=0.0, own_tiles=False):

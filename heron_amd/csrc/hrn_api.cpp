@@ -555,11 +555,15 @@ bool with_waves(hrn_kernel_desc d, hrn_kernel_desc* out) {
 }
 
 // Of an input window's tile whose workgroup has a CU to itself (more than half of the LDS), the phases - window in, filter taps,
-// result out - take turns: half the rows leave room for a second workgroup, whose phases fill the gaps.  Row-major results with as many
-// waves as before, channels-first ones with half (their strips are as long as a wave has rows) and two stages (a third workgroup).
-//   fp16 512x64 -> 256x64, 3x3: 64x56x56x64 -> 128 52.5 -> 41.1 us, 128x56x56x64 -> 64 52.0 -> 42.2, 32x56x56x64 -> 64 15.5 -> 14.5; 1x1
-// 16x111x111x64 -> 128 22.3 -> 18.7; transposed conv 16x56x56x64 -> 128, stride 2, channels first 35.7 -> 31.0 (25.5 with stores that
-// allocate, see the template).
+// result out - take turns: where two workgroups of half the rows fit a CU, the phases of one fill the gaps of the other.  Where
+// only one does, or the columns are halved, each window is loaded for half the results and nothing fills the gaps.
+// Row-major results with as many waves as before, channels-first ones with half (their strips are as long as a wave has rows) and two
+// stages (a third workgroup).
+//   fp16 512x64 -> 256x64, two fit: 3x3 64x56x56x64 -> 64 26.8 -> 24.8 us, 128x56x56x64 52.5 -> 43.0, 32x60x60x64 15.0 -> 14.2, 5x5 128x31x31x64
+// 30.4 -> 30.0; 1x1 16x111x111x64 -> 128 22.3 -> 18.7; transposed conv 16x56x56x64 -> 128, stride 2, channels first 35.7 -> 31.0 (25.5
+// with stores that allocate, see the template).  One fits, kept whole: 3x3 64x64x64x64 29.6 (34.3 halved), 16x112x112x64 27.3 (33.4), 5x5
+// 16x80x80x64 27.9 (33.9), 1x1 32x56x56x128 8.5 (10.2); 5x5 64x48x48x64, a round of 256 tiles and one of 32, 53.5 (48.8).  64x128 ->
+// 64x64: 1x1 16x28x28x512 -> 128 6.9 (15.1).
 constexpr int kOnePerCu = 163840 / 2;
 
 // fit_desc[0]: the own tile with more waves, if it has few; then the halves, [*first_half, *end_half); behind them the half of
@@ -594,14 +598,27 @@ int64_t tiles_of(const hrn_kernel_desc& d, const hrn_problem* p) {
     return (((int64_t)p->m + d.bm - 1) / d.bm) * (((int64_t)p->n + d.bn - 1) / d.bn) * p->batch;
 }
 
-// which of the instance's tiles a launch takes: -1 its own (`lds`: what a workgroup of that needs)
-int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw, int lds) {
+// LDS bytes of a workgroup of a conv_window instance: the stages and, one behind the other in the rest, the window and the epilogue
+// region (column sums, strips)
+int64_t window_lds(const hrn_module* m, const hrn_problem* p, bool chw) {
+    const int es = m->desc.dtype == HRN_DT_F16 ? 2 : 1;
+    const int64_t rows = m->desc.bm + 2 * ((int64_t)p->cpad * p->cw + p->cpad_w);
+    const int64_t window = (rows * (p->ci * es / 16) + 63) / 64 * 1024;
+    return m->info.lds_bytes + std::max<int64_t>(window, chw ? std::max(m->chw_bytes, m->epi_bytes) : m->epi_bytes);
+}
+
+// which of the instance's tiles a launch that fill_args takes may take: -1 its own
+int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw) {
     if (!p || p->m < 1 || p->n < 1 || p->batch < 1 || m->fits == 0 || m->own_tiles.load(std::memory_order_relaxed)) return -1;
     const int halves = m->first_half;
     int pick = -1;
     const hrn_kernel_desc* d = &m->desc;
     for (int i = halves; i < m->end_half && tiles_of(*d, p) * 2 <= m->cus; ++i) { pick = i; d = &m->fit_desc[i]; }
-    if (pick < 0 && m->desc.conv_window && lds > kOnePerCu) pick = chw ? (m->fits > m->end_half ? m->end_half : -1) : (halves < m->end_half ? halves : -1);
+    if (pick < 0 && m->desc.conv_window && window_lds(m, p, chw) > kOnePerCu) {
+        const int half = chw ? m->end_half : halves;
+        const bool rows = half < (chw ? m->fits : m->end_half) && m->fit_desc[half].bn == m->desc.bn;
+        if (rows && m->fit[half] && window_lds(m->fit[half], p, chw) <= kOnePerCu) pick = half;
+    }
     const int64_t row_bytes = (int64_t)p->k * (m->desc.dtype == HRN_DT_F16 ? 2 : 1), tiles = tiles_of(m->desc, p);
     if (pick < 0 && halves == 1 && tiles <= 6 * (int64_t)m->cus && (tiles <= m->cus ? row_bytes > 2 * m->desc.bkb : !chw)) pick = 0;
     return pick;
@@ -661,10 +678,8 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
                 return fail(HRN_E_BADPARAM, "conv_window needs stride 1, dilation 1 and 'same' padding");
             if ((p->ci * es) % d.bkb) return fail(HRN_E_BADPARAM, "conv_window needs CI*%d to be a multiple of bkb %d", es, d.bkb);
             if (p->kh * p->kw > 32) return fail(HRN_E_BADPARAM, "conv_window supports at most 32 filter taps");
-            const int64_t rows = d.bm + 2 * ((int64_t)p->cpad * p->cw + p->cpad_w);
-            const int64_t instr = (rows * (p->ci * es / 16) + 63) / 64;
-            // dynamic LDS: the window, reused by the epilogue region (column sums, strips) once the last tap is read
-            const int64_t dyn = std::max<int64_t>(instr * 1024, mod->epi_bytes);
+            // dynamic LDS: the window, reused by the epilogue region once the last tap is read
+            const int64_t dyn = window_lds(mod, p, false) - mod->info.lds_bytes;
             if (dyn + mod->info.lds_bytes > 163840)
                 return fail(HRN_E_BADPARAM, "conv_window: window of %lld bytes + %d static LDS exceeds 163840", (long long)dyn, mod->info.lds_bytes);
             plan->dyn_lds = (unsigned)dyn;
@@ -780,7 +795,7 @@ int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, con
     const size_t ws_bytes = p ? p->workspace_bytes : 0;
     int rc = fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);          // (the instance says what is refused)
     if (rc) return rc;
-    const int i = fitting_tiles(*mod, p, part != PART_MAIN, (*mod)->info.lds_bytes + (int)plan->dyn_lds);
+    const int i = fitting_tiles(*mod, p, part != PART_MAIN);
     const hrn_module* f = i < 0 ? nullptr : (*mod)->fit[i];
     if (f && !f->part[part].path.empty() && (!load || tile_kernels(f, part))) {
         const std::string keep = g_err;

@@ -210,7 +210,7 @@ int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
 /*
  * A launch of at most half as many tiles as the device has CUs takes the instance's tile cut in halves (same MFMA shape, same order
  * along K: same result bit for bit), a tile of one to three waves takes more of them on grids of at most six tiles a CU, and a conv window
- * tile that has a CU to itself takes half the rows; persistent and split-K instances keep theirs.  Such a tile is an instance of its own.
+ * tile that has a CU to itself takes half the rows where two of those fit; persistent and split-K instances keep theirs.  Such a tile is an instance of its own.
  * hrn_build looks which of them the cache holds; only those are taken, each loaded (never compiled) at the first launch that does, and
  * a launch whose kernel the cache lacks or that cannot be loaded is the instance's own.  hrn_tiles lists those of an instance (returns
  * how many, at most `cap` are written), for hrn_compile and hrn_compile_chw; hrn_compile_tiles

@@ -222,3 +222,37 @@ def test_a_tile_that_cannot_be_loaded(no_compiler, hrn):
     torch.cuda.synchronize()
     mod.close()
     own.close()
+
+
+# a window tile that has a CU to itself, on more tiles than half the CUs: (image width, channels, filter, whether two of the half fit a
+# CU).  The 512x64 record's half: 32 KiB of stages, and 256 + 2 pad (width + 1) rows of 2 ci bytes in 48 KiB at width 63 (3x3) and 31 (5x5).
+@pytest.mark.parametrize("w,ci,k,two", [(56, 64, 3, True), (60, 64, 3, True), (63, 64, 3, True), (64, 64, 3, False), (160, 64, 3, False),
+                                        (31, 64, 5, True), (32, 64, 5, False), (80, 64, 5, False), (111, 64, 1, True), (57, 128, 1, False)])
+def test_half_a_window_where_two_fit(w, ci, k, two, hrn):
+    d = CONVS["f16-window"]
+    mod, own = B.Module(d), B.Module(d, own_tiles=True)
+    n = -(-200 * d.bm // (w * w))
+    p = B.conv2d_problem(n, w, w, ci, 64, k, k, 1, k // 2, 1)
+    t = mod.launch_tile(p)
+    half = d.bm // 2 + 2 * (k // 2) * (w + 1)
+    lds = t.stages * t.bn * t.bkb + -(-half * ci * 2 // 1024) * 1024
+    assert two == (lds <= 80 * 1024)
+    assert (t.bm, t.bn) == ((d.bm // 2 if two else d.bm), d.bn)
+    X, F = _operands(True, (n, w, w, ci), (64, k, k, ci), w)
+    print("half a window", w, ci, k, t.as_tuple(), flush=True)
+    assert torch.equal(hostops.conv2d_nhwc(mod, X, F, 1, k // 2, 1), hostops.conv2d_nhwc(own, X, F, 1, k // 2, 1))
+    mod.close()
+    own.close()
+
+
+def test_half_a_window_in_rows_only(hrn, tmp_path, monkeypatch):
+    """A window tile wider than high is halved in columns where the grid leaves CUs idle, and never to share a CU."""
+    monkeypatch.setenv("HRN_CACHE_DIR", str(tmp_path))
+    d = D(F16, CONV, 64, 128, 256, 2, 4, 32, 2, 1, epi=1, win=1)
+    for t in [d, B.tiles(d)[0]]:
+        B.compile_desc(t)
+    mod = B.Module(d)
+    for n, tile in ((8, (64, 64)), (16, (64, 128))):                      # 98 and 196 tiles; 96 KiB of LDS, 64 KiB with half the columns
+        t = mod.launch_tile(B.conv2d_problem(n, 28, 28, 256, 128, 1, 1, 1, 0, 1))
+        assert (t.bm, t.bn) == tile
+    mod.close()
