@@ -110,7 +110,7 @@ def settle(torch, mod, prob, a, b, c, stream, min_ms=200.0, max_ms=4000.0):
 def measure(torch, B, w, steps, warmup, keep_rows=0, cold=False):
     """One workload: returns dict(wall_s, kernel_s, settle_ms, info[, cold_s][, rows])."""
     inst = w["inst"]
-    mod = B.Module(inst.desc, own_tiles=True)          # (the row is about the record it names)
+    mod = B.Module(inst.desc)
     a, b, c, prob = w["build"]()
     mod.bind_workspace(prob)
     stream = torch.cuda.current_stream().cuda_stream

@@ -72,6 +72,8 @@ class KernelDesc(ctypes.Structure):
     KEYS = ("dtype", "op", "bm", "bn", "bkb", "wm", "wn", "mfma", "stages", "swizzle", "epilogue", "waves_per_eu",
             "conv_window", "persistent", "split_k", "sched", "load_spread", "colsum", "nt_store")
 
+    tuned_for = None                # the Problem it was searched for, where it is the instance of a record
+
     def as_tuple(self):
         return tuple(int(getattr(self, k)) for k in self.KEYS)
 
@@ -175,6 +177,7 @@ SYMBOLS = {
     "hrn_compile_tiles": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
     "hrn_launch_tile": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(KernelDesc)]),
     "hrn_module_own_tiles": (None, [_vp, _i]),
+    "hrn_module_tuned_for": (None, [_vp, ctypes.POINTER(Problem)]),
     "hrn_launch_conv2d_chw": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(ConvView), _vp, _vp, _vp, _vp]),
     "hrn_launch_is_deep": (_i, [_vp, ctypes.POINTER(Problem)]),
     "hrn_launch_splitk_static": (_i, [_vp, ctypes.POINTER(Problem), _vp, _vp, _vp, _vp]),
@@ -396,8 +399,9 @@ def probe_copy(src_ptr, dst_ptr, nbytes, repeat=10, stream=0):
 
 class Module:
     """One loaded template instance (``hrn_module``).  Launches whose grid leaves half of the device idle, tiles of one to three
-    waves on grids of at most six tiles a CU and conv windows that fill a CU's LDS where two halves would fit take another tile of the same instance
-    (``launch_tile``, same bits) where the cache holds it, unless ``own_tiles`` is set."""
+    waves on grids of at most six tiles a CU and conv windows that fill a CU's LDS where two halves would fit take another tile
+    of the same instance (``launch_tile``, same bits) where the cache holds it, except on the problem the instance was searched for
+    (``desc.tuned_for``) and where ``own_tiles`` is set."""
 
     def __init__(self, desc, timeout_s=0.0, own_tiles=False):
         self.desc = desc
@@ -406,6 +410,8 @@ class Module:
         self._h = h
         if own_tiles:
             lib().hrn_module_own_tiles(h, 1)
+        if desc.tuned_for is not None:
+            lib().hrn_module_tuned_for(h, ctypes.byref(desc.tuned_for))
         self.native = (h.value, ctypes.addressof(desc))      # what the functions of ext() take for this instance
         self.has_chw = bool(lib().hrn_module_has_chw(h))     # launch_conv2d_chw takes it
         info = KernelInfo()

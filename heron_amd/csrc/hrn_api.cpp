@@ -77,6 +77,8 @@ struct hrn_module {
     hrn_kernel_desc fit_desc[kMaxFits];
     hrn_module* fit[kMaxFits];
     std::atomic<bool> own_tiles;    // launches keep to the instance's own tile
+    bool tuned;                     // and those of the problem it was searched for (sizes of tuned_for) do in any case
+    hrn_problem tuned_for;
     hrn_kernel_info info;
     mutable CodeObject part[PARTS]; // those of hrn_launch_conv2d_chw are there from hrn_build on or from their first launch
     mutable std::mutex part_mutex;
@@ -607,9 +609,20 @@ int64_t window_lds(const hrn_module* m, const hrn_problem* p, bool chw) {
     return m->info.lds_bytes + std::max<int64_t>(window, chw ? std::max(m->chw_bytes, m->epi_bytes) : m->epi_bytes);
 }
 
-// which of the instance's tiles a launch that fill_args takes may take: -1 its own
+bool same_sizes(const hrn_problem& a, const hrn_problem& b) {
+    if (a.op != b.op || a.batch != b.batch || a.m != b.m || a.n != b.n || a.k != b.k) return false;
+    return a.op != HRN_OP_CONV2D || (a.cn == b.cn && a.ch == b.ch && a.cw == b.cw && a.ci == b.ci && a.co == b.co && a.kh == b.kh && a.kw == b.kw &&
+                                     a.cstride == b.cstride && a.cpad == b.cpad && a.cdil == b.cdil && a.cstride_w == b.cstride_w &&
+                                     a.cpad_w == b.cpad_w && a.cdil_w == b.cdil_w);
+}
+
+// which of the instance's tiles a launch that fill_args takes may take: -1 its own.  On the problem an instance was searched for its tile
+// is the one that was timed against others.  Six records would be changed by the rules below (fp16 convs, own tile / the other, us):
+// ResNet-50 28x28x128 9.1 / 9.4, 14x14x256 11.3 / 11.6, InceptionV3 35x35x192 4.7 / 4.9, 17x17x768 6.9 / 6.6, 8x8x1280 8.0 / 8.0, and
+// 32x56x56x64 14.1 / 13.7.
 int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw) {
     if (!p || p->m < 1 || p->n < 1 || p->batch < 1 || m->fits == 0 || m->own_tiles.load(std::memory_order_relaxed)) return -1;
+    if (m->tuned && same_sizes(*p, m->tuned_for)) return -1;
     const int halves = m->first_half;
     int pick = -1;
     const hrn_kernel_desc* d = &m->desc;
@@ -1661,6 +1674,12 @@ int hrn_launch_tile(const hrn_module* mod, const hrn_problem* p, hrn_kernel_desc
 
 void hrn_module_own_tiles(hrn_module* mod, int on) {
     if (mod) mod->own_tiles.store(on != 0, std::memory_order_relaxed);
+}
+
+void hrn_module_tuned_for(hrn_module* mod, const hrn_problem* p) {
+    if (!mod) return;
+    mod->tuned = p != nullptr;
+    if (p) mod->tuned_for = *p;
 }
 
 int hrn_build(const hrn_kernel_desc* desc, double timeout_s, hrn_module** out) {

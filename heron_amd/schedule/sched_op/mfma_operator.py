@@ -29,10 +29,12 @@ class TemplateSchedule:
         p = self.params
         dtype = B.HRN_DT_F16 if self.info['kind'] == 'f16' else B.HRN_DT_U8S8
         op = B.HRN_OP_CONV2D if self.info['operator'] == 'conv2d_nhwc' else B.HRN_OP_GEMM
-        return B.make_desc(dtype, op, p['bm'], p['bn'], p['bkb'], p['wm'], p['wn'], p['mfma'], p['stages'],
+        desc = B.make_desc(dtype, op, p['bm'], p['bn'], p['bkb'], p['wm'], p['wn'], p['mfma'], p['stages'],
                            p['swizzle'], p.get('epilogue', 0), p['waves_per_eu'],
                            p.get('conv_window', 0), p.get('persistent', 0), 1 if p.get('split_k', 1) > 1 else 0,
                            p.get('sched', 1), p.get('load_spread', 2), p.get('colsum', 0), p.get('nt_store', 0))
+        desc.tuned_for = self.to_problem()
+        return desc
 
     def to_problem(self):
         from ... import backend as B

@@ -256,3 +256,33 @@ def test_half_a_window_in_rows_only(hrn, tmp_path, monkeypatch):
         t = mod.launch_tile(B.conv2d_problem(n, 28, 28, 256, 128, 1, 1, 1, 0, 1))
         assert (t.bm, t.bn) == tile
     mod.close()
+
+
+@pytest.mark.parametrize("name", sorted(tuned.CASES))
+def test_a_record_runs_its_own_tile_on_its_own_problem(name, hrn):
+    t = tuned.load(name)
+    _, op, shape, dtype = tuned.CASES[name]
+    sched, _ = tuned.instantiate(name, op, shape, dtype, t.records)
+    mod = B.Module(t.desc)
+    assert not _cut(mod, sched.to_problem())
+    mod.close()
+
+
+def test_a_record_of_few_tiles(hrn):
+    """On its own sizes, in any raster order, it keeps its tile; elsewhere the rule decides."""
+    d = D(F16, GEMM, 256, 256, 128, 2, 4, 16, 2, 2)
+    d.tuned_for = B.gemm_problem(1, 700, 520, 256)
+    mod = B.Module(d)
+    assert not _cut(mod, B.gemm_problem(1, 700, 520, 256, group_m=2))
+    for other in (B.gemm_problem(1, 700, 520, 264), B.gemm_problem(1, 701, 520, 256), B.gemm_problem(1, 700, 528, 256), B.gemm_problem(2, 700, 520, 256)):
+        assert _cut(mod, other)
+    mod.close()
+    d = CONVS["f16-128"]
+    args = [2, 14, 14, 64, 48, 3, 3, 1, 1, 1]
+    d.tuned_for = B.conv2d_problem(*args)
+    mod = B.Module(d)
+    assert not _cut(mod, B.conv2d_problem(*args))
+    for i, v in [(0, 3), (4, 64), (5, 5), (6, 1), (7, (1, 2)), (8, 2), (9, 2)]:
+        assert _cut(mod, B.conv2d_problem(*args[:i], v, *args[i + 1:])), (i, v)
+    assert _cut(mod, B.conv2d_problem(1, 28, 14, *args[3:]))             # as many pixels in another image
+    mod.close()
