@@ -176,6 +176,7 @@ SYMBOLS = {
     "hrn_tiles": (_i, [ctypes.POINTER(KernelDesc), ctypes.POINTER(KernelDesc), _i]),
     "hrn_compile_tiles": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
     "hrn_launch_tile": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(KernelDesc)]),
+    "hrn_launch_chw_tile": (_i, [_vp, ctypes.POINTER(Problem), _i, ctypes.POINTER(KernelDesc)]),
     "hrn_module_own_tiles": (None, [_vp, _i]),
     "hrn_module_tuned_for": (None, [_vp, ctypes.POINTER(Problem)]),
     "hrn_launch_conv2d_chw": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(ConvView), _vp, _vp, _vp, _vp]),
@@ -463,10 +464,14 @@ class Module:
         self.bind_colsum(problem, b_ptr, stream)
         _check(self._launcher(problem)(self._h, ctypes.byref(problem), a_ptr, b_ptr, c_ptr, stream))
 
-    def launch_tile(self, problem):
-        """The descriptor of the instance whose kernel a launch of ``problem`` takes."""
+    def launch_tile(self, problem, chw=False, expand=False):
+        """The descriptor of the instance whose kernel a launch of ``problem`` takes (``chw``: one of ``launch_conv2d_chw``, of a
+        zero-expanded input with ``expand``)."""
         out = KernelDesc()
-        _check(lib().hrn_launch_tile(self._h, ctypes.byref(problem), ctypes.byref(out)))
+        if chw:
+            _check(lib().hrn_launch_chw_tile(self._h, ctypes.byref(problem), 1 if expand else 0, ctypes.byref(out)))
+        else:
+            _check(lib().hrn_launch_tile(self._h, ctypes.byref(problem), ctypes.byref(out)))
         return out
 
     def is_deep(self, problem):

@@ -445,13 +445,15 @@ int chw_kernels(const hrn_module* m, int part, const CodeObject** out) {
     return rc ? rc : load_late(m, path, part);
 }
 
-// The same of a tile of an instance (hrn_module.fit), which no launch compiles; false: the launch is the instance's own.
-bool tile_kernels(const hrn_module* f, int part) {
+// The same of a tile of an instance (hrn_module.fit), which no launch compiles; false: the launch is the instance's own.  Without
+// `load` the answer for a launch to come.
+bool tile_kernels(const hrn_module* f, int part, bool load) {
     CodeObject& c = f->part[part];
+    if (c.path.empty()) return false;
     if (c.ready.load(std::memory_order_acquire)) return true;
     std::lock_guard<std::mutex> lock(f->part_mutex);
     if (c.ready.load(std::memory_order_acquire)) return true;
-    if (c.failed) return false;
+    if (c.failed || !load) return !c.failed;
     const std::string keep = g_err;
     c.failed = load_late(f, c.path, part) != HRN_OK;
     if (c.failed) {
@@ -810,7 +812,7 @@ int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, con
     if (rc) return rc;
     const int i = fitting_tiles(*mod, p, part != PART_MAIN);
     const hrn_module* f = i < 0 ? nullptr : (*mod)->fit[i];
-    if (f && !f->part[part].path.empty() && (!load || tile_kernels(f, part))) {
+    if (f && tile_kernels(f, part, load)) {
         const std::string keep = g_err;
         if (fill_args(f, p, A, B, C, ws, ws_bytes, plan) == HRN_OK) {
             *mod = f;
@@ -1667,6 +1669,16 @@ int hrn_launch_tile(const hrn_module* mod, const hrn_problem* p, hrn_kernel_desc
     if (!mod || !p || !out) return fail(HRN_E_BADPARAM, "null argument");
     LaunchPlan plan;
     int rc = launch_plan_only(&mod, p, &plan);
+    if (rc) return rc;
+    *out = mod->desc;
+    return HRN_OK;
+}
+
+int hrn_launch_chw_tile(const hrn_module* mod, const hrn_problem* p, int expand, hrn_kernel_desc* out) {
+    if (!mod || !p || !out) return fail(HRN_E_BADPARAM, "null argument");
+    if (!mod->has_chw) return fail(HRN_E_BADPARAM, "the instance has no channels-first kernels");
+    LaunchPlan plan;
+    int rc = launch_plan_only(&mod, p, &plan, expand ? PART_EXPAND : PART_CHW);
     if (rc) return rc;
     *out = mod->desc;
     return HRN_OK;

@@ -215,13 +215,14 @@ int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
  * a launch whose kernel the cache lacks or that cannot be loaded is the instance's own.  hrn_tiles lists those of an instance (returns
  * how many, at most `cap` are written), for hrn_compile and hrn_compile_chw; hrn_compile_tiles
  * compiles them ahead (part 0: the kernels of plain launches, 1 and 2: those of hrn_launch_conv2d_chw without and with
- * expand), hrn_launch_tile says which a row-major launch takes without loading it, and hrn_module_own_tiles(mod, 1) keeps a module to its own,
+ * expand), hrn_launch_tile and hrn_launch_chw_tile say which a row-major launch and one of hrn_launch_conv2d_chw take, without loading it, and hrn_module_own_tiles(mod, 1) keeps a module to its own,
  * as a search over tiles needs.  hrn_module_tuned_for names the problem an instance was searched for, before the module's first launch: on
  * its sizes (strides, slices and raster order count for nothing) the launches keep the tile that was found (null: no such problem).
  */
 int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap);
 int hrn_compile_tiles(const hrn_kernel_desc* desc, int part, double timeout_s);
 int hrn_launch_tile(const hrn_module* mod, const hrn_problem* p, hrn_kernel_desc* out);
+int hrn_launch_chw_tile(const hrn_module* mod, const hrn_problem* p, int expand, hrn_kernel_desc* out);
 void hrn_module_own_tiles(hrn_module* mod, int on);
 void hrn_module_tuned_for(hrn_module* mod, const hrn_problem* p);
 

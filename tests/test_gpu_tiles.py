@@ -44,8 +44,14 @@ def _declared(op, args, f16):
     return ctx.info, list(_operands(f16, ref["input"], ref["filter"], len(args)))
 
 
-def _cut(mod, p):
-    return mod.launch_tile(p).as_tuple() != mod.desc.as_tuple()
+def _cut(mod, p, **how):
+    return mod.launch_tile(p, **how).as_tuple() != mod.desc.as_tuple()
+
+
+def _conv_problem(info):
+    c = info["conv"]
+    return B.conv2d_problem(*(c[n] for n in ("N", "H", "W", "CI", "CO", "KH", "KW")), (c["stride"], c["stride_w"]), (c["pad"], c["pad_w"]),
+                            (c["dil"], c["dil_w"]))
 
 
 @pytest.mark.parametrize("name", sorted(GEMMS))
@@ -101,14 +107,21 @@ def test_conv(name, hrn):
 def test_channels_first(name, hrn):
     d = CONVS[name]
     mod, own, f16 = B.Module(d), B.Module(d, own_tiles=True), d.dtype == F16
+    cut = 0
     for op, args in [("c2d_nchw", [3, 13, 11, 64, 72, 3, 3, 1, 1, 1]), ("c1d", [2, 301, 64, 64, 3, 1, 1, 1]), ("t2d", [2, 9, 7, 64, 96, 1, 1, 2, 0, 1, 0]),
                      ("t2d", [16, 56, 56, 64, 128, 1, 1, 2, 0, 1, 0]), ("t2d", [2, 9, 7, 128, 40, 3, 3, 2, 1, 1, 1])]:
         info, inputs = _declared(op, args, f16)
         c = info["conv"]
         if d.conv_window and (2 * c["pad"] != c["KH"] - 1 or 2 * c["pad_w"] != c["KW"] - 1):
             continue
-        print("tiles channels first", name, op, args, flush=True)
+        p, expand = _conv_problem(info), op == "t2d" and args[7] > 1
+        took = _cut(mod, p, chw=True, expand=expand)
+        cut += took
+        print("tiles channels first", name, op, args, mod.launch_tile(p, chw=True, expand=expand).as_tuple(), flush=True)
+        assert not _cut(own, p, chw=True, expand=expand)
         assert torch.equal(hostops.run_operator(mod, info, inputs), hostops.run_operator(own, info, inputs))
+        assert _cut(mod, p, chw=True, expand=expand) == took             # (also after its kernels were loaded)
+    assert cut >= 3
     mod.close()
     own.close()
 
@@ -131,9 +144,12 @@ def test_first_launch_under_capture(hrn):
     out = torch.empty((300, 260), dtype=torch.int32, device="cuda")
     hostops.gemm(own, A, W, bsum=bsum)
     torch.cuda.synchronize()
+    p = B.gemm_problem(1, 300, 260, 528)
+    assert _cut(mod, p)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         hostops.gemm(mod, A, W, out=out, bsum=bsum)
+    assert _cut(mod, p)                                                  # the tile was loaded inside the capture, else it is passed by
     for _ in range(3):
         A.random_(0, 256)
         out.fill_(1)
@@ -194,6 +210,8 @@ def test_channels_first_without_the_tiles_kernels(no_compiler, hrn):
     _copy_parts(cache, (d, "main"), (d, "chw"), *((t, "main") for t in B.tiles(d)))
     use()
     mod = B.Module(d)
+    p = _conv_problem(info)
+    assert _cut(mod, p) and not _cut(mod, p, chw=True)
     assert torch.equal(hostops.run_operator(mod, info, inputs), want)
     assert not mark.exists()
     mod.close()
@@ -217,6 +235,7 @@ def test_a_tile_that_cannot_be_loaded(no_compiler, hrn):
     assert _cut(mod, p)
     for _ in range(2):
         assert torch.equal(hostops.conv2d_nhwc(mod, X, F, 1, 1, 1), want)
+        assert not _cut(mod, p)
     assert "hipModule" not in B.lib().hrn_last_error().decode()
     torch.zeros(4, device="cuda").add_(1)
     torch.cuda.synchronize()
