@@ -777,6 +777,8 @@ hrn_module* module_of(const hrn_kernel_desc* desc, const std::string& stem, doub
 typedef float rv4f __attribute__((ext_vector_type(4)));
 typedef int rv4i __attribute__((ext_vector_type(4)));
 typedef _Float16 rv4h __attribute__((ext_vector_type(4)));
+typedef rv4h rv4h_any __attribute__((aligned(2)));      // (a result starts at any element)
+typedef rv4i rv4i_any __attribute__((aligned(4)));
 
 template <bool F16>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restrict__ ws, void* __restrict__ C, int split,
@@ -796,9 +798,9 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restri
         if constexpr (F16) {
             rv4h o;
             for (int r = 0; r < 4; ++r) o[r] = (_Float16)acc[r];
-            *(rv4h*)((_Float16*)C + dst) = o;
+            *(rv4h_any*)((_Float16*)C + dst) = o;
         } else {
-            *(rv4i*)((int*)C + dst) = acc;
+            *(rv4i_any*)((int*)C + dst) = acc;
         }
     }
 }

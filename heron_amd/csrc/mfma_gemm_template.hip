@@ -146,7 +146,6 @@ static_assert(NS >= 2 && NS <= 5, "stages");
 // with write 8 bytes here and there, 32 bytes of a row per instruction at best, and with the non-temporal hint each of them on
 // its own.  (32-bit results go out 16 bytes at a time either way; staged, one wave's 64x64 tile of them takes 0.4 us longer.)  Unlike HRN_EPI = 1 it takes rows of any alignment.  fp16, 128x128 tiles, stored non-temporally / not: 2000x2000x1024
 // 25.4 / 16.4 -> 13.0 us, 3000x2304x512 34.5 / 15.6 -> 11.9, 4000x1024x512 19.7 / 13.1 -> 8.2.
-constexpr bool ANY_ALIGNMENT = HRN_EPI == 0;
 constexpr bool STAGE_DIRECT = HRN_EPI == 0 && OES == 2 && !CW && !PERS && (MT * (WTN * OES / 16)) % 64 == 0 &&
                               NW * MT * (WTN * OES + 16) <= NS * STAGE_BYTES;
 constexpr int EPI = STAGE_DIRECT ? 1 : HRN_EPI;
@@ -236,6 +235,13 @@ __device__ __forceinline__ void wait_only() {
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 constexpr int AGENT_SCOPE = 16;             // cache policy (sc1): a load or store that all XCDs of the device see
+// pieces of a result in memory: rows and results start at any element with HRN_EPI = 0 and where split-K slices are added up.  (The
+// attribute belongs to these names: template arguments and `auto` drop it, so stores name the type.)
+typedef v4i out16_t __attribute__((aligned(HRN_EPI == 0 ? OES : 16)));
+typedef long out8_t __attribute__((aligned(HRN_EPI == 0 ? OES : 8)));
+typedef v4h sum8_t __attribute__((aligned(2)));
+typedef v4i sum16_t __attribute__((aligned(4)));
+static_assert(HRN_EPI != 0 || (alignof(out16_t) == OES && alignof(out8_t) == OES), "results of any alignment");
 
 // raw buffer (stride 0): a lane offset >= `bytes` reads as zero instead of touching memory (the scalar offset of a
 // load is not part of that check)
@@ -750,9 +756,13 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
 
         char* Cb = (char*)a.C + ((int64_t)slice * a.batch + c_bz) * a.sC * OES;
         [[maybe_unused]] const rsrc_t rsrcC = make_rsrc(Cb, (uint32_t)a.M * (uint32_t)a.ldc * OES);
-        auto put = [&](auto* ptr, auto val) __attribute__((always_inline)) {
-            if constexpr (NTS) __builtin_nontemporal_store(val, ptr);
-            else *ptr = val;
+        [[maybe_unused]] auto put16 = [&](char* dst, v4i val) __attribute__((always_inline)) {
+            if constexpr (NTS) __builtin_nontemporal_store(val, (out16_t*)dst);
+            else *(out16_t*)dst = val;
+        };
+        [[maybe_unused]] auto put8 = [&](char* dst, long val) __attribute__((always_inline)) {
+            if constexpr (NTS) __builtin_nontemporal_store(val, (out8_t*)dst);
+            else *(out8_t*)dst = val;
         };
         [[maybe_unused]] auto put_partial = [&](int m, int n, auto val) __attribute__((always_inline)) {
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rsrcC, (m * a.ldc + n) * 4, 0, AGENT_SCOPE);
@@ -852,8 +862,6 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             char* strip = epi + EPI_BASE + wave * (MT * EPI_PITCH);
             constexpr int CPRW = SW * OES / 16;                // 16-byte chunks per strip row
             constexpr int EPC = 16 / OES;                      // output elements per chunk
-            typedef v4i any_t __attribute__((aligned(OES)));
-            using piece_t = typename std::conditional<ANY_ALIGNMENT, any_t, v4i>::type;
             constexpr int TNS = TN / ESPLIT;                   // MFMA column tiles per strip
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -902,8 +910,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                         } else {
                             char* dst = Cb + ((int64_t)m * a.ldc + n) * OES;
                             if (m < a.M) {
-                                if (n + EPC <= a.N) put((piece_t*)dst, val);
-                                else if (OES == 2 && n + 4 <= a.N) put((long*)dst, (long)(((long)(uint32_t)val.y << 32) | (uint32_t)val.x));
+                                if (n + EPC <= a.N) put16(dst, val);
+                                else if (OES == 2 && n + 4 <= a.N) put8(dst, (long)(((long)(uint32_t)val.y << 32) | (uint32_t)val.x));
                             }
                         }
                     }
@@ -926,7 +934,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                                 v4h o;
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) o[r] = (_Float16)acc[i][j][g * 4 + r];
-                                put((v4h*)dst, o);
+                                put8(dst, __builtin_bit_cast(long, o));
                             } else if constexpr (DT == 0) {
                                 v4f o;
 #pragma unroll
@@ -938,7 +946,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r] + 128 * bs[r];
                                 if constexpr (SPLITK) put_partial(m, n, o);
-                                else put((v4i*)dst, o);
+                                else put16(dst, o);
                             }
                         }
                     }
@@ -1031,9 +1039,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                             v4h o;
 #pragma unroll
                             for (int r = 0; r < 4; ++r) o[r] = (_Float16)sum[u][r];
-                            *(v4h*)((_Float16*)a.out + at) = o;
+                            *(sum8_t*)((_Float16*)a.out + at) = o;
                         } else {
-                            *(v4i*)((int*)a.out + at) = __builtin_bit_cast(v4i, sum[u]);
+                            *(sum16_t*)((int*)a.out + at) = __builtin_bit_cast(v4i, sum[u]);
                         }
                     }
                 }
