@@ -706,7 +706,8 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     int64_t total = (int64_t)k->tiles_m * k->tiles_n * p->batch;
     plan->C = C; plan->ldc = p->ldc; plan->stride_c = p->stride_c;
     if (d.split_k) {
-        // the kernel writes raw partial sums, slice by slice, into the workspace; hrn's reduction pass writes C
+        // the kernel writes raw partial sums, slice by slice, into the workspace; its last slices write C, or the reduction kernel
+        // where the workspace ends before the arrivals
         if (p->split_k < 1) return fail(HRN_E_BADPARAM, "a split_k instance needs problem.split_k >= 1 (got %d)", p->split_k);
         int kps, split;
         split_shape(d, p, &kps, &split);

@@ -9,7 +9,7 @@
 //   HRN_MFMA    32 | 16 (MFMA tile edge), HRN_STAGES LDS stages, HRN_SWZ LDS chunk swizzle,
 //   HRN_EPI     0 result of any alignment, staged where there is room, 1 LDS-staged epilogue with 16-byte coalesced
 //               stores, 2 the same with half-width staging strips, HRN_WPE waves-per-SIMD hint, HRN_CONVWIN conv input window in LDS, HRN_PERSIST persistent
-//               launch, HRN_SPLITK K split over several workgroups with raw partial sums as output.
+//               launch, HRN_SPLITK K split over several workgroups whose partial sums the last one adds up.
 //
 // Data movement: both operands are K-contiguous, so a tile is a set of rows of HRN_BKB bytes.
 // Rows are cut into 16-byte chunks; every lane moves one chunk per load straight from HBM/L2
@@ -86,7 +86,8 @@ constexpr bool CW = (HRN_CONVWIN != 0);
 #endif
 constexpr bool PERS = (HRN_PERSIST != 0);
 // Split-K: the grid holds `split` copies of the tile grid; copy z multiplies k-tiles [z*kt_per_slice, (z+1)*kt_per_slice)
-// and stores its raw fp32 / int32 partial sums to slice z of the output buffer (a workspace); a second kernel adds the slices.
+// and stores its raw fp32 / int32 partial sums to slice z of a workspace; the slice that finishes a tile last adds them up (fold_slices),
+// or, where the workspace has no room for the arrivals, a second kernel (splitk_reduce_kernel) does.
 #ifndef HRN_SPLITK
 #define HRN_SPLITK 0
 #endif
@@ -99,8 +100,8 @@ constexpr bool SPLITK = (HRN_SPLITK != 0);
 #endif
 constexpr bool COLSUM = (HRN_DTYPE == 1) && (HRN_COLSUM != 0);
 // the results leave with the non-temporal hint: C is written once and not read by this kernel, and a round's 8 MiB of it
-// per XCD would otherwise push the operand slabs of the next round out of the 4 MiB L2 (split-K partial sums, which the
-// reduction reads right away, keep the default policy)
+// per XCD would otherwise push the operand slabs of the next round out of the 4 MiB L2 (split-K partial sums go out at device scope
+// instead, whoever adds them up: the other XCDs' slices are read from memory)
 #ifndef HRN_NTSTORE
 #define HRN_NTSTORE 0
 #endif
@@ -144,8 +145,8 @@ static_assert(BM % (WM * MT) == 0 && BN % (WN * MT) == 0, "wave tile");
 static_assert(NS >= 2 && NS <= 5, "stages");
 // HRN_EPI = 0 stages fp16 results as well, where the strips fit into the LDS of the stages: lanes that store what the MFMAs leave them
 // with write 8 bytes here and there, 32 bytes of a row per instruction at best, and with the non-temporal hint each of them on
-// its own.  (32-bit results go out 16 bytes at a time either way; staged, one wave's 64x64 tile of them takes 0.4 us longer.)  Unlike HRN_EPI = 1 it takes rows of any alignment.  fp16, 128x128 tiles, stored non-temporally / not: 2000x2000x1024
-// 25.4 / 16.4 -> 13.0 us, 3000x2304x512 34.5 / 15.6 -> 11.9, 4000x1024x512 19.7 / 13.1 -> 8.2.
+// its own.  (32-bit results go out 16 bytes at a time either way; staged, one wave's 64x64 tile of them takes 0.4 us longer.)  Unlike HRN_EPI = 1
+// it takes rows of any alignment.  fp16, 128x128 tiles, stored non-temporally / not: 2000x2000x1024 25.4 / 16.4 -> 13.0 us, 3000x2304x512 34.5 / 15.6 -> 11.9, 4000x1024x512 19.7 / 13.1 -> 8.2.
 constexpr bool STAGE_DIRECT = HRN_EPI == 0 && OES == 2 && !CW && !PERS && (MT * (WTN * OES / 16)) % 64 == 0 &&
                               NW * MT * (WTN * OES + 16) <= NS * STAGE_BYTES;
 constexpr int EPI = STAGE_DIRECT ? 1 : HRN_EPI;
