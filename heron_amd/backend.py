@@ -174,7 +174,6 @@ SYMBOLS = {
     "hrn_compile_chw": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
     "hrn_module_has_chw": (_i, [_vp]),
     "hrn_tiles": (_i, [ctypes.POINTER(KernelDesc), ctypes.POINTER(KernelDesc), _i]),
-    "hrn_compile_tiles": (_i, [ctypes.POINTER(KernelDesc), _i, _d]),
     "hrn_launch_tile": (_i, [_vp, ctypes.POINTER(Problem), ctypes.POINTER(KernelDesc)]),
     "hrn_launch_chw_tile": (_i, [_vp, ctypes.POINTER(Problem), _i, ctypes.POINTER(KernelDesc)]),
     "hrn_module_own_tiles": (None, [_vp, _i]),

@@ -1642,22 +1642,6 @@ int hrn_compile_chw(const hrn_kernel_desc* desc, int expand, double timeout_s) {
     return compile_desc(desc, expand ? PART_EXPAND : PART_CHW, timeout_s, &path);
 }
 
-int hrn_compile_tiles(const hrn_kernel_desc* desc, int part, double timeout_s) {
-    int rc = derive(desc, nullptr);
-    if (rc) return rc;
-    hrn_kernel_desc fit[kMaxFits];
-    int first_half, end_half;
-    const int n = cut_tiles(*desc, fit, &first_half, &end_half);
-    for (int i = 0; i < n; ++i) {
-        Derived dv;
-        (void)derive(&fit[i], &dv);
-        std::string path;
-        if (part == PART_MAIN || dv.has_chw) rc = compile_desc(&fit[i], part, timeout_s, &path);
-        if (rc) return rc;
-    }
-    return n;
-}
-
 int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap) {
     int rc = derive(desc, nullptr);
     if (rc) return rc;

@@ -208,19 +208,19 @@ int hrn_launch_conv2d_nhwc_u8s8(const hrn_module* mod, const hrn_problem* p, con
 int hrn_launch_is_deep(const hrn_module* mod, const hrn_problem* p);
 
 /*
- * A launch of at most half as many tiles as the device has CUs takes the instance's tile cut in halves (same MFMA shape, same order
- * along K: same result bit for bit), a tile of one to three waves takes more of them on grids of at most six tiles a CU, and a conv window
- * tile that has a CU to itself takes half the rows where two of those fit; persistent and split-K instances keep theirs.  Such a tile is an instance of its own.
- * hrn_build looks which of them the cache holds; only those are taken, each loaded (never compiled) at the first launch that does, and
- * a launch whose kernel the cache lacks or that cannot be loaded is the instance's own.  hrn_tiles lists those of an instance (returns
- * how many, at most `cap` are written), for hrn_compile and hrn_compile_chw; hrn_compile_tiles
- * compiles them ahead (part 0: the kernels of plain launches, 1 and 2: those of hrn_launch_conv2d_chw without and with
- * expand), hrn_launch_tile and hrn_launch_chw_tile say which a row-major launch and one of hrn_launch_conv2d_chw take, without loading it, and hrn_module_own_tiles(mod, 1) keeps a module to its own,
- * as a search over tiles needs.  hrn_module_tuned_for names the problem an instance was searched for, before the module's first launch: on
- * its sizes (strides, slices and raster order count for nothing) the launches keep the tile that was found (null: no such problem).
+ * Other tiles of an instance, same MFMA shape and same order along K, so the same result bit for bit.  A launch of at most half as
+ * many tiles as the device has CUs takes the instance's tile cut in halves, a tile of one to three waves takes more of them on grids
+ * of at most six tiles a CU, and a conv window tile that has a CU to itself takes half the rows where two of those fit.  Persistent and
+ * split-K instances keep theirs.  Such a tile is an instance of its own: hrn_build looks which of them the cache holds, only those are
+ * taken, each loaded (never compiled) at the first launch that does, and a launch whose kernel is not there or cannot be loaded is the
+ * instance's own.
+ *   hrn_tiles lists those of an instance (returns how many, at most `cap` are written), for hrn_compile and hrn_compile_chw ahead of
+ * hrn_build.  hrn_launch_tile and hrn_launch_chw_tile say which a row-major launch and one of hrn_launch_conv2d_chw take, and load
+ * nothing.  hrn_module_own_tiles(mod, 1) keeps a module to its own, as a search over tiles needs.  hrn_module_tuned_for names the problem
+ * an instance was searched for, before the module's first launch: on its sizes (strides, slices and raster order count for nothing) the
+ * launches keep the tile that was found (null: no such problem).
  */
 int hrn_tiles(const hrn_kernel_desc* desc, hrn_kernel_desc* out, int cap);
-int hrn_compile_tiles(const hrn_kernel_desc* desc, int part, double timeout_s);
 int hrn_launch_tile(const hrn_module* mod, const hrn_problem* p, hrn_kernel_desc* out);
 int hrn_launch_chw_tile(const hrn_module* mod, const hrn_problem* p, int expand, hrn_kernel_desc* out);
 void hrn_module_own_tiles(hrn_module* mod, int on);
