@@ -61,8 +61,7 @@ def main():
             else:
                 host = np.zeros(shp, dtype=np.int32 if dt == "int32" else np.float16)
             tens.append(torch.from_numpy(host).cuda().to(torch_dt.get(dt, torch.float16)))
-        layers.append(dict(name=name, mod=mod, prob=prob, a=tens[0], b=tens[1], c=tens[-1], times=int(times),
-                           split=int(sched.params.get('split_k', 1))))
+        layers.append(dict(name=name, mod=mod, prob=prob, a=tens[0], b=tens[1], c=tens[-1], times=int(times)))
     launches = sum(l["times"] for l in layers)
     stream = torch.cuda.Stream()
     st = stream.cuda_stream
@@ -113,8 +112,8 @@ def main():
         e1.record(stream)
         e1.synchronize()
         graph_us = e0.elapsed_time(e1) * 1e3 / args.reps
-    out = dict(config=args.config, layers=len(layers), launches=launches, kernel_launches=launches + sum(
-                   l["times"] for l in layers if l["split"] > 1),
+    out = dict(config=args.config, layers=len(layers), launches=launches,
+               kernel_launches=launches,             # (a split-K launch adds its slices up itself)
                isolated_sum_us=isolated, stream_us=stream_us, graph_us=graph_us, graph_rounds_checked=checked,
                per_launch_us=dict(isolated=isolated / launches, stream=stream_us / launches, graph=graph_us / launches))
     print("%d layers, %d launches per pass" % (len(layers), launches))
