@@ -51,7 +51,7 @@ WINDOW_CASES = [
                          ids=sorted(INSTANCES) + [n + "-carry" for n in INSTANCES if "window" in n])
 def test_equals_the_separate_passes(name, cases, hrn):
     f16 = name.startswith("f16")
-    mod, own = B.Module(INSTANCES[name]), B.Module(INSTANCES[name], own_tiles=True)
+    mod = B.Module(INSTANCES[name])
     ran = 0
     for op, args in cases:
         ctx = Ctx()
@@ -69,17 +69,15 @@ def test_equals_the_separate_passes(name, cases, hrn):
             X = torch.randint(0, 256, ref["input"], device="cuda", generator=gen, dtype=torch.uint8)
             F = torch.randint(-128, 128, ref["filter"], device="cuda", generator=gen, dtype=torch.int8)
         print("channels first", name, op, args, flush=True)
-        got = hostops.run_operator(own, info, [X, F])
+        got = hostops.run_operator(mod, info, [X, F])
         act, const, fin = hostops.ADAPTERS[info["adapter"]]
-        want = fin(info, hostops.conv2d_nhwc(own, act(info, X, F), const(info, X, F), (c["stride"], c["stride_w"]), (c["pad"], c["pad_w"]),
+        want = fin(info, hostops.conv2d_nhwc(mod, act(info, X, F), const(info, X, F), (c["stride"], c["stride_w"]), (c["pad"], c["pad_w"]),
                                              (c["dil"], c["dil_w"])))
         torch.cuda.synchronize()
         assert got.shape == want.shape and torch.equal(got, want), (name, op, args)
-        assert torch.equal(hostops.run_operator(mod, info, [X, F]), want), (name, op, args)      # the tile a caller gets
         ran += 1
     assert ran >= 2
     mod.close()
-    own.close()
 
 
 def test_bad_views_are_refused(hrn):

@@ -37,7 +37,7 @@ def _inputs(f16, b, m, n, k):
 @pytest.mark.parametrize("rest", [0, 16, 112])
 def test_equals_the_plain_kernel(name, k_tiles, rest, hrn):
     d = INSTANCES[name]
-    mod, f16 = B.Module(d, own_tiles=True), d.dtype == F16
+    mod, f16 = B.Module(d), d.dtype == F16
     m, n, slices = (1025, 1028, 3) if d.split_k else ((1700, 1732, 0) if d.bkb == 128 else (3100, 3300, 0))
     kb = (k_tiles * d.bkb - min(rest, d.bkb - 16)) * max(1, slices)
     assert (m + n) * kb >= 2 << 20 or k_tiles < 6
@@ -58,7 +58,7 @@ def test_equals_the_plain_kernel(name, k_tiles, rest, hrn):
 def test_conv_images_in_one_launch_and_apart(dtype, hrn):
     f16 = dtype == "f16"
     d = D(F16, CONV, 128, 64, 128, 2, 1, 32, 2, 1, epi=1) if f16 else instances.int8_conv_descs()[0]
-    mod = B.Module(d, own_tiles=True)
+    mod = B.Module(d)
     gen = torch.Generator(device="cuda").manual_seed(3)
     shape, filt = (16, 33, 31, 1024 if f16 else 2048), (72, 3, 3, 1024 if f16 else 2048)
     if f16:
@@ -101,7 +101,7 @@ def _oracle(op, args, X, F):
 @pytest.mark.parametrize("name", sorted(CHW_INSTANCES))
 @pytest.mark.parametrize("op,args", CHW_CASES, ids=["%s-%d" % (o, i) for i, (o, _) in enumerate(CHW_CASES)])
 def test_channels_first(name, op, args, hrn):
-    mod, f16 = B.Module(CHW_INSTANCES[name], own_tiles=True), name.startswith("f16")
+    mod, f16 = B.Module(CHW_INSTANCES[name]), name.startswith("f16")
     ctx = type("Ctx", (), dict(set_info=lambda self, i: setattr(self, "info", i), set_axis_map=lambda self, m: None))()
     getOpFromName(op)(ctx, *args, *(["float16"] * 2 if f16 else ["int8"] * 2))
     info, c = ctx.info, ctx.info["conv"]

@@ -20,8 +20,7 @@ PAIRS = [(F16, (128, 128, 128, 2, 2, 32, 2, 1)), (U8, (128, 128, 128, 2, 2, 32, 
 @pytest.mark.parametrize("n", [4, 36, 100, 128, 132, 260])
 def test_rows_and_starts(kind, shape, n, hrn):
     f16 = kind == F16
-    mods = [B.Module(D(kind, GEMM, *shape, epi=e), own_tiles=True) for e in (0, 1)]
-    mods.append(B.Module(D(kind, GEMM, *shape, epi=0)))                   # the tile a caller gets on these grids
+    mods = [B.Module(D(kind, GEMM, *shape, epi=e)) for e in (0, 1)]
     rng = np.random.default_rng(n)
     for m in (1, 127, 131):
         k = 160
@@ -34,10 +33,8 @@ def test_rows_and_starts(kind, shape, n, hrn):
             buf = torch.full((m * n + 64,), -3, dtype=torch.float16 if f16 else torch.int32, device="cuda")
             out = buf[16 + start:16 + start + m * n].view(m, n)
             print("direct epilogue", kind, shape, (m, n, k), start, flush=True)
-            hostops.gemm(mods[2], a, w, out=out)
-            cut = out.clone()
-            hostops.gemm(mods[0], a, w, out=out.fill_(-3))
-            assert (buf[:16 + start] == -3).all() and (buf[16 + start + m * n:] == -3).all() and torch.equal(cut, out)
+            hostops.gemm(mods[0], a, w, out=out)
+            assert (buf[:16 + start] == -3).all() and (buf[16 + start + m * n:] == -3).all()
             if f16:
                 check_f16(out.cpu().numpy(), oracle.gemm_f32(A, W))
             else:

@@ -31,7 +31,7 @@ INSTANCES = {
 @pytest.mark.parametrize("kb", [16, 128, 144, 256, 272, 384, 400, 1024, 1040])
 def test_k_tiles(name, kb, hrn):
     f16 = name.startswith("f16")
-    mod = B.Module(INSTANCES[name], own_tiles=True)
+    mod = B.Module(INSTANCES[name])
     K = kb // 2 if f16 else kb
     for M, N in [(256, 256), (257, 264), (13, 520), (700, 248)]:
         A, Bm = (workloads.gemm_f16_inputs if f16 else workloads.gemm_u8s8_inputs)(M, K, N, seed=kb + M)
