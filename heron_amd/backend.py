@@ -72,7 +72,8 @@ class KernelDesc(ctypes.Structure):
     KEYS = ("dtype", "op", "bm", "bn", "bkb", "wm", "wn", "mfma", "stages", "swizzle", "epilogue", "waves_per_eu",
             "conv_window", "persistent", "split_k", "sched", "load_spread", "colsum", "nt_store")
 
-    tuned_for = None                # the Problem it was searched for, where it is the instance of a record
+    # the sizes it was searched for, where it is the instance of a record: the leading arguments of gemm_problem or conv2d_problem
+    tuned_for = None
 
     def as_tuple(self):
         return tuple(int(getattr(self, k)) for k in self.KEYS)
@@ -411,7 +412,8 @@ class Module:
         if own_tiles:
             lib().hrn_module_own_tiles(h, 1)
         if desc.tuned_for is not None:
-            lib().hrn_module_tuned_for(h, ctypes.byref(desc.tuned_for))
+            problem = conv2d_problem if desc.op == HRN_OP_CONV2D else gemm_problem
+            lib().hrn_module_tuned_for(h, ctypes.byref(problem(*desc.tuned_for)))
         self.native = (h.value, ctypes.addressof(desc))      # what the functions of ext() take for this instance
         self.has_chw = bool(lib().hrn_module_has_chw(h))     # launch_conv2d_chw takes it
         info = KernelInfo()

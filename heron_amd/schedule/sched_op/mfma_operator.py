@@ -33,18 +33,21 @@ class TemplateSchedule:
                            p['swizzle'], p.get('epilogue', 0), p['waves_per_eu'],
                            p.get('conv_window', 0), p.get('persistent', 0), 1 if p.get('split_k', 1) > 1 else 0,
                            p.get('sched', 1), p.get('load_spread', 2), p.get('colsum', 0), p.get('nt_store', 0))
-        desc.tuned_for = self.to_problem()
+        desc.tuned_for = self.sizes()
         return desc
+
+    def sizes(self):
+        if self.info['operator'] == 'conv2d_nhwc':
+            c = self.info['conv']
+            return (c['N'], c['H'], c['W'], c['CI'], c['CO'], c['KH'], c['KW'], (c['stride'], c['stride_w']), (c['pad'], c['pad_w']),
+                    (c['dil'], c['dil_w']))
+        g = self.info['gemm_view']
+        return g['batch'], g['M'], g['N'], g['K']
 
     def to_problem(self):
         from ... import backend as B
-        g = self.info['gemm_view']
-        if self.info['operator'] == 'conv2d_nhwc':
-            c = self.info['conv']
-            return B.conv2d_problem(c['N'], c['H'], c['W'], c['CI'], c['CO'], c['KH'], c['KW'],
-                                    (c['stride'], c['stride_w']), (c['pad'], c['pad_w']), (c['dil'], c['dil_w']),
-                                    self.params['group_m'], self.params.get('split_k', 1))
-        return B.gemm_problem(g['batch'], g['M'], g['N'], g['K'], self.params['group_m'], self.params.get('split_k', 1))
+        make = B.conv2d_problem if self.info['operator'] == 'conv2d_nhwc' else B.gemm_problem
+        return make(*self.sizes(), self.params['group_m'], self.params.get('split_k', 1))
 
     def describe(self):
         return ", ".join("%s=%s" % kv for kv in sorted(self.params.items()))

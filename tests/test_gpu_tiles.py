@@ -290,7 +290,7 @@ def test_a_record_runs_its_own_tile_on_its_own_problem(name, hrn):
 def test_a_record_of_few_tiles(hrn):
     """On its own sizes, in any raster order, it keeps its tile; elsewhere the rule decides."""
     d = D(F16, GEMM, 256, 256, 128, 2, 4, 16, 2, 2)
-    d.tuned_for = B.gemm_problem(1, 700, 520, 256)
+    d.tuned_for = (1, 700, 520, 256)
     mod = B.Module(d)
     assert not _cut(mod, B.gemm_problem(1, 700, 520, 256, group_m=2))
     for other in (B.gemm_problem(1, 700, 520, 264), B.gemm_problem(1, 701, 520, 256), B.gemm_problem(1, 700, 528, 256), B.gemm_problem(2, 700, 520, 256)):
@@ -298,7 +298,7 @@ def test_a_record_of_few_tiles(hrn):
     mod.close()
     d = CONVS["f16-128"]
     args = [2, 14, 14, 64, 48, 3, 3, 1, 1, 1]
-    d.tuned_for = B.conv2d_problem(*args)
+    d.tuned_for = tuple(args)
     mod = B.Module(d)
     assert not _cut(mod, B.conv2d_problem(*args))
     for i, v in [(0, 3), (4, 64), (5, 5), (6, 1), (7, (1, 2)), (8, 2), (9, 2)]:
