@@ -30,6 +30,15 @@
 #include <type_traits>
 #include <vector>
 
+// n / d for 0 <= n < 2^31 and 1 <= d < 2^31 by a multiplication: with L = ceil(log2 d) and m = ceil(2^(31+L) / d), which fits into
+// 32 bits, n*m / 2^(31+L) exceeds n / d by less than 1 / d (Granlund and Montgomery, Division by Invariant Integers).
+struct FastDiv {
+    uint32_t m, shift;
+    FastDiv() = default;
+    explicit FastDiv(uint32_t d) : shift(d > 1 ? 32 - __builtin_clz(d - 1) : 0) { m = (uint32_t)(((1ull << (31 + shift)) + d - 1) / d); }
+    __device__ __forceinline__ uint32_t operator()(uint32_t n) const { return __umulhi(n << 1, m) >> shift; }
+};
+
 #define HRN_KARGS_DEFINED
 struct HrnKArgs {  // must match mfma_gemm_template.hip
     const void* A;
@@ -50,6 +59,7 @@ struct HrnKArgs {  // must match mfma_gemm_template.hip
     uint64_t* arrivals;
     uint64_t ticket;
     int32_t out_ld;
+    FastDiv by_total, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
 };
 
 // An instance's kernels lie in up to three code objects, so that a caller pays the compiler only for those it launches: a
@@ -702,8 +712,21 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     }
     k->tiles_m = (p->m + d.bm - 1) / d.bm;
     k->tiles_n = (p->n + d.bn - 1) / d.bn;
-    k->group_m = p->group_m > 0 ? p->group_m : 8;
+    k->group_m = std::min(p->group_m > 0 ? p->group_m : 8, k->tiles_m);
     int64_t total = (int64_t)k->tiles_m * k->tiles_n * p->batch;
+    if (total >= (1ll << 31)) return fail(HRN_E_BADPARAM, "grid size");
+    k->by_total = FastDiv((uint32_t)total);
+    k->by_tiles = FastDiv((uint32_t)(k->tiles_m * k->tiles_n));
+    k->by_group = FastDiv((uint32_t)(k->group_m * k->tiles_n));
+    k->by_gm = FastDiv((uint32_t)k->group_m);
+    k->by_gm_last = FastDiv((uint32_t)std::max(1, k->tiles_m % k->group_m));
+    if (d.op == HRN_OP_CONV2D) {
+        k->by_kwci = FastDiv((uint32_t)(k->KW * k->CI));
+        k->by_ci = FastDiv((uint32_t)k->CI);
+        k->by_hw = FastDiv((uint32_t)(k->HO * k->WO));
+        k->by_wo = FastDiv((uint32_t)k->WO);
+        k->by_cpp = FastDiv((uint32_t)(k->CI * es / 16));
+    }
     plan->C = C; plan->ldc = p->ldc; plan->stride_c = p->stride_c;
     if (d.split_k) {
         // the kernel writes raw partial sums, slice by slice, into the workspace; its last slices write C, or the reduction kernel
@@ -1078,15 +1101,6 @@ __global__ void __launch_bounds__(256) pad_rows_kernel(const unsigned char* __re
         dst[t] = v;
     }
 }
-
-// n / d for 0 <= n < 2^31 and 1 <= d < 2^31 by a multiplication: with L = ceil(log2 d) and m = ceil(2^(31+L) / d), which fits into
-// 32 bits, n*m / 2^(31+L) exceeds n / d by less than 1 / d (Granlund and Montgomery, Division by Invariant Integers).
-struct FastDiv {
-    uint32_t m, shift;
-    FastDiv() = default;
-    explicit FastDiv(uint32_t d) : shift(d > 1 ? 32 - __builtin_clz(d - 1) : 0) { m = (uint32_t)(((1ull << (31 + shift)) + d - 1) / d); }
-    __device__ __forceinline__ uint32_t operator()(uint32_t n) const { return __umulhi(n << 1, m) >> shift; }
-};
 
 // hrn_gather as its kernel reads it: the innermost extent counts lanes.  IDX = uint32_t when every extent, numerator, coordinate
 // and offset fits (the host has checked), else uint64_t.
@@ -1795,6 +1809,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
     if (view->out_plane < 1 || p->m % view->out_plane)
         return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
     plan.k.out_plane = view->out_plane;
+    plan.k.by_plane = FastDiv((uint32_t)view->out_plane);
     if (mod->desc.conv_window) plan.dyn_lds = std::max(plan.dyn_lds, (unsigned)mod->chw_bytes);
     if (view->expand) {
         if (view->expand < 1 || (view->expand & (view->expand - 1)) || view->in_h < 1 || view->in_w < 1 || view->top < 0 || view->left < 0 ||

@@ -35,6 +35,7 @@
 
 #ifndef HRN_KARGS_DEFINED
 #define HRN_KARGS_DEFINED
+struct HrnDiv { uint32_t m, shift; };    // n / d for 0 <= n < 2^31 is (2n * m >> 32) >> shift (FastDiv of hrn_api.cpp)
 struct HrnKArgs {
     const void* A;
     const void* B;
@@ -57,6 +58,9 @@ struct HrnKArgs {
     uint64_t* arrivals;                  // one word per output tile, of any content
     uint64_t ticket;                     // of this launch, its low 16 bits zero
     int32_t out_ld;
+    // divisors of the launch: output tiles, those of a batch entry, of a raster group, rows of a group and of the last one, conv: elements of
+    // a filter row and of a tap, output pixels of an image and of a row, 16-byte pieces of a pixel, pixels of a plane (out_plane)
+    HrnDiv by_total, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
 };
 #endif
 
@@ -213,6 +217,12 @@ template <> struct AccT<16> { using F = v16f; using I = v16i; };
 template <> struct AccT<4> { using F = v4f; using I = v4i; };
 using acc_t = typename std::conditional<DT == 0, typename AccT<ACC_N>::F, typename AccT<ACC_N>::I>::type;
 
+// Divisions by what is fixed for a launch, by multiplication.  A division proper is some 30 instructions, and a kernel starts with four
+// (GEMM) to eight of them, each waiting for the one before, in front of its first load: 194 instructions to it instead of 127 (u8 64x128
+// tiles), 435 instead of 283 (fp16 im2col 128x128).  fp16 3x3 32x56x56x64 -> 64 13.67 -> 13.24 us, transposed conv 16x56x56x64 -> 128
+// 24.1 -> 23.0, fp16 batch_matmul 192x512x512x64 21.2 -> 20.8, u8 x s8 1111x1500x2064 11.5 -> 11.4; u8 1972x408x2672 10.1 -> 10.3.
+__device__ __forceinline__ int div_by(int n, HrnDiv d) { return (int)(__umulhi((uint32_t)n << 1, d.m) >> d.shift); }
+
 __device__ __forceinline__ int swz_of_row(int row) {
     if (SWZ == 0) return 0;
     return (row >> (SWZ - 1)) & (CPR - 1);
@@ -306,10 +316,14 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     if constexpr (TM * TN * ACC_N < 256) {      // (not where every register holds an accumulator)
         asm volatile("" ::"s"(a.A), "s"(a.B), "s"(a.C), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.lda), "s"(a.ldb), "s"(a.ldc), "s"(a.sA), "s"(a.sB),
                      "s"(a.sC), "s"(a.tiles_m), "s"(a.tiles_n), "s"(a.group_m), "s"(a.batch));
+        asm volatile("" ::"s"(a.by_tiles.m), "s"(a.by_tiles.shift), "s"(a.by_group.m), "s"(a.by_group.shift), "s"(a.by_gm.m), "s"(a.by_gm.shift),
+                     "s"(a.by_gm_last.m), "s"(a.by_gm_last.shift));
         if constexpr (OP == 1)
             asm volatile("" ::"s"(a.H), "s"(a.W), "s"(a.CI), "s"(a.HO), "s"(a.WO), "s"(a.KH), "s"(a.KW), "s"(a.cstride), "s"(a.cpad), "s"(a.cdil),
-                         "s"(a.cstride_w), "s"(a.cpad_w), "s"(a.cdil_w));
-        if constexpr (SPLITK) asm volatile("" ::"s"(a.split), "s"(a.kt_per_slice));
+                         "s"(a.cstride_w), "s"(a.cpad_w), "s"(a.cdil_w), "s"(a.by_hw.m), "s"(a.by_hw.shift), "s"(a.by_wo.m), "s"(a.by_wo.shift));
+        if constexpr (OP == 1 && !CW) asm volatile("" ::"s"(a.by_kwci.m), "s"(a.by_kwci.shift), "s"(a.by_ci.m), "s"(a.by_ci.shift));
+        if constexpr (CW) asm volatile("" ::"s"(a.by_cpp.m), "s"(a.by_cpp.shift));
+        if constexpr (SPLITK) asm volatile("" ::"s"(a.split), "s"(a.kt_per_slice), "s"(a.by_total.m), "s"(a.by_total.shift));
         if constexpr (COLSUM) asm volatile("" ::"s"(a.bsum));
     }
     const int tid = threadIdx.x;
@@ -322,24 +336,25 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     const uint32_t Kb = (uint32_t)a.K * ES;           // bytes of K
     const int KT_all = (Kb + BKB - 1) / BKB;
     int first_pid = blockIdx.x, slice = 0;
-    if constexpr (SPLITK) { slice = first_pid / total; first_pid -= slice * total; }
+    if constexpr (SPLITK) { slice = div_by(first_pid, a.by_total); first_pid -= slice * total; }
     const int kt0 = SPLITK ? slice * a.kt_per_slice : 0;                                   // first k-tile of this workgroup
     const int KT = SPLITK ? min(a.kt_per_slice, KT_all - kt0) : KT_all;                    // k-tiles of this workgroup
 
     // ---- tile raster: spread over the 8 XCDs so that each XCD's L2 sees a compact block ----
     auto tile_coords = [&](int pid, int& bz, int& tile_m, int& tile_n) {
         if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
-        bz = pid / tiles_mn;
+        bz = div_by(pid, a.by_tiles);
         const int t = pid - bz * tiles_mn;
         const int group_sz = a.group_m * a.tiles_n;
-        const int gid = t / group_sz;
+        const int gid = div_by(t, a.by_group);
         const int first_m = gid * a.group_m;
         const int gsz = min(a.tiles_m - first_m, a.group_m);
         const int tin = t - gid * group_sz;
-        // (the divisions run on the vector ALU; everything here is wave-uniform, and saying so keeps what is derived
-        // from it - descriptors, scalar offsets - in scalar registers)
-        tile_m = __builtin_amdgcn_readfirstlane(first_m + tin % gsz);
-        tile_n = __builtin_amdgcn_readfirstlane(tin / gsz);
+        const int col = div_by(tin, gsz == a.group_m ? a.by_gm : a.by_gm_last);
+        // (everything here is wave-uniform, and saying so keeps what is derived from it - descriptors, scalar offsets - in
+        // scalar registers)
+        tile_m = __builtin_amdgcn_readfirstlane(first_m + tin - col * gsz);
+        tile_n = __builtin_amdgcn_readfirstlane(col);
         bz = __builtin_amdgcn_readfirstlane(bz);
     };
 
@@ -363,7 +378,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     uint32_t a_bytes;
     const uint32_t b_bytes = (uint32_t)a.N * (uint32_t)a.ldb * ES;
     if constexpr (OP == 0) a_bytes = (uint32_t)a.M * (uint32_t)a.lda * ES;
-    else a_bytes = (uint32_t)(a.M / (a.HO * a.WO)) * (uint32_t)(in_h * in_w * a.CI) * ES;
+    else a_bytes = (uint32_t)div_by(a.M, a.by_hw) * (uint32_t)(in_h * in_w * a.CI) * ES;
     const char* baseA = (const char*)a.A;
     const char* baseB = (const char*)a.B;
     bool issue_alive = true;
@@ -428,14 +443,14 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                           "conv: the lane's chunk column must not depend on the load index");
             const int chunk = lpos ^ swz_of_row(wave * RPI + lrow);
             int ke = chunk * (16 / ES) + kt0 * (BKB / ES);      // element index inside K of this workgroup's first k-tile
-            cr = ke / (a.KW * a.CI); ke -= cr * (a.KW * a.CI);
-            cs = ke / a.CI; cc = ke - cs * a.CI;
+            cr = div_by(ke, a.by_kwci); ke -= cr * (a.KW * a.CI);
+            cs = div_by(ke, a.by_ci); cc = ke - cs * a.CI;
             // output pixel of the lane's first row by division, of the following rows (NW*RPI further each) by carry
             const int hw = a.HO * a.WO;
             int m = im0 + wave * RPI + lrow;
-            int img = m / hw;
+            int img = div_by(m, a.by_hw);
             int rem = m - img * hw;
-            int oy = rem / a.WO, ox = rem - oy * a.WO;
+            int oy = div_by(rem, a.by_wo), ox = rem - oy * a.WO;
 #pragma unroll
             for (int i = 0; i < A_LPW; ++i) {
                 const bool ok = m < a.M;
@@ -562,8 +577,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         // A lane's chunk moves on by NW * 64 chunks from load to load.  Its window row and its position in the row (EXPAND:
         // and the row's pixel) are divided out once and then carried: a division is some 40 instructions, and with three of
         // them per load (and one per stored piece, see HOIST below) the transposed conv below took 38.0 us instead of 33.8.
-        const int d_row = NW * 64 / cpp, d_pos = NW * 64 - d_row * cpp;
-        int wrow = (wave * 64 + lane) / cpp, pos = wave * 64 + lane - wrow * cpp;
+        const int d_row = div_by(NW * 64, a.by_cpp), d_pos = NW * 64 - d_row * cpp;
+        int wrow = div_by(wave * 64 + lane, a.by_cpp), pos = wave * 64 + lane - wrow * cpp;
         [[maybe_unused]] int w_img = 0, w_y = 0, w_x = 0, d_img = 0, d_y = 0, d_x = 0;
         if constexpr (EXPAND) {
             const int gp = gp0 + wrow;
@@ -602,9 +617,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         // masks: pixel of fragment row i by one division, the following rows (MT further each) by carry
         const int hw = a.H * a.W;
         int m = m0 + wm_idx * WTM + lr;
-        int img = m / hw;
+        int img = div_by(m, a.by_hw);          // ('same' padding: the image and its result are of one size)
         int rem = m - img * hw;
-        int oy = rem / a.W, ox = rem - oy * a.W;
+        int oy = div_by(rem, a.by_wo), ox = rem - oy * a.W;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             uint32_t bits = 0;
@@ -791,7 +806,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
 #pragma unroll
                 for (int b = 0; b < NIB; ++b) {
                     const unsigned m = (unsigned)(m0 + wm_idx * WTM + b * CSW + (lane_e % CPRW) * EPC);
-                    h_img[b] = m / plane;
+                    h_img[b] = (unsigned)div_by((int)m, a.by_plane);
                     h_px[b] = m - h_img[b] * plane;
                 }
             }
@@ -835,7 +850,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                         const int m = m0 + wm_idx * WTM + ib * MT + cc2 * EPC;
                         if (c < MT * CPRW && n < a.N && m < a.M) {
                             const v4i val = *(const v4i*)(strip + row * CHW_PITCH + cc2 * 16);
-                            const unsigned img = HOIST ? h_img[HOIST ? ib / IT : 0] : (unsigned)m / plane;
+                            const unsigned img = HOIST ? h_img[HOIST ? ib / IT : 0] : (unsigned)div_by(m, a.by_plane);
                             const unsigned px = HOIST ? h_px[HOIST ? ib / IT : 0] : (unsigned)m - img * plane;
                             oel_t* dst = (oel_t*)a.C + ((int64_t)img * a.N + n) * plane + px;
                             if (px + EPC <= plane && m + EPC <= a.M) {
