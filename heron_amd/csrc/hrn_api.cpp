@@ -60,6 +60,8 @@ struct HrnKArgs {  // must match mfma_gemm_template.hip
     uint64_t ticket;
     int32_t out_ld;
     FastDiv by_total, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
+    int32_t kw_end, kh_end, x_row, y_img, px;
+    uint32_t tap_bytes, taprow_bytes, row_bytes, img_bytes;
 };
 
 // An instance's kernels lie in up to three code objects, so that a caller pays the compiler only for those it launches: a
@@ -726,6 +728,14 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         k->by_hw = FastDiv((uint32_t)(k->HO * k->WO));
         k->by_wo = FastDiv((uint32_t)k->WO);
         k->by_cpp = FastDiv((uint32_t)(k->CI * es / 16));
+        k->kw_end = k->KW * k->cdil_w; k->kh_end = k->KH * k->cdil;
+        k->x_row = k->WO * k->cstride_w; k->y_img = k->HO * k->cstride;
+        k->px = k->CI * es;
+        const uint32_t px = (uint32_t)k->px, W = (uint32_t)k->W;               // (modulo 2^32, as the kernel adds them)
+        k->tap_bytes = ((uint32_t)k->cdil_w - 1u) * px;
+        k->taprow_bytes = ((uint32_t)k->cdil * W - (uint32_t)k->kw_end) * px;
+        k->row_bytes = ((uint32_t)k->cstride * W - (uint32_t)k->x_row) * px;
+        k->img_bytes = ((uint32_t)k->H - (uint32_t)k->y_img) * W * px;
     }
     plan->C = C; plan->ldc = p->ldc; plan->stride_c = p->stride_c;
     if (d.split_k) {
@@ -1819,6 +1829,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
         plan.k.in_h = view->in_h; plan.k.in_w = view->in_w;
         plan.k.top = view->top; plan.k.left = view->left;
         plan.k.expand_shift = __builtin_ctz((unsigned)view->expand);
+        plan.k.img_bytes = (uint32_t)view->in_h * (uint32_t)view->in_w * (uint32_t)plan.k.px;
     }
     const CodeObject* kernels;
     rc = chw_kernels(mod, part, &kernels);

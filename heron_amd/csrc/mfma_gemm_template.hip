@@ -61,6 +61,10 @@ struct HrnKArgs {
     // divisors of the launch: output tiles, those of a batch entry, of a raster group, rows of a group and of the last one, conv: elements of
     // a filter row and of a tap, output pixels of an image and of a row, 16-byte pieces of a pixel, pixels of a plane (out_plane)
     HrnDiv by_total, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
+    // conv, im2col: extents of all taps (dilated) and of the result (times the stride) in input pixels, the bytes of a pixel, and what
+    // a byte offset changes by beyond the step itself where K goes on to the next tap and filter row, the pixels to the next row and image
+    int32_t kw_end, kh_end, x_row, y_img, px;
+    uint32_t tap_bytes, taprow_bytes, row_bytes, img_bytes;
 };
 #endif
 
@@ -321,7 +325,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         if constexpr (OP == 1)
             asm volatile("" ::"s"(a.H), "s"(a.W), "s"(a.CI), "s"(a.HO), "s"(a.WO), "s"(a.KH), "s"(a.KW), "s"(a.cstride), "s"(a.cpad), "s"(a.cdil),
                          "s"(a.cstride_w), "s"(a.cpad_w), "s"(a.cdil_w), "s"(a.by_hw.m), "s"(a.by_hw.shift), "s"(a.by_wo.m), "s"(a.by_wo.shift));
-        if constexpr (OP == 1 && !CW) asm volatile("" ::"s"(a.by_kwci.m), "s"(a.by_kwci.shift), "s"(a.by_ci.m), "s"(a.by_ci.shift));
+        if constexpr (OP == 1 && !CW)
+            asm volatile("" ::"s"(a.by_kwci.m), "s"(a.by_kwci.shift), "s"(a.by_ci.m), "s"(a.by_ci.shift), "s"(a.kw_end), "s"(a.kh_end), "s"(a.x_row),
+                         "s"(a.y_img), "s"(a.px), "s"(a.tap_bytes), "s"(a.taprow_bytes), "s"(a.row_bytes), "s"(a.img_bytes));
         if constexpr (CW) asm volatile("" ::"s"(a.by_cpp.m), "s"(a.by_cpp.shift));
         if constexpr (SPLITK) asm volatile("" ::"s"(a.split), "s"(a.kt_per_slice), "s"(a.by_total.m), "s"(a.by_total.shift));
         if constexpr (COLSUM) asm volatile("" ::"s"(a.bsum));
@@ -410,7 +416,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     // GEMM: byte offset of the lane's chunk in k-tile 0.  Conv: pixel bookkeeping.
     uint32_t voffA[(A_LPW > 0 ? A_LPW : 1)];
     int iy0[OP == 1 ? (A_LPW > 0 ? A_LPW : 1) : 1], ix0[OP == 1 ? (A_LPW > 0 ? A_LPW : 1) : 1];
-    int cc = 0, cs = 0, cr = 0;  // conv: channel / kw / kh position of the lane's chunk
+    // conv: where the lane's chunk is in K: its channel, its tap in pixels from tap (0, 0), and (koff) that as a byte offset
+    int cc = 0, dx = 0, dy = 0;
+    uint32_t koff = 0;
     int itile = first_pid;
     int issue_kt = 0;            // next k-tile (relative to kt0) of tile `itile` to fetch
 
@@ -443,23 +451,33 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                           "conv: the lane's chunk column must not depend on the load index");
             const int chunk = lpos ^ swz_of_row(wave * RPI + lrow);
             int ke = chunk * (16 / ES) + kt0 * (BKB / ES);      // element index inside K of this workgroup's first k-tile
-            cr = div_by(ke, a.by_kwci); ke -= cr * (a.KW * a.CI);
-            cs = div_by(ke, a.by_ci); cc = ke - cs * a.CI;
-            // output pixel of the lane's first row by division, of the following rows (NW*RPI further each) by carry
-            const int hw = a.HO * a.WO;
+            const int r = div_by(ke, a.by_kwci); ke -= r * (a.KW * a.CI);
+            const int s = div_by(ke, a.by_ci); cc = ke - s * a.CI;
+            dy = r * a.cdil; dx = s * a.cdil_w;
+            koff = (uint32_t)(dy * in_w + dx) * a.px + (uint32_t)cc * ES;
+            // input position (y, x) of tap (0, 0) of the lane's first row by division, of the following rows (NW*RPI output pixels
+            // further each) by carry; its byte offset `off` with it, modulo 2^32: the position may lie in the padding
             int m = im0 + wave * RPI + lrow;
-            int img = div_by(m, a.by_hw);
-            int rem = m - img * hw;
-            int oy = div_by(rem, a.by_wo), ox = rem - oy * a.WO;
+            const int img = div_by(m, a.by_hw);
+            const int rem = m - img * (a.HO * a.WO);
+            const int oy = div_by(rem, a.by_wo);
+            int y = oy * a.cstride - a.cpad, x = (rem - oy * a.WO) * a.cstride_w - a.cpad_w;
+            uint32_t off = EXPAND ? (uint32_t)img * a.img_bytes : ((uint32_t)((img * in_h + y) * in_w) + (uint32_t)x) * (uint32_t)a.px;
+            const int x_step = NW * RPI * a.cstride_w, x_end = a.x_row - a.cpad_w, y_end = a.y_img - a.cpad;
 #pragma unroll
             for (int i = 0; i < A_LPW; ++i) {
-                const bool ok = m < a.M;
-                voffA[i] = (uint32_t)img * (uint32_t)(in_h * in_w * a.CI) * ES;
-                iy0[i] = ok ? oy * a.cstride - a.cpad : -(1 << 28);
-                ix0[i] = ox * a.cstride_w - a.cpad_w;
+                iy0[i] = (m < a.M) ? y : -(1 << 28);
+                ix0[i] = x;
+                voffA[i] = off;
                 m += NW * RPI;
-                ox += NW * RPI;
-                while (ox >= a.WO) { ox -= a.WO; if (++oy == a.HO) { oy = 0; ++img; } }
+                x += x_step;
+                if constexpr (!EXPAND) off += (uint32_t)(x_step * a.px);
+                while (x >= x_end) {
+                    x -= a.x_row;
+                    y += a.cstride;
+                    if constexpr (!EXPAND) off += a.row_bytes;
+                    if (y >= y_end) { y -= a.y_img; off += a.img_bytes; }
+                }
             }
         }
     };
@@ -497,10 +515,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         ks_cur = live ? koff_cur : 0u;
         return live && koff_cur + BKB > Kb;                                      // ragged: the last tile is not full
     };
-    [[maybe_unused]] int conv_iyr = 0, conv_ixs = 0;
-    [[maybe_unused]] bool conv_kvalid = false;
+    [[maybe_unused]] int conv_dy = 0;            // past the last tap: below every image
     auto conv_tap = [&]() {
-        if constexpr (OP == 1 && !CW) { conv_iyr = cr * a.cdil; conv_ixs = cs * a.cdil_w; conv_kvalid = cr < a.KH; }
+        if constexpr (OP == 1 && !CW) conv_dy = dy < a.kh_end ? dy : 1 << 29;
     };
     auto issue_loads = [&](auto ragc, int stage, auto firstc, auto countc) {
         constexpr bool RAG = decltype(ragc)::value;
@@ -522,11 +539,15 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                     if constexpr (RAG) { if (koff_rag + chunk_of(i) >= Kb) v = OOB; }
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, ks_cur);
                 } else if constexpr (!CW) {
-                    int iy = iy0[i] + conv_iyr, ix = ix0[i] + conv_ixs;
-                    bool ok = conv_kvalid;
-                    if constexpr (EXPAND) ok = ok && unexpand(iy, ix);
-                    else ok = ok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-                    const uint32_t v = ok ? voffA[i] + (uint32_t)((iy * in_w + ix) * a.CI + cc) * ES : OOB;
+                    int iy = iy0[i] + conv_dy, ix = ix0[i] + dx;
+                    uint32_t v;
+                    if constexpr (EXPAND) {
+                        const bool ok = dy < a.kh_end && unexpand(iy, ix);
+                        v = ok ? voffA[i] + (uint32_t)((iy * in_w + ix) * a.CI + cc) * ES : OOB;
+                    } else {
+                        const bool ok = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+                        v = ok ? voffA[i] + koff : OOB;
+                    }
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, 0u);
                 }
             } else {
@@ -545,9 +566,28 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     };
     auto end_issue = [&]() {
         if constexpr (OP == 1 && !CW) {
-            // advance the lane's (kh, kw, ci) position by one k-tile
+            // advance the lane's (kh, kw, ci) position by one k-tile.  A load's address is then its row's plus koff; resolved anew for
+            // every load it took some twelve vector instructions, two of them quarter-rate multiplications, now six: fp16 3x3
+            // 9x46x49x240 -> 64 19.4 -> 17.8 us, 5x5 14x39x42x80 -> 80 24.0 -> 22.8, u8 3x3 19x26x25x352 -> 352 41.5 -> 39.4; where few
+            // k-tiles repay the longer start, fp16 3x3 21x20x432 -> 240 in 9 slices 11.6 -> 11.8, u8 3x3, stride 2, 3x48x48x72 -> 64 10.2 -> 10.5.
             cc += BKB / ES;
-            while (cc >= a.CI) { cc -= a.CI; if (++cs == a.KW) { cs = 0; ++cr; } }
+            if (a.CI >= BKB / ES) {                              // (one tap further at most)
+                const bool wrap = cc >= a.CI;
+                cc -= wrap ? a.CI : 0;
+                dx += wrap ? a.cdil_w : 0;
+                koff += BKB + (wrap ? a.tap_bytes : 0u);
+                const bool row = dx == a.kw_end;
+                dx = row ? 0 : dx;
+                dy += row ? a.cdil : 0;
+                koff += row ? a.taprow_bytes : 0u;
+            } else {
+                while (cc >= a.CI) {
+                    cc -= a.CI;
+                    dx += a.cdil_w;
+                    if (dx == a.kw_end) { dx = 0; dy += a.cdil; }
+                }
+                koff = (uint32_t)(dy * in_w + dx) * a.px + (uint32_t)cc * ES;
+            }
         }
         advance_issue();
     };
