@@ -109,7 +109,7 @@ constexpr bool SPLITK = (HRN_SPLITK != 0);
 constexpr bool COLSUM = (HRN_DTYPE == 1) && (HRN_COLSUM != 0);
 // the results leave with the non-temporal hint: C is written once and not read by this kernel, and a round's 8 MiB of it
 // per XCD would otherwise push the operand slabs of the next round out of the 4 MiB L2 (split-K partial sums go out at device scope
-// instead, whoever adds them up: the other XCDs' slices are read from memory)
+// instead, whoever adds them up: the other XCDs' slices are read from memory).  Staged results whose rows end inside lines go without it (row_lines)
 #ifndef HRN_NTSTORE
 #define HRN_NTSTORE 0
 #endif
@@ -811,13 +811,24 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         };
 
         char* Cb = (char*)a.C + ((int64_t)slice * a.batch + c_bz) * a.sC * OES;
+        using NtC = std::integral_constant<bool, NTS>;
+        // The non-temporal hint only where no line is written in pieces: rows of whole lines, or of whole half lines as long as the
+        // memory-side cache has room for the result.  Elsewhere the L2 joins the pieces that tiles side by side and the strips of a tile
+        // leave of a line.  Hint / no hint, us: rows at 16 or 32 bytes u8 x s8 4653x3384x208 34.0 / 24.5, 8190x4040x128 47.9 / 27.3, fp16
+        // 8190x8184x128 59.0 / 37.3, batch_matmul 192x512x520x64 55.2 / 25.4; half lines fp16 8190x8160x128 (134 MB) 58.5 / 43.0, batch_matmul
+        // 192x512x544x64 (107 MB) 29.5 / 27.4, 4330x6624x1120 (57 MB) 63.4 / 63.3, 3000x2336x512 15.1 / 15.7, 100x300x352x64 10.8 / 12.7, u8 conv
+        // 1x1 16x56x56x64 -> 112 7.4 / 8.3.
+        [[maybe_unused]] const uint32_t row_ends = (uint32_t)a.ldc * OES | (uint32_t)(uintptr_t)Cb;
+        [[maybe_unused]] const bool row_lines =
+            (row_ends & 127) == 0 || ((row_ends & 63) == 0 && (uint64_t)a.batch * (uint32_t)a.M * (uint32_t)a.ldc <= (64u << 20) / OES);
         [[maybe_unused]] const rsrc_t rsrcC = make_rsrc(Cb, (uint32_t)a.M * (uint32_t)a.ldc * OES);
-        [[maybe_unused]] auto put16 = [&](char* dst, v4i val) __attribute__((always_inline)) {
-            if constexpr (NTS) __builtin_nontemporal_store(val, (out16_t*)dst);
+        // (the hint only where rows of C are whole lines: see row_lines)
+        [[maybe_unused]] auto put16 = [&](auto ntc, char* dst, v4i val) __attribute__((always_inline)) {
+            if constexpr (decltype(ntc)::value) __builtin_nontemporal_store(val, (out16_t*)dst);
             else *(out16_t*)dst = val;
         };
-        [[maybe_unused]] auto put8 = [&](char* dst, long val) __attribute__((always_inline)) {
-            if constexpr (NTS) __builtin_nontemporal_store(val, (out8_t*)dst);
+        [[maybe_unused]] auto put8 = [&](auto ntc, char* dst, long val) __attribute__((always_inline)) {
+            if constexpr (decltype(ntc)::value) __builtin_nontemporal_store(val, (out8_t*)dst);
             else *(out8_t*)dst = val;
         };
         [[maybe_unused]] auto put_partial = [&](int m, int n, auto val) __attribute__((always_inline)) {
@@ -919,60 +930,70 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             constexpr int CPRW = SW * OES / 16;                // 16-byte chunks per strip row
             constexpr int EPC = 16 / OES;                      // output elements per chunk
             constexpr int TNS = TN / ESPLIT;                   // MFMA column tiles per strip
+            // (two copies of the loop and one branch: a branch per strip costs u8 x s8 1205x1392x656 6.4 -> 6.95 us)
+            auto staged = [&](auto ntc) __attribute__((always_inline)) {
+                constexpr bool NT_HINT = decltype(ntc)::value;
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {
+                for (int i = 0; i < TM; ++i) {
 #pragma unroll
-                for (int h = 0; h < ESPLIT; ++h) {
+                    for (int h = 0; h < ESPLIT; ++h) {
 #pragma unroll
-                    for (int js = 0; js < TNS; ++js) {
-                        const int j = h * TNS + js;
+                        for (int js = 0; js < TNS; ++js) {
+                            const int j = h * TNS + js;
 #pragma unroll
-                        for (int g = 0; g < ACC_N / 4; ++g) {
-                            const int cl = js * MT + g * 8 + lq_e * 4;         // column inside the strip
-                            char* dst = strip + lr_e * EPI_PITCH + cl * OES;
-                            if constexpr (DT == 0 && !SPLITK) {
-                                v4h o;
+                            for (int g = 0; g < ACC_N / 4; ++g) {
+                                const int cl = js * MT + g * 8 + lq_e * 4;         // column inside the strip
+                                char* dst = strip + lr_e * EPI_PITCH + cl * OES;
+                                if constexpr (DT == 0 && !SPLITK) {
+                                    v4h o;
 #pragma unroll
-                                for (int r = 0; r < 4; ++r) o[r] = (_Float16)acc[i][j][g * 4 + r];
-                                *(v4h*)dst = o;
-                            } else if constexpr (DT == 0) {
-                                v4f o;
+                                    for (int r = 0; r < 4; ++r) o[r] = (_Float16)acc[i][j][g * 4 + r];
+                                    *(v4h*)dst = o;
+                                } else if constexpr (DT == 0) {
+                                    v4f o;
 #pragma unroll
-                                for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r];
-                                *(v4f*)dst = o;
+                                    for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r];
+                                    *(v4f*)dst = o;
+                                } else {
+                                    const v4i bs = colsum4(wn_idx * WTN + h * SW + cl);
+                                    v4i o;
+#pragma unroll
+                                    for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r] + 128 * bs[r];
+                                    *(v4i*)dst = o;
+                                }
+                            }
+                        }
+                        asm volatile("" ::: "memory");     // LDS serves one wave's requests in order: the reads below see the writes
+#pragma unroll
+                        for (int it = 0; it < MT * CPRW / 64; ++it) {
+                            const int c = it * 64 + lane_e;
+                            const int row = c / CPRW, cc2 = c % CPRW;
+                            const v4i val = *(const v4i*)(strip + row * EPI_PITCH + cc2 * 16);
+                            const int m = m0 + wm_idx * WTM + i * MT + row;
+                            const int n = n0 + wn_idx * WTN + h * SW + cc2 * EPC;
+                            if constexpr (PERS) {
+                                // always issued, so that every wave has exactly STORES_PER_TILE stores per tile in flight
+                                const uint32_t off = (m < a.M && n + EPC <= a.N) ? (uint32_t)(m * a.ldc + n) * OES : OOB;
+                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rsrcC, (int)off, 0, NT_HINT ? 2 : 0);
+                            } else if constexpr (SPLITK) {
+                                if (m < a.M && n < a.N) put_partial(m, n, val);
                             } else {
-                                const v4i bs = colsum4(wn_idx * WTN + h * SW + cl);
-                                v4i o;
-#pragma unroll
-                                for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r] + 128 * bs[r];
-                                *(v4i*)dst = o;
+                                char* dst = Cb + ((int64_t)m * a.ldc + n) * OES;
+                                if (m < a.M) {
+                                    if (n + EPC <= a.N) put16(ntc, dst, val);
+                                    else if (OES == 2 && n + 4 <= a.N) put8(ntc, dst, (long)(((long)(uint32_t)val.y << 32) | (uint32_t)val.x));
+                                }
                             }
                         }
+                        asm volatile("" ::: "memory");
                     }
-                    asm volatile("" ::: "memory");     // LDS serves one wave's requests in order: the reads below see the writes
-#pragma unroll
-                    for (int it = 0; it < MT * CPRW / 64; ++it) {
-                        const int c = it * 64 + lane_e;
-                        const int row = c / CPRW, cc2 = c % CPRW;
-                        const v4i val = *(const v4i*)(strip + row * EPI_PITCH + cc2 * 16);
-                        const int m = m0 + wm_idx * WTM + i * MT + row;
-                        const int n = n0 + wn_idx * WTN + h * SW + cc2 * EPC;
-                        if constexpr (PERS) {
-                            // always issued, so that every wave has exactly STORES_PER_TILE stores per tile in flight
-                            const uint32_t off = (m < a.M && n + EPC <= a.N) ? (uint32_t)(m * a.ldc + n) * OES : OOB;
-                            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rsrcC, (int)off, 0, NTS ? 2 : 0);
-                        } else if constexpr (SPLITK) {
-                            if (m < a.M && n < a.N) put_partial(m, n, val);
-                        } else {
-                            char* dst = Cb + ((int64_t)m * a.ldc + n) * OES;
-                            if (m < a.M) {
-                                if (n + EPC <= a.N) put16(dst, val);
-                                else if (OES == 2 && n + 4 <= a.N) put8(dst, (long)(((long)(uint32_t)val.y << 32) | (uint32_t)val.x));
-                            }
-                        }
-                    }
-                    asm volatile("" ::: "memory");
                 }
+            };
+            if constexpr (NTS) {
+                if (row_lines) staged(TrueC{});
+                else staged(FalseC{});
+            } else {
+                staged(FalseC{});
             }
         } else {
 #pragma unroll
@@ -990,7 +1011,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                                 v4h o;
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) o[r] = (_Float16)acc[i][j][g * 4 + r];
-                                put8(dst, __builtin_bit_cast(long, o));
+                                put8(NtC{}, dst, __builtin_bit_cast(long, o));
                             } else if constexpr (DT == 0) {
                                 v4f o;
 #pragma unroll
@@ -1002,7 +1023,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) o[r] = acc[i][j][g * 4 + r] + 128 * bs[r];
                                 if constexpr (SPLITK) put_partial(m, n, o);
-                                else put16(dst, o);
+                                else put16(NtC{}, dst, o);
                             }
                         }
                     }
