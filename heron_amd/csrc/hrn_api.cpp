@@ -59,7 +59,7 @@ struct HrnKArgs {  // must match mfma_gemm_template.hip
     uint64_t* arrivals;
     uint64_t ticket;
     int32_t out_ld;
-    FastDiv by_total, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
+    FastDiv by_split, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
     int32_t kw_end, kh_end, x_row, y_img, px;
     uint32_t tap_bytes, taprow_bytes, row_bytes, img_bytes;
 };
@@ -717,7 +717,6 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     k->group_m = std::min(p->group_m > 0 ? p->group_m : 8, k->tiles_m);
     int64_t total = (int64_t)k->tiles_m * k->tiles_n * p->batch;
     if (total >= (1ll << 31)) return fail(HRN_E_BADPARAM, "grid size");
-    k->by_total = FastDiv((uint32_t)total);
     k->by_tiles = FastDiv((uint32_t)(k->tiles_m * k->tiles_n));
     k->by_group = FastDiv((uint32_t)(k->group_m * k->tiles_n));
     k->by_gm = FastDiv((uint32_t)k->group_m);
@@ -752,6 +751,7 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         if ((int64_t)p->m * p->n * 4 >= (1ll << 31)) return fail(HRN_E_BADPARAM, "split_k: one slice of C exceeds 2 GiB");
         k->C = workspace; k->ldc = p->n; k->sC = (int64_t)p->m * p->n;
         k->split = split; k->kt_per_slice = kps;
+        k->by_split = FastDiv((uint32_t)split);
         plan->split = split;
         if (split <= kMaxArrivals && (int64_t)workspace_bytes >= need + total * 8) {
             k->out = C; k->out_ld = p->ldc; k->out_stride = p->stride_c;

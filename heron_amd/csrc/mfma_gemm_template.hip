@@ -58,9 +58,9 @@ struct HrnKArgs {
     uint64_t* arrivals;                  // one word per output tile, of any content
     uint64_t ticket;                     // of this launch, its low 16 bits zero
     int32_t out_ld;
-    // divisors of the launch: output tiles, those of a batch entry, of a raster group, rows of a group and of the last one, conv: elements of
+    // divisors of the launch: K slices, output tiles of a batch entry, of a raster group, rows of a group and of the last one, conv: elements of
     // a filter row and of a tap, output pixels of an image and of a row, 16-byte pieces of a pixel, pixels of a plane (out_plane)
-    HrnDiv by_total, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
+    HrnDiv by_split, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
     // conv, im2col: extents of all taps (dilated) and of the result (times the stride) in input pixels, the bytes of a pixel, and what
     // a byte offset changes by beyond the step itself where K goes on to the next tap and filter row, the pixels to the next row and image
     int32_t kw_end, kh_end, x_row, y_img, px;
@@ -329,7 +329,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             asm volatile("" ::"s"(a.by_kwci.m), "s"(a.by_kwci.shift), "s"(a.by_ci.m), "s"(a.by_ci.shift), "s"(a.kw_end), "s"(a.kh_end), "s"(a.x_row),
                          "s"(a.y_img), "s"(a.px), "s"(a.tap_bytes), "s"(a.taprow_bytes), "s"(a.row_bytes), "s"(a.img_bytes));
         if constexpr (CW) asm volatile("" ::"s"(a.by_cpp.m), "s"(a.by_cpp.shift));
-        if constexpr (SPLITK) asm volatile("" ::"s"(a.split), "s"(a.kt_per_slice), "s"(a.by_total.m), "s"(a.by_total.shift));
+        if constexpr (SPLITK) asm volatile("" ::"s"(a.split), "s"(a.kt_per_slice), "s"(a.by_split.m), "s"(a.by_split.shift));
         if constexpr (COLSUM) asm volatile("" ::"s"(a.bsum));
     }
     const int tid = threadIdx.x;
@@ -342,13 +342,24 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     const uint32_t Kb = (uint32_t)a.K * ES;           // bytes of K
     const int KT_all = (Kb + BKB - 1) / BKB;
     int first_pid = blockIdx.x, slice = 0;
-    if constexpr (SPLITK) { slice = div_by(first_pid, a.by_total); first_pid -= slice * total; }
+    if constexpr (SPLITK) {
+        // Eighths of the (tile, slice) pairs, one per XCD: the slices of a tile count and fold where most of their partial sums were
+        // written, and tiles side by side, which read the same rows of B, come into one L2.
+        // Before, tiles went round the XCDs within each slice (eighths where 8 divides them).  Before / now, us: u8 x s8 149x1776x5056 in 3
+        // slices 11.5 / 10.0, fp16 300x900x1592 in 3 9.8 / 8.7, 540x784x864 in 2 8.0 / 7.4, 97x840x7192 in 9 12.7 / 12.3, conv 3x3
+        // 4x14x14x256 -> 256 in 4 10.3 / 9.8; where 8 divides the tiles as before.  Eighths of the slices instead: 500x500x1000 8.0 / 9.6,
+        // conv u8 3x3 8x9x9x512 -> 512 10.6 / 12.4.
+        const int all = total * a.split, xcd = blockIdx.x & 7;
+        const int pair = xcd * (all >> 3) + min(xcd, all & 7) + (int)(blockIdx.x >> 3);
+        first_pid = div_by(pair, a.by_split);
+        slice = pair - first_pid * a.split;
+    }
     const int kt0 = SPLITK ? slice * a.kt_per_slice : 0;                                   // first k-tile of this workgroup
     const int KT = SPLITK ? min(a.kt_per_slice, KT_all - kt0) : KT_all;                    // k-tiles of this workgroup
 
     // ---- tile raster: spread over the 8 XCDs so that each XCD's L2 sees a compact block ----
     auto tile_coords = [&](int pid, int& bz, int& tile_m, int& tile_n) {
-        if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+        if (!SPLITK && (total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
         bz = div_by(pid, a.by_tiles);
         const int t = pid - bz * tiles_mn;
         const int group_sz = a.group_m * a.tiles_n;

@@ -1,0 +1,44 @@
+"""Split-K launches give every XCD an eighth of the (tile, slice) pairs: each pair belongs to one workgroup, whatever the counts, and
+results are right for counts that 8 does and does not divide."""
+import pytest
+import torch
+
+from heron_amd import backend as B
+from heron_amd import hostops, instances
+
+
+def pair_of(block, pairs):
+    xcd = block & 7
+    return xcd * (pairs >> 3) + min(xcd, pairs & 7) + (block >> 3)
+
+
+@pytest.mark.parametrize("pairs", list(range(1, 40)) + [63, 64, 65, 252, 255, 256, 257, 1001])
+def test_every_pair_once(pairs):
+    assert sorted(pair_of(b, pairs) for b in range(pairs)) == list(range(pairs))
+    for xcd in range(min(8, pairs)):
+        own = [pair_of(b, pairs) for b in range(xcd, pairs, 8)]
+        assert own == list(range(own[0], own[0] + len(own)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", [0, 1, 2, 3, 6])
+@pytest.mark.parametrize("m,n", [(1, 64), (65, 68), (130, 200), (64, 512), (200, 452)])
+def test_products(which, m, n, hrn):
+    d = instances.splitk_descs()[which]
+    f16 = d.dtype == instances.F16
+    mod = B.Module(d)
+    gen = torch.Generator(device="cuda").manual_seed(m * n)
+    for split, k in ((1, 64), (2, 272), (3, 400), (7, 1040)):
+        for batch in (1, 3):
+            a, w = (batch, m, k), (batch, n, k)
+            if f16:      # sums of k products of -1, 0, 1: exact in fp16
+                A = torch.randint(-1, 2, a, device="cuda", generator=gen).half()
+                W = torch.randint(-1, 2, w, device="cuda", generator=gen).half()
+            else:
+                A = torch.randint(0, 2, a, device="cuda", generator=gen).to(torch.uint8)
+                W = torch.randint(-128, 128, w, device="cuda", generator=gen, dtype=torch.int8)
+            print("split-K raster", d.as_tuple(), (batch, m, n, k), split, flush=True)
+            C = hostops.gemm(mod, A, W, split_k=split)
+            for b in range(batch):
+                assert torch.equal(C[b].float(), A[b].float() @ W[b].float().t())
+    mod.close()
