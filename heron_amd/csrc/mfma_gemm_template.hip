@@ -318,10 +318,10 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     // every argument the start of the kernel needs, fetched at once: left to itself the compiler reads them where they are
     // used and waits for memory several times before the first load is out (1700 - 1900 cycles, 850 like this)
     if constexpr (TM * TN * ACC_N < 256) {      // (not where every register holds an accumulator)
-        asm volatile("" ::"s"(a.A), "s"(a.B), "s"(a.C), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.lda), "s"(a.ldb), "s"(a.ldc), "s"(a.sA), "s"(a.sB),
-                     "s"(a.sC), "s"(a.tiles_m), "s"(a.tiles_n), "s"(a.group_m), "s"(a.batch));
-        asm volatile("" ::"s"(a.by_tiles.m), "s"(a.by_tiles.shift), "s"(a.by_group.m), "s"(a.by_group.shift), "s"(a.by_gm.m), "s"(a.by_gm.shift),
-                     "s"(a.by_gm_last.m), "s"(a.by_gm_last.shift));
+        asm volatile("" ::"s"(a.A), "s"(a.B), "s"(a.C), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.ldb), "s"(a.ldc), "s"(a.tiles_m), "s"(a.tiles_n),
+                     "s"(a.group_m), "s"(a.by_group.m), "s"(a.by_group.shift), "s"(a.by_gm.m), "s"(a.by_gm.shift), "s"(a.by_gm_last.m),
+                     "s"(a.by_gm_last.shift));
+        if constexpr (OP == 0) asm volatile("" ::"s"(a.lda), "s"(a.sA), "s"(a.sB), "s"(a.sC), "s"(a.batch), "s"(a.by_tiles.m), "s"(a.by_tiles.shift));
         if constexpr (OP == 1)
             asm volatile("" ::"s"(a.H), "s"(a.W), "s"(a.CI), "s"(a.HO), "s"(a.WO), "s"(a.KH), "s"(a.KW), "s"(a.cstride), "s"(a.cpad), "s"(a.cdil),
                          "s"(a.cstride_w), "s"(a.cpad_w), "s"(a.cdil_w), "s"(a.by_hw.m), "s"(a.by_hw.shift), "s"(a.by_wo.m), "s"(a.by_wo.shift));
@@ -338,7 +338,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     const int wm_idx = wave / WN, wn_idx = wave % WN;
 
     const int tiles_mn = a.tiles_m * a.tiles_n;
-    const int total = tiles_mn * a.batch;             // output tiles (of one K slice)
+    const int batch = OP == 1 ? 1 : a.batch;          // (the images of a conv are rows of one product)
+    const int total = tiles_mn * batch;               // output tiles (of one K slice)
     const uint32_t Kb = (uint32_t)a.K * ES;           // bytes of K
     const int KT_all = (Kb + BKB - 1) / BKB;
     int first_pid = blockIdx.x, slice = 0;
@@ -360,7 +361,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     // ---- tile raster: spread over the 8 XCDs so that each XCD's L2 sees a compact block ----
     auto tile_coords = [&](int pid, int& bz, int& tile_m, int& tile_n) {
         if (!SPLITK && (total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
-        bz = div_by(pid, a.by_tiles);
+        bz = OP == 1 ? 0 : div_by(pid, a.by_tiles);
         const int t = pid - bz * tiles_mn;
         const int group_sz = a.group_m * a.tiles_n;
         const int gid = div_by(t, a.by_group);
@@ -821,7 +822,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             return bs;
         };
 
-        char* Cb = (char*)a.C + ((int64_t)slice * a.batch + c_bz) * a.sC * OES;
+        char* Cb = (char*)a.C + ((int64_t)slice * batch + c_bz) * a.sC * OES;
         using NtC = std::integral_constant<bool, NTS>;
         // The non-temporal hint only where no line is written in pieces: rows of whole lines, or of whole half lines as long as the
         // memory-side cache has room for the result.  Elsewhere the L2 joins the pieces that tiles side by side and the strips of a tile
@@ -831,7 +832,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         // 1x1 16x56x56x64 -> 112 7.4 / 8.3.
         [[maybe_unused]] const uint32_t row_ends = (uint32_t)a.ldc * OES | (uint32_t)(uintptr_t)Cb;
         [[maybe_unused]] const bool row_lines =
-            (row_ends & 127) == 0 || ((row_ends & 63) == 0 && (uint64_t)a.batch * (uint32_t)a.M * (uint32_t)a.ldc <= (64u << 20) / OES);
+            (row_ends & 127) == 0 || ((row_ends & 63) == 0 && (uint64_t)batch * (uint32_t)a.M * (uint32_t)a.ldc <= (64u << 20) / OES);
         [[maybe_unused]] const rsrc_t rsrcC = make_rsrc(Cb, (uint32_t)a.M * (uint32_t)a.ldc * OES);
         // (the hint only where rows of C are whole lines: see row_lines)
         [[maybe_unused]] auto put16 = [&](auto ntc, char* dst, v4i val) __attribute__((always_inline)) {
@@ -1084,7 +1085,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         const int cpr = min(BN, a.N - n0) / 4, count = min(BM, a.M - m0) * cpr;   // 16-byte pieces of the tile
         const float inv = 1.0f / (float)cpr;
         const uint32_t slice_bytes = (uint32_t)a.M * (uint32_t)a.N * 4;
-        const int64_t step = (int64_t)a.batch * a.sC * 4;
+        const int64_t step = (int64_t)batch * a.sC * 4;
         // U pieces of a lane at a time, Z slices of each on the way
         auto fold = [&](auto uc, auto zc) __attribute__((always_inline)) {
             constexpr int U = decltype(uc)::value, Z = decltype(zc)::value;
