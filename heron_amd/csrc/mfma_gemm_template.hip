@@ -1451,12 +1451,18 @@ __device__ __forceinline__ void body_if(BodyArgs a) {
     if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND, DEEP>(a);
 }
 
+// Where 256 registers are enough for a wave, the compiler is told so: it then keeps the accumulators in them and the MFMAs add in place.  Given 512,
+// it takes the other half for the accumulators and copies them from one half to the other in the k-loop (20 - 28 instructions and the
+// waits between them a k-tile of four MFMA tiles).  u8 conv 5x5 16x21x24x176 -> 288 33.0 -> 28.9 us, 3x3 4x30x30x448 -> 320 24.3 -> 20.3, fp16 3x3
+// in 4 slices 2x20x20x432 -> 240 13.2 -> 12.3.  (Deep kernels fill the LDS with one workgroup, and the compiler then goes by that.)
+constexpr int MIN_WPE = NT > 256 ? (NT + 255) / 256 : (TM * TN * ACC_N <= 128 ? 2 : 1);
+
 }  // namespace
 
 #if HRN_WPE > 0
 #define HRN_ENTRY extern "C" __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(HRN_WPE, HRN_WPE)))
 #else
-#define HRN_ENTRY extern "C" __global__ void __launch_bounds__(NT)
+#define HRN_ENTRY extern "C" __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(MIN_WPE)))
 #endif
 
 // Which kernels this code object holds: those of the instance's own launches, the channels-first ones, or those that also
