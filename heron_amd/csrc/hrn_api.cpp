@@ -98,6 +98,7 @@ struct hrn_module {
     int device;                     // the code objects are loaded on
     double timeout_s;               // of a compilation
     int deep_grid;      // workgroups of the deep kernels that the device holds at once
+    int deep_lds;       // LDS bytes of a deep kernel (of a product's: all of them dynamic)
     int persist_grid;   // persistent instances: workgroups that fit the device at once (multiple of 8 when >= 8)
     int epi_bytes;      // LDS bytes of the epilogue region (column sums + strips)
     int chw_bytes;      // the same of the channels-first epilogue
@@ -768,6 +769,7 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     const int64_t a_bytes = d.op == HRN_OP_GEMM ? (int64_t)p->m * p->k * es : (int64_t)p->cn * p->ch * p->cw * p->ci * es;
     plan->deep = deep_fits(mod, total, d.split_k ? k->kt_per_slice : (int)(((int64_t)p->k * es + d.bkb - 1) / d.bkb),
                            p->batch * (a_bytes + b_bytes));
+    if (plan->deep && d.op == HRN_OP_GEMM) plan->dyn_lds = (unsigned)mod->deep_lds;       // (DYN_LDS of the template)
     if (d.persistent) {
         if ((int64_t)p->n * oes % 16) return fail(HRN_E_BADPARAM, "persistent instances store whole 16-byte chunks: N*%d must be a multiple of 16", oes);
         if ((int64_t)p->m * p->ldc * oes >= (1ll << 31)) return fail(HRN_E_BADPARAM, "persistent: C exceeds 2 GiB per batch entry");
@@ -794,6 +796,7 @@ hrn_module* module_of(const hrn_kernel_desc* desc, const std::string& stem, doub
     m->chw_bytes = dv.chw_bytes;
     m->has_chw = dv.has_chw;
     m->has_deep = dv.has_deep;
+    m->deep_lds = dv.deep_lds;
     m->timeout_s = timeout_s;
     m->device = dev;
     m->cus = cus;

@@ -312,8 +312,10 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     constexpr int NS = DEEP ? DEEP_NS : HRN_STAGES;
     constexpr int OWN_LDS = CHW ? CHW_LDS_BYTES : LDS_BYTES;
     constexpr int KERNEL_LDS = (DEEP && NS * STAGE_BYTES > OWN_LDS) ? NS * STAGE_BYTES : OWN_LDS;
-    __shared__ __attribute__((aligned(1024))) char lds[KERNEL_LDS];
-    extern __shared__ __attribute__((aligned(1024))) char win[];   // window mode: input window, later the epilogue region
+    constexpr bool DYN_LDS = DEEP && OP == 0;
+    __shared__ __attribute__((aligned(1024))) char own_lds[DYN_LDS ? 1024 : KERNEL_LDS];
+    extern __shared__ __attribute__((aligned(1024))) char win[];   // window mode: input window, later the epilogue region; DYN_LDS: all of it
+    char* const lds = DYN_LDS ? win : own_lds;
 
     // every argument the start of the kernel needs, fetched at once: left to itself the compiler reads them where they are
     // used and waits for memory several times before the first load is out (1700 - 1900 cycles, 850 like this)
@@ -1454,7 +1456,9 @@ __device__ __forceinline__ void body_if(BodyArgs a) {
 // Where 256 registers are enough for a wave, the compiler is told so: it then keeps the accumulators in them and the MFMAs add in place.  Given 512,
 // it takes the other half for the accumulators and copies them from one half to the other in the k-loop (20 - 28 instructions and the
 // waits between them a k-tile of four MFMA tiles).  u8 conv 5x5 16x21x24x176 -> 288 33.0 -> 28.9 us, 3x3 4x30x30x448 -> 320 24.3 -> 20.3, fp16 3x3
-// in 4 slices 2x20x20x432 -> 240 13.2 -> 12.3.  (Deep kernels fill the LDS with one workgroup, and the compiler then goes by that.)
+// in 4 slices 2x20x20x432 -> 240 13.2 -> 12.3.  Deep kernels fill the LDS with one workgroup,
+// which would be reason enough for 512 registers, so those of products take their LDS dynamically: u8 x s8 1500x1536x4112 25.9 -> 23.1 us, fp16
+// 1500x1536x2048 18.2 -> 17.9.  (Those of convs gain nothing by it: 5x5 10x30x30x208 -> 128 35.4 -> 36.6, 3x3 16x28x28x256 -> 160 23.9 -> 23.5.)
 constexpr int MIN_WPE = NT > 256 ? (NT + 255) / 256 : (TM * TN * ACC_N <= 128 ? 2 : 1);
 
 }  // namespace
