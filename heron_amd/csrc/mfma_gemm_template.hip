@@ -1472,7 +1472,7 @@ __device__ __forceinline__ void body_if(BodyArgs a) {
 // in 4 slices 2x20x20x432 -> 240 13.2 -> 12.3.  Deep kernels fill the LDS with one workgroup,
 // which would be reason enough for 512 registers, so those of products take their LDS dynamically: u8 x s8 1500x1536x4112 25.9 -> 23.1 us, fp16
 // 1500x1536x2048 18.2 -> 17.9.  (Those of convs gain nothing by it: 5x5 10x30x30x208 -> 128 35.4 -> 36.6, 3x3 16x28x28x256 -> 160 23.9 -> 23.5.)
-constexpr int MIN_WPE = NT > 256 ? (NT + 255) / 256 : (TM * TN * ACC_N <= 128 ? 2 : 1);
+constexpr int MIN_WPE = NT > 256 ? (NT + 255) / 256 : (TM * TN * ACC_N + 8 * (TM + TN) <= 208 ? 2 : 1);      // (accumulators, two sets of fragments)
 
 }  // namespace
 
