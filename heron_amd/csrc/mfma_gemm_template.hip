@@ -582,8 +582,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         if constexpr (OP == 1 && !CW) {
             // advance the lane's (kh, kw, ci) position by one k-tile.  A load's address is then its row's plus koff; resolved anew for
             // every load it took some twelve vector instructions, two of them quarter-rate multiplications, now six: fp16 3x3
-            // 9x46x49x240 -> 64 19.4 -> 17.8 us, 5x5 14x39x42x80 -> 80 24.0 -> 22.8, u8 3x3 19x26x25x352 -> 352 41.5 -> 39.4; where few
-            // k-tiles repay the longer start, fp16 3x3 21x20x432 -> 240 in 9 slices 11.6 -> 11.8, u8 3x3, stride 2, 3x48x48x72 -> 64 10.2 -> 10.5.
+            // 9x46x49x240 -> 64 19.4 -> 17.8 us, 5x5 14x39x42x80 -> 80 24.0 -> 22.8, u8 3x3 19x26x25x352 -> 352 41.5 -> 39.4; calls of few k-tiles
+            // start 0.1 - 0.3 us later for it (u8 3x3, stride 2, 3x48x48x80 -> 64 6.6 -> 6.8).
             cc += BKB / ES;
             if (a.CI >= BKB / ES) {                              // (one tap further at most)
                 const bool wrap = cc >= a.CI;
@@ -846,9 +846,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             else *(out8_t*)dst = val;
         };
         // partial sums that this kernel adds up lie tile by tile (the rows of tiles one behind the other), so that a tile's are stored and
-        // read in one piece: as rows of the result, which
-        // rarely are whole lines, fp16 500x500x1000 in 4 slices took 7.8 us (7.2 like this), 97x840x7192 in 9 12.2 (11.9), 40x864x560 in 2 5.9 (5.8); where
-        // N is whole lines nothing changes.  Those for splitk_reduce_kernel are row-major.
+        // read in one piece: as rows of the result, which rarely are whole lines, fp16 500x500x1000 in 4 slices took 7.8 us (7.2 like this),
+        // 97x840x7192 in 9 12.2 (11.9), 40x864x560 in 2 5.9 (5.8); where N is whole lines nothing changes.  Those for splitk_reduce_kernel are row-major.
         [[maybe_unused]] const bool by_tile = SPLITK && a.arrivals;
         [[maybe_unused]] const int part_ld = by_tile ? min(BN, a.N - n0) : a.ldc;
         [[maybe_unused]] const int part_base = m0 * a.ldc + n0 * (by_tile ? min(BM, a.M - m0) : 1);
