@@ -30,39 +30,7 @@
 #include <type_traits>
 #include <vector>
 
-// n / d for 0 <= n < 2^31 and 1 <= d < 2^31 by a multiplication: with L = ceil(log2 d) and m = ceil(2^(31+L) / d), which fits into
-// 32 bits, n*m / 2^(31+L) exceeds n / d by less than 1 / d (Granlund and Montgomery, Division by Invariant Integers).
-struct FastDiv {
-    uint32_t m, shift;
-    FastDiv() = default;
-    explicit FastDiv(uint32_t d) : shift(d > 1 ? 32 - __builtin_clz(d - 1) : 0) { m = (uint32_t)(((1ull << (31 + shift)) + d - 1) / d); }
-    __device__ __forceinline__ uint32_t operator()(uint32_t n) const { return __umulhi(n << 1, m) >> shift; }
-};
-
-#define HRN_KARGS_DEFINED
-struct HrnKArgs {  // must match mfma_gemm_template.hip
-    const void* A;
-    const void* B;
-    void* C;
-    int32_t M, N, K;
-    int32_t lda, ldb, ldc;
-    int64_t sA, sB, sC;
-    int32_t tiles_m, tiles_n, group_m, batch;
-    int32_t H, W, CI, HO, WO, KH, KW, cstride, cpad, cdil;
-    int32_t cstride_w, cpad_w, cdil_w;
-    int32_t split, kt_per_slice;
-    const void* bsum;
-    int32_t out_plane;
-    int32_t expand_shift, in_h, in_w, top, left;
-    void* out;
-    int64_t out_stride;
-    uint64_t* arrivals;
-    uint64_t ticket;
-    int32_t out_ld;
-    FastDiv by_split, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
-    int32_t kw_end, kh_end, x_row, y_img, px;
-    uint32_t tap_bytes, taprow_bytes, row_bytes, img_bytes;
-};
+#include "hrn_args.h"
 
 // An instance's kernels lie in up to three code objects, so that a caller pays the compiler only for those it launches: a
 // 128x128 im2col conv instance takes 1.8 s for its own, 5.1 s for all.
@@ -154,17 +122,21 @@ std::string env_or(const char* name, const std::string& dflt) {
     return (v && *v) ? std::string(v) : dflt;
 }
 
-std::string kernel_source() { return env_or("HRN_KERNEL_DIR", lib_dir()) + "/mfma_gemm_template.hip"; }
-std::string cache_dir() { return env_or("HRN_CACHE_DIR", lib_dir() + "/cache"); }
-
 bool file_exists(const std::string& p) {
     struct stat st;
     return stat(p.c_str(), &st) == 0 && st.st_size > 0;
 }
 
-uint64_t fnv1a_file(const std::string& p) {
+std::string kernel_source() { return env_or("HRN_KERNEL_DIR", lib_dir()) + "/mfma_gemm_template.hip"; }
+// the header that the template includes: the one beside it, else the library's
+std::string kernel_header(const std::string& src) {
+    const std::string beside = src.substr(0, src.rfind('/')) + "/hrn_args.h";
+    return file_exists(beside) ? beside : lib_dir() + "/hrn_args.h";
+}
+std::string cache_dir() { return env_or("HRN_CACHE_DIR", lib_dir() + "/cache"); }
+
+uint64_t fnv1a_file(const std::string& p, uint64_t h = 1469598103934665603ull) {
     std::ifstream f(p, std::ios::binary);
-    uint64_t h = 1469598103934665603ull;
     char buf[4096];
     while (f) {
         f.read(buf, sizeof buf);
@@ -342,9 +314,9 @@ int run_hipcc(const std::vector<std::string>& args, const std::string& log_path,
     return HRN_OK;
 }
 
-// what the template is compiled from: its text and extra compiler flags (e.g. -D switches of the template under study)
+// what the template is compiled from: its text, its header's and extra compiler flags (e.g. -D switches of the template under study)
 uint64_t template_hash(const std::string& src, const std::string& extra) {
-    uint64_t h = fnv1a_file(src);
+    uint64_t h = fnv1a_file(kernel_header(src), fnv1a_file(src));
     for (unsigned char ch : extra) { h ^= ch; h *= 1099511628211ull; }
     return h;
 }
@@ -390,6 +362,7 @@ int compile_desc(const hrn_kernel_desc* d, int part, double timeout_s, std::stri
         std::string tok;
         while (es >> tok) args.push_back(tok);
     }
+    args.push_back("-I" + lib_dir());
     args.push_back(src);
     args.push_back("-o");
     args.push_back(co_tmp);
@@ -718,16 +691,16 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     k->group_m = std::min(p->group_m > 0 ? p->group_m : 8, k->tiles_m);
     int64_t total = (int64_t)k->tiles_m * k->tiles_n * p->batch;
     if (total >= (1ll << 31)) return fail(HRN_E_BADPARAM, "grid size");
-    k->by_tiles = FastDiv((uint32_t)(k->tiles_m * k->tiles_n));
-    k->by_group = FastDiv((uint32_t)(k->group_m * k->tiles_n));
-    k->by_gm = FastDiv((uint32_t)k->group_m);
-    k->by_gm_last = FastDiv((uint32_t)std::max(1, k->tiles_m % k->group_m));
+    k->by_tiles = HrnDiv((uint32_t)(k->tiles_m * k->tiles_n));
+    k->by_group = HrnDiv((uint32_t)(k->group_m * k->tiles_n));
+    k->by_gm = HrnDiv((uint32_t)k->group_m);
+    k->by_gm_last = HrnDiv((uint32_t)std::max(1, k->tiles_m % k->group_m));
     if (d.op == HRN_OP_CONV2D) {
-        k->by_kwci = FastDiv((uint32_t)(k->KW * k->CI));
-        k->by_ci = FastDiv((uint32_t)k->CI);
-        k->by_hw = FastDiv((uint32_t)(k->HO * k->WO));
-        k->by_wo = FastDiv((uint32_t)k->WO);
-        k->by_cpp = FastDiv((uint32_t)(k->CI * es / 16));
+        k->by_kwci = HrnDiv((uint32_t)(k->KW * k->CI));
+        k->by_ci = HrnDiv((uint32_t)k->CI);
+        k->by_hw = HrnDiv((uint32_t)(k->HO * k->WO));
+        k->by_wo = HrnDiv((uint32_t)k->WO);
+        k->by_cpp = HrnDiv((uint32_t)(k->CI * es / 16));
         k->kw_end = k->KW * k->cdil_w; k->kh_end = k->KH * k->cdil;
         k->x_row = k->WO * k->cstride_w; k->y_img = k->HO * k->cstride;
         k->px = k->CI * es;
@@ -752,7 +725,7 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         if ((int64_t)p->m * p->n * 4 >= (1ll << 31)) return fail(HRN_E_BADPARAM, "split_k: one slice of C exceeds 2 GiB");
         k->C = workspace; k->ldc = p->n; k->sC = (int64_t)p->m * p->n;
         k->split = split; k->kt_per_slice = kps;
-        k->by_split = FastDiv((uint32_t)split);
+        k->by_split = HrnDiv((uint32_t)split);
         plan->split = split;
         if (split <= kMaxArrivals && (int64_t)workspace_bytes >= need + total * 8) {
             k->out = C; k->out_ld = p->ldc; k->out_stride = p->stride_c;
@@ -1124,20 +1097,20 @@ struct GatherArgs {
     CO ext[HRN_GATHER_DIMS], live[HRN_GATHER_DIMS], dst_stride[HRN_GATHER_DIMS];
     CO dim[HRN_GATHER_DIMS], src_stride[HRN_GATHER_DIMS], add[HRN_GATHER_DIMS], div[HRN_GATHER_DIMS];
     CO mul[HRN_GATHER_DIMS][HRN_GATHER_DIMS];
-    FastDiv by_ext[HRN_GATHER_DIMS], by_div[HRN_GATHER_DIMS];           // IDX = uint32_t only
+    HrnDiv by_ext[HRN_GATHER_DIMS], by_div[HRN_GATHER_DIMS];           // IDX = uint32_t only
     GatherArgs(const hrn_gather& g, int v) : ndim(g.ndim), nsrc(g.nsrc), op(g.op) {
         for (int d = 0; d < ndim; ++d) {
             ext[d] = (CO)(d == ndim - 1 ? g.dst_dim[d] / v : g.dst_dim[d]);
             live[d] = (CO)g.dst_live[d];
             dst_stride[d] = (CO)g.dst_stride[d];
-            if (sizeof(IDX) == 4) by_ext[d] = FastDiv((uint32_t)ext[d]);
+            if (sizeof(IDX) == 4) by_ext[d] = HrnDiv((uint32_t)ext[d]);
         }
         for (int s = 0; s < nsrc; ++s) {
             dim[s] = (CO)g.src_dim[s];
             src_stride[s] = (CO)g.src_stride[s];
             add[s] = (CO)g.add[s];
             div[s] = (CO)g.div[s];
-            if (sizeof(IDX) == 4) by_div[s] = FastDiv((uint32_t)div[s]);
+            if (sizeof(IDX) == 4) by_div[s] = HrnDiv((uint32_t)div[s]);
             for (int d = 0; d < ndim; ++d) mul[s][d] = (CO)g.mul[s][d];
         }
     }
@@ -1822,7 +1795,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
     if (view->out_plane < 1 || p->m % view->out_plane)
         return fail(HRN_E_BADPARAM, "conv2d_chw: %d result pixels are not whole planes of %d", p->m, view->out_plane);
     plan.k.out_plane = view->out_plane;
-    plan.k.by_plane = FastDiv((uint32_t)view->out_plane);
+    plan.k.by_plane = HrnDiv((uint32_t)view->out_plane);
     if (mod->desc.conv_window) plan.dyn_lds = std::max(plan.dyn_lds, (unsigned)mod->chw_bytes);
     if (view->expand) {
         if (view->expand < 1 || (view->expand & (view->expand - 1)) || view->in_h < 1 || view->in_w < 1 || view->top < 0 || view->left < 0 ||

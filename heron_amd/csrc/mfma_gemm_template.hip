@@ -29,44 +29,12 @@
 #include <stdint.h>
 #include <type_traits>
 
+#include "hrn_args.h"
+
 #ifndef HRN_DTYPE
 #error "instantiate with -DHRN_DTYPE=... (see hrn_api.cpp)"
 #endif
 
-#ifndef HRN_KARGS_DEFINED
-#define HRN_KARGS_DEFINED
-struct HrnDiv { uint32_t m, shift; };    // n / d for 0 <= n < 2^31 is (2n * m >> 32) >> shift (FastDiv of hrn_api.cpp)
-struct HrnKArgs {
-    const void* A;
-    const void* B;
-    void* C;
-    int32_t M, N, K;            // K in elements
-    int32_t lda, ldb, ldc;      // elements
-    int64_t sA, sB, sC;         // batch strides, elements
-    int32_t tiles_m, tiles_n, group_m, batch;
-    // conv
-    int32_t H, W, CI, HO, WO, KH, KW, cstride, cpad, cdil;
-    int32_t cstride_w, cpad_w, cdil_w;   // conv: the width-direction values (cstride/cpad/cdil are the height ones)
-    int32_t split, kt_per_slice;         // split-K: number of K slices and k-tiles per slice
-    const void* bsum;                    // uint8 path: per batch entry N column sums of B (sum_k B[n,k], int32), or null
-    int32_t out_plane;                   // CHW kernels: row m, column n of the result goes to C[m / out_plane][n][m % out_plane]
-    int32_t expand_shift;                // EXPAND kernels: the H x W input is not in memory: pixel (y, x) of the in_h x in_w
-    int32_t in_h, in_w, top, left;       // one that is stands at (top + (y << shift), left + (x << shift)), zeros elsewhere
-    // split-K: the result and what tells the last slice of a tile to add them all up; arrivals null: a kernel behind this one does
-    void* out;
-    int64_t out_stride;                  // batch stride of the result, elements
-    uint64_t* arrivals;                  // one word per output tile, of any content
-    uint64_t ticket;                     // of this launch, its low 16 bits zero
-    int32_t out_ld;
-    // divisors of the launch: K slices, output tiles of a batch entry, of a raster group, rows of a group and of the last one, conv: elements of
-    // a filter row and of a tap, output pixels of an image and of a row, 16-byte pieces of a pixel, pixels of a plane (out_plane)
-    HrnDiv by_split, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
-    // conv, im2col: extents of all taps (dilated) and of the result (times the stride) in input pixels, the bytes of a pixel, and what
-    // a byte offset changes by beyond the step itself where K goes on to the next tap and filter row, the pixels to the next row and image
-    int32_t kw_end, kh_end, x_row, y_img, px;
-    uint32_t tap_bytes, taprow_bytes, row_bytes, img_bytes;
-};
-#endif
 
 namespace {
 
@@ -221,11 +189,7 @@ template <> struct AccT<16> { using F = v16f; using I = v16i; };
 template <> struct AccT<4> { using F = v4f; using I = v4i; };
 using acc_t = typename std::conditional<DT == 0, typename AccT<ACC_N>::F, typename AccT<ACC_N>::I>::type;
 
-// Divisions by what is fixed for a launch, by multiplication.  A division proper is some 30 instructions, and a kernel starts with four
-// (GEMM) to eight of them, each waiting for the one before, in front of its first load: 194 instructions to it instead of 127 (u8 64x128
-// tiles), 435 instead of 283 (fp16 im2col 128x128).  fp16 3x3 32x56x56x64 -> 64 13.67 -> 13.24 us, transposed conv 16x56x56x64 -> 128
-// 24.1 -> 23.0, fp16 batch_matmul 192x512x512x64 21.2 -> 20.8, u8 x s8 1111x1500x2064 11.5 -> 11.4; u8 1972x408x2672 10.1 -> 10.3.
-__device__ __forceinline__ int div_by(int n, HrnDiv d) { return (int)(__umulhi((uint32_t)n << 1, d.m) >> d.shift); }
+__device__ __forceinline__ int div_by(int n, HrnDiv d) { return (int)d((uint32_t)n); }
 
 __device__ __forceinline__ int swz_of_row(int row) {
     if (SWZ == 0) return 0;
@@ -352,8 +316,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         // slices 11.5 / 10.0, fp16 300x900x1592 in 3 9.8 / 8.7, 540x784x864 in 2 8.0 / 7.4, 97x840x7192 in 9 12.7 / 12.3, conv 3x3
         // 4x14x14x256 -> 256 in 4 10.3 / 9.8; where 8 divides the tiles as before.  Eighths of the slices instead: 500x500x1000 8.0 / 9.6,
         // conv u8 3x3 8x9x9x512 -> 512 10.6 / 12.4.
-        const int all = total * a.split, xcd = blockIdx.x & 7;
-        const int pair = xcd * (all >> 3) + min(xcd, all & 7) + (int)(blockIdx.x >> 3);
+        const int pair = hrn_pair_of((int)blockIdx.x, total * a.split);
         first_pid = div_by(pair, a.by_split);
         slice = pair - first_pid * a.split;
     }

@@ -5,15 +5,12 @@ import torch
 
 from heron_amd import backend as B
 from heron_amd import hostops, instances
-
-
-def pair_of(block, pairs):
-    xcd = block & 7
-    return xcd * (pairs >> 3) + min(xcd, pairs & 7) + (block >> 3)
+from launch_args import library
 
 
 @pytest.mark.parametrize("pairs", list(range(1, 40)) + [63, 64, 65, 252, 255, 256, 257, 1001])
 def test_every_pair_once(pairs):
+    pair_of = library().pair_of
     assert sorted(pair_of(b, pairs) for b in range(pairs)) == list(range(pairs))
     for xcd in range(min(8, pairs)):
         own = [pair_of(b, pairs) for b in range(xcd, pairs, 8)]
