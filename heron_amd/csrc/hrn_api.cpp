@@ -625,6 +625,9 @@ int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw) {
     return pick;
 }
 
+// rows of a tile that one load of every wave covers
+int load_rows(const hrn_kernel_desc& d) { return d.wm * d.wn * 1024 / d.bkb; }
+
 int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
               size_t workspace_bytes, LaunchPlan* plan) {
     HrnKArgs* k = &plan->k;
@@ -701,14 +704,7 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         k->by_hw = HrnDiv((uint32_t)(k->HO * k->WO));
         k->by_wo = HrnDiv((uint32_t)k->WO);
         k->by_cpp = HrnDiv((uint32_t)(k->CI * es / 16));
-        k->kw_end = k->KW * k->cdil_w; k->kh_end = k->KH * k->cdil;
-        k->x_row = k->WO * k->cstride_w; k->y_img = k->HO * k->cstride;
-        k->px = k->CI * es;
-        const uint32_t px = (uint32_t)k->px, W = (uint32_t)k->W;               // (modulo 2^32, as the kernel adds them)
-        k->tap_bytes = ((uint32_t)k->cdil_w - 1u) * px;
-        k->taprow_bytes = ((uint32_t)k->cdil * W - (uint32_t)k->kw_end) * px;
-        k->row_bytes = ((uint32_t)k->cstride * W - (uint32_t)k->x_row) * px;
-        k->img_bytes = ((uint32_t)k->H - (uint32_t)k->y_img) * W * px;
+        hrn_walk_args(k, es, load_rows(d), false);
     }
     plan->C = C; plan->ldc = p->ldc; plan->stride_c = p->stride_c;
     if (d.split_k) {
@@ -1805,7 +1801,7 @@ int hrn_launch_conv2d_chw(const hrn_module* mod, const hrn_problem* p, const hrn
         plan.k.in_h = view->in_h; plan.k.in_w = view->in_w;
         plan.k.top = view->top; plan.k.left = view->left;
         plan.k.expand_shift = __builtin_ctz((unsigned)view->expand);
-        plan.k.img_bytes = (uint32_t)view->in_h * (uint32_t)view->in_w * (uint32_t)plan.k.px;
+        hrn_walk_args(&plan.k, mod->desc.dtype == HRN_DT_F16 ? 2 : 1, load_rows(mod->desc), true);
     }
     const CodeObject* kernels;
     rc = chw_kernels(mod, part, &kernels);

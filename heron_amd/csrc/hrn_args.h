@@ -53,10 +53,13 @@ struct HrnKArgs {
     // divisors of the launch: K slices, output tiles of a batch entry, of a raster group, rows of a group and of the last one, conv: elements of
     // a filter row and of a tap, output pixels of an image and of a row, 16-byte pieces of a pixel, pixels of a plane (out_plane)
     HrnDiv by_split, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
-    // conv, im2col: extents of all taps (dilated) and of the result (times the stride) in input pixels, the bytes of a pixel, and what
-    // a byte offset changes by beyond the step itself where K goes on to the next tap and filter row, the pixels to the next row and image
-    int32_t kw_end, kh_end, x_row, y_img, px;
-    uint32_t tap_bytes, taprow_bytes, row_bytes, img_bytes;
+    // conv, im2col (hrn_walk_args): the bytes of a pixel; the width of all taps; whether taps are carried along K (CI, or 0); what a byte offset changes by, beyond the step itself, where K goes on to the next
+    // tap and filter row; the step from one row of A that a lane loads to the next in output pixels, input pixels and bytes, and what
+    // changes where it leaves a row or an image of the result.  Modulo 2^32, as the kernel adds them: pads, strides and dilations
+    // may be of any size, and only what lies inside an image is used.
+    uint32_t px, kw_end, tap_bytes, taprow_bytes;
+    int32_t carry_ci;
+    uint32_t d_ox, d_oy, x_step, y_step, off_step, x_row, row_bytes, y_img, img_bytes;
 };
 
 // The (output tile, K slice) pair of a split-K workgroup, slices fastest: workgroup i runs on XCD i % 8, and each XCD has an eighth of
@@ -64,6 +67,106 @@ struct HrnKArgs {
 HRN_BOTH int hrn_pair_of(int block, int pairs) {
     const int xcd = block & 7, more = pairs & 7;
     return xcd * (pairs >> 3) + (xcd < more ? xcd : more) + (block >> 3);
+}
+
+// What the walks below need of a launch whose conv fields are set; `rows`: output pixels from one load of a lane to its next.
+// expanded: the input in memory is the in_h x in_w one.
+inline void hrn_walk_args(HrnKArgs* k, int es, int rows, bool expanded) {
+    const uint32_t px = (uint32_t)k->CI * es, H = k->H, W = k->W, sh = k->cstride, sw = k->cstride_w, hw = (uint32_t)k->HO * k->WO;
+    const uint32_t images = rows / hw, rest = rows % hw;
+    k->px = px;
+    k->tap_bytes = ((uint32_t)k->cdil_w - 1u) * px;
+    k->kw_end = (uint32_t)k->KW * k->cdil_w;
+    k->carry_ci = (uint64_t)k->KW * k->cdil_w >> 32 ? 0 : k->CI;      // (then no other tap of a row is where the row ends)
+    k->taprow_bytes = ((uint32_t)k->cdil * W - k->kw_end) * px;
+    k->d_oy = rest / k->WO; k->d_ox = rest % k->WO;
+    k->x_step = k->d_ox * sw; k->y_step = k->d_oy * sh;
+    k->x_row = k->WO * sw; k->y_img = k->HO * sh;
+    k->row_bytes = (sh * W - k->x_row) * px;
+    if (expanded) {
+        k->img_bytes = (uint32_t)k->in_h * k->in_w * px;
+        k->off_step = images * k->img_bytes;
+    } else {
+        k->img_bytes = (H - k->y_img) * W * px;
+        k->off_step = ((images * H + k->y_step) * W + k->x_step) * px;
+    }
+}
+
+// Where a row of A begins: the output pixel, the input position of tap (0, 0), which may lie in the padding, and its byte offset
+// modulo 2^32 (EXPAND: that of the image).  Rows follow one another by carry: each sum is less than twice its modulus.
+struct HrnRow {
+    uint32_t oy, ox;
+    int32_t y, x;
+    uint32_t off;
+};
+
+template <bool EXPAND>
+HRN_BOTH HrnRow hrn_row_at(const HrnKArgs& a, int m) {
+    HrnRow r;
+    const uint32_t img = a.by_hw((uint32_t)m), rem = (uint32_t)m - img * ((uint32_t)a.HO * a.WO);
+    r.oy = a.by_wo(rem);
+    r.ox = rem - r.oy * a.WO;
+    r.y = (int)(r.oy * a.cstride - a.cpad);
+    r.x = (int)(r.ox * a.cstride_w - a.cpad_w);
+    r.off = EXPAND ? img * a.img_bytes : ((img * a.H + (uint32_t)r.y) * a.W + (uint32_t)r.x) * a.px;
+    return r;
+}
+
+template <bool EXPAND>
+HRN_BOTH void hrn_next_row(const HrnKArgs& a, HrnRow& r) {
+    r.ox += a.d_ox;
+    r.oy += a.d_oy;
+    r.x = (int)((uint32_t)r.x + a.x_step);
+    r.y = (int)((uint32_t)r.y + a.y_step);
+    r.off += a.off_step;
+    const bool row = r.ox >= (uint32_t)a.WO;
+    r.ox -= row ? a.WO : 0;
+    r.oy += row ? 1 : 0;
+    r.x = (int)((uint32_t)r.x - (row ? a.x_row : 0u));
+    r.y = (int)((uint32_t)r.y + (row ? a.cstride : 0));
+    if (!EXPAND) r.off += row ? a.row_bytes : 0u;
+    const bool image = r.oy >= (uint32_t)a.HO;
+    r.oy -= image ? a.HO : 0;
+    r.y = (int)((uint32_t)r.y - (image ? a.y_img : 0u));
+    r.off += image ? a.img_bytes : 0u;
+}
+
+// Where a lane's chunk is in K: its channel, its tap in input pixels from tap (0, 0), and that and the channel as a byte offset
+// modulo 2^32.  Past the end of K it means nothing.
+struct HrnTap {
+    int32_t c, dy, dx;
+    uint32_t off;
+};
+
+HRN_BOTH HrnTap hrn_tap_at(const HrnKArgs& a, int ke, int in_w, int es) {
+    HrnTap t;
+    const int r = (int)a.by_kwci((uint32_t)ke);
+    ke -= r * (a.KW * a.CI);
+    const int s = (int)a.by_ci((uint32_t)ke);
+    t.c = ke - s * a.CI;
+    t.dy = (int)((uint32_t)r * a.cdil);
+    t.dx = (int)((uint32_t)s * a.cdil_w);
+    t.off = ((uint32_t)t.dy * in_w + (uint32_t)t.dx) * a.px + (uint32_t)t.c * es;
+    return t;
+}
+
+// ELEMS further along K, to element ke.  Carried where a step goes one tap further at most and a filter row's end shows in dx; a count of the
+// taps instead costs 2 - 12 % (fp16 3x3 32x7x7x512 -> 512 27.7 us, 31.0 with the count).
+template <int ELEMS, int ES>
+HRN_BOTH void hrn_next_tap(const HrnKArgs& a, HrnTap& t, int ke, int in_w) {
+    if (a.carry_ci >= ELEMS) {
+        t.c += ELEMS;
+        const bool tap = t.c >= a.CI;
+        t.c -= tap ? a.CI : 0;
+        t.dx = (int)((uint32_t)t.dx + (tap ? a.cdil_w : 0));
+        t.off += ELEMS * ES + (tap ? a.tap_bytes : 0u);
+        const bool row = (uint32_t)t.dx == a.kw_end;
+        t.dx = row ? 0 : t.dx;
+        t.dy = (int)((uint32_t)t.dy + (row ? a.cdil : 0));
+        t.off += row ? a.taprow_bytes : 0u;
+    } else {
+        t = hrn_tap_at(a, ke, in_w, ES);
+    }
 }
 
 #endif

@@ -292,8 +292,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             asm volatile("" ::"s"(a.H), "s"(a.W), "s"(a.CI), "s"(a.HO), "s"(a.WO), "s"(a.KH), "s"(a.KW), "s"(a.cstride), "s"(a.cpad), "s"(a.cdil),
                          "s"(a.cstride_w), "s"(a.cpad_w), "s"(a.cdil_w), "s"(a.by_hw.m), "s"(a.by_hw.shift), "s"(a.by_wo.m), "s"(a.by_wo.shift));
         if constexpr (OP == 1 && !CW)
-            asm volatile("" ::"s"(a.by_kwci.m), "s"(a.by_kwci.shift), "s"(a.by_ci.m), "s"(a.by_ci.shift), "s"(a.kw_end), "s"(a.kh_end), "s"(a.x_row),
-                         "s"(a.y_img), "s"(a.px), "s"(a.tap_bytes), "s"(a.taprow_bytes), "s"(a.row_bytes), "s"(a.img_bytes));
+            asm volatile("" ::"s"(a.by_kwci.m), "s"(a.by_kwci.shift), "s"(a.by_ci.m), "s"(a.by_ci.shift), "s"(a.px), "s"(a.kw_end), "s"(a.tap_bytes),
+                         "s"(a.taprow_bytes), "s"(a.carry_ci), "s"(a.d_ox), "s"(a.d_oy), "s"(a.x_step), "s"(a.y_step), "s"(a.off_step), "s"(a.x_row), "s"(a.row_bytes),
+                         "s"(a.y_img), "s"(a.img_bytes));
         if constexpr (CW) asm volatile("" ::"s"(a.by_cpp.m), "s"(a.by_cpp.shift));
         if constexpr (SPLITK) asm volatile("" ::"s"(a.split), "s"(a.kt_per_slice), "s"(a.by_split.m), "s"(a.by_split.shift));
         if constexpr (COLSUM) asm volatile("" ::"s"(a.bsum));
@@ -393,9 +394,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     // GEMM: byte offset of the lane's chunk in k-tile 0.  Conv: pixel bookkeeping.
     uint32_t voffA[(A_LPW > 0 ? A_LPW : 1)];
     int iy0[OP == 1 ? (A_LPW > 0 ? A_LPW : 1) : 1], ix0[OP == 1 ? (A_LPW > 0 ? A_LPW : 1) : 1];
-    // conv: where the lane's chunk is in K: its channel, its tap in pixels from tap (0, 0), and (koff) that as a byte offset
-    int cc = 0, dx = 0, dy = 0;
-    uint32_t koff = 0;
+    HrnTap tap = {};             // conv: where the lane's chunk is in K
     int itile = first_pid;
     int issue_kt = 0;            // next k-tile (relative to kt0) of tile `itile` to fetch
 
@@ -427,34 +426,17 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
             static_assert(OP == 0 || CW || SWZ == 0 || ((NW * RPI) % (CPR << (SWZ > 0 ? SWZ - 1 : 0))) == 0,
                           "conv: the lane's chunk column must not depend on the load index");
             const int chunk = lpos ^ swz_of_row(wave * RPI + lrow);
-            int ke = chunk * (16 / ES) + kt0 * (BKB / ES);      // element index inside K of this workgroup's first k-tile
-            const int r = div_by(ke, a.by_kwci); ke -= r * (a.KW * a.CI);
-            const int s = div_by(ke, a.by_ci); cc = ke - s * a.CI;
-            dy = r * a.cdil; dx = s * a.cdil_w;
-            koff = (uint32_t)(dy * in_w + dx) * a.px + (uint32_t)cc * ES;
-            // input position (y, x) of tap (0, 0) of the lane's first row by division, of the following rows (NW*RPI output pixels
-            // further each) by carry; its byte offset `off` with it, modulo 2^32: the position may lie in the padding
+            tap = hrn_tap_at(a, chunk * (16 / ES) + kt0 * (BKB / ES), in_w, ES);      // of this workgroup's first k-tile
+            // the lane's first row by division, the following ones (NW*RPI output pixels further each) by carry
             int m = im0 + wave * RPI + lrow;
-            const int img = div_by(m, a.by_hw);
-            const int rem = m - img * (a.HO * a.WO);
-            const int oy = div_by(rem, a.by_wo);
-            int y = oy * a.cstride - a.cpad, x = (rem - oy * a.WO) * a.cstride_w - a.cpad_w;
-            uint32_t off = EXPAND ? (uint32_t)img * a.img_bytes : ((uint32_t)((img * in_h + y) * in_w) + (uint32_t)x) * (uint32_t)a.px;
-            const int x_step = NW * RPI * a.cstride_w, x_end = a.x_row - a.cpad_w, y_end = a.y_img - a.cpad;
+            HrnRow row = hrn_row_at<EXPAND>(a, m);
 #pragma unroll
             for (int i = 0; i < A_LPW; ++i) {
-                iy0[i] = (m < a.M) ? y : -(1 << 28);
-                ix0[i] = x;
-                voffA[i] = off;
+                iy0[i] = (m < a.M) ? row.y : -(1 << 28);
+                ix0[i] = row.x;
+                voffA[i] = row.off;
                 m += NW * RPI;
-                x += x_step;
-                if constexpr (!EXPAND) off += (uint32_t)(x_step * a.px);
-                while (x >= x_end) {
-                    x -= a.x_row;
-                    y += a.cstride;
-                    if constexpr (!EXPAND) off += a.row_bytes;
-                    if (y >= y_end) { y -= a.y_img; off += a.img_bytes; }
-                }
+                if (i + 1 < A_LPW) hrn_next_row<EXPAND>(a, row);
             }
         }
     };
@@ -492,9 +474,24 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         ks_cur = live ? koff_cur : 0u;
         return live && koff_cur + BKB > Kb;                                      // ragged: the last tile is not full
     };
-    [[maybe_unused]] int conv_dy = 0;            // past the last tap: below every image
-    auto conv_tap = [&]() {
-        if constexpr (OP == 1 && !CW) conv_dy = dy < a.kh_end ? dy : 1 << 29;
+    // conv: the byte offsets of the next k-tile's loads of A.  Made in front of the barrier that lets the loads go: left to itself the compiler
+    // makes all but the first between the loads (fp16 3x3 9x46x49x240 -> 64 18.5 us, 18.2 like this, stride 2 16x28x28x96 -> 144 8.1 and 8.0, u8 3x3
+    // 4x30x30x448 -> 320 19.7 and 19.3).
+    [[maybe_unused]] uint32_t addr[(A_LPW > 0 ? A_LPW : 1)];
+    auto conv_addresses = [&]() __attribute__((always_inline)) {
+        if constexpr (OP == 1 && !CW) {
+#pragma unroll
+            for (int i = 0; i < A_LPW; ++i) {
+                int iy = iy0[i] + tap.dy, ix = ix0[i] + tap.dx;
+                if constexpr (EXPAND) {
+                    addr[i] = unexpand(iy, ix) ? voffA[i] + (uint32_t)((iy * in_w + ix) * a.CI + tap.c) * ES : OOB;
+                } else {
+                    const bool ok = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+                    addr[i] = ok ? voffA[i] + tap.off : OOB;
+                }
+                asm volatile("" : "+v"(addr[i]));
+            }
+        }
     };
     auto issue_loads = [&](auto ragc, int stage, auto firstc, auto countc) {
         constexpr bool RAG = decltype(ragc)::value;
@@ -516,15 +513,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                     if constexpr (RAG) { if (koff_rag + chunk_of(i) >= Kb) v = OOB; }
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, ks_cur);
                 } else if constexpr (!CW) {
-                    int iy = iy0[i] + conv_dy, ix = ix0[i] + dx;
-                    uint32_t v;
-                    if constexpr (EXPAND) {
-                        const bool ok = dy < a.kh_end && unexpand(iy, ix);
-                        v = ok ? voffA[i] + (uint32_t)((iy * in_w + ix) * a.CI + cc) * ES : OOB;
-                    } else {
-                        const bool ok = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-                        v = ok ? voffA[i] + koff : OOB;
-                    }
+                    uint32_t v = addr[i];
+                    if constexpr (RAG) { if (koff_rag + lane_chunk >= Kb) v = OOB; }      // (past the last tap)
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, 0u);
                 }
             } else {
@@ -543,28 +533,9 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     };
     auto end_issue = [&]() {
         if constexpr (OP == 1 && !CW) {
-            // advance the lane's (kh, kw, ci) position by one k-tile.  A load's address is then its row's plus koff; resolved anew for
-            // every load it took some twelve vector instructions, two of them quarter-rate multiplications, now six: fp16 3x3
-            // 9x46x49x240 -> 64 19.4 -> 17.8 us, 5x5 14x39x42x80 -> 80 24.0 -> 22.8, u8 3x3 19x26x25x352 -> 352 41.5 -> 39.4; calls of few k-tiles
-            // start 0.1 - 0.3 us later for it (u8 3x3, stride 2, 3x48x48x80 -> 64 6.6 -> 6.8).
-            cc += BKB / ES;
-            if (a.CI >= BKB / ES) {                              // (one tap further at most)
-                const bool wrap = cc >= a.CI;
-                cc -= wrap ? a.CI : 0;
-                dx += wrap ? a.cdil_w : 0;
-                koff += BKB + (wrap ? a.tap_bytes : 0u);
-                const bool row = dx == a.kw_end;
-                dx = row ? 0 : dx;
-                dy += row ? a.cdil : 0;
-                koff += row ? a.taprow_bytes : 0u;
-            } else {
-                while (cc >= a.CI) {
-                    cc -= a.CI;
-                    dx += a.cdil_w;
-                    if (dx == a.kw_end) { dx = 0; dy += a.cdil; }
-                }
-                koff = (uint32_t)(dy * in_w + dx) * a.px + (uint32_t)cc * ES;
-            }
+            // advance the lane's (kh, kw, ci) position by one k-tile.  A load's address is then its row's plus the tap's; resolved anew for
+            // every load it took some twelve vector instructions, two of them quarter-rate multiplications, now six.
+            hrn_next_tap<BKB / ES, ES>(a, tap, (int)(koff_cur + BKB + lane_chunk) / ES, in_w);
         }
         advance_issue();
     };
@@ -572,7 +543,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     using FalseC = std::integral_constant<bool, false>;
     auto issue_tile = [&](int stage) {          // the whole tile at once (prologue)
         const bool rag = begin_issue();
-        conv_tap();
+        conv_addresses();
         if (rag) issue_loads(TrueC{}, stage, std::integral_constant<int, 0>{}, std::integral_constant<int, LPT>{});
         else issue_loads(FalseC{}, stage, std::integral_constant<int, 0>{}, std::integral_constant<int, LPT>{});
         end_issue();
@@ -1196,6 +1167,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
         for (int kk = 0; kk < KS; ++kk) {
             const int cur = (kk + P) & 1;
             if (kk == KS - 1) {
+                conv_addresses();
                 // every fragment of tile kt is in registers: publish tile kt+1, recycle this stage
                 if constexpr (PERS) {
                     if (stores_between && kt <= NS - 2) wait_and_barrier<(NS - 2) * LPT + STORES_PER_TILE, 0>();
@@ -1204,8 +1176,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
                     wait_and_barrier<(NS - 2) * LPT, 0>();
                 }
                 const bool rag = begin_issue();
-                conv_tap();
-                advance_reader();
+                        advance_reader();
                 kstep(TrueC{}, mayragc, rag, cur, next_stage * STAGE_BYTES, 0, kt, kt * KS + kk);
                 end_issue();
             } else {
