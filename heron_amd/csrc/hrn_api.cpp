@@ -465,7 +465,7 @@ void read_info(const std::string& path, hrn_kernel_info* o) {
 
 // What one launch consists of: the template kernel and, for a split-K instance, the pass that adds the K slices.
 struct LaunchPlan {
-    HrnKArgs k;
+    HrnConvArgs k;             // (of a product's launch: the HrnKArgs in front)
     bool deep;                 // the deep kernel of the instance
     hipFunction_t fn;
     unsigned grid, dyn_lds;
@@ -604,7 +604,7 @@ bool same_sizes(const hrn_problem& a, const hrn_problem& b) {
                                      a.cpad_w == b.cpad_w && a.cdil_w == b.cdil_w);
 }
 
-// which of the instance's tiles a launch that fill_args takes may take: -1 its own.  On the problem an instance was searched for its tile
+// which of the instance's tiles a launch that check_args takes may take: -1 its own.  On the problem an instance was searched for its tile
 // is the one that was timed against others.  Six records would be changed by the rules below (fp16 convs, own tile / the other, us):
 // ResNet-50 28x28x128 9.1 / 9.4, 14x14x256 11.3 / 11.6, InceptionV3 35x35x192 4.7 / 4.9, 17x17x768 6.9 / 6.6, 8x8x1280 8.0 / 8.0, and
 // 32x56x56x64 14.1 / 13.7.
@@ -628,9 +628,9 @@ int fitting_tiles(const hrn_module* m, const hrn_problem* p, bool chw) {
 // rows of a tile that one load of every wave covers
 int load_rows(const hrn_kernel_desc& d) { return d.wm * d.wn * 1024 / d.bkb; }
 
-int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
+int check_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
               size_t workspace_bytes, LaunchPlan* plan) {
-    HrnKArgs* k = &plan->k;
+    HrnConvArgs* k = &plan->k;
     plan->dyn_lds = 0;
     plan->split = 1;
     plan->deep = false;
@@ -639,7 +639,7 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     if (p->op != d.op) return fail(HRN_E_BADPARAM, "problem op %d does not match module op %d", p->op, d.op);
     const int es = d.dtype == HRN_DT_F16 ? 2 : 1;
     const int oes = d.dtype == HRN_DT_F16 ? 2 : 4;     // bytes of an element of the caller's C
-    memset(k, 0, sizeof *k);
+    memset(k, 0, d.op == HRN_OP_GEMM ? sizeof(HrnKArgs) : sizeof(HrnConvArgs));
     k->A = A; k->B = B; k->C = C;
     if (p->m <= 0 || p->n <= 0 || p->k <= 0 || p->batch <= 0) return fail(HRN_E_BADPARAM, "empty problem");
     if ((int64_t)p->k * es % 16) return fail(HRN_E_BADPARAM, "K*%d must be a multiple of 16 bytes", es);
@@ -694,18 +694,6 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
     k->group_m = std::min(p->group_m > 0 ? p->group_m : 8, k->tiles_m);
     int64_t total = (int64_t)k->tiles_m * k->tiles_n * p->batch;
     if (total >= (1ll << 31)) return fail(HRN_E_BADPARAM, "grid size");
-    k->by_tiles = HrnDiv((uint32_t)(k->tiles_m * k->tiles_n));
-    k->by_group = HrnDiv((uint32_t)(k->group_m * k->tiles_n));
-    k->by_gm = HrnDiv((uint32_t)k->group_m);
-    k->by_gm_last = HrnDiv((uint32_t)std::max(1, k->tiles_m % k->group_m));
-    if (d.op == HRN_OP_CONV2D) {
-        k->by_kwci = HrnDiv((uint32_t)(k->KW * k->CI));
-        k->by_ci = HrnDiv((uint32_t)k->CI);
-        k->by_hw = HrnDiv((uint32_t)(k->HO * k->WO));
-        k->by_wo = HrnDiv((uint32_t)k->WO);
-        k->by_cpp = HrnDiv((uint32_t)(k->CI * es / 16));
-        hrn_walk_args(k, es, load_rows(d), false);
-    }
     plan->C = C; plan->ldc = p->ldc; plan->stride_c = p->stride_c;
     if (d.split_k) {
         // the kernel writes raw partial sums, slice by slice, into the workspace; its last slices write C, or the reduction kernel
@@ -721,7 +709,6 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         if ((int64_t)p->m * p->n * 4 >= (1ll << 31)) return fail(HRN_E_BADPARAM, "split_k: one slice of C exceeds 2 GiB");
         k->C = workspace; k->ldc = p->n; k->sC = (int64_t)p->m * p->n;
         k->split = split; k->kt_per_slice = kps;
-        k->by_split = HrnDiv((uint32_t)split);
         plan->split = split;
         if (split <= kMaxArrivals && (int64_t)workspace_bytes >= need + total * 8) {
             k->out = C; k->out_ld = p->ldc; k->out_stride = p->stride_c;
@@ -751,6 +738,32 @@ int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const 
         plan->grid = (unsigned)g;
     }
     return HRN_OK;
+}
+
+// What the kernels divide by and step by, of the kernel that a launch takes.  (A 64-bit division each, so not in check_args, which a launch
+// that takes another tile of its instance calls twice.)
+void derived_args(const hrn_kernel_desc& d, HrnConvArgs* k) {
+    k->by_tiles = HrnDiv((uint32_t)(k->tiles_m * k->tiles_n));
+    k->by_group = HrnDiv((uint32_t)(k->group_m * k->tiles_n));
+    k->by_gm = HrnDiv((uint32_t)k->group_m);
+    k->by_gm_last = HrnDiv((uint32_t)std::max(1, k->tiles_m % k->group_m));
+    if (d.split_k) k->by_split = HrnDiv((uint32_t)k->split);
+    if (d.op == HRN_OP_CONV2D) {
+        const int es = d.dtype == HRN_DT_F16 ? 2 : 1;
+        k->by_kwci = HrnDiv((uint32_t)(k->KW * k->CI));
+        k->by_ci = HrnDiv((uint32_t)k->CI);
+        k->by_hw = HrnDiv((uint32_t)(k->HO * k->WO));
+        k->by_wo = HrnDiv((uint32_t)k->WO);
+        k->by_cpp = HrnDiv((uint32_t)(k->CI * es / 16));
+        hrn_walk_args(k, es, load_rows(d), false);
+    }
+}
+
+int fill_args(const hrn_module* mod, const hrn_problem* p, const void* A, const void* B, void* C, void* workspace,
+              size_t workspace_bytes, LaunchPlan* plan) {
+    const int rc = check_args(mod, p, A, B, C, workspace, workspace_bytes, plan);
+    if (rc == HRN_OK) derived_args(mod->desc, &plan->k);
+    return rc;
 }
 
 // A module of `desc` with nothing loaded yet, whose code objects lie at `stem`: the main one is there.
@@ -816,21 +829,23 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const void* __restri
 int plan_launch(const hrn_module** mod, const hrn_problem* p, const void* A, const void* B, void* C, LaunchPlan* plan, int part, bool load) {
     void* ws = p ? p->workspace : nullptr;
     const size_t ws_bytes = p ? p->workspace_bytes : 0;
-    int rc = fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);          // (the instance says what is refused)
+    int rc = check_args(*mod, p, A, B, C, ws, ws_bytes, plan);          // (the instance says what is refused)
     if (rc) return rc;
     const int i = fitting_tiles(*mod, p, part != PART_MAIN);
     const hrn_module* f = i < 0 ? nullptr : (*mod)->fit[i];
     if (f && tile_kernels(f, part, load)) {
         const std::string keep = g_err;
-        if (fill_args(f, p, A, B, C, ws, ws_bytes, plan) == HRN_OK) {
+        if (check_args(f, p, A, B, C, ws, ws_bytes, plan) == HRN_OK) {
             *mod = f;
         } else {
             g_err = keep;
-            rc = fill_args(*mod, p, A, B, C, ws, ws_bytes, plan);
+            rc = check_args(*mod, p, A, B, C, ws, ws_bytes, plan);
         }
     }
+    if (rc) return rc;
+    derived_args((*mod)->desc, &plan->k);
     if (load && part == PART_MAIN) plan->fn = (*mod)->part[part].fn[plan->deep];
-    return rc;
+    return HRN_OK;
 }
 
 // The plan of a launch that is not made: the operands' addresses decide nothing, and what a launch would have to bring is filled in.
@@ -851,7 +866,7 @@ int launch_plan_only(const hrn_module** mod, const hrn_problem* p, LaunchPlan* p
 }
 
 int run_plan(const hrn_module* mod, const hrn_problem* p, const LaunchPlan& plan, void* workspace, hipStream_t st) {
-    size_t sz = sizeof plan.k;
+    size_t sz = mod->desc.op == HRN_OP_GEMM ? sizeof(HrnKArgs) : sizeof(HrnConvArgs);
     void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void*)&plan.k, HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz, HIP_LAUNCH_PARAM_END};
     HIP_TRY(hipModuleLaunchKernel(plan.fn, plan.grid, 1, 1, (unsigned)mod->info.threads, 1, 1, plan.dyn_lds, st, nullptr, extra));
     if (mod->desc.split_k && !plan.k.arrivals) {

@@ -28,6 +28,7 @@ struct HrnDiv {
     }
 };
 
+// What every launch hands over, and all of it for a product
 struct HrnKArgs {
     const void* A;
     const void* B;
@@ -36,27 +37,32 @@ struct HrnKArgs {
     int32_t lda, ldb, ldc;      // elements
     int64_t sA, sB, sC;         // batch strides, elements
     int32_t tiles_m, tiles_n, group_m, batch;
-    // conv
-    int32_t H, W, CI, HO, WO, KH, KW, cstride, cpad, cdil;
-    int32_t cstride_w, cpad_w, cdil_w;   // conv: the width-direction values (cstride/cpad/cdil are the height ones)
     int32_t split, kt_per_slice;         // split-K: number of K slices and k-tiles per slice
     const void* bsum;                    // uint8 path: per batch entry N column sums of B (sum_k B[n,k], int32), or null
-    int32_t out_plane;                   // CHW kernels: row m, column n of the result goes to C[m / out_plane][n][m % out_plane]
-    int32_t expand_shift;                // EXPAND kernels: the H x W input is not in memory: pixel (y, x) of the in_h x in_w
-    int32_t in_h, in_w, top, left;       // one that is stands at (top + (y << shift), left + (x << shift)), zeros elsewhere
     // split-K: the result and what tells the last slice of a tile to add them all up; arrivals null: a kernel behind this one does
     void* out;
     int64_t out_stride;                  // batch stride of the result, elements
     uint64_t* arrivals;                  // one word per output tile, of any content
     uint64_t ticket;                     // of this launch, its low 16 bits zero
     int32_t out_ld;
-    // divisors of the launch: K slices, output tiles of a batch entry, of a raster group, rows of a group and of the last one, conv: elements of
-    // a filter row and of a tap, output pixels of an image and of a row, 16-byte pieces of a pixel, pixels of a plane (out_plane)
-    HrnDiv by_split, by_tiles, by_group, by_gm, by_gm_last, by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
-    // conv, im2col (hrn_walk_args): the bytes of a pixel; the width of all taps; whether taps are carried along K (CI, or 0); what a byte offset changes by, beyond the step itself, where K goes on to the next
-    // tap and filter row; the step from one row of A that a lane loads to the next in output pixels, input pixels and bytes, and what
-    // changes where it leaves a row or an image of the result.  Modulo 2^32, as the kernel adds them: pads, strides and dilations
-    // may be of any size, and only what lies inside an image is used.
+    // divisors of the launch: K slices, output tiles of a batch entry, of a raster group, rows of a group and of the last one
+    HrnDiv by_split, by_tiles, by_group, by_gm, by_gm_last;
+};
+
+// What a conv's launch adds; a product's does without
+struct HrnConvArgs : HrnKArgs {
+    int32_t H, W, CI, HO, WO, KH, KW, cstride, cpad, cdil;
+    int32_t cstride_w, cpad_w, cdil_w;   // the width-direction values (cstride/cpad/cdil are the height ones)
+    int32_t out_plane;                   // CHW kernels: row m, column n of the result goes to C[m / out_plane][n][m % out_plane]
+    int32_t expand_shift;                // EXPAND kernels: the H x W input is not in memory: pixel (y, x) of the in_h x in_w
+    int32_t in_h, in_w, top, left;       // one that is stands at (top + (y << shift), left + (x << shift)), zeros elsewhere
+    // divisors of the launch: elements of a filter row and of a tap, output pixels of an image and of a row, 16-byte pieces of a pixel, pixels
+    // of a plane (out_plane)
+    HrnDiv by_kwci, by_ci, by_hw, by_wo, by_cpp, by_plane;
+    // im2col (hrn_walk_args): the bytes of a pixel; the width of all taps; whether taps are carried along K (CI, or 0); what a byte offset
+    // changes by, beyond the step itself, where K goes on to the next tap and filter row; the step from one row of A that a lane
+    // loads to the next in output pixels, input pixels and bytes, and what changes where it leaves a row or an image of the result.  Modulo
+    // 2^32, as the kernel adds them: pads, strides and dilations may be of any size, and only what lies inside an image is used.
     uint32_t px, kw_end, tap_bytes, taprow_bytes;
     int32_t carry_ci;
     uint32_t d_ox, d_oy, x_step, y_step, off_step, x_row, row_bytes, y_img, img_bytes;
@@ -71,7 +77,7 @@ HRN_BOTH int hrn_pair_of(int block, int pairs) {
 
 // What the walks below need of a launch whose conv fields are set; `rows`: output pixels from one load of a lane to its next.
 // expanded: the input in memory is the in_h x in_w one.
-inline void hrn_walk_args(HrnKArgs* k, int es, int rows, bool expanded) {
+inline void hrn_walk_args(HrnConvArgs* k, int es, int rows, bool expanded) {
     const uint32_t px = (uint32_t)k->CI * es, H = k->H, W = k->W, sh = k->cstride, sw = k->cstride_w, hw = (uint32_t)k->HO * k->WO;
     const uint32_t images = rows / hw, rest = rows % hw;
     k->px = px;
@@ -101,7 +107,7 @@ struct HrnRow {
 };
 
 template <bool EXPAND>
-HRN_BOTH HrnRow hrn_row_at(const HrnKArgs& a, int m) {
+HRN_BOTH HrnRow hrn_row_at(const HrnConvArgs& a, int m) {
     HrnRow r;
     const uint32_t img = a.by_hw((uint32_t)m), rem = (uint32_t)m - img * ((uint32_t)a.HO * a.WO);
     r.oy = a.by_wo(rem);
@@ -113,7 +119,7 @@ HRN_BOTH HrnRow hrn_row_at(const HrnKArgs& a, int m) {
 }
 
 template <bool EXPAND>
-HRN_BOTH void hrn_next_row(const HrnKArgs& a, HrnRow& r) {
+HRN_BOTH void hrn_next_row(const HrnConvArgs& a, HrnRow& r) {
     r.ox += a.d_ox;
     r.oy += a.d_oy;
     r.x = (int)((uint32_t)r.x + a.x_step);
@@ -138,7 +144,7 @@ struct HrnTap {
     uint32_t off;
 };
 
-HRN_BOTH HrnTap hrn_tap_at(const HrnKArgs& a, int ke, int in_w, int es) {
+HRN_BOTH HrnTap hrn_tap_at(const HrnConvArgs& a, int ke, int in_w, int es) {
     HrnTap t;
     const int r = (int)a.by_kwci((uint32_t)ke);
     ke -= r * (a.KW * a.CI);
@@ -153,7 +159,7 @@ HRN_BOTH HrnTap hrn_tap_at(const HrnKArgs& a, int ke, int in_w, int es) {
 // ELEMS further along K, to element ke.  Carried where a step goes one tap further at most and a filter row's end shows in dx; a count of the
 // taps instead costs 2 - 12 % (fp16 3x3 32x7x7x512 -> 512 27.7 us, 31.0 with the count).
 template <int ELEMS, int ES>
-HRN_BOTH void hrn_next_tap(const HrnKArgs& a, HrnTap& t, int ke, int in_w) {
+HRN_BOTH void hrn_next_tap(const HrnConvArgs& a, HrnTap& t, int ke, int in_w) {
     if (a.carry_ci >= ELEMS) {
         t.c += ELEMS;
         const bool tap = t.c >= a.CI;

@@ -270,9 +270,10 @@ __device__ __forceinline__ void sched_hint() {
 // How the arguments are handed in decides what the compiler does with the scalar registers.  Persistent instances take them by
 // value (fp16 192 x 512x512x64: 4 spills and 24 idle instructions instead of 7 and 41, 21.3 us instead of 21.55), the others by
 // reference (u8 x s8 8192^3: 418 us instead of 425; the rest of the cases within their spread either way).
-using BodyArgs = typename std::conditional<PERS, const HrnKArgs, const HrnKArgs&>::type;
-template <bool CHW, bool EXPAND, bool DEEP>
-__device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
+using KArgs = typename std::conditional<OP == 1, HrnConvArgs, HrnKArgs>::type;
+using BodyArgs = typename std::conditional<PERS, const KArgs, const KArgs&>::type;
+template <bool CHW, bool EXPAND, bool DEEP, class Args>       // (Args: BodyArgs, a parameter so that a product need not have a conv's)
+__device__ __forceinline__ void hrn_mfma_body(Args a) {
     constexpr int NS = DEEP ? DEEP_NS : HRN_STAGES;
     constexpr int OWN_LDS = CHW ? CHW_LDS_BYTES : LDS_BYTES;
     constexpr int KERNEL_LDS = (DEEP && NS * STAGE_BYTES > OWN_LDS) ? NS * STAGE_BYTES : OWN_LDS;
@@ -348,14 +349,18 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     int m0 = c_tile_m * BM, n0 = c_tile_n * BN;
 
     // conv: the input that is in memory, and the way from a position of the expanded one to it
-    const int in_h = EXPAND ? a.in_h : a.H, in_w = EXPAND ? a.in_w : a.W;
+    [[maybe_unused]] int in_h = 0, in_w = 0;
+    if constexpr (OP == 1) { in_h = EXPAND ? a.in_h : a.H; in_w = EXPAND ? a.in_w : a.W; }
     [[maybe_unused]] auto unexpand = [&](int& y, int& x) {
-        y -= a.top;
-        x -= a.left;
-        const bool hit = ((y | x) & ((1 << a.expand_shift) - 1)) == 0;
-        y >>= a.expand_shift;                                  // (a negative position stays negative)
-        x >>= a.expand_shift;
-        return hit && (unsigned)y < (unsigned)in_h && (unsigned)x < (unsigned)in_w;
+        if constexpr (!EXPAND) return true;
+        else {
+            y -= a.top;
+            x -= a.left;
+            const bool hit = ((y | x) & ((1 << a.expand_shift) - 1)) == 0;
+            y >>= a.expand_shift;                                  // (a negative position stays negative)
+            x >>= a.expand_shift;
+            return hit && (unsigned)y < (unsigned)in_h && (unsigned)x < (unsigned)in_w;
+        }
     };
 
     // ---- issue side: the tile whose k-tiles are being fetched (the same tile unless the launch is persistent) ----
@@ -553,7 +558,8 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
     const int lr = lane % MT, lq = lane / MT;
 
     // ---- conv window mode: the window itself (dynamic LDS) and the per-row tap masks ----
-    const int w_pitch = a.CI * ES;                       // bytes of one pixel (all channels)
+    int w_pitch = 0;                                     // bytes of one pixel (all channels)
+    if constexpr (CW) w_pitch = a.CI * ES;
     const int w_cch = CW ? w_pitch / BKB : 1;            // k-tiles per tap
     uint32_t tapmask[CW ? TM : 1];                       // bit t: tap t of this lane's pixel i is inside the image
     if constexpr (CW) {
@@ -1396,7 +1402,7 @@ __device__ __forceinline__ void hrn_mfma_body(BodyArgs a) {
 // kernel is scheduled 0.6 % slower, NCW conv1d 16 x 892 x 512 -> 512 30.56 -> 30.73 us)
 template <bool ROOM, bool CHW, bool EXPAND, bool DEEP>
 __device__ __forceinline__ void body_if(BodyArgs a) {
-    if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND, DEEP>(a);
+    if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND, DEEP, BodyArgs>(a);
 }
 
 // Where 256 registers are enough for a wave, the compiler is told so: it then keeps the accumulators in them and the MFMAs add in place.  Given 512,
@@ -1422,12 +1428,12 @@ constexpr int MIN_WPE = NT > 256 ? (NT + 255) / 256 : (TM * TN * ACC_N + 8 * (TM
 #endif
 
 #if HRN_PART == 0
-HRN_ENTRY hrn_mfma_kernel(const HrnKArgs a) { hrn_mfma_body<false, false, false>(a); }
-HRN_ENTRY hrn_mfma_kernel_deep(const HrnKArgs a) { body_if<HAS_DEEP, false, false, true>(a); }
+HRN_ENTRY hrn_mfma_kernel(const KArgs a) { hrn_mfma_body<false, false, false, BodyArgs>(a); }
+HRN_ENTRY hrn_mfma_kernel_deep(const KArgs a) { body_if<HAS_DEEP, false, false, true>(a); }
 #elif HRN_PART == 1
-HRN_ENTRY hrn_mfma_kernel_chw(const HrnKArgs a) { body_if<HAS_CHW, true, false, false>(a); }
-HRN_ENTRY hrn_mfma_kernel_chw_deep(const HrnKArgs a) { body_if<HAS_DEEP, true, false, true>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw(const KArgs a) { body_if<HAS_CHW, true, false, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_deep(const KArgs a) { body_if<HAS_DEEP, true, false, true>(a); }
 #else
-HRN_ENTRY hrn_mfma_kernel_chw_expand(const HrnKArgs a) { body_if<HAS_CHW, true, true, false>(a); }
-HRN_ENTRY hrn_mfma_kernel_chw_expand_deep(const HrnKArgs a) { body_if<HAS_DEEP, true, true, true>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand(const KArgs a) { body_if<HAS_CHW, true, true, false>(a); }
+HRN_ENTRY hrn_mfma_kernel_chw_expand_deep(const KArgs a) { body_if<HAS_DEEP, true, true, true>(a); }
 #endif

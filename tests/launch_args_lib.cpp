@@ -11,7 +11,7 @@ using i64 = long long;
 // im2col loads of an instance (`row_bytes` of K in a tile row, `rows` of a tile a load of every wave, `loads` a lane) over a conv: how many
 // (row, K position) pairs find another address, or another answer to whether it is in the image, than the definition gives.
 template <int ELEMS, int ES, bool EXPAND>
-i64 walk_errors(HrnKArgs a, int images, int rows, int loads, const int* starts, int n_starts) {
+i64 walk_errors(HrnConvArgs a, int images, int rows, int loads, const int* starts, int n_starts) {
     const int hw = a.HO * a.WO, M = images * hw, K = a.KH * a.KW * a.CI, kts = (K + ELEMS - 1) / ELEMS, tile = rows * loads;
     const int in_w = EXPAND ? a.in_w : a.W, in_h = EXPAND ? a.in_h : a.H;
     a.by_kwci = HrnDiv((uint32_t)(a.KW * a.CI)); a.by_ci = HrnDiv((uint32_t)a.CI);
@@ -66,7 +66,7 @@ void div_all(const uint32_t* ns, uint32_t* out, int count, uint32_t d) {
 
 // conv: images, H, W, CI, HO, WO, KH, KW, then (stride, pad, dilation) of the height and of the width, then in_h, in_w (0: not expanded)
 long long conv_walk_errors(const int* conv, int es, int row_bytes, int rows, int loads, const int* starts, int n_starts) {
-    HrnKArgs a = {};
+    HrnConvArgs a = {};
     a.H = conv[1]; a.W = conv[2]; a.CI = conv[3]; a.HO = conv[4]; a.WO = conv[5]; a.KH = conv[6]; a.KW = conv[7];
     a.cstride = conv[8]; a.cpad = conv[9]; a.cdil = conv[10];
     a.cstride_w = conv[11]; a.cpad_w = conv[12]; a.cdil_w = conv[13];
@@ -86,6 +86,8 @@ long long conv_walk_errors(const int* conv, int es, int row_bytes, int rows, int
     }
     return -1;
 }
+
+int args_bytes(int conv) { return conv ? (int)sizeof(HrnConvArgs) : (int)sizeof(HrnKArgs); }
 
 int pair_of(int block, int pairs) { return hrn_pair_of(block, pairs); }
 }
