@@ -1130,11 +1130,6 @@ __device__ __forceinline__ void hrn_mfma_body(Args a) {
             }
         };
         if constexpr (LROWS == 0 && NLD > 0) loads(std::integral_constant<int, 0>{}, std::integral_constant<int, NLD>{});
-        // All reads of the next step go out in front of the first MFMAs (at most two rows): the fragments of this one are waited for
-        // before, in a form that the compiler counts.  Left to itself it waits behind them, and for all of them.
-        // fp16 3x3 in 4 slices 2x20x20x432 -> 240 12.2 -> 11.6 us, 4x14x14x256 -> 256 9.7 -> 9.4, in 2, stride 2, 8x28x28x512 -> 256 18.6 -> 17.7,
-        // batch_matmul 192x512x512x64 (persistent) 23.8 -> 22.7.
-        if constexpr (!LAST && RROWS == 1) __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0)
         v4i av = a_operand(cur, 0);
         auto row = [&](auto ic) {
             constexpr int i = decltype(ic)::value;
