@@ -14,7 +14,7 @@
 // 32 bits, n*m / 2^(31+L) exceeds n / d by less than 1 / d (Granlund and Montgomery, Division by Invariant Integers).
 // Kernels divide by what is fixed for a launch.  A division proper is some 30 instructions, and a kernel starts with four
 // (GEMM) to eight of them, each waiting for the one before, in front of its first load: 194 instructions to it instead of 127 (u8 64x128
-// tiles), 435 instead of 283 (fp16 im2col 128x128).
+// tiles), 435 instead of 283 (fp16 im2col 128x128) when the multipliers came.
 struct HrnDiv {
     uint32_t m, shift;
     HrnDiv() = default;

@@ -61,9 +61,10 @@ constexpr bool CW = (HRN_CONVWIN != 0);
 #define HRN_PERSIST 0
 #endif
 constexpr bool PERS = (HRN_PERSIST != 0);
-// Split-K: the grid holds `split` copies of the tile grid; copy z multiplies k-tiles [z*kt_per_slice, (z+1)*kt_per_slice)
-// and stores its raw fp32 / int32 partial sums to slice z of a workspace; the slice that finishes a tile last adds them up (fold_slices),
-// or, where the workspace has no room for the arrivals, a second kernel (splitk_reduce_kernel) does.
+// Split-K: the grid holds `split` workgroups for every tile, side by side; number z of them multiplies k-tiles
+// [z*kt_per_slice, (z+1)*kt_per_slice) and stores its raw fp32 / int32 partial sums in slice z of a workspace, tile by tile; the one that
+// finishes a tile last adds them up (fold_slices).  Where the workspace has no room for the arrivals, slices are row-major and a second
+// kernel (splitk_reduce_kernel) adds them up.
 #ifndef HRN_SPLITK
 #define HRN_SPLITK 0
 #endif
@@ -77,7 +78,8 @@ constexpr bool SPLITK = (HRN_SPLITK != 0);
 constexpr bool COLSUM = (HRN_DTYPE == 1) && (HRN_COLSUM != 0);
 // the results leave with the non-temporal hint: C is written once and not read by this kernel, and a round's 8 MiB of it
 // per XCD would otherwise push the operand slabs of the next round out of the 4 MiB L2 (split-K partial sums go out at device scope
-// instead, whoever adds them up: the other XCDs' slices are read from memory).  Staged results whose rows end inside lines go without it (row_lines)
+// instead, whoever adds them up: the other XCDs' slices are read from memory).  Staged results go without it where row_lines says so; those
+// straight from the accumulators, which no strip gathers, keep it whatever their rows
 #ifndef HRN_NTSTORE
 #define HRN_NTSTORE 0
 #endif
@@ -766,8 +768,8 @@ __device__ __forceinline__ void hrn_mfma_body(Args a) {
 
         char* Cb = (char*)a.C + ((int64_t)slice * batch + c_bz) * a.sC * OES;
         using NtC = std::integral_constant<bool, NTS>;
-        // The non-temporal hint only where no line is written in pieces: rows of whole lines, or of whole half lines as long as the
-        // memory-side cache has room for the result.  Elsewhere the L2 joins the pieces that tiles side by side and the strips of a tile
+        // Staged results: the non-temporal hint for rows of whole lines, and for rows of whole half lines up to 64 MiB of result, a limit between
+        // the 57 MB and the 107 MB below.  Elsewhere the L2 joins the pieces that tiles side by side and the strips of a tile
         // leave of a line.  Hint / no hint, us: rows at 16 or 32 bytes u8 x s8 4653x3384x208 34.0 / 24.5, 8190x4040x128 47.9 / 27.3, fp16
         // 8190x8184x128 59.0 / 37.3, batch_matmul 192x512x520x64 55.2 / 25.4; half lines fp16 8190x8160x128 (134 MB) 58.5 / 43.0, batch_matmul
         // 192x512x544x64 (107 MB) 29.5 / 27.4, 4330x6624x1120 (57 MB) 63.4 / 63.3, 3000x2336x512 15.1 / 15.7, 100x300x352x64 10.8 / 12.7, u8 conv
@@ -776,7 +778,7 @@ __device__ __forceinline__ void hrn_mfma_body(Args a) {
         [[maybe_unused]] const bool row_lines =
             (row_ends & 127) == 0 || ((row_ends & 63) == 0 && (uint64_t)batch * (uint32_t)a.M * (uint32_t)a.ldc <= (64u << 20) / OES);
         [[maybe_unused]] const rsrc_t rsrcC = make_rsrc(Cb, (uint32_t)a.M * (uint32_t)a.ldc * OES);
-        // (the hint only where rows of C are whole lines: see row_lines)
+        // (ntc: with the hint.  Staged results ask row_lines, the others take NtC)
         [[maybe_unused]] auto put16 = [&](auto ntc, char* dst, v4i val) __attribute__((always_inline)) {
             if constexpr (decltype(ntc)::value) __builtin_nontemporal_store(val, (out16_t*)dst);
             else *(out16_t*)dst = val;
@@ -1400,12 +1402,17 @@ __device__ __forceinline__ void body_if(BodyArgs a) {
     if constexpr (ROOM) hrn_mfma_body<CHW, EXPAND, DEEP, BodyArgs>(a);
 }
 
-// Where 256 registers are enough for a wave, the compiler is told so: it then keeps the accumulators in them and the MFMAs add in place.  Given 512,
-// it takes the other half for the accumulators and copies them from one half to the other in the k-loop (20 - 28 instructions and the
-// waits between them a k-tile of four MFMA tiles).  u8 conv 5x5 16x21x24x176 -> 288 33.0 -> 28.9 us, 3x3 4x30x30x448 -> 320 24.3 -> 20.3, fp16 3x3
-// in 4 slices 2x20x20x432 -> 240 13.2 -> 12.3.  Deep kernels fill the LDS with one workgroup,
-// which would be reason enough for 512 registers, so those of products take their LDS dynamically: u8 x s8 1500x1536x4112 25.9 -> 23.1 us, fp16
-// 1500x1536x2048 18.2 -> 17.9.  (Those of convs gain nothing by it: 5x5 10x30x30x208 -> 128 35.4 -> 36.6, 3x3 16x28x28x256 -> 160 23.9 -> 23.5.)
+// Where 256 registers are enough for a wave, the compiler is told so.  Kernels of 16x16 MFMAs that are given 512 can get accumulators in the
+// other half, copied through the lower one in the k-loop (60 and 100 moves in two u8 instances; those of 32x32 MFMAs that were looked
+// at have none).  Given 512 / told, us: fp16 3x3 in 4 slices 2x20x20x432 -> 240 11.2 / 10.4, 3x3 32x7x7x512 -> 512 28.8 / 26.8, u8 3x3
+// 15x34x33x384 -> 144 21.9 / 21.6.  Deep kernels fill the LDS with one workgroup, which would be reason enough for 512 registers, so those of
+// products take their LDS dynamically: u8 x s8 1500x1536x4112 26.2 / 22.9, fp16 1500x1536x2048 17.25 / 17.2.  (Those of convs gain nothing by
+// it: 5x5 10x30x30x208 -> 128 35.4 -> 36.6, 3x3 16x28x28x256 -> 160 23.9 -> 23.5.)
+// The rule counts registers, not the waves that the LDS lets in.  Two instances whose LDS admits more end two registers above a wave's share and
+// run with one wave less: u8 window conv 64x128x64, 4x1 waves, 4 stages (130), as fast with it (asked for four waves it spills 8 bytes:
+// 28x28x128 -> 128 at batch 32 15.93 / 15.92, at 128 39.6 / 39.6), and u8 GEMM 128x128x64, 4x1 waves, 3 stages (170; asked for three, 16
+// bytes spilled: 2048x2048x1024 14.5 / 14.1, 4096x4096x256 22.9 / 23.5, 3000x2504x720 17.5 / 17.7).  Others keep 512 registers as their
+// static LDS admits one wave.
 constexpr int MIN_WPE = NT > 256 ? (NT + 255) / 256 : (TM * TN * ACC_N + 8 * (TM + TN) <= 208 ? 2 : 1);      // (accumulators, two sets of fragments)
 
 }  // namespace

@@ -82,9 +82,10 @@ typedef struct hrn_kernel_desc {
                              fetching the next tile's operands while the current result is stored (needs epilogue 1 and
                              N*out_bytes a multiple of 16) */
     int32_t split_k;      /* 1 = K is cut into hrn_problem.split_k slices that run as separate workgroups; the kernel
-                             stores raw fp32 / int32 partial sums per slice into hrn_problem.workspace and a second
-                             pass of the library adds them into C (for small M*N with long K: more workgroups than
-                             output tiles).  Not with persistent or conv_window. */
+                             stores raw fp32 / int32 partial sums per slice into hrn_problem.workspace, and the slice that
+                             finishes an output tile last adds them into C, or, where the workspace has no room for a word
+                             per tile, a second launch does (for small M*N with long K: more workgroups than output
+                             tiles).  Not with persistent or conv_window. */
     int32_t sched;        /* issue order of a k-step: 1 = the template's own interleaving of fragment reads, tile loads
                              and MFMAs is pinned with scheduling fences, 0 = left to the compiler under group hints,
                              2 = another name of 1 (the same code object).  256x256 tiles of 128-byte rows in two stages

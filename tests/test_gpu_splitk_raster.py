@@ -39,3 +39,21 @@ def test_products(which, m, n, hrn):
             for b in range(batch):
                 assert torch.equal(C[b].float(), A[b].float() @ W[b].float().t())
     mod.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", [4, 5])
+@pytest.mark.parametrize("n,h,w,co", [(1, 5, 5, 64), (3, 6, 5, 192), (8, 8, 8, 64), (2, 9, 7, 128)])     # 1, 6, 8 and 4 tiles
+def test_convs(which, n, h, w, co, hrn):
+    d = instances.splitk_descs()[which]
+    f16 = d.dtype == instances.F16
+    mod = B.Module(d)
+    gen = torch.Generator(device="cuda").manual_seed(n * h + co)
+    X = torch.randint(-1 if f16 else 0, 2, (n, h, w, 80), device="cuda", generator=gen)
+    W = torch.randint(-1, 2, (co, 3, 3, 80), device="cuda", generator=gen)
+    want = torch.nn.functional.conv2d(X.cpu().float().permute(0, 3, 1, 2), W.cpu().float().permute(0, 3, 1, 2), padding=1).permute(0, 2, 3, 1)
+    for split in (1, 2, 3, 5):      # sums of at most 720 products of -1, 0, 1: exact in fp16
+        print("split-K raster", d.as_tuple(), (n, h, w, 80, co), split, flush=True)
+        Y = hostops.conv2d_nhwc(mod, X.to(torch.float16 if f16 else torch.uint8), W.to(torch.float16 if f16 else torch.int8), 1, 1, 1, split_k=split)
+        assert torch.equal(Y.cpu().float(), want), split
+    mod.close()
