@@ -773,7 +773,8 @@ __device__ __forceinline__ void hrn_mfma_body(Args a) {
         // leave of a line.  Hint / no hint, us: rows at 16 or 32 bytes u8 x s8 4653x3384x208 34.0 / 24.5, 8190x4040x128 47.9 / 27.3, fp16
         // 8190x8184x128 59.0 / 37.3, batch_matmul 192x512x520x64 55.2 / 25.4; half lines fp16 8190x8160x128 (134 MB) 58.5 / 43.0, batch_matmul
         // 192x512x544x64 (107 MB) 29.5 / 27.4, 4330x6624x1120 (57 MB) 63.4 / 63.3, 3000x2336x512 15.1 / 15.7, 100x300x352x64 10.8 / 12.7, u8 conv
-        // 1x1 16x56x56x64 -> 112 7.4 / 8.3.
+        // 1x1 16x56x56x64 -> 112 7.4 / 8.3.  Long products hide the pieces: fp16 4330x6616x2048 102.8 / 98.9, x4096 186.1 / 188.7, x8192 364.5 / 363.3,
+        // 2308x6904x5560 240.8 / 244.0, u8 4653x3384x4096 100.3 / 90.8.
         [[maybe_unused]] const uint32_t row_ends = (uint32_t)a.ldc * OES | (uint32_t)(uintptr_t)Cb;
         [[maybe_unused]] const bool row_lines =
             (row_ends & 127) == 0 || ((row_ends & 63) == 0 && (uint64_t)batch * (uint32_t)a.M * (uint32_t)a.ldc <= (64u << 20) / OES);
@@ -1132,6 +1133,11 @@ __device__ __forceinline__ void hrn_mfma_body(Args a) {
             }
         };
         if constexpr (LROWS == 0 && NLD > 0) loads(std::integral_constant<int, 0>{}, std::integral_constant<int, NLD>{});
+        // uint8 products whose reads of the next step all go out in front of the first MFMAs (at most two rows): the fragments of this one, which go
+        // through the vector ALU first, are waited for before, in a form that the compiler counts.  Without / with, us: 250x2500x8192 23.1 / 22.6,
+        // 291x2704x4352 14.2 / 14.0, 150x3000x4096 12.9 / 12.7.  fp16 loses: 250x2500x8192 32.2 / 32.8, conv 3x3 32x56x56x64 -> 64 13.4 / 13.6; u8
+        // convs are equal.
+        if constexpr (DT == 1 && OP == 0 && !LAST && RROWS == 1) __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0)
         v4i av = a_operand(cur, 0);
         auto row = [&](auto ic) {
             constexpr int i = decltype(ic)::value;
