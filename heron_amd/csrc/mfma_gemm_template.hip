@@ -481,21 +481,32 @@ __device__ __forceinline__ void hrn_mfma_body(Args a) {
         ks_cur = live ? koff_cur : 0u;
         return live && koff_cur + BKB > Kb;                                      // ragged: the last tile is not full
     };
-    // conv: the byte offsets of the next k-tile's loads of A.  Made in front of the barrier that lets the loads go: left to itself the compiler
-    // makes all but the first between the loads (fp16 3x3 9x46x49x240 -> 64 18.5 us, 18.2 like this, stride 2 16x28x28x96 -> 144 8.1 and 8.0, u8 3x3
-    // 4x30x30x448 -> 320 19.7 and 19.3).
+    // conv: the byte offset of load i of the next k-tile of A
+    [[maybe_unused]] auto conv_address = [&](int i) __attribute__((always_inline)) {
+        if constexpr (OP == 1) {
+            int iy = iy0[i] + tap.dy, ix = ix0[i] + tap.dx;
+            if constexpr (EXPAND) {
+                return unexpand(iy, ix) ? voffA[i] + (uint32_t)((iy * in_w + ix) * a.CI + tap.c) * ES : OOB;
+            } else {
+                const bool ok = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+                return ok ? voffA[i] + tap.off : OOB;
+            }
+        } else {
+            return 0u;
+        }
+    };
+    // They are made in front of the barrier that lets the loads go; left to itself the compiler makes all but the first between the loads.
+    // Between / in front, us: fp16 3x3 in 2 slices 16x7x7x512 -> 512 15.8 / 14.9, 9x46x49x240 -> 64 18.1 / 17.9, u8 3x3 4x30x30x448 -> 320 19.7 / 18.6,
+    // 5x5 16x21x24x176 -> 288 26.9 / 26.5.  Not with one MFMA tile a wave and one wave a SIMD, whose barrier then comes later: fp16 64x64 tiles, 3x3
+    // 32x7x7x512 -> 512 25.5 / 26.3, 5x5 12x19x18x96 -> 80 15.3 / 16.0, stride 2, 2x54x54x352 -> 368 46.2 / 48.2 (u8 in slices 4x14x14x512 -> 256 11.1 /
+    // 11.0).  Of 128x128 tiles on four waves one call was better off between its loads, stride 2 17x35x38x288 -> 272 25.7 / 27.0.
+    constexpr bool ADDR_FIRST = OP == 1 && !CW && !(DT == 0 && TM * TN == 1 && NW <= 4);
     [[maybe_unused]] uint32_t addr[(A_LPW > 0 ? A_LPW : 1)];
     auto conv_addresses = [&]() __attribute__((always_inline)) {
-        if constexpr (OP == 1 && !CW) {
+        if constexpr (ADDR_FIRST) {
 #pragma unroll
             for (int i = 0; i < A_LPW; ++i) {
-                int iy = iy0[i] + tap.dy, ix = ix0[i] + tap.dx;
-                if constexpr (EXPAND) {
-                    addr[i] = unexpand(iy, ix) ? voffA[i] + (uint32_t)((iy * in_w + ix) * a.CI + tap.c) * ES : OOB;
-                } else {
-                    const bool ok = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-                    addr[i] = ok ? voffA[i] + tap.off : OOB;
-                }
+                addr[i] = conv_address(i);
                 asm volatile("" : "+v"(addr[i]));
             }
         }
@@ -520,7 +531,7 @@ __device__ __forceinline__ void hrn_mfma_body(Args a) {
                     if constexpr (RAG) { if (koff_rag + chunk_of(i) >= Kb) v = OOB; }
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, ks_cur);
                 } else if constexpr (!CW) {
-                    uint32_t v = addr[i];
+                    uint32_t v = ADDR_FIRST ? addr[i] : conv_address(i);
                     if constexpr (RAG) { if (koff_rag + lane_chunk >= Kb) v = OOB; }      // (past the last tap)
                     load_chunk_to_lds(rA_cur, sbase + (i * NW + wave) * 1024, v, 0u);
                 }
